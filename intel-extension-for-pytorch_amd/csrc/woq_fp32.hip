@@ -9,9 +9,7 @@
 //
 // y[M, N] = x[M, K] * w[N, K]^T on v_mfma_f32_32x32x2_f32: workgroup tile 128 x 128, K step 32,
 // 4 waves in a 2 x 2 grid, each owning 64 x 64 as 2 x 2 MFMA tiles (A = activations, B = weights:
-// a lane's accumulator registers hold consecutive rows of its own output column); up to 64 rows
-// (SMALL) the tile is 32 x 128 and a wave owns one 32 x 32 MFMA tile, a quarter of the MFMA work
-// per K step.  Weights are dequantized once per workgroup and K step into LDS.  One MFMA consumes the K pair (2t, 2t + 1),
+// a lane's accumulator registers hold consecutive rows of its own output column).  Weights are dequantized once per workgroup and K step into LDS.  One MFMA consumes the K pair (2t, 2t + 1),
 // lanes 0..31 the even element and lanes 32..63 the odd one; both LDS tiles keep the even elements
 // of a row in floats 0..15 and the odd ones in floats 16..31, so that a lane reads the operands of
 // four MFMAs with one 16-byte load.
@@ -25,22 +23,22 @@ constexpr int F_BM = 128, F_BN = 128, F_BK = 32;
 constexpr int F_STRIDE = F_BK + 4;  // floats; keeps 16-byte alignment, spreads rows over the banks
 }  // namespace
 
-template <int WBITS, bool NF4, bool SMALL>
+template <int WBITS, bool NF4>
 __global__ __launch_bounds__(256) void woq_fp32_kernel(const Fp32Args f) {
   static_assert(!NF4 || WBITS == 4, "NF4 codes are 4 bits wide");
   constexpr int TK = WBITS == 4 ? kTileK4 : kTileK8;
-  constexpr int BM = SMALL ? 32 : F_BM;
+  constexpr int BM = F_BM;
   constexpr int XI = BM / 32;         // 16-byte activation pieces per thread and K step
-  constexpr int TM = SMALL ? 1 : 2;   // MFMA tiles per wave along M and N
-  constexpr int TN = SMALL ? 1 : 2;
+  constexpr int TM = 2;               // MFMA tiles per wave along M and N
+  constexpr int TN = 2;
   __shared__ __align__(16) float sA[BM * F_STRIDE];
   __shared__ __align__(16) float sB[F_BN * F_STRIDE];
   __shared__ float sTab[16];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const int row0 = SMALL ? 0 : (wave >> 1) * 64;             // first row / column of this wave
-  const int col0 = SMALL ? wave * 32 : (wave & 1) * 64;
+  const int row0 = (wave >> 1) * 64;  // first row / column of this wave
+  const int col0 = (wave & 1) * 64;
   const int64_t m0 = (int64_t)blockIdx.y * BM;
   const int64_t n0 = (int64_t)blockIdx.x * F_BN;
   const int64_t nt0 = n0 / kTileN;
@@ -182,21 +180,243 @@ __global__ __launch_bounds__(256) void woq_fp32_kernel(const Fp32Args f) {
     }
 }
 
+// Few rows (decode, short prompts): a workgroup owns NTW row-blocks of 16 output columns for all K, its W waves split
+// K, and every operand goes from memory straight into the registers that feed the MFMA.  A packed weight tile already
+// has the B layout of v_mfma_f32_16x16x4_f32: lane r + 16 c holds consecutive K values of row r, so MFMA number e of a
+// tile takes each lane's value e, and the A operand of lane m + 16 c is x[m] at the same K, read as 16-byte pieces.
+// Up to four rows (RT 0) the MFMA is v_mfma_f32_4x4x1_16b: its block l / 4 has the columns 4 (l / 4 % 4) .. + 3 and
+// the K values of c = l / 16, so the four K quarters of a tile become four sums that are added with the waves'.
+// A 16-row MFMA would spend three quarters of its time on absent rows (9 us of fp32 matrix work at 4096 -> 11008
+// against 2.3 us).
+// Bound: HBM and the launch up to four rows, the fp32 matrix pipes from 16 rows (16 rows, 4096 -> 11008: 9.2 us at 157 TFLOP/s).
+// Against the tiles of 32 / 128 x 128 outputs below, whose workgroups (86 at N = 11008) go through K alone with two barriers
+// every 32 values (us, INT8 per channel): 4096 -> 11008 M = 1 / 4 / 16 / 64 / 128: 16.4 / 17.3 / 25.5 / 64 / 123 against
+// 223 / 224 / 223 / 223 / 521; 4096 -> 28672: 32 / 33 / 51 / 153 / 297 against 225 / 226 / 226 / 254 / 570;
+// 14336 -> 1024: 18 / 29 / 34 / 107 / 108 against 665 / 691 / 700 / 712 / 1777.  128 rows (two workgroups along M) is where
+// the measurements end; beyond it the weights would be dequantized a third time.  Error against 64 bits 2e-7 .. 8e-7 in the
+// 2-norm (one chain over all of K: 1.1e-6 .. 2.2e-6).
+enum { kFmtInt8, kFmtFp8, kFmtInt4, kFmtNf4 };
+
+template <int RT, int NTW>
+struct Fp32Decode {
+  static constexpr int kRows = RT ? RT : 1;  // row tiles of a wave
+  static constexpr int kWaves = (RT <= 1 && NTW == 1) ? 16 : 8;  // narrow layers: more of K in flight per workgroup
+  static constexpr int kMinWaves = RT <= 1 ? 4 : 2;              // per SIMD: 128 or 256 registers
+};
+
+template <int FMT, int RT, int NTW>
+__global__ __launch_bounds__((Fp32Decode<RT, NTW>::kWaves * 64), (Fp32Decode<RT, NTW>::kMinWaves))
+void woq_fp32_decode_kernel(const Fp32Args f) {
+  using S = Fp32Decode<RT, NTW>;
+  constexpr int W = S::kWaves, R = S::kRows;
+  constexpr bool kBytes = FMT == kFmtInt8 || FMT == kFmtFp8;
+  constexpr int TK = kBytes ? kTileK8 : kTileK4;
+  constexpr int CH = TK / 4;        // K values of a lane in a tile, taken 16 at a time
+  constexpr int SUB = CH / 16;
+  constexpr bool kAheadX = RT <= 2;  // activations one step ahead; with three or four row tiles there are no registers for it
+  __shared__ f4 red[W][NTW][64];
+  __shared__ float tab[16];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, c = lane >> 4;
+  const int64_t nt0 = (int64_t)blockIdx.x * NTW;
+  const int64_t m0 = (int64_t)blockIdx.y * (RT ? 16 * RT : 4);
+  const int KT = (int)f.KT;
+  if (FMT == kFmtNf4) {
+    if (tid < 16) tab[tid] = kNf4Values[tid];
+    __syncthreads();
+  }
+
+  // absent rows and row-blocks repeat the last real one; their results are not stored
+  const float* xrow[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int64_t m = m0 + 16 * i + (RT ? r : lane & 3);
+    xrow[i] = f.x + (m < f.M ? m : f.M - 1) * f.K + c * CH;
+  }
+  int64_t nt[NTW];
+#pragma unroll
+  for (int j = 0; j < NTW; ++j) nt[j] = nt0 + j < f.NT ? nt0 + j : f.NT - 1;
+
+  float s0[NTW], z0[NTW], s1[NTW], z1[NTW];
+  u4 q0[NTW], q1[NTW];
+  auto params = [&](int g, float* s, float* z) {
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) {
+      const int64_t qi = (nt[j] * f.KG + g) * kTileN + r;
+      s[j] = f.scales[qi];
+      if (FMT == kFmtInt8 || FMT == kFmtInt4) z[j] = f.zeros ? (float)f.zeros[qi] : (FMT == kFmtInt4 ? 8.0f : 128.0f);
+    }
+  };
+  auto request_w = [&](int kt, u4* q, float* s, float* z) {
+#pragma unroll
+    for (int j = 0; j < NTW; ++j)
+      q[j] = __builtin_nontemporal_load((const u4*)(f.qweight + ((nt[j] * f.KT + kt) * 64 + lane) * 16));
+    if (f.KG > 1) {  // (a lane's K values of a tile lie in one group: groups are multiples of 32)
+      const unsigned g = ((unsigned)kt * TK + c * CH) / (unsigned)f.G;
+      params((int)(g < (unsigned)f.KG ? g : (unsigned)f.KG - 1), s, z);
+    }
+  };
+  const bool xvec = (f.K % 4) == 0;
+  auto request_x = [&](int kt, int sub, f4 (*x)[4]) {
+    const int64_t k = (int64_t)kt * TK + sub * 16;
+    if ((int64_t)(kt + 1) * TK <= f.K && xvec) {
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[i][q] = *(const f4*)(xrow[i] + k + 4 * q);
+    } else {
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[i][q][e] = c * CH + k + 4 * q + e < f.K ? xrow[i][k + 4 * q + e] : 0.0f;
+    }
+  };
+
+  f4 acc[NTW][R];
+#pragma unroll
+  for (int j = 0; j < NTW; ++j)
+#pragma unroll
+    for (int i = 0; i < R; ++i) acc[j][i] = f4{0.f, 0.f, 0.f, 0.f};
+
+  f4 x0[R][4], x1[R][4];
+  if (f.KG <= 1) params(0, s0, z0);
+  if (wave < KT) {
+    request_w(wave, q0, s0, z0);
+    if (kAheadX) request_x(wave, 0, x0);
+  }
+  for (int kt = wave; kt < KT; kt += W) {
+    const bool more = kt + W < KT;
+    if (more) request_w(kt + W, q1, s1, z1);
+#pragma unroll
+    for (int sub = 0; sub < SUB; ++sub) {
+      if (!kAheadX)
+        request_x(kt, sub, x0);
+      else if (sub + 1 < SUB)
+        request_x(kt, sub + 1, x1);
+      else if (more)
+        request_x(kt + W, 0, x1);
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) {
+        float w[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const uint32_t q = kBytes ? (q0[j][e >> 2] >> (8 * (e & 3))) & 0xFFu
+                                    : (q0[j][2 * sub + (e >> 3)] >> (4 * nibble_pos(e & 7))) & 0xFu;
+          if (FMT == kFmtNf4)
+            w[e] = __fmul_rn(tab[q], s0[j]);
+          else if (FMT == kFmtFp8)
+            w[e] = __fmul_rn(fp8_e4m3fn_to_f32(q), s0[j]);
+          else
+            w[e] = __fmul_rn(__fsub_rn((float)q, z0[j]), s0[j]);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+#pragma unroll
+          for (int i = 0; i < R; ++i)
+            acc[j][i] = RT ? __builtin_amdgcn_mfma_f32_16x16x4f32(x0[i][e >> 2][e & 3], w[e], acc[j][i], 0, 0, 0)
+                           : __builtin_amdgcn_mfma_f32_4x4x1f32(x0[i][e >> 2][e & 3], w[e], acc[j][i], 0, 0, 0);
+      }
+      if (kAheadX)
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) x0[i][q] = x1[i][q];
+    }
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) {
+      q0[j] = q1[j];
+      if (f.KG > 1) { s0[j] = s1[j]; z0[j] = z1[j]; }
+    }
+  }
+
+  // ---- the waves' sums, in wave order (RT 0: and inside a wave the four K quarters) ----
+  Epilogue ep{f.bias, f.fusion, f.other0, f.other1, f.out, WOQ_HIP_ACT_FP32, WOQ_HIP_ACT_FP32, f.N};
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (i) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) red[wave][j][lane] = acc[j][i];
+    __syncthreads();
+    const int j = tid >> 6;  // (W >= NTW: one wave per row-block)
+    if (j >= NTW || nt0 + j >= f.NT) continue;
+    if (RT == 0) {
+      const int e = lane & 3, col = lane >> 2;
+      float sum = 0.0f;
+#pragma unroll
+      for (int w = 0; w < W; ++w)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sum += red[w][j][16 * q + col][e];
+      const int64_t m = m0 + e, n = (nt0 + j) * kTileN + col;
+      if (m < f.M && n < f.N) epilogue_store<kRegimeBF16>(ep, m, n, sum);
+    } else {  // D[m][n]: lane holds n = lane % 16, m = 4 (lane / 16) + e
+      f4 sum = red[0][j][lane];
+#pragma unroll
+      for (int w = 1; w < W; ++w) sum += red[w][j][lane];
+      const int64_t n = (nt0 + j) * kTileN + r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t m = m0 + 16 * i + 4 * c + e;
+        if (m < f.M && n < f.N) epilogue_store<kRegimeBF16>(ep, m, n, sum[e]);
+      }
+    }
+  }
+}
+
+template <int FMT, int RT>
+static void launch_fp32_decode_rows(const Fp32Args& f, unsigned gy, hipStream_t st) {
+  // row-blocks per workgroup: the shortest schedule, generations of 256 workgroups times a workgroup's length (its
+  // row-blocks and about half a one for the activations), ties to the larger count
+  int best = 1;
+  double best_cost = 1e300;
+  for (int n = 1; n <= 4; ++n) {
+    const int64_t wg = (f.NT + n - 1) / n * gy;
+    const double cost = (double)((wg + 255) / 256) * (n + 0.5);
+    if (cost <= best_cost) { best = n; best_cost = cost; }
+  }
+  const dim3 grid((unsigned)((f.NT + best - 1) / best), gy);
+#define WOQ_FP32_DECODE(N) woq_fp32_decode_kernel<FMT, RT, N><<<grid, Fp32Decode<RT, N>::kWaves * 64, 0, st>>>(f)
+  switch (best) {
+    case 1: WOQ_FP32_DECODE(1); break;
+    case 2: WOQ_FP32_DECODE(2); break;
+    case 3: WOQ_FP32_DECODE(3); break;
+    default: WOQ_FP32_DECODE(4);
+  }
+#undef WOQ_FP32_DECODE
+}
+
+template <int FMT>
+static void launch_fp32_decode(const Fp32Args& f, hipStream_t st) {
+  if (f.M <= 4) return launch_fp32_decode_rows<FMT, 0>(f, 1, st);
+  const int64_t tiles = (f.M + 15) / 16, gy = (tiles + 3) / 4;
+  switch ((tiles + gy - 1) / gy) {
+    case 1: return launch_fp32_decode_rows<FMT, 1>(f, (unsigned)gy, st);
+    case 2: return launch_fp32_decode_rows<FMT, 2>(f, (unsigned)gy, st);
+    case 3: return launch_fp32_decode_rows<FMT, 3>(f, (unsigned)gy, st);
+    default: return launch_fp32_decode_rows<FMT, 4>(f, (unsigned)gy, st);
+  }
+}
+
 int launch_fp32(const Fp32Args& f, int wbits, hipStream_t st) {
   if (f.G <= 0 || f.G % F_BK != 0) return set_error("woq_linear: fp32 compute needs groups that are multiples of 32");
-  const bool small = f.M <= 64;
-  const int bm = small ? 32 : F_BM;
-  dim3 grid((unsigned)((f.NT * kTileN + F_BN - 1) / F_BN), (unsigned)((f.M + bm - 1) / bm));
-#define WOQ_FP32(WB, NF)                                          \
-  (small ? woq_fp32_kernel<WB, NF, true><<<grid, 256, 0, st>>>(f) \
-         : woq_fp32_kernel<WB, NF, false><<<grid, 256, 0, st>>>(f))
+  // up to 128 rows the kernel for few rows (figures there); its group index is 32 bits wide
+  if (f.M <= 128 && f.KT * kTileK4 < (1ll << 31)) {
+    if (wbits == 8)
+      f.fp8 ? launch_fp32_decode<kFmtFp8>(f, st) : launch_fp32_decode<kFmtInt8>(f, st);
+    else
+      f.nf4 ? launch_fp32_decode<kFmtNf4>(f, st) : launch_fp32_decode<kFmtInt4>(f, st);
+    return check_launch("woq_fp32_decode_kernel");
+  }
+  const dim3 grid((unsigned)((f.NT * kTileN + F_BN - 1) / F_BN), (unsigned)((f.M + F_BM - 1) / F_BM));
   if (wbits == 8)
-    WOQ_FP32(8, false);
+    woq_fp32_kernel<8, false><<<grid, 256, 0, st>>>(f);
   else if (f.nf4)
-    WOQ_FP32(4, true);
+    woq_fp32_kernel<4, true><<<grid, 256, 0, st>>>(f);
   else
-    WOQ_FP32(4, false);
-#undef WOQ_FP32
+    woq_fp32_kernel<4, false><<<grid, 256, 0, st>>>(f);
   return check_launch("woq_fp32_kernel");
 }
 

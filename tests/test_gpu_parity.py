@@ -2174,6 +2174,39 @@ def test_fp32_compute(cuda, kind, M, K, N, G, bias):
         assert torch.equal(ctx8.run(x.cuda()), y)
 
 
+@pytest.mark.parametrize(
+    "kind,M,K,N,G",
+    [
+        # four-row matrix instructions, one to three row-blocks per workgroup (narrow: sixteen waves), ragged widths
+        ("int8", 1, 4096, 512, -1), ("int8", 2, 1000, 4100, -1), ("int8", 4, 2048, 8720, 64), ("nf4", 4, 1024, 4112, 64), ("fp8", 3, 1024, 528, 128),
+        # one, two, three and four row tiles, the first and last row of each; more waves than K tiles
+        ("int8", 5, 4096, 528, -1), ("int8", 16, 192, 80, -1), ("int4", 17, 1408, 96, 32), ("int8", 32, 1001, 272, -1), ("int4", 33, 512, 4112, 128),
+        ("int8", 48, 640, 8224, -1), ("nf4", 49, 512, 272, 64), ("fp8", 64, 1024, 4112, 128), ("int8", 64, 512, 12304, -1),
+        # two workgroups along the rows, and the tiled kernel from 129 rows on
+        ("int8", 65, 640, 528, -1), ("int8", 97, 512, 4112, 64), ("int4", 128, 512, 272, 32), ("int8", 129, 512, 272, -1),
+    ],
+)
+def test_fp32_few_rows(cuda, kind, M, K, N, G):
+    """The kernel for few rows against the products in 64 bits; fp32 sums of K terms in any order lie within
+    K * 2^-24 of the terms' absolute sum, and well inside 1e-5 in the 2-norm at these widths."""
+    syn = _synthetic()
+    if kind == "int8":
+        case = syn.make_int8_case(430, M, K, N, bias=True, group_size=G)
+    elif kind == "fp8":
+        case = syn.make_fp8_case(430, M, K, N, bias=True, group_size=G, x_dtype=torch.float32)
+    elif kind == "nf4":
+        case = syn.make_nf4_case(430, M, K, N, G, bias=True, scale_dtype=torch.float32)
+    else:
+        case = syn.make_int4_case(430, M, K, N, G, bias=True, scale_dtype=torch.float32)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(431))
+    y = make_context(case, O.LOWP_NONE).run(x.cuda()).cpu().numpy()
+    assert _lib_last_kernel() == ("woq_fp32_decode_kernel" if M <= 128 else "woq_fp32_kernel")
+    c = case_np(case)
+    acc, _ = O.woq_linear_ref(x.numpy(), "fp32", c["qw"], N, K, c["scales"], c["zps"], c["bias"], case["weight_dtype"], G, "fp32")
+    assert rel_l2(y, acc) <= 1e-5
+    assert max_abs(y, acc) <= 2e-4 * max(1.0, float(np.abs(acc).max()))
+
+
 def test_fp32_compute_post_ops(cuda):
     from ipex_amd import _lib
     import torch.nn.functional as F
