@@ -395,6 +395,8 @@ int woq_hip_moe_scale_add_rows(void* out, int dtype, int64_t T, int64_t H, const
  *   woq_hip_moe_scale_add_rows call per expert, experts ascending, leaves.
  */
 #define WOQ_HIP_MOE_ROUTE_MAX 2048
+#define WOQ_HIP_MOE_TILES_MAX 8192
+#define WOQ_HIP_MOE_TILES_EXPERTS 1024
 typedef struct woq_hip_moe_group {
   const int32_t* slot_expert;      /* [slots] expert of the slot or -1 */
   const int32_t* slot_row0;        /* [slots] */
@@ -409,6 +411,19 @@ int woq_hip_moe_route(const int64_t* topk_ids, int64_t T, int64_t topk, int64_t 
                       int64_t split_mid, int use_single, int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of,
                       int32_t* slot_of, void* stream);
 int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, int64_t slots);
+/*
+ * The same layer for prompts: woq_hip_moe_route_tiles sorts at most WOQ_HIP_MOE_TILES_MAX entries over at most
+ * WOQ_HIP_MOE_TILES_EXPERTS experts and cuts the routed rows into slots, int32 [4][3][S], S >= experts + T * topk /
+ * tile_rows: class 0 the experts with fewer than split_lo rows, 1 at most split_mid, 2 at most 64, one slot each; class 3
+ * the others, in slots of at most tile_rows (64 or 128) rows; split_lo and split_mid at most 64.  x_row, row_of and slot_of as from woq_hip_moe_route.
+ * woq_hip_linear_grouped_tiles runs one linear over the slots of class 3 on the prefill kernel: p as for
+ * woq_hip_linear_grouped (M is ignored), INT4 weights with power-of-two groups of at least 32 or INT8 weights with
+ * power-of-two groups of at least 128, or per-channel; K a multiple of 128, rows in the compute type of five and more rows.
+ */
+int woq_hip_moe_route_tiles(const int64_t* topk_ids, int64_t T, int64_t topk, int64_t experts, int64_t split_lo,
+                            int64_t split_mid, int64_t tile_rows, int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of,
+                            int32_t* slot_of, void* stream);
+int woq_hip_linear_grouped_tiles(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows);
 int woq_hip_moe_combine_rows(void* out, int dtype, int64_t T, int64_t H, const void* expert_out,
                              const void* routing_weights, int64_t topk, const int32_t* row_of, const int32_t* slot_of,
                              int accumulate, void* stream);

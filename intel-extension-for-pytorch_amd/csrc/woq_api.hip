@@ -393,16 +393,17 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
                      : launch_gemm(f, wbits, regime, st);
 }
 
-int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, int64_t slots) {
+// The problem of one expert of a grouped launch: arguments checked, FpArgs and compute type filled in (rows: the bound on a
+// slot's rows that selects the compute type).
+static int grouped_problem(const woq_hip_linear_params* p, const void* group, int64_t rows, FpArgs& f, int& wbits, int& regime) {
   if (!p || !group) return set_error("woq_linear_grouped: null params or group table");
   if (p->struct_size != sizeof(woq_hip_linear_params))
     return set_error("woq_linear_grouped: struct_size %u does not match this library (%zu)", p->struct_size,
                      sizeof(woq_hip_linear_params));
   if (p->weight_dtype != WOQ_HIP_DTYPE_INT4 && p->weight_dtype != WOQ_HIP_DTYPE_INT8)
     return set_error("woq_linear_grouped: INT4 and INT8 weights, got dtype %d", p->weight_dtype);
-  if (p->M < 1 || p->M > 64 || p->K <= 0 || p->N <= 0)
-    return set_error("woq_linear_grouped: 1..64 rows per slot, got M=%lld K=%lld N=%lld", (long long)p->M, (long long)p->K,
-                     (long long)p->N);
+  if (p->K <= 0 || p->N <= 0)
+    return set_error("woq_linear_grouped: bad shape K=%lld N=%lld", (long long)p->K, (long long)p->N);
   if (p->x_dtype != WOQ_HIP_ACT_BF16 && p->x_dtype != WOQ_HIP_ACT_FP16)
     return set_error("woq_linear_grouped: bf16 or fp16 rows, got x_dtype %d", p->x_dtype);
   if (p->out_dtype != p->x_dtype) return set_error("woq_linear_grouped: out_dtype must equal x_dtype");
@@ -414,26 +415,33 @@ int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, in
   if (p->fusion != WOQ_HIP_FUSE_NONE && p->fusion != WOQ_HIP_FUSE_SILU && p->fusion != WOQ_HIP_FUSE_MUL)
     return set_error("woq_linear_grouped: post-op none, silu or mul, got 0x%x", p->fusion);
   if (p->fusion == WOQ_HIP_FUSE_MUL && !p->others[0]) return set_error("woq_linear_grouped: mul needs others[0]");
-  const int wbits = p->weight_dtype == WOQ_HIP_DTYPE_INT8 ? 8 : 4;
+  wbits = p->weight_dtype == WOQ_HIP_DTYPE_INT8 ? 8 : 4;
   const int tk = wbits == 4 ? kTileK4 : kTileK8;
   const int64_t NT = woq_hip_padded_n(p->N) / kTileN;
   const int64_t KT = woq_hip_padded_k(p->weight_dtype, p->K) / tk;
   const int64_t G = p->group_size > 0 ? p->group_size : KT * tk;
   const int64_t KG = p->group_size > 0 ? (p->K + G - 1) / G : 1;
-  // the regimes of woq_hip_linear (csrc/cpu/aten/kernels/WoqLinearKrnl.cpp:75-112), with M the bound on a slot's rows
-  int regime;
+  // the regimes of woq_hip_linear (csrc/cpu/aten/kernels/WoqLinearKrnl.cpp:75-112), with the bound on a slot's rows
   if (p->lowp_mode == WOQ_HIP_LOWP_FP16 || (p->lowp_mode == WOQ_HIP_LOWP_NONE && p->x_dtype == WOQ_HIP_ACT_FP16) ||
-      (p->lowp_mode == WOQ_HIP_LOWP_BF16 && p->M < small_batch_threshold()))
+      (p->lowp_mode == WOQ_HIP_LOWP_BF16 && rows < small_batch_threshold()))
     regime = kRegimeF16;
   else
     regime = kRegimeBF16;
-  FpArgs f;
-  f.x = p->x; f.x_dtype = p->x_dtype; f.M = p->M; f.K = p->K; f.N = p->N; f.NT = NT; f.KT = KT;
+  f.x = p->x; f.x_dtype = p->x_dtype; f.M = rows; f.K = p->K; f.N = p->N; f.NT = NT; f.KT = KT;
   f.qweight = nullptr; f.scales = nullptr; f.zeros = nullptr;  // per expert, from the group table
   f.szb = nullptr;
   f.G = G; f.KG = KG; f.bias = nullptr; f.fusion = p->fusion;
   f.other0 = p->others[0]; f.other1 = nullptr; f.out = p->out; f.out_dtype = p->out_dtype;
   f.nf4 = 0; f.fp8 = 0;
+  return 0;
+}
+
+int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, int64_t slots) {
+  FpArgs f;
+  int wbits, regime;
+  if (p && p->struct_size == sizeof(woq_hip_linear_params) && (p->M < 1 || p->M > 64))
+    return set_error("woq_linear_grouped: 1..64 rows per slot, got M=%lld", (long long)p->M);
+  if (int rc = grouped_problem(p, group, p ? p->M : 0, f, wbits, regime)) return rc;
   if (p->scale_zero_f16x2) {
     // up to four routed rows per slot on the integer-weight decode kernels: the group's scales table holds the
     // experts' (fp16 scale, fp16 128 + zero) dword tables
@@ -445,6 +453,18 @@ int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, in
     return launch_decode_grouped(f, (const MoeGroup*)group, slots, (hipStream_t)p->stream);
   }
   return launch_decode_dq_grouped(f, wbits, regime, (const MoeGroup*)group, slots, (hipStream_t)p->stream);
+}
+
+int woq_hip_linear_grouped_tiles(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows) {
+  FpArgs f;
+  int wbits, regime;
+  if (tile_rows != 64 && tile_rows != 128) return set_error("woq_linear_grouped_tiles: 64 or 128 rows per slot, got %d", tile_rows);
+  if (slots < 1 || slots > 65535) return set_error("woq_linear_grouped_tiles: bad slot count %lld", (long long)slots);
+  if (int rc = grouped_problem(p, group, tile_rows, f, wbits, regime)) return rc;
+  if (!gemm_w4_applies(f, wbits, regime))
+    return set_error("woq_linear_grouped_tiles: K a multiple of 128, power-of-two groups (INT4: 32 and more, INT8: 128 and "
+                     "more) or per-channel, 16-byte aligned rows in the compute type");
+  return launch_gemm_w4_grouped(f, wbits, regime, (const MoeGroup*)group, slots, tile_rows, (hipStream_t)p->stream);
 }
 
 int woq_hip_dequant_weight(const void* qweight, int weight_dtype, int64_t N, int64_t K, const float* scales_f32,
@@ -518,6 +538,17 @@ int woq_hip_moe_route(const int64_t* topk_ids, int64_t T, int64_t topk, int64_t 
   if (T > 0 && (!topk_ids || !x_row || !slots || !row_of || !slot_of)) return set_error("moe_route: null pointer");
   return launch_moe_route(topk_ids, T, topk, experts, split_lo, split_mid, use_single, S, x_row, slots, row_of, slot_of,
                           (hipStream_t)stream);
+}
+
+int woq_hip_moe_route_tiles(const int64_t* topk_ids, int64_t T, int64_t topk, int64_t experts, int64_t split_lo,
+                            int64_t split_mid, int64_t tile_rows, int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of,
+                            int32_t* slot_of, void* stream) {
+  if (T < 0 || topk <= 0 || experts <= 0) return set_error("moe_route_tiles: bad size");
+  if (split_lo < 0 || split_lo > 64 || split_mid < 0 || split_mid > 64 || (tile_rows != 64 && tile_rows != 128))
+    return set_error("moe_route_tiles: split_lo and split_mid are 0..64, tile_rows 64 or 128");
+  if (T > 0 && (!topk_ids || !x_row || !slots || !row_of || !slot_of)) return set_error("moe_route_tiles: null pointer");
+  return launch_moe_route_tiles(topk_ids, T, topk, experts, split_lo, split_mid, tile_rows, S, x_row, slots, row_of, slot_of,
+                                (hipStream_t)stream);
 }
 
 int woq_hip_moe_combine_rows(void* out, int dtype, int64_t T, int64_t H, const void* expert_out,

@@ -107,9 +107,14 @@ __device__ __forceinline__ u4 g4_dequant_m(uint32_t d, const G4Masks& k, uint32_
   return r;
 }
 
-template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false>
-__global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs f, const int g_shift, float* const sk_partial,
-                                                          int* const sk_counters, const int kts) {
+// GROUPED (mixture of experts): the row tile of a workgroup is a slot of the routing tables -- at most G4_BM routed rows of
+// one expert, whose tensors come from the group's pointer tables; a slot without an expert ends at once.
+// 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3832 us with three launches per expert (each on 32 to 192 workgroups),
+// 794 us with one launch per linear.
+template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false>
+__global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const int g_shift, float* const sk_partial,
+                                                          int* const sk_counters, const int kts, const MoeGroup* const grp) {
+  static_assert(!GROUPED || !MERGED, "the pointer tables hold scales and zero points apart");
   constexpr int TPS = WBITS / 4;  // packed tiles per row-block and K step of 128
   constexpr int G4_MT = S::MT, G4_NTW = S::NTW, G4_BM = S::BM, G4_XBYTES = S::XBYTES, G4_XLOADS = S::XLOADS,
                 G4_WSTAGE = S::WSTAGE * TPS, G4_SSTRIDE = S::SSTRIDE;
@@ -117,6 +122,31 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs f, const 
   extern __shared__ __align__(1024) uint8_t sX[];
   uint8_t* const sW = sX + 2 * G4_XBYTES;
 
+  int bx, by;  // this workgroup's tile, by XCD (xcd_tile)
+  xcd_tile(bx, by);
+  FpArgs fg;                        // GROUPED: this slot's problem
+  const int64_t* xrow = nullptr;    // GROUPED: routed row of the slot -> row of x, or null: x has the routed rows
+  if constexpr (GROUPED) {
+    const MoeGroup& g = *grp;
+    const int e = __builtin_amdgcn_readfirstlane(g.slot_expert[by]);
+    if (e < 0) return;
+    const int64_t row0 = __builtin_amdgcn_readfirstlane(g.slot_row0[by]);
+    const int rows = __builtin_amdgcn_readfirstlane(g.slot_rows[by]);
+    fg = fa;
+    fg.M = rows < G4_BM ? rows : G4_BM;
+    fg.qweight = dq_uniform((const uint8_t*)g.qweight[e]);
+    fg.scales = dq_uniform((const uint16_t*)g.scales[e]);
+    fg.zeros = g.zeros ? dq_uniform(g.zeros[e]) : nullptr;
+    fg.bias = g.bias ? dq_uniform(g.bias[e]) : nullptr;
+    fg.out = (uint8_t*)fa.out + row0 * fa.N * 2;  // (16-bit rows)
+    if (fa.other0) fg.other0 = (const uint8_t*)fa.other0 + row0 * fa.N * 2;
+    if (g.x_row)
+      xrow = g.x_row + row0;
+    else
+      fg.x = (const uint8_t*)fa.x + row0 * fa.K * 2;
+    by = 0;
+  }
+  const FpArgs& f = GROUPED ? fg : fa;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -127,8 +157,6 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs f, const 
   // that of its number whatever the split
   const int kt_lo = (int)blockIdx.z * kts;
   const int KT = KTW / TPS < kt_lo + kts ? KTW / TPS : kt_lo + kts;
-  int bx, by;  // this workgroup's tile, by XCD (xcd_tile)
-  xcd_tile(bx, by);
   const int m0 = by * G4_BM;
   const int nt0 = (bx * G4_WAVES + wave) * G4_NTW;  // first row-block of this wave
 
@@ -152,7 +180,10 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs f, const 
 #pragma unroll
   for (int i = 0; i < G4_XLOADS; ++i) {
     const int rowl = (wave * G4_XLOADS + i) * 4 + c;
-    const int rowc = m0 + rowl < M ? rowl : M - 1 - m0;
+    int rowc = m0 + rowl < M ? rowl : M - 1 - m0;
+    if constexpr (GROUPED) {
+      if (xrow) rowc = (int)xrow[rowc];  // (the host bounds rows of x * K * 2 below 2^31)
+    }
     // (4-bit weights: the chunk 4 c + j of lane column c and sub-step j is kept at slot 4 j + c, so that the four
     // lane columns of a row read slots that differ in their low bits: chunks 8 apart share their banks)
     const int slot = r ^ (rowl & 15);
@@ -559,13 +590,45 @@ static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits
       if (lds_optin_m != hipSuccess)
         return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin_m));
       woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, true><<<grid, 256, kLds, st>>>(
-          f, g_shift, splits > 1 ? scratch->partial : nullptr, splits > 1 ? scratch->counters : nullptr, kts);
+          f, g_shift, splits > 1 ? scratch->partial : nullptr, splits > 1 ? scratch->counters : nullptr, kts, nullptr);
       return check_launch("woq_gemm_w4_kernel");
     }
   }
   woq_gemm_w4_kernel<REGIME, S, WBITS, FP8><<<grid, 256, kLds, st>>>(f, g_shift, splits > 1 ? scratch->partial : nullptr,
-                                                                 splits > 1 ? scratch->counters : nullptr, kts);
+                                                                 splits > 1 ? scratch->counters : nullptr, kts, nullptr);
   return check_launch("woq_gemm_w4_kernel");
+}
+
+// Row tiles of the routed rows of all experts in one launch (woq_hip_linear_grouped_tiles).
+template <int REGIME, class S, int WBITS>
+static int launch_grouped_shape(const FpArgs& f, int g_shift, const MoeGroup* grp, int64_t slots, hipStream_t st) {
+  constexpr int kLds = g4_lds_bytes<S, WBITS>();
+  static const hipError_t lds_optin =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, false, false, true>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+  if (lds_optin != hipSuccess)
+    return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin));
+  const dim3 grid((unsigned)((f.NT * kTileN + S::BN - 1) / S::BN), (unsigned)slots);
+  woq_gemm_w4_kernel<REGIME, S, WBITS, false, false, true>
+      <<<grid, 256, kLds, st>>>(f, g_shift, nullptr, nullptr, (int)(f.KT / (WBITS / 4)), grp);
+  return check_launch("woq_gemm_w4_kernel (grouped)");
+}
+
+int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGroup* grp, int64_t slots, int tile_rows,
+                           hipStream_t st) {
+  int g_shift = 30;
+  if (f.G < f.KT * (wbits == 4 ? kTileK4 : kTileK8)) {
+    g_shift = 0;
+    while (((int64_t)1 << g_shift) < f.G) ++g_shift;
+  }
+  using S2 = G4Shape<8, 2>;
+  using S42 = G4Shape<4, 2>;
+#define WOQ_GROUPED(RG, WB)                                                         \
+  (tile_rows == 64 ? launch_grouped_shape<RG, S42, WB>(f, g_shift, grp, slots, st) \
+                   : launch_grouped_shape<RG, S2, WB>(f, g_shift, grp, slots, st))
+  if (wbits == 4) return regime == kRegimeF16 ? WOQ_GROUPED(kRegimeF16, 4) : WOQ_GROUPED(kRegimeBF16, 4);
+  return regime == kRegimeF16 ? WOQ_GROUPED(kRegimeF16, 8) : WOQ_GROUPED(kRegimeBF16, 8);
+#undef WOQ_GROUPED
 }
 
 // Relative time of a shape: generations of 256 workgroups times the length of one K step, which

@@ -82,6 +82,8 @@ int launch_moe_scale_add_rows(void* out, int dtype, int64_t T, int64_t H, const 
 int launch_moe_route(const int64_t* ids, int64_t T, int64_t topk, int64_t experts, int64_t split_lo, int64_t split_mid,
                      int use_single, int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of, int32_t* slot_of,
                      hipStream_t st);
+int launch_moe_route_tiles(const int64_t* ids, int64_t T, int64_t topk, int64_t experts, int64_t split_lo, int64_t split_mid, int64_t tile_rows,
+                           int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of, int32_t* slot_of, hipStream_t st);
 int launch_moe_combine_rows(void* out, int dtype, int64_t T, int64_t H, const void* cur, const void* rw, int64_t topk,
                             const int32_t* row_of, const int32_t* slot_of, int accumulate, hipStream_t st);
 int launch_dequant_weight(const void* qweight, int weight_dtype, int64_t N, int64_t K, const float* s32,
@@ -155,6 +157,9 @@ bool gemm_w4s_applies(const FpArgs& f, int wbits, int regime);
 int launch_gemm_w4s(const FpArgs& f, int regime, hipStream_t st);
 int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int shape = 0, int splits = 0,
                    const SplitKScratch* scratch = nullptr);
+// The same kernel over the slots of a routed layer (at most tile_rows = 64 or 128 routed rows of one expert each)
+int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGroup* grp, int64_t slots, int tile_rows,
+                           hipStream_t st);
 // Dense bf16 GEMM on the fragment-laid copy that launch_dense_weight writes (woq_gemm_dense.hip): bf16 activations,
 // K % 128 == 0; wbits selects the assignment of K values to lanes that the copy was written with;
 // shape: row-blocks per wave (7, 4 or 2), 0 = by cost model

@@ -183,6 +183,87 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const int64_t* __restric
   for (int i = valid + threadIdx.x; i < R; i += blockDim.x) x_row[i] = 0;
 }
 
+// The same routing for batches beyond the pairwise kernel: a counting sort by one workgroup.  Per entry one LDS atomic counts
+// its expert; a wave then walks the entries expert by expert and numbers them with ballots (stable), which costs
+// entries / 64 x experts / 16 steps a wave instead of entries x entries / 256 comparisons a thread.
+//   slots   [4 classes][expert, first row, rows][S]: 0: experts with fewer than split_lo rows, 1: at most split_mid, 2: at most
+//           64, one slot each; 3: the others in slots of at most tile_rows rows, an expert's slots one after the other;
+//           unused entries expert -1.
+//   x_row, row_of, slot_of as above.
+constexpr int kMoeTilesMax = WOQ_HIP_MOE_TILES_MAX;
+constexpr int kMoeTilesExperts = WOQ_HIP_MOE_TILES_EXPERTS;
+__global__ __launch_bounds__(1024) void moe_route_tiles_kernel(const int64_t* __restrict__ ids, int R, int topk, int experts,
+                                                               int split_lo, int split_mid, int tile_rows, int S,
+                                                               int64_t* __restrict__ x_row,
+                                                               int32_t* __restrict__ slots, int32_t* __restrict__ row_of,
+                                                               int32_t* __restrict__ slot_of) {
+  __shared__ int16_t se[kMoeTilesMax];
+  __shared__ int16_t pos[kMoeTilesMax];
+  __shared__ int cnt[kMoeTilesExperts], off[kMoeTilesExperts];
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int e = tid; e < experts; e += 1024) cnt[e] = 0;
+  __syncthreads();
+  for (int i = tid; i < R; i += 1024) {
+    const int64_t e = ids[i];
+    const bool ok = e >= 0 && e < experts;
+    se[i] = ok ? (int16_t)e : (int16_t)-1;
+    if (ok) atomicAdd(&cnt[(int)e], 1);
+  }
+  __syncthreads();
+  if (tid < experts) {  // (experts <= 1024: one thread each)
+    int before = 0, used[4] = {0, 0, 0, 0};
+    auto cls_of = [&](int n) { return n < split_lo ? 0 : n <= split_mid ? 1 : n <= kMoeSlotRowsMax ? 2 : 3; };
+    auto slots_of = [&](int n) { return n == 0 ? 0 : n <= kMoeSlotRowsMax ? 1 : (n + tile_rows - 1) / tile_rows; };
+    for (int k = 0; k <= tid; ++k) {
+      const int n = cnt[k], cls = cls_of(n), add = slots_of(n);
+      if (k == tid) {
+        off[tid] = before;
+        int idx = cls == 0 ? used[0] : cls == 1 ? used[1] : cls == 2 ? used[2] : used[3];
+        int32_t* const tab = slots + cls * 3 * S;
+        const int step = cls == 3 ? tile_rows : kMoeSlotRowsMax;
+        for (int row = 0; row < n; row += step, ++idx) {
+          if (idx >= S) break;  // (the host gives S entries for every case)
+          tab[idx] = tid;
+          tab[S + idx] = before + row;
+          tab[2 * S + idx] = n - row < step ? n - row : step;
+        }
+      }
+      before += n;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) used[u] += u == cls ? add : 0;
+    }
+    if (tid == experts - 1) {  // the unused ends of the tables
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        for (int i = used[u]; i < S; ++i) slots[u * 3 * S + i] = -1;
+    }
+  }
+  __syncthreads();
+  for (int e = wave; e < experts; e += 16) {
+    int next = off[e];
+    for (int i0 = 0; i0 < R; i0 += 64) {
+      const int i = i0 + lane;
+      const bool mine = i < R && se[i] == e;
+      const uint64_t b = __ballot(mine);
+      if (mine) pos[i] = (int16_t)(next + __popcll(b & ((1ull << lane) - 1)));
+      next += __popcll(b);
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < R; i += 1024) {
+    const int e = se[i], t = i / topk, j = i - t * topk;
+    const int order = e < 0 ? 32767 : e;  // (an id outside [0, experts) comes last and is no row)
+    int ord = 0;
+    for (int jj = 0; jj < topk; ++jj) {
+      const int ek = se[t * topk + jj] < 0 ? 32767 : se[t * topk + jj];
+      ord += ek < order || (ek == order && jj < j) ? 1 : 0;
+    }
+    if (e >= 0) x_row[pos[i]] = t;
+    row_of[t * topk + ord] = e >= 0 ? (int)pos[i] : -1;
+    slot_of[t * topk + ord] = j;
+  }
+}
+
 // out[t, :] accumulates token t's contributions in the order row_of gives (ascending expert), each step rounded to the
 // output dtype -- what one moe_scale_add_rows launch per expert leaves in memory between the experts.
 template <int DTYPE>
@@ -266,6 +347,19 @@ int launch_moe_route(const int64_t* ids, int64_t T, int64_t topk, int64_t expert
   moe_route_kernel<<<1, 256, 0, st>>>(ids, (int)R, (int)topk, (int)experts, (int)split_lo, (int)split_mid, use_single, (int)S,
                                        x_row, slots, row_of, slot_of);
   return check_launch("moe_route");
+}
+
+int launch_moe_route_tiles(const int64_t* ids, int64_t T, int64_t topk, int64_t experts, int64_t split_lo, int64_t split_mid, int64_t tile_rows,
+                           int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of, int32_t* slot_of, hipStream_t st) {
+  const int64_t R = T * topk;
+  if (R == 0) return 0;
+  if (R > kMoeTilesMax || experts > kMoeTilesExperts)
+    return set_error("moe_route_tiles: at most %d (token, slot) entries and %d experts, got %lld and %lld", kMoeTilesMax,
+                     kMoeTilesExperts, (long long)R, (long long)experts);
+  if (S < experts + R / tile_rows) return set_error("moe_route_tiles: the slot tables are too short");
+  moe_route_tiles_kernel<<<1, 1024, 0, st>>>(ids, (int)R, (int)topk, (int)experts, (int)split_lo, (int)split_mid, (int)tile_rows, (int)S,
+                                             x_row, slots, row_of, slot_of);
+  return check_launch("moe_route_tiles");
 }
 
 int launch_moe_combine_rows(void* out, int dtype, int64_t T, int64_t H, const void* cur, const void* rw, int64_t topk,

@@ -14,6 +14,8 @@ LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libwoq_hip.so")
 DTYPE_INT8, DTYPE_INT4, DTYPE_NF4, DTYPE_FP8 = 1, 2, 3, 4
 DTYPES_8BIT = (DTYPE_INT8, DTYPE_FP8)
 MOE_ROUTE_MAX = 2048  # WOQ_HIP_MOE_ROUTE_MAX
+MOE_TILES_MAX = 8192  # WOQ_HIP_MOE_TILES_MAX
+MOE_TILES_EXPERTS = 1024  # WOQ_HIP_MOE_TILES_EXPERTS
 LOWP_NONE, LOWP_FP16, LOWP_BF16, LOWP_INT8 = 0, 1, 2, 3
 ACT_FP32, ACT_FP16, ACT_BF16 = 0, 1, 2
 FUSE_NONE, FUSE_GELU_ERF, FUSE_GELU_TANH, FUSE_RELU, FUSE_SILU = 0x0, 0x1, 0x2, 0x3, 0x4
@@ -50,6 +52,8 @@ EXPORTS = [
     "woq_hip_moe_scale_add_rows",
     "woq_hip_moe_route",
     "woq_hip_linear_grouped",
+    "woq_hip_moe_route_tiles",
+    "woq_hip_linear_grouped_tiles",
     "woq_hip_moe_combine_rows",
 ]
 
@@ -167,6 +171,10 @@ def load():
         lib.woq_hip_moe_route.argtypes = [vp, i64, i64, i64, i64, i64, i32, i64, vp, vp, vp, vp, vp]
         lib.woq_hip_linear_grouped.restype = i32
         lib.woq_hip_linear_grouped.argtypes = [ctypes.POINTER(LinearParams), vp, i64]
+        lib.woq_hip_moe_route_tiles.restype = i32
+        lib.woq_hip_moe_route_tiles.argtypes = [vp, i64, i64, i64, i64, i64, i64, i64, vp, vp, vp, vp, vp]
+        lib.woq_hip_linear_grouped_tiles.restype = i32
+        lib.woq_hip_linear_grouped_tiles.argtypes = [ctypes.POINTER(LinearParams), vp, i64, i32]
         lib.woq_hip_moe_combine_rows.restype = i32
         lib.woq_hip_moe_combine_rows.argtypes = [vp, i32, i64, i64, vp, vp, i64, vp, vp, i32, vp]
         if lib.woq_hip_abi_version() != 3:

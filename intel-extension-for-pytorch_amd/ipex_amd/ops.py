@@ -748,7 +748,20 @@ class _MoeGroupedPlan:
             for x in self.shapes)
         self.structs = {}
         self.device = device
+        self.tiles = None
+        # the prefill kernel over row tiles of the routed rows: whole K steps of 128, power-of-two or per-channel groups
+        self.tiles_ok = len(gate_ctx) <= _lib.MOE_TILES_EXPERTS and all(
+            x["K"] % 128 == 0 and (x["G"] <= 0 or (x["G"] >= (32 if x["wd"] == _lib.DTYPE_INT4 else 128) and x["G"] & (x["G"] - 1) == 0))
+            for x in self.shapes)
         self.ok = True
+
+    def tile_routing(self):
+        """Routing buffers of woq_hip_moe_route_tiles, made at the first prompt."""
+        if self.tiles is None:
+            R, S = _lib.MOE_TILES_MAX, self.S + _lib.MOE_TILES_MAX // 64
+            i32 = lambda *n: torch.empty(n, dtype=torch.int32, device=self.device)
+            self.tiles = dict(x_row=torch.empty(R, dtype=torch.int64, device=self.device), slots=i32(4, 3, S), row_of=i32(R), slot_of=i32(R), S=S)
+        return self.tiles
 
     def buffers(self, dtype, stream):
         N1, H = self.shapes[0]["N"], self.shapes[0]["K"]
@@ -759,15 +772,17 @@ class _MoeGroupedPlan:
             have = _MOE_ROWS[key] = (mk(N1), mk(N1), mk(H))
         return have
 
-    def group_struct(self, linear, cls, f16_scales, gather, sz=False):
+    def group_struct(self, linear, cls, f16_scales, gather, sz=False, tiles=False):
         """Device copy of the woq_hip_moe_group of one launch (built once).  ``sz``: for the integer-weight decode
-        kernels, with the (scale, zero) dword tables in place of the scales."""
-        key = (linear, cls, f16_scales, gather, sz)
+        kernels, with the (scale, zero) dword tables in place of the scales.  ``tiles``: over the slots of
+        woq_hip_moe_route_tiles."""
+        key = (linear, cls, f16_scales, gather, sz, tiles)
         st = self.structs.get(key)
         if st is None:
             t = self.tables[linear]
             ptr = lambda x: 0 if x is None else x.data_ptr()
-            tab = [ptr(self.slots[cls, i]) for i in range(3)] + [ptr(self.x_row) if gather else 0]
+            slots, x_row = (self.tiles["slots"], self.tiles["x_row"]) if tiles else (self.slots, self.x_row)
+            tab = [ptr(slots[cls, i]) for i in range(3)] + [ptr(x_row) if gather else 0]
             if sz:
                 fields = tab + [ptr(t["qweight"]), ptr(t["sz"]), 0, ptr(t["bias"])]
             else:
@@ -800,10 +815,10 @@ def _f16_regime(lowp, x_dtype, rows):
 
 
 def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, routing_weights):
-    """The layer in five to fourteen launches and without reading the routing on the host: the routing is sorted on the
+    """The layer in five to fourteen launches and, up to 64 tokens, without reading the routing on the host: the routing is sorted on the
     device, every linear runs once per compute type over all experts that have tokens (woq_hip_linear_grouped), and
     the contributions of a token are added in ascending expert order.  Returns None when the layer does not fit
-    (more than 64 tokens, mixed experts, act-order, NF4 / FP8 / lowp INT8 ...): the caller then takes the per-expert path."""
+    (more than 8192 routed rows, mixed experts, act-order, NF4 / FP8 / lowp INT8 ...): the caller then takes the per-expert path."""
     x = hidden_states
     if x.dim() != 2 or x.dtype not in (torch.bfloat16, torch.float16) or not x.is_contiguous() or x.data_ptr() % 16:
         return None
@@ -813,7 +828,8 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     if topk_ids.dim() != 2 or topk_ids.shape[0] != T or not topk_ids.is_cuda or topk_ids.device != x.device:
         return None
     topk = topk_ids.shape[1]
-    if T == 0 or T > 64 or T * topk > _lib.MOE_ROUTE_MAX or T * H * 2 >= 2**31:
+    tiles = T > 64 or T * topk > _lib.MOE_ROUTE_MAX
+    if T == 0 or T * topk > (_lib.MOE_TILES_MAX if tiles else _lib.MOE_ROUTE_MAX) or T * H * 2 >= 2**31:
         return None
     if routing_weights.dtype != x.dtype or routing_weights.dim() != 2 or tuple(routing_weights.shape) != (T, topk) or not routing_weights.is_cuda:
         return None
@@ -821,6 +837,8 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     plan = _moe_plan(gate_ctx, up_ctx, down_ctx, x.device, raw_stream)
     if not plan.ok or plan.shapes[0]["K"] != H:
         return None
+    if tiles:
+        return _deepseek_moe_tiles(plan, x, topk_ids, routing_weights) if plan.tiles_ok else None
     lowp = plan.shapes[0]["lowp"]
     # experts with fewer than five rows on the integer-weight decode kernels, as woq_hip_linear serves them, where
     # such rows compute in fp16 and the layer has the kernels' tables; those with exactly one row (most of them in a
@@ -881,13 +899,82 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     return out
 
 
+def _moe_tile_rows(rows, experts):
+    """Rows of a slot of the prefill kernel: 128 from 192 rows per expert on.  Tiles of 128 rows dequantize half as often, but
+    waste more of an expert's last tile (INT4 g128, us with 64 / 128 rows): 128 rows per expert 794 / 846 and 192 / 234,
+    200 rows 603 / 538, 512 rows 413 / 385."""
+    return 128 if rows >= 192 * experts else 64
+
+
+def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights):
+    """The layer for prompts (more than 64 tokens): the routed rows of all experts in row tiles of the prefill kernel, one
+    launch per linear (woq_hip_linear_grouped_tiles), experts with at most 64 rows on the decode kernels as above (which are
+    the kernels that the per-expert path runs for them).  The routing is read on the host to refuse ids that name no
+    expert, as the per-expert path does, and says which of the size classes are empty."""
+    T, H = x.shape
+    topk, experts, lowp = topk_ids.shape[1], plan.S, plan.shapes[0]["lowp"]
+    f16 = _f16_regime(lowp, x.dtype, 64)
+    if f16 != (x.dtype == torch.float16):  # rows must be in the compute type
+        return None
+    R, N1 = T * topk, plan.shapes[0]["N"]
+    single = plan.single_row and _f16_regime(lowp, x.dtype, 1)
+    split = 5 if (lowp == 2 or single) else 0
+    host_ids = topk_ids.detach().to("cpu", torch.int64)
+    if int(host_ids.min()) < 0 or int(host_ids.max()) >= experts:
+        raise RuntimeError(f"torch_ipex::deepseek_moe_woq: expert ids must lie in [0, {experts})")
+    counts = torch.bincount(host_ids.reshape(-1), minlength=experts).tolist()
+    rows = _moe_tile_rows(R, experts)
+    used = [0, 0, 0, 0]  # slots of each size class
+    for n in counts:
+        if n:
+            used[0 if n < split else 1 if n <= 16 else 2 if n <= 64 else 3] += 1 if n <= 64 else -(-n // rows)
+    lib = _lib.load()
+    ids = topk_ids.to(torch.int64).contiguous()
+    rw = routing_weights.contiguous()
+    buf = plan.tile_routing()
+    code = _kernels._ACT_CODE[x.dtype]
+    with torch.cuda.device(x.device):
+        stream = _kernels._stream()
+        out = torch.empty_like(x)
+        act, inter, y = (torch.empty((R, n), dtype=x.dtype, device=x.device) for n in (N1, N1, H))
+        _lib.check(lib.woq_hip_moe_route_tiles(ids.data_ptr(), T, topk, experts, split, 16, rows, buf["S"], buf["x_row"].data_ptr(),
+                                               buf["slots"].data_ptr(), buf["row_of"].data_ptr(), buf["slot_of"].data_ptr(), stream),
+                   "moe_route_tiles")
+        p = _lib.LinearParams()
+        p.struct_size = ctypes.sizeof(_lib.LinearParams)
+        p.x_dtype = p.out_dtype = code
+        p.stream = torch.cuda.current_stream().cuda_stream
+        p.lowp_mode = lowp
+        p.act_quant_mode = -1
+        for li, src, dst, fusion, other, gather in ((0, x, act, _lib.FUSE_SILU, None, True), (1, x, inter, _lib.FUSE_MUL, act, True),
+                                                    (2, inter, y, _lib.FUSE_NONE, None, False)):
+            sh = plan.shapes[li]
+            p.K, p.N, p.weight_dtype, p.group_size = sh["K"], sh["N"], sh["wd"], sh["G"]
+            p.x, p.out, p.fusion = src.data_ptr(), dst.data_ptr(), fusion
+            p.others[0] = other.data_ptr() if other is not None else None
+            for cls, bound in ((0, 4), (1, 16), (2, 64), (3, rows)):
+                if not used[cls]:
+                    continue
+                p.M = bound
+                sz = cls == 0 and single
+                p.scale_zero_f16x2 = plan.tables[li]["sz"].data_ptr() if sz else None
+                g = plan.group_struct(li, cls, _f16_regime(lowp, x.dtype, bound), gather, sz, tiles=True)
+                if cls == 3:
+                    _lib.check(lib.woq_hip_linear_grouped_tiles(ctypes.byref(p), g.data_ptr(), used[cls], rows), "woq_linear_grouped_tiles")
+                else:
+                    _lib.check(lib.woq_hip_linear_grouped(ctypes.byref(p), g.data_ptr(), used[cls]), "woq_linear_grouped")
+        _lib.check(lib.woq_hip_moe_combine_rows(out.data_ptr(), code, T, H, y.data_ptr(), rw.data_ptr(), topk,
+                                                buf["row_of"].data_ptr(), buf["slot_of"].data_ptr(), 0, stream), "moe_combine_rows")
+    return out
+
+
 def deepseek_moe_woq(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, routing_weights, is_distributed):
     """All experts of a layer (csrc/cpu/aten/MoE.cpp:290-328): ``topk_ids`` [tokens, top-k] names the
     experts of every token, the three lists hold one WoqLinearOpContext per expert.  Experts are
     visited in ascending order and, inside an expert, tokens in ascending order (get_expert_topx_idx,
     MoE.cpp:64-81), which fixes the order of the additions into a token's row.
-    The routing table is read on the host (one synchronizing copy of [tokens, top-k] int64) to size
-    the per-expert launches."""
+    Beyond 64 tokens, and on layers that take no grouped launches, the routing table is read on the host (one
+    synchronizing copy of [tokens, top-k] int64)."""
     _require_gpu_input(hidden_states, "torch_ipex::deepseek_moe_woq")
     _no_all_reduce(is_distributed, "deepseek_moe_woq")
     num_experts = len(gate_ctx)

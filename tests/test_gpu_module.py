@@ -998,6 +998,41 @@ def test_deepseek_moe_grouped_groups_of_128_and_rejections(cuda, monkeypatch):
     assert lib.woq_hip_linear_grouped(ctypes.byref(p), None, 4) != 0
 
 
+@pytest.mark.parametrize("T,E,topk,tile", [(65, 3, 2, 64), (65, 40, 2, 128), (200, 5, 4, 64), (333, 9, 3, 128), (1024, 8, 8, 128)])
+@pytest.mark.parametrize("weight_dtype,G,lowp", [("INT4", 128, "BF16"), ("INT4", 32, "FP16"), ("INT8", -1, "BF16")])
+def test_deepseek_moe_prompts_in_row_tiles(cuda, monkeypatch, T, E, topk, tile, weight_dtype, G, lowp):
+    """More than 64 tokens: an expert without tokens, experts with few rows, one that ends at a tile's edge, a token that names
+    an expert twice; both tile heights.  The per-expert path rounds the same weights and sums in another order: bf16
+    (2^-9) flips of the intermediate rows and the output, each in the 2-norm well below 4e-3."""
+    from ipex_amd import _lib, ops
+
+    ipex = _ipex()
+    H, I = 256, 384
+    mk = lambda k, n, s: _woq_module(ipex, k, n, weight_dtype, G, lowp, bias=True, seed=s)
+    ctxs = [[mk(H, I, 700 + 3 * e)._op_context for e in range(E)], [mk(H, I, 701 + 3 * e)._op_context for e in range(E)],
+            [mk(I, H, 702 + 3 * e)._op_context for e in range(E)]]
+    g = torch.Generator().manual_seed(T)
+    xdt = torch.float16 if lowp == "FP16" else torch.bfloat16
+    hidden = torch.randn(T, H, generator=g).to(xdt).to(cuda)
+    ids = torch.randint(0, E, (T, topk), generator=g)
+    ids[:, 0] = torch.where(torch.arange(T) < 64, torch.zeros(T, dtype=torch.long), torch.ones(T, dtype=torch.long))
+    ids[ids == E - 1] = E - 2  # the last expert has no token
+    ids = ids.to(cuda)
+    rw = torch.softmax(torch.randn(T, topk, generator=g), -1).to(xdt).to(cuda)
+    op = torch.ops.torch_ipex.deepseek_moe_woq
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
+    want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False).double()
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
+    monkeypatch.setattr(ops, "_moe_tile_rows", lambda rows, experts: tile)
+    got = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    assert _lib.last_kernel() == "moe_combine_rows"
+    assert float((got.double() - want).norm() / want.norm()) < 4e-3
+    bad = ids.clone()
+    bad[T - 1, 0] = E
+    with pytest.raises(RuntimeError, match="expert ids must lie in"):
+        op(hidden, bad, ctxs[0], ctxs[1], ctxs[2], rw, False)
+
+
 def test_mixtral_moe_woq_single_expert_and_errors(cuda):
     ipex = _ipex()
     H, I, T = 128, 256, 6
