@@ -329,9 +329,9 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
   if (kernel == 0 && p->dense_bf16 && lowp == WOQ_HIP_LOWP_BF16 && regime == kRegimeBF16 &&
       p->M >= weight_cache_batch_threshold() && p->M > 64 && gemm_dense_applies(f)) {
     // ... where it is the faster kernel: against the prefill kernel that dequantizes in registers (a quarter of the
-    // bytes for the same MFMAs, and shapes of 64 rows) by the two cost models; weights that kernel does not take
-    // (NF4, groups that split a lane's K values) run on the general tiled kernel, which the dense one always beats
-    if (!gemm_w4_applies(f, wbits, regime) || gemm_dense_cost(f) < 0.97 * gemm_w4_cost(f, wbits))
+    // bytes for the same MFMAs, and shapes of 64 rows) by the two cost models, which leave NF4 out: it and weights that
+    // kernel does not take (groups that split a lane's K values) always go to the dense one
+    if (nf4 || !gemm_w4_applies(f, wbits, regime) || gemm_dense_cost(f) < 0.97 * gemm_w4_cost(f, wbits))
       return launch_gemm_dense(f, p->dense_bf16, wbits, st, 0);
   }
   if (nf4) {
@@ -340,6 +340,7 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
     if (kernel == 0) kernel = decode_dq_applies(f, wbits, regime) ? 7 : (p->M <= 64 ? 1 : 2);
     if (kernel != 1 && kernel != 2 && (kernel < 7 || kernel > 9) && kernel != 13 && kernel != 14 && kernel != 16)
       return set_error("woq_linear: NF4 weights run on kernels 1, 2, 7..9, 13, 14 and 16 only");
+    if (p->force_kernel == 0 && kernel != 7 && p->M > 64 && gemm_w4_applies(f, wbits, regime) && gemm_w4_nf4_faster(f)) kernel = 3;
   }
   if (kernel == 0 && decode_kernel_applies(f, wbits, regime, p->scale_zero_f16x2))
     return launch_decode(f, p->scale_zero_f16x2, st);

@@ -111,9 +111,14 @@ __device__ __forceinline__ u4 g4_dequant_m(uint32_t d, const G4Masks& k, uint32_
 // one expert, whose tensors come from the group's pointer tables; a slot without an expert ends at once.
 // 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3832 us with three launches per expert (each on 32 to 192 workgroups),
 // 794 us with one launch per linear.
-template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false>
+// NF4: a dword's eight table values come from the 256-entry table of value pairs in LDS (nf4_dequant), built before the first
+// request; four 8-byte reads, eight products and four conversions against 17 instructions for integers.
+template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false, bool NF4 = false>
 __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const int g_shift, float* const sk_partial,
                                                           int* const sk_counters, const int kts, const MoeGroup* const grp) {
+  static_assert(!NF4 || (WBITS == 4 && !FP8 && !MERGED && !GROUPED), "NF4 codes have a table and a scale");
+  __shared__ f2 sNf4[NF4 ? kNf4LutEntries : 1];
+  if constexpr (NF4) nf4_fill_lut(sNf4, (int)threadIdx.x, 256);  // (the barrier before the first use is the K loop's first)
   static_assert(!GROUPED || !MERGED, "the pointer tables hold scales and zero points apart");
   constexpr int TPS = WBITS / 4;  // packed tiles per row-block and K step of 128
   constexpr int G4_MT = S::MT, G4_NTW = S::NTW, G4_BM = S::BM, G4_XBYTES = S::XBYTES, G4_XLOADS = S::XLOADS,
@@ -268,10 +273,12 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
   G4Consts<REGIME> qc[WBITS == 4 ? G4_NTW : 1];
   G4ConstsM qm[G4_NTW];
   uint32_t mr[G4_NTW];
-  float q8s[WBITS == 8 ? G4_NTW : 1], q8c[WBITS == 8 ? G4_NTW : 1];  // 8-bit: scale, -(128 + z) * scale
+  float q8s[WBITS == 8 || NF4 ? G4_NTW : 1], q8c[WBITS == 8 ? G4_NTW : 1];  // 8-bit: scale, -(128 + z) * scale
   auto set_q = [&](int t, uint16_t sbits, float z) {
     if constexpr (MERGED) {
       qm[t].set(mr[t]);
+    } else if constexpr (NF4) {
+      q8s[t] = REGIME == kRegimeF16 ? f16_bits_to_f32(sbits) : bf16_bits_to_f32(sbits);
     } else if constexpr (WBITS == 4) {
       qc[t].set(sbits, z);
     } else {
@@ -283,6 +290,8 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
   auto deq = [&](int t, int j) -> u4 {
     if constexpr (MERGED) {
       return g4_dequant_m(wr[t][0][j], km, magic64, qm[t]);
+    } else if constexpr (NF4) {
+      return nf4_dequant<REGIME>(wr[t][0][j], sNf4, q8s[t]);
     } else if constexpr (WBITS == 4) {
       return g4_dequant(wr[t][0][j], km, qc[t]);
     } else {
@@ -547,23 +556,34 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
 
 // The kernel needs whole K steps of 128, activations already in the regime's dtype, and a group size
 // whose boundaries never split a lane's 32 consecutive K values (8-bit weights: a K step, so groups of
-// at least 128 or one scale per channel).  NF4 codes are not taken.
+// at least 128 or one scale per channel).  NF4 codes like the 4-bit integers.
 bool gemm_w4_applies(const FpArgs& f, int wbits, int regime) {
   const int want = regime == kRegimeF16 ? WOQ_HIP_ACT_FP16 : WOQ_HIP_ACT_BF16;
-  if ((wbits != 4 && wbits != 8) || f.nf4 || f.x_dtype != want || ((uintptr_t)f.x & 15) != 0) return false;
+  if ((wbits != 4 && wbits != 8) || f.x_dtype != want || ((uintptr_t)f.x & 15) != 0) return false;
   if (f.K % kTileK4 != 0 || f.K * 256 * 2 >= (int64_t)1 << 31) return false;
   if (f.G >= f.KT * (wbits == 4 ? kTileK4 : kTileK8)) return true;  // per-channel: one group
   return f.G >= (wbits == 4 ? 32 : 128) && (f.G & (f.G - 1)) == 0;
 }
 
-template <int REGIME, class S, int WBITS = 4, bool FP8 = false>
+// NF4 weights above 32 rows: this kernel or the general tiled one.  Measured at K = 4096: 64 x 128 tiles 40 us while they fit
+// one generation (the general kernel: 98 us at M = 77, N = 11008); beyond that 83 us per 256 workgroups of 128 x 256 or 512 of
+// 128 x 128, the general kernel 105 us and 0.22 us per 128 x 128 tile: M = 2048, 4096 -> 11008 247 against 283 us, M = 1024,
+// 4096 -> 14336 165 against 230 us, but M = 1000, 4096 -> 11008 (688 tiles, two generations here) 165 against 155 us.
+bool gemm_w4_nf4_faster(const FpArgs& f) {
+  auto wgs = [&](int bm, int bn) { return ((f.NT * kTileN + bn - 1) / bn) * ((f.M + bm - 1) / bm); };
+  if (wgs(64, 128) <= 256) return true;
+  const int64_t w2 = wgs(128, 128), gens = std::min((wgs(128, 256) + 255) / 256, (w2 + 511) / 512);
+  return 83.0 * (double)gens < std::max(105.0, 0.22 * (double)w2);
+}
+
+template <int REGIME, class S, int WBITS = 4, bool FP8 = false, bool NF4 = false>
 static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits = 1,
                         const SplitKScratch* scratch = nullptr) {
   constexpr int kLds = g4_lds_bytes<S, WBITS>();
   static_assert(kLds <= 160 * 1024, "a workgroup's LDS");
   // more than 64 KiB of LDS per workgroup needs an opt-in (once per kernel and process)
   static const hipError_t lds_optin =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, FP8>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   if (lds_optin != hipSuccess)
     return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin));
@@ -582,7 +602,7 @@ static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits
       return set_error("woq_gemm_w4_kernel: split K needs %lld bytes of workspace, the counter array and at most %d "
                        "tiles", (long long)need, kSplitKCounters);
   }
-  if constexpr (REGIME == kRegimeBF16 && WBITS == 4) {
+  if constexpr (REGIME == kRegimeBF16 && WBITS == 4 && !NF4) {
     if (f.szb) {  // scale and zero point of a (row, group) in one dword
       static const hipError_t lds_optin_m =
           hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, true>),
@@ -594,7 +614,7 @@ static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits
       return check_launch("woq_gemm_w4_kernel");
     }
   }
-  woq_gemm_w4_kernel<REGIME, S, WBITS, FP8><<<grid, 256, kLds, st>>>(f, g_shift, splits > 1 ? scratch->partial : nullptr,
+  woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4><<<grid, 256, kLds, st>>>(f, g_shift, splits > 1 ? scratch->partial : nullptr,
                                                                  splits > 1 ? scratch->counters : nullptr, kts, nullptr);
   return check_launch("woq_gemm_w4_kernel");
 }
@@ -703,6 +723,19 @@ int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int s
   using S2 = G4Shape<8, 2>;
   using ST = G4Shape<16, 3>;
   using S42 = G4Shape<4, 2>;
+  if (f.nf4) {
+    // NF4: the 128 x 256, 128 x 128 and 64 x 128 tiles
+    if (shape != 0 || splits > 1) return set_error("woq_gemm_w4_kernel: NF4 weights take the automatic shape only");
+    const int64_t wgs42 = ((f.NT * kTileN + S42::BN - 1) / S42::BN) * ((f.M + S42::BM - 1) / S42::BM);
+#define WOQ_NF4(S, ...)                                                                    \
+  (regime == kRegimeF16 ? launch_shape<kRegimeF16, S, 4, false, true>(f, g_shift, st, ##__VA_ARGS__) \
+                        : launch_shape<kRegimeBF16, S, 4, false, true>(f, g_shift, st, ##__VA_ARGS__))
+    if (wgs42 <= 256) return WOQ_NF4(S42, pick_splits(f, 4, wgs42, scratch), scratch);
+    const int64_t wgs4 = ((f.NT * kTileN + S4::BN - 1) / S4::BN) * ((f.M + S4::BM - 1) / S4::BM);
+    const int64_t wgs2 = ((f.NT * kTileN + S2::BN - 1) / S2::BN) * ((f.M + S2::BM - 1) / S2::BM);
+    return (wgs4 + 255) / 256 < (wgs2 + 511) / 512 ? WOQ_NF4(S4) : WOQ_NF4(S2);  // (two 128 x 128 tiles share a CU)
+#undef WOQ_NF4
+  }
   if (wbits == 8) {
     // 8-bit weights: twice the tile bytes per K step, so at most four row-blocks per wave fit the LDS
     // (128 x 256, 128 x 128 and 64 x 128 workgroup tiles), chosen like the 4-bit ones

@@ -338,7 +338,7 @@ __global__ __launch_bounds__(512) void woq_gemm_w4s_kernel(const FpArgs f, const
 }
 
 // What the register-resident prefill kernel takes, 4-bit integer weights only.
-bool gemm_w4s_applies(const FpArgs& f, int wbits, int regime) { return wbits == 4 && gemm_w4_applies(f, wbits, regime); }
+bool gemm_w4s_applies(const FpArgs& f, int wbits, int regime) { return wbits == 4 && !f.nf4 && gemm_w4_applies(f, wbits, regime); }
 
 template <int REGIME>
 static int launch_w4s(const FpArgs& f, int g_shift, hipStream_t st) {
