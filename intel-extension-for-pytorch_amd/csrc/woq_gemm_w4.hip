@@ -107,6 +107,24 @@ __device__ __forceinline__ u4 g4_dequant_m(uint32_t d, const G4Masks& k, uint32_
   return r;
 }
 
+__device__ __forceinline__ float act_bits_to_f32(uint16_t bits, int dtype) {
+  return dtype == WOQ_HIP_ACT_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
+}
+
+// Post-op of epilogue_store on a value of the activation dtype; the result is rounded by the store.
+__device__ __forceinline__ float post_op(float y, int fusion, int act_dtype, float other0, float other1) {
+  switch (fusion) {
+    case WOQ_HIP_FUSE_GELU_ERF: return gelu_erf(y);
+    case WOQ_HIP_FUSE_GELU_TANH: return gelu_tanh(y);
+    case WOQ_HIP_FUSE_RELU: return y > 0.0f ? y : 0.0f;
+    case WOQ_HIP_FUSE_SILU: return silu(y);
+    case WOQ_HIP_FUSE_ADD: return y + other0;
+    case WOQ_HIP_FUSE_ADD_ADD: return round_to_act(y + other0, act_dtype) + other1;
+    case WOQ_HIP_FUSE_MUL: return y * other0;
+    default: return y;
+  }
+}
+
 // GROUPED (mixture of experts): the row tile of a workgroup is a slot of the routing tables -- at most G4_BM routed rows of
 // one expert, whose tensors come from the group's pointer tables; a slot without an expert ends at once.
 // 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3832 us with three launches per expert (each on 32 to 192 workgroups),
@@ -533,6 +551,75 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
           }
           if (ncol0 + t * kTileN + 4 * c < f.N) *(u2*)(row + t * kTileN) = o;  // (N % 4 == 0: all four or none)
         }
+      }
+    }
+    return;
+  }
+  // Post-ops in the activation type on rows of whole 8-byte pieces: ECH row tiles at a time through the wave's stage (inside
+  // the activation buffers: the weight stages can still be written by the other waves' last requests), four columns a lane,
+  // the operands of the next pair of pieces requested before the current pair is worked on.  One element a lane and
+  // iteration, each waiting for its operand, took 20 us of a 88 us launch (M = 333, 11008 -> 4096 with a residual).
+  constexpr int kStageBytes = G4_WAVES * 16 * G4_SSTRIDE * (int)sizeof(float);  // one row tile of all waves
+  constexpr int ECH = G4_MT % 8 == 0 && 8 * kStageBytes <= 2 * G4_XBYTES   ? 8
+                      : G4_MT % 4 == 0 && 4 * kStageBytes <= 2 * G4_XBYTES ? 4
+                      : 2 * kStageBytes <= 2 * G4_XBYTES                   ? 2
+                                                                           : 1;
+  const bool vec4 = f.fusion != WOQ_HIP_FUSE_NONE && f.out_dtype == f.x_dtype && (f.N % 4) == 0 &&
+                    (((uintptr_t)f.out | (uintptr_t)f.other0 | (uintptr_t)f.other1) & 7) == 0 && ((uintptr_t)f.bias & 15) == 0;
+  // (not for 128 x 448 tiles, whose K loop has no register to spare)
+  if constexpr (G4_MT * G4_NTW <= 48) if (vec4) {
+    float* const st4 = (float*)sX + wave * (ECH * 16 * G4_SSTRIDE);
+    constexpr int ITS = ECH * G4_NTW;  // pieces of 64 lanes x 4 columns
+#pragma unroll
+    for (int mc = 0; mc < G4_MT; mc += ECH) {
+#pragma unroll
+      for (int i = 0; i < ECH; ++i)
+#pragma unroll
+        for (int t = 0; t < G4_NTW; ++t) *(f4*)(st4 + (16 * i + r) * G4_SSTRIDE + t * kTileN + 4 * c) = acc[mc + i][t];
+      struct Piece {
+        u2 a, b;
+        int64_t at;  // element of the output, or -1
+        int stage;
+        f4 bias;
+      };
+      auto request = [&](int it) {
+        Piece p;
+        const int q = it * 64 + lane, row = q / (G4_NTW * 4), col = (q - row * (G4_NTW * 4)) * 4;
+        const int m = m0 + mc * 16 + row;
+        const int64_t n = ncol0 + col;
+        p.stage = row * G4_SSTRIDE + col;
+        p.at = it < ITS && m < M && n < f.N ? (int64_t)m * f.N + n : -1;
+        p.a = p.b = u2{0u, 0u};
+        p.bias = f4{0.f, 0.f, 0.f, 0.f};
+        if (p.at >= 0) {
+          if (f.other0) p.a = *(const u2*)((const uint16_t*)f.other0 + p.at);
+          if (f.other1) p.b = *(const u2*)((const uint16_t*)f.other1 + p.at);
+          if (hb) p.bias = *(const f4*)(f.bias + n);
+        }
+        return p;
+      };
+      auto finish = [&](const Piece& p) {
+        if (p.at < 0) return;
+        const f4 v = *(const f4*)(st4 + p.stage);
+        u2 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float y = post_op(round_to_act(finalize_acc<REGIME>(v[e], hb, p.bias[e]), f.x_dtype), f.fusion, f.x_dtype,
+                                  act_bits_to_f32((uint16_t)(p.a[e / 2] >> (16 * (e % 2))), f.x_dtype),
+                                  act_bits_to_f32((uint16_t)(p.b[e / 2] >> (16 * (e % 2))), f.x_dtype));
+          const uint32_t bits = out_f16 ? f32_to_f16_bits(y) : f32_to_bf16_bits(y);
+          o[e / 2] = e % 2 ? o[e / 2] | (bits << 16) : bits;
+        }
+        *(u2*)((uint16_t*)f.out + p.at) = o;
+      };
+      Piece p0 = request(0), p1 = request(1);
+#pragma unroll 1
+      for (int it = 0; it < ITS; it += 2) {
+        const Piece n0 = request(it + 2), n1 = request(it + 3);
+        finish(p0);
+        finish(p1);
+        p0 = n0;
+        p1 = n1;
       }
     }
     return;

@@ -1054,6 +1054,30 @@ def test_nf4_prefill_kernel(cuda, M, K, N, G):
     assert _lib_last_kernel() == "woq_gemm_w4_kernel"
 
 
+@pytest.mark.parametrize("M,N,shape", [(65, 80, 12), (200, 272, 12), (200, 272, 6), (131, 272, 5), (130, 460, 4), (300, 400, 11)])  # (4: 128 x 448, one element a lane)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_prefill_kernel_post_ops_four_columns_at_a_time(cuda, M, N, shape, dtype):
+    """Every post-op through the vector epilogue of each tile shape, with a bias, rows and columns that end inside a tile: bit
+    for bit the post-op on the rounded output (silu and gelu to one rounding of the type)."""
+    from ipex_amd import _lib
+    import torch.nn.functional as F
+
+    case = _synthetic().make_int4_case(27, M, 256, N, 128, bias=True)
+    ctx = make_context(case, O.LOWP_BF16 if dtype == torch.bfloat16 else O.LOWP_FP16)
+    g = torch.Generator().manual_seed(28)
+    x = case["x"].to(dtype).cuda()
+    o1, o2 = (torch.randn(M, N, generator=g).to(dtype).cuda() for _ in range(2))
+    run = lambda **kw: ctx.run(x, force_kernel=shape, **kw)
+    base = run()
+    assert torch.equal(run(fusion=_lib.FUSE_ADD, others=(o1,)), base + o1)
+    assert torch.equal(run(fusion=_lib.FUSE_MUL, others=(o1,)), base * o1)
+    assert torch.equal(run(fusion=_lib.FUSE_ADD_ADD, others=(o1, o2)), (base + o1) + o2)
+    assert torch.equal(run(fusion=_lib.FUSE_RELU), F.relu(base))
+    eps = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    for fusion, f in ((_lib.FUSE_SILU, F.silu), (_lib.FUSE_GELU_ERF, F.gelu), (_lib.FUSE_GELU_TANH, lambda v: F.gelu(v, approximate="tanh"))):
+        assert torch.allclose(run(fusion=fusion).float(), f(base.float()), rtol=eps, atol=1e-6)
+
+
 def test_nf4_rejections(cuda):
     syn = _synthetic()
     case = syn.make_nf4_case(25, 4, 256, 32, 64)
