@@ -328,13 +328,36 @@ int launch_dense_weight(const void* qweight, int weight_dtype, int64_t N, int64_
 // (csrc/cpu/jit/cpu/kernels/LinearWoqPacked.cpp:777-954).  Channel j moves to position
 // g_idx[j] * group_size + (number of earlier channels of the same group); `src` is that map
 // read backwards (src[p] = the channel that lands at position p), which serves both directions.
+// Few rows, or rows too long for the LDS: columns along x, rows along y.
 template <typename T>
-__global__ void shuffle_activations_kernel(const T* __restrict__ x, int64_t M, int64_t K,
-                                           const int32_t* __restrict__ src, T* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M * K) return;
-  const int64_t m = i / K, p = i - m * K;
-  out[i] = x[m * K + src[p]];
+__global__ __launch_bounds__(256) void shuffle_activations_kernel(const T* __restrict__ x, int64_t M, int64_t K,
+                                                                  const int32_t* __restrict__ src, T* __restrict__ out) {
+  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (p >= K) return;
+  const int64_t j = src[p];
+  for (int64_t m = blockIdx.y; m < M; m += gridDim.y) out[m * K + p] = x[m * K + j];
+}
+
+// A row per workgroup through LDS: read and written in 16-byte pieces, the scattered two-byte reads are the LDS's (from
+// memory each of them is a cache line request of its own).  Rows and pointers are multiples of 16 bytes.
+template <typename T>
+__global__ __launch_bounds__(512) void shuffle_rows_kernel(const T* __restrict__ x, int K, const int32_t* __restrict__ src,
+                                                           T* __restrict__ out) {
+  extern __shared__ __align__(16) uint8_t srow[];
+  constexpr int PER = 16 / (int)sizeof(T);
+  const int64_t base = (int64_t)blockIdx.x * K;
+  for (int i = threadIdx.x * PER; i < K; i += 512 * PER) *(u4*)(srow + (size_t)i * sizeof(T)) = *(const u4*)(x + base + i);
+  __syncthreads();
+  for (int i = threadIdx.x * PER; i < K; i += 512 * PER) {
+    int32_t j[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) j[e] = src[i + e];
+    u4 o;
+    T* const v = (T*)&o;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) v[e] = ((const T*)srow)[j[e]];
+    *(u4*)(out + base + i) = o;
+  }
 }
 
 // plain int4 rows (two values per byte, low nibble first): one thread per output byte
@@ -396,14 +419,21 @@ int launch_convert_activations(const void* src, int src_dtype, void* dst, int ds
 
 int launch_shuffle_activations(const void* x, int x_dtype, int64_t M, int64_t K, const int32_t* src, void* out,
                                hipStream_t st) {
-  const int64_t total = M * K;
-  if (total == 0) return 0;
+  if (M * K == 0) return 0;
+  const int64_t row_bytes = K * (x_dtype == WOQ_HIP_ACT_FP32 ? 4 : 2);
+  // from 64 rows on a workgroup per row fills enough of the chip; 64 KiB is the LDS a launch gets without opting in
+  if (M >= 64 && M < (1ll << 31) && row_bytes <= 65536 && row_bytes % 16 == 0 && (((uintptr_t)x | (uintptr_t)out) & 15) == 0) {
+    if (x_dtype == WOQ_HIP_ACT_FP32)
+      shuffle_rows_kernel<uint32_t><<<(unsigned)M, 512, row_bytes, st>>>((const uint32_t*)x, (int)K, src, (uint32_t*)out);
+    else
+      shuffle_rows_kernel<uint16_t><<<(unsigned)M, 512, row_bytes, st>>>((const uint16_t*)x, (int)K, src, (uint16_t*)out);
+    return check_launch("shuffle_activations");
+  }
+  const dim3 grid(blocks_for(K, 256), (unsigned)(M < 65535 ? M : 65535));
   if (x_dtype == WOQ_HIP_ACT_FP32)
-    shuffle_activations_kernel<uint32_t><<<blocks_for(total, 256), 256, 0, st>>>((const uint32_t*)x, M, K, src,
-                                                                                   (uint32_t*)out);
+    shuffle_activations_kernel<uint32_t><<<grid, 256, 0, st>>>((const uint32_t*)x, M, K, src, (uint32_t*)out);
   else
-    shuffle_activations_kernel<uint16_t><<<blocks_for(total, 256), 256, 0, st>>>((const uint16_t*)x, M, K, src,
-                                                                                   (uint16_t*)out);
+    shuffle_activations_kernel<uint16_t><<<grid, 256, 0, st>>>((const uint16_t*)x, M, K, src, (uint16_t*)out);
   return check_launch("shuffle_activations");
 }
 

@@ -1078,6 +1078,16 @@ def test_prefill_kernel_post_ops_four_columns_at_a_time(cuda, M, N, shape, dtype
         assert torch.allclose(run(fusion=fusion).float(), f(base.float()), rtol=eps, atol=1e-6)
 
 
+@pytest.mark.parametrize("M,K,dtype", [(63, 264, torch.bfloat16), (64, 264, torch.bfloat16), (65, 4104, torch.float16), (70, 30, torch.bfloat16),
+                                       (64, 32768, torch.bfloat16), (64, 32776, torch.bfloat16), (80, 1000, torch.float32), (3, 16392, torch.float32)])
+def test_shuffle_activations_rows(cuda, M, K, dtype):
+    """Rows through the LDS from 64 rows on, element by element otherwise (few rows, odd or longer widths): whole values."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).to(dtype).cuda()
+    src = torch.randperm(K, generator=g).to(torch.int32).cuda()
+    assert torch.equal(_kernels().shuffle_activations(x, src), x[:, src.long()])
+
+
 def test_nf4_rejections(cuda):
     syn = _synthetic()
     case = syn.make_nf4_case(25, 4, 256, 32, 64)
