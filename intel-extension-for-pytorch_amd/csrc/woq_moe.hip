@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const int64_t* __restric
                                                         int split_lo, int split_mid, int use_single, int S,
                                                         int64_t* __restrict__ x_row, int32_t* __restrict__ slots,
                                                         int32_t* __restrict__ row_of, int32_t* __restrict__ slot_of) {
-  __shared__ int se[kMoeRouteMax];
+  __shared__ __align__(16) int se[kMoeRouteMax];
   __shared__ int8_t cls_of[kMoeRouteMax];  // size class of the expert whose first sorted position this is, or -1
   for (int i = threadIdx.x; i < R; i += blockDim.x) {
     const int64_t e = ids[i];
@@ -117,6 +117,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const int64_t* __restric
     row_of[i] = -1;
     slot_of[i] = 0;
   }
+  if ((int)threadIdx.x < 4 && R + (int)threadIdx.x < ((R + 3) & ~3)) se[R + threadIdx.x] = -1;  // to a multiple of four (kMoeRouteMax is one)
   for (int i = threadIdx.x; i < 12 * S; i += blockDim.x) slots[i] = (i / S) % 3 == 0 ? -1 : 0;
   __syncthreads();
   int my_p[kMoeRouteMax / 256], my_e[kMoeRouteMax / 256], my_n[kMoeRouteMax / 256];
@@ -128,11 +129,15 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const int64_t* __restric
     const int e = se[i];
     if (e < 0) continue;
     int before = 0, rank = 0, count = 0;
-    for (int k = 0; k < R; ++k) {
-      const int ek = se[k];
-      before += (ek >= 0 && ek < e) ? 1 : 0;
-      rank += (ek == e && k < i) ? 1 : 0;
-      count += (ek == e) ? 1 : 0;
+#pragma unroll 2
+    for (int k = 0; k < R; k += 4) {
+      const i4 ek = *(const i4*)(se + k);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        before += (ek[q] >= 0 && ek[q] < e) ? 1 : 0;
+        rank += (ek[q] == e && k + q < i) ? 1 : 0;
+        count += (ek[q] == e) ? 1 : 0;
+      }
     }
     const int p = before + rank;
     const int t = i / topk, j = i - t * topk;
@@ -179,7 +184,10 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const int64_t* __restric
   }
   // positions past the valid entries read token 0 (never used: no slot covers them)
   int valid = 0;
-  for (int k = 0; k < R; ++k) valid += se[k] >= 0 ? 1 : 0;
+  for (int k = 0; k < R; k += 4) {
+    const i4 ek = *(const i4*)(se + k);
+    valid += (ek[0] >= 0 ? 1 : 0) + (ek[1] >= 0 ? 1 : 0) + (ek[2] >= 0 ? 1 : 0) + (ek[3] >= 0 ? 1 : 0);
+  }
   for (int i = valid + threadIdx.x; i < R; i += blockDim.x) x_row[i] = 0;
 }
 
@@ -266,7 +274,8 @@ __global__ __launch_bounds__(1024) void moe_route_tiles_kernel(const int64_t* __
 
 // out[t, :] accumulates token t's contributions in the order row_of gives (ascending expert), each step rounded to the
 // output dtype -- what one moe_scale_add_rows launch per expert leaves in memory between the experts.
-template <int DTYPE>
+// VEC (16-bit types, H a multiple of 8, 16-byte aligned rows): a contribution's eight values are one load instead of eight.
+template <int DTYPE, bool VEC>
 __global__ void moe_combine_rows_kernel(void* __restrict__ out, const void* __restrict__ cur, const void* __restrict__ rw,
                                         int64_t topk, const int32_t* __restrict__ row_of,
                                         const int32_t* __restrict__ slot_of, int64_t T, int64_t H, int64_t R,
@@ -289,7 +298,19 @@ __global__ void moe_combine_rows_kernel(void* __restrict__ out, const void* __re
       have[i] = (uint64_t)r < (uint64_t)R;
       w[i] = have[i] ? load_act(rw, DTYPE, t * topk + slot_of[t * topk + i0 + i]) : 0.0f;
 #pragma unroll
-      for (int e = 0; e < PER; ++e) v[i][e] = (have[i] && j0 + e < H) ? load_act(cur, DTYPE, r * H + j0 + e) : 0.0f;
+      for (int e = 0; e < PER; ++e) v[i][e] = 0.0f;
+      if constexpr (VEC) {
+        const u4 raw = have[i] ? *(const u4*)((const uint16_t*)cur + r * H + j0) : u4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+          const uint16_t bits = (uint16_t)(raw[e / 2] >> (16 * (e % 2)));
+          v[i][e] = DTYPE == WOQ_HIP_ACT_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < PER; ++e)
+          if (have[i] && j0 + e < H) v[i][e] = load_act(cur, DTYPE, r * H + j0 + e);
+      }
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -303,7 +324,17 @@ __global__ void moe_combine_rows_kernel(void* __restrict__ out, const void* __re
       }
     }
   }
-  for (int e = 0; e < PER && j0 + e < H; ++e) store_act(out, DTYPE, t * H + j0 + e, o[e]);
+  if constexpr (VEC) {
+    u4 q;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)  // (o holds values of the type: exact)
+      q[e] = DTYPE == WOQ_HIP_ACT_BF16
+                 ? (uint32_t)f32_to_bf16_bits(o[(2 * e) % PER]) | ((uint32_t)f32_to_bf16_bits(o[(2 * e + 1) % PER]) << 16)
+                 : (uint32_t)f32_to_f16_bits(o[(2 * e) % PER]) | ((uint32_t)f32_to_f16_bits(o[(2 * e + 1) % PER]) << 16);
+    *(u4*)((uint16_t*)out + t * H + j0) = q;
+  } else {
+    for (int e = 0; e < PER && j0 + e < H; ++e) store_act(out, DTYPE, t * H + j0 + e, o[e]);
+  }
 }
 
 static inline unsigned moe_blocks(int64_t n) { return (unsigned)((n + 255) / 256); }
@@ -366,14 +397,18 @@ int launch_moe_combine_rows(void* out, int dtype, int64_t T, int64_t H, const vo
                             const int32_t* row_of, const int32_t* slot_of, int accumulate, hipStream_t st) {
   if (T == 0 || H == 0 || topk == 0) return 0;
   const int per = dtype == WOQ_HIP_ACT_FP32 ? 4 : 8;
-  const unsigned blocks = moe_blocks(T * ((H + per - 1) / per));
-  const int64_t R = T * topk;
+  const int64_t n = T * ((H + per - 1) / per), R = T * topk;
+  const unsigned threads = n < 65536 ? 64 : 256;  // few tokens: a wave per workgroup, spread over more CUs
+  const unsigned blocks = (unsigned)((n + threads - 1) / threads);
+  const bool vec = H % 8 == 0 && (((uintptr_t)out | (uintptr_t)cur) & 15) == 0;
+#define WOQ_COMBINE(D, V) moe_combine_rows_kernel<D, V><<<blocks, threads, 0, st>>>(out, cur, rw, topk, row_of, slot_of, T, H, R, accumulate != 0)
   if (dtype == WOQ_HIP_ACT_BF16)
-    moe_combine_rows_kernel<WOQ_HIP_ACT_BF16><<<blocks, 256, 0, st>>>(out, cur, rw, topk, row_of, slot_of, T, H, R, accumulate != 0);
+    vec ? WOQ_COMBINE(WOQ_HIP_ACT_BF16, true) : WOQ_COMBINE(WOQ_HIP_ACT_BF16, false);
   else if (dtype == WOQ_HIP_ACT_FP16)
-    moe_combine_rows_kernel<WOQ_HIP_ACT_FP16><<<blocks, 256, 0, st>>>(out, cur, rw, topk, row_of, slot_of, T, H, R, accumulate != 0);
+    vec ? WOQ_COMBINE(WOQ_HIP_ACT_FP16, true) : WOQ_COMBINE(WOQ_HIP_ACT_FP16, false);
   else
-    moe_combine_rows_kernel<WOQ_HIP_ACT_FP32><<<blocks, 256, 0, st>>>(out, cur, rw, topk, row_of, slot_of, T, H, R, accumulate != 0);
+    WOQ_COMBINE(WOQ_HIP_ACT_FP32, false);
+#undef WOQ_COMBINE
   return check_launch("moe_combine_rows");
 }
 
