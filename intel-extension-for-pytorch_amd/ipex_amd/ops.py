@@ -686,6 +686,9 @@ _MOE_PLAN_LIMIT = 128
 # path takes, allocated once and never moved, so that a HIP graph captured over a layer keeps valid addresses; shared
 # by all layers of those widths (calls on one stream follow each other).
 _MOE_ROWS = {}
+# Threads that share a stream share those buffers too: a layer's launches are queued as a whole, never between those of
+# another thread's layer (whose routing would name other slots and more rows than this call's buffers hold).
+_moe_launch_lock = threading.Lock()
 
 
 def _context_epochs():
@@ -865,10 +868,10 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     rw = routing_weights.contiguous()
     R = T * topk
     N1 = plan.shapes[0]["N"]
-    act, inter, y = plan.buffers(x.dtype, raw_stream)  # calls on one stream follow each other
     out = torch.empty_like(x)
     code = _kernels._ACT_CODE[x.dtype]
-    with torch.cuda.device(x.device):
+    with _moe_launch_lock, torch.cuda.device(x.device):
+        act, inter, y = plan.buffers(x.dtype, raw_stream)  # calls on one stream follow each other
         stream = _kernels._stream()
         _lib.check(lib.woq_hip_moe_route(ids.data_ptr(), T, topk, len(gate_ctx), split, 16, 2 if each else int(single), plan.S,
                                          plan.x_row.data_ptr(), plan.slots.data_ptr(), plan.row_of.data_ptr(),
@@ -931,9 +934,9 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights):
     lib = _lib.load()
     ids = topk_ids.to(torch.int64).contiguous()
     rw = routing_weights.contiguous()
-    buf = plan.tile_routing()
     code = _kernels._ACT_CODE[x.dtype]
-    with torch.cuda.device(x.device):
+    with _moe_launch_lock, torch.cuda.device(x.device):
+        buf = plan.tile_routing()
         stream = _kernels._stream()
         out = torch.empty_like(x)
         act, inter, y = (torch.empty((R, n), dtype=x.dtype, device=x.device) for n in (N1, N1, H))

@@ -1033,6 +1033,37 @@ def test_deepseek_moe_prompts_in_row_tiles(cuda, monkeypatch, T, E, topk, tile, 
         op(hidden, bad, ctxs[0], ctxs[1], ctxs[2], rw, False)
 
 
+def test_deepseek_moe_threads_on_one_stream(cuda):
+    """Layers called from several threads share their stream's routing buffers: every call has the bits it has alone."""
+    import threading
+
+    ipex = _ipex()
+    H, I, E, topk = 256, 384, 5, 2
+    mk = lambda k, n, s: _woq_module(ipex, k, n, "INT4", 128, "BF16", bias=False, seed=s)._op_context
+    ctxs = [[mk(H, I, 900 + 3 * e) for e in range(E)], [mk(H, I, 901 + 3 * e) for e in range(E)], [mk(I, H, 902 + 3 * e) for e in range(E)]]
+    calls = []
+    for T in (16, 65, 200, 333):
+        g = torch.Generator().manual_seed(T)
+        calls.append((torch.randn(T, H, generator=g).to(torch.bfloat16).to(cuda), torch.randint(0, E, (T, topk), generator=g).to(cuda),
+                      torch.softmax(torch.randn(T, topk, generator=g), -1).to(torch.bfloat16).to(cuda)))
+    layer = lambda x, ids, rw: torch.ops.torch_ipex.deepseek_moe_woq(x, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    want = [layer(*c) for c in calls]
+    got = [[] for _ in calls]
+
+    def work(i):
+        for _ in range(10):
+            got[i].append(layer(*calls[i]))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(calls))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for w, outs in zip(want, got):
+        assert len(outs) == 10 and all(torch.equal(w, o) for o in outs)
+
+
 def test_mixtral_moe_woq_single_expert_and_errors(cuda):
     ipex = _ipex()
     H, I, T = 128, 256, 6
