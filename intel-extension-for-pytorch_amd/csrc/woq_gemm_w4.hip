@@ -128,7 +128,7 @@ __device__ __forceinline__ float post_op(float y, int fusion, int act_dtype, flo
 // GROUPED (mixture of experts): the row tile of a workgroup is a slot of the routing tables -- at most G4_BM routed rows of
 // one expert, whose tensors come from the group's pointer tables; a slot without an expert ends at once.
 // 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3832 us with three launches per expert (each on 32 to 192 workgroups),
-// 794 us with one launch per linear.
+// 619 us with one launch per linear (three of about 200 us).
 // NF4: a dword's eight table values come from the 256-entry table of value pairs in LDS (nf4_dequant), built before the first
 // request; four 8-byte reads, eight products and four conversions against 17 instructions for integers.
 template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false, bool NF4 = false>
