@@ -415,11 +415,17 @@ int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, in
  * The same layer for prompts: woq_hip_moe_route_tiles sorts at most WOQ_HIP_MOE_TILES_MAX entries over at most
  * WOQ_HIP_MOE_TILES_EXPERTS experts and cuts the routed rows into slots, int32 [4][3][S], S >= experts + T * topk /
  * tile_rows: class 0 the experts with fewer than split_lo rows, 1 at most split_mid, 2 at most 64, one slot each; class 3
- * the others, in slots of at most tile_rows (64 or 128) rows; split_lo and split_mid at most 64.  x_row, row_of and slot_of as from woq_hip_moe_route.
+ * the others, in slots of at most tile_rows (64 or 128) rows, each slot's rows plus the expert's rows << 16;
+ * split_lo and split_mid at most 64.  x_row, row_of and slot_of as from woq_hip_moe_route.
  * woq_hip_linear_grouped_tiles runs one linear over the slots of class 3 on the prefill kernel: p as for
  * woq_hip_linear_grouped (M is ignored), INT4 weights with power-of-two groups of at least 32 or INT8 weights with
  * power-of-two groups of at least 128, or per-channel; K a multiple of 128, rows in the compute type of five and more rows.
+ * With slots of 64 rows an expert whose own launch would split K over workgroups (woq_hip_linear with the scratch that
+ * woq_hip_linear_auto_split_k_workspace_bytes asks for) runs the same K ranges one after the other and adds them in that
+ * launch's order, so it has that launch's bits; woq_hip_moe_chained_rows: the most rows of such an expert, 0 if there is none
+ * at this K and N.  Slots of 128 rows run K in one chain, as do slots whose table does not say the expert's rows.
  */
+int64_t woq_hip_moe_chained_rows(int64_t K, int64_t N);
 int woq_hip_moe_route_tiles(const int64_t* topk_ids, int64_t T, int64_t topk, int64_t experts, int64_t split_lo,
                             int64_t split_mid, int64_t tile_rows, int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of,
                             int32_t* slot_of, void* stream);

@@ -190,7 +190,7 @@ int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_
   const bool int8 = lowp_mode == WOQ_HIP_LOWP_INT8;
   // the dequantizing decode kernel (launch_decode_dq) and the 64 x 128 tiles of the prefill GEMMs (pick_splits)
   const bool decode = !int8 && M >= 5 && M <= 32 && K >= 8192 && N <= 4096;
-  const bool prefill = M > 64 && K >= 4096 && M * N <= 1048576;
+  const bool prefill = M > 64 && K >= kSplitKPrefillMinK && M * N <= kSplitKPrefillElems;
   return decode || prefill ? woq_hip_linear_split_k_workspace_bytes(M, N) : 0;
 }
 
@@ -455,6 +455,8 @@ int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, in
   }
   return launch_decode_dq_grouped(f, wbits, regime, (const MoeGroup*)group, slots, (hipStream_t)p->stream);
 }
+
+int64_t woq_hip_moe_chained_rows(int64_t K, int64_t N) { return K > 0 && N > 0 ? gemm_w4_split_rows(K, N) : 0; }
 
 int woq_hip_linear_grouped_tiles(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows) {
   FpArgs f;

@@ -129,15 +129,22 @@ __device__ __forceinline__ float post_op(float y, int fusion, int act_dtype, flo
 // one expert, whose tensors come from the group's pointer tables; a slot without an expert ends at once.
 // 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3832 us with three launches per expert (each on 32 to 192 workgroups),
 // 619 us with one launch per linear (three of about 200 us).
+// Where an expert's own launch would split K over workgroups (pick_splits), the workgroup runs the same K steps in as many
+// chains, one after the other, and adds them in the same order: the expert has the bits of its own launch.
 // NF4: a dword's eight table values come from the 256-entry table of value pairs in LDS (nf4_dequant), built before the first
 // request; four 8-byte reads, eight products and four conversions against 17 instructions for integers.
-template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false, bool NF4 = false>
+struct G4Group {
+  const MoeGroup* tables;
+  int rows4, kts4, rows2, kts2;  // experts of at most rows4 / rows2 rows (0: none): chains of kts4 / kts2 K steps
+};
+template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false, bool NF4 = false, bool CHAINS = false>
 __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const int g_shift, float* const sk_partial,
-                                                          int* const sk_counters, const int kts, const MoeGroup* const grp) {
+                                                          int* const sk_counters, const int kts, const G4Group grp) {
   static_assert(!NF4 || (WBITS == 4 && !FP8 && !MERGED && !GROUPED), "NF4 codes have a table and a scale");
   __shared__ f2 sNf4[NF4 ? kNf4LutEntries : 1];
   if constexpr (NF4) nf4_fill_lut(sNf4, (int)threadIdx.x, 256);  // (the barrier before the first use is the K loop's first)
   static_assert(!GROUPED || !MERGED, "the pointer tables hold scales and zero points apart");
+  static_assert(GROUPED || !CHAINS, "an ungrouped launch splits K over workgroups");
   constexpr int TPS = WBITS / 4;  // packed tiles per row-block and K step of 128
   constexpr int G4_MT = S::MT, G4_NTW = S::NTW, G4_BM = S::BM, G4_XBYTES = S::XBYTES, G4_XLOADS = S::XLOADS,
                 G4_WSTAGE = S::WSTAGE * TPS, G4_SSTRIDE = S::SSTRIDE;
@@ -149,12 +156,16 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
   xcd_tile(bx, by);
   FpArgs fg;                        // GROUPED: this slot's problem
   const int64_t* xrow = nullptr;    // GROUPED: routed row of the slot -> row of x, or null: x has the routed rows
+  int chain = kts;                  // CHAINS: K steps of a chain
   if constexpr (GROUPED) {
-    const MoeGroup& g = *grp;
+    const MoeGroup& g = *grp.tables;
     const int e = __builtin_amdgcn_readfirstlane(g.slot_expert[by]);
     if (e < 0) return;
     const int64_t row0 = __builtin_amdgcn_readfirstlane(g.slot_row0[by]);
-    const int rows = __builtin_amdgcn_readfirstlane(g.slot_rows[by]);
+    const int packed = __builtin_amdgcn_readfirstlane(g.slot_rows[by]);
+    const int rows = packed & 0xFFFF, expert_rows = packed >> 16;  // (0: not known, one chain)
+    if constexpr (CHAINS)
+      chain = expert_rows == 0 ? kts : expert_rows <= grp.rows4 ? grp.kts4 : expert_rows <= grp.rows2 ? grp.kts2 : kts;
     fg = fa;
     fg.M = rows < G4_BM ? rows : G4_BM;
     fg.qweight = dq_uniform((const uint8_t*)g.qweight[e]);
@@ -367,80 +378,107 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
 #pragma unroll
     for (int t = 0; t < G4_NTW; ++t) asm volatile("" : "+a"(acc[mt][t]));
 
-  for (int kt = kt_lo; kt < KT; ++kt) {
-    const uint8_t* xs = sX + (kt & 1) * G4_XBYTES;
-    const uint8_t* xsn = sX + ((kt & 1) ^ 1) * G4_XBYTES;
-    // ---- requests, in this order (s_waitcnt vmcnt counts from the youngest): parameters and
-    // activations of step kt + 1, then (behind the first MFMA block) the weight tiles of step
-    // kt + 2 into the stage that held step kt.  Past the end the last step is requested again. ----
-    const int kt1 = kt + 1 < KT ? kt + 1 : KT - 1;
-    const int kt2 = kt + 2 < KT ? kt + 2 : KT - 1;
-    if constexpr (MERGED) load_m(kt1, mr); else load_q(kt1, sr, zr);
-    load_x(kt1, (kt & 1) ^ 1);
-    __builtin_amdgcn_sched_barrier(0);
+  // (the requests of a chain's last steps are the next chain's first ones; -0 + x is x for every x)
+  f4 total[CHAINS ? G4_MT : 1][CHAINS ? G4_NTW : 1];
+  if constexpr (CHAINS) {
+#pragma unroll
+    for (int mt = 0; mt < G4_MT; ++mt)
+#pragma unroll
+      for (int t = 0; t < G4_NTW; ++t) total[mt][t] = f4{-0.f, -0.f, -0.f, -0.f};
+  }
+  for (int kt = kt_lo; kt < KT;) {  // (CHAINS: chain after chain, else once)
+    const int kt_end = CHAINS && kt + chain < KT ? kt + chain : KT;
+    for (; kt < kt_end; ++kt) {
+      const uint8_t* xs = sX + (kt & 1) * G4_XBYTES;
+      const uint8_t* xsn = sX + ((kt & 1) ^ 1) * G4_XBYTES;
+      // ---- requests, in this order (s_waitcnt vmcnt counts from the youngest): parameters and
+      // activations of step kt + 1, then (behind the first MFMA block) the weight tiles of step
+      // kt + 2 into the stage that held step kt.  Past the end the last step is requested again. ----
+      const int kt1 = kt + 1 < KT ? kt + 1 : KT - 1;
+      const int kt2 = kt + 2 < KT ? kt + 2 : KT - 1;
+      if constexpr (MERGED) load_m(kt1, mr); else load_q(kt1, sr, zr);
+      load_x(kt1, (kt & 1) ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
 
-    // 4 NTW blocks of MT MFMAs (one row-block t of one K sub-step j against the MT row tiles); the VALU
-    // dequantizes the B operand of the next block meanwhile.  Block FETCH_T of a sub-step also
-    // fetches the A fragments of the next sub-step; in the last sub-step these come from the other
-    // buffer, so that block starts with the wait for this step's activations and the barrier.  Block t of the last sub-step reads the
-    // tile of row-block t for the next step from LDS; its registers were last used one block before.
+      // 4 NTW blocks of MT MFMAs (one row-block t of one K sub-step j against the MT row tiles); the VALU
+      // dequantizes the B operand of the next block meanwhile.  Block FETCH_T of a sub-step also
+      // fetches the A fragments of the next sub-step; in the last sub-step these come from the other
+      // buffer, so that block starts with the wait for this step's activations and the barrier.  Block t of the last sub-step reads the
+      // tile of row-block t for the next step from LDS; its registers were last used one block before.
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < 4; ++j) {
 #pragma unroll
-      for (int t = 0; t < G4_NTW; ++t) {
-        const int cur = (j * G4_NTW + t) & 1;
-        const bool last_t = t == G4_NTW - 1;
-        const bool fetch_t = t == S::FETCH_T;
-        if (j == 0 && t == 1) {
-          // the LDS reads of the previous step's last blocks have returned: their stage is free
-          __builtin_amdgcn_s_waitcnt(kLgkmcnt0);
-          dma_w(kt2, kt & 1);
+        for (int t = 0; t < G4_NTW; ++t) {
+          const int cur = (j * G4_NTW + t) & 1;
+          const bool last_t = t == G4_NTW - 1;
+          const bool fetch_t = t == S::FETCH_T;
+          if (j == 0 && t == 1) {
+            // the LDS reads of the previous step's last blocks have returned: their stage is free
+            __builtin_amdgcn_s_waitcnt(kLgkmcnt0);
+            dma_w(kt2, kt & 1);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (j == 3 && t == 0) __builtin_amdgcn_s_waitcnt(kVmcntStep);  // tiles of step kt + 1 are in LDS
+          if constexpr (STAG_MAX == 0) {
+            if (fetch_t && j == 3) {
+              // Written as an instruction, not as the barrier builtin: before that one the compiler
+              // waits for every outstanding load, the tiles requested for step kt + 2 included.
+              __builtin_amdgcn_s_waitcnt(kVmcntW);
+              asm volatile("s_barrier" ::: "memory");
+            }
+          } else {
+            // this wave's meeting block (see bar_t)
+            if (j == 3 && t <= S::FETCH_T && t >= S::FETCH_T - STAG_MAX && bar_t == t) {
+              __builtin_amdgcn_s_waitcnt(kVmcntW);
+              __builtin_amdgcn_s_barrier();
+            }
+          }
+          if (last_t && j == 3) {
+#pragma unroll
+            for (int u = 0; u < G4_NTW; ++u) set_q(u, sr[u], (float)zr[u]);
+            bop[cur ^ 1] = deq(0, 0);
+          } else if (last_t) {
+            bop[cur ^ 1] = deq(0, j + 1);
+          } else {
+            bop[cur ^ 1] = deq(t + 1, j);
+          }
+#pragma unroll
+          for (int mt = 0; mt < G4_MT; ++mt) {
+            acc[mt][t] = g4_mfma<REGIME>(bop[cur], xa[(j & 1) % S::XA_SETS][mt], acc[mt][t]);
+            if (fetch_t)
+              xa[((j & 1) ^ 1) % S::XA_SETS][mt] = j == 3 ? *(const u4*)(xsn + mt * 4096 + rd[0])
+                                           : *(const u4*)(xs + mt * 4096 + rd[j + 1]);
+          }
+          if (j == 3) {
+#pragma unroll
+            for (int u = 0; u < TPS; ++u) wr[t][u] = read_w((kt & 1) ^ 1, t, u);
+          }
+#pragma unroll
+          for (int mt = 0; mt < G4_MT; ++mt) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (fetch_t) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (j == 3 && t == 0) __builtin_amdgcn_s_waitcnt(kVmcntStep);  // tiles of step kt + 1 are in LDS
-        if constexpr (STAG_MAX == 0) {
-          if (fetch_t && j == 3) {
-            // Written as an instruction, not as the barrier builtin: before that one the compiler
-            // waits for every outstanding load, the tiles requested for step kt + 2 included.
-            __builtin_amdgcn_s_waitcnt(kVmcntW);
-            asm volatile("s_barrier" ::: "memory");
-          }
-        } else {
-          // this wave's meeting block (see bar_t)
-          if (j == 3 && t <= S::FETCH_T && t >= S::FETCH_T - STAG_MAX && bar_t == t) {
-            __builtin_amdgcn_s_waitcnt(kVmcntW);
-            __builtin_amdgcn_s_barrier();
-          }
-        }
-        if (last_t && j == 3) {
-#pragma unroll
-          for (int u = 0; u < G4_NTW; ++u) set_q(u, sr[u], (float)zr[u]);
-          bop[cur ^ 1] = deq(0, 0);
-        } else if (last_t) {
-          bop[cur ^ 1] = deq(0, j + 1);
-        } else {
-          bop[cur ^ 1] = deq(t + 1, j);
-        }
-#pragma unroll
-        for (int mt = 0; mt < G4_MT; ++mt) {
-          acc[mt][t] = g4_mfma<REGIME>(bop[cur], xa[(j & 1) % S::XA_SETS][mt], acc[mt][t]);
-          if (fetch_t)
-            xa[((j & 1) ^ 1) % S::XA_SETS][mt] = j == 3 ? *(const u4*)(xsn + mt * 4096 + rd[0])
-                                         : *(const u4*)(xs + mt * 4096 + rd[j + 1]);
-        }
-        if (j == 3) {
-#pragma unroll
-          for (int u = 0; u < TPS; ++u) wr[t][u] = read_w((kt & 1) ^ 1, t, u);
-        }
-#pragma unroll
-        for (int mt = 0; mt < G4_MT; ++mt) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          if (fetch_t) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
       }
     }
+    if constexpr (CHAINS) {
+#pragma unroll
+      for (int mt = 0; mt < G4_MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < G4_NTW; ++t) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) total[mt][t][e] += acc[mt][t][e];
+          acc[mt][t] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+  if constexpr (CHAINS) {
+#pragma unroll
+    for (int mt = 0; mt < G4_MT; ++mt)
+#pragma unroll
+      for (int t = 0; t < G4_NTW; ++t) acc[mt][t] = total[mt][t];
   }
 
   // The requests past the last step are still writing LDS: drain them before the workgroup can end.
@@ -663,6 +701,31 @@ bool gemm_w4_nf4_faster(const FpArgs& f) {
   return 83.0 * (double)gens < std::max(105.0, 0.22 * (double)w2);
 }
 
+// Even, so that every split starts on buffer 0.
+static int split_k_steps(int ksteps, int splits) { return ((ksteps + splits - 1) / splits + 1) & ~1; }
+
+constexpr int kSplitWorkgroups = 256, kSplitMinSteps = 16;
+// K splits of the 64 x 128 shape: 4 or 2 workgroups per tile while that stays within 256 workgroups,
+// leaves each at least 16 K steps and the caller's scratch suffices (14336 -> 4096, M = 128: 64 tiles).
+static int pick_splits(const FpArgs& f, int wbits, int64_t tiles, const SplitKScratch* scratch) {
+  if (!scratch || !scratch->partial || !scratch->counters || tiles > kSplitKCounters) return 1;
+  const int64_t ksteps = f.KT / (wbits / 4);
+  for (int s = 4; s >= 2; s -= 2) {
+    const int64_t need = (int64_t)s * tiles * 64 * 128 * (int64_t)sizeof(float);
+    if (tiles * s <= kSplitWorkgroups && ksteps / s >= kSplitMinSteps && scratch->bytes >= need) return s;
+  }
+  return 1;
+}
+
+// The same choice for one expert of a grouped launch, as its own launch makes it with the scratch that
+// woq_hip_linear_auto_split_k_workspace_bytes asks for: experts of at most this many rows run in `splits` chains (0: none).
+static int split_rows(int64_t K, int64_t N, int splits) {
+  if (K < kSplitKPrefillMinK || K / kTileK4 / splits < kSplitMinSteps) return 0;
+  const int64_t columns = (N + 127) / 128;
+  return (int)std::min(kSplitWorkgroups / (splits * columns) * 64, kSplitKPrefillElems / N);
+}
+int gemm_w4_split_rows(int64_t K, int64_t N) { return split_rows(K, N, 2); }
+
 template <int REGIME, class S, int WBITS = 4, bool FP8 = false, bool NF4 = false>
 static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits = 1,
                         const SplitKScratch* scratch = nullptr) {
@@ -680,7 +743,7 @@ static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits
   int kts = ksteps;
   if (splits > 1) {
     if (S::MT * S::NTW > 8) return set_error("woq_gemm_w4_kernel: K is split for the 64 x 128 shape only");
-    kts = ((ksteps + splits - 1) / splits + 1) & ~1;  // even, so that every workgroup starts on buffer 0
+    kts = split_k_steps(ksteps, splits);
     const int64_t tiles = (int64_t)grid.x * grid.y;
     const int64_t need = (int64_t)splits * tiles * S::BM * S::BN * (int64_t)sizeof(float);
     if ((int64_t)(splits - 1) * kts >= ksteps)
@@ -697,27 +760,27 @@ static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits
       if (lds_optin_m != hipSuccess)
         return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin_m));
       woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, true><<<grid, 256, kLds, st>>>(
-          f, g_shift, splits > 1 ? scratch->partial : nullptr, splits > 1 ? scratch->counters : nullptr, kts, nullptr);
+          f, g_shift, splits > 1 ? scratch->partial : nullptr, splits > 1 ? scratch->counters : nullptr, kts, G4Group{});
       return check_launch("woq_gemm_w4_kernel");
     }
   }
   woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4><<<grid, 256, kLds, st>>>(f, g_shift, splits > 1 ? scratch->partial : nullptr,
-                                                                 splits > 1 ? scratch->counters : nullptr, kts, nullptr);
+                                                                 splits > 1 ? scratch->counters : nullptr, kts, G4Group{});
   return check_launch("woq_gemm_w4_kernel");
 }
 
 // Row tiles of the routed rows of all experts in one launch (woq_hip_linear_grouped_tiles).
-template <int REGIME, class S, int WBITS>
-static int launch_grouped_shape(const FpArgs& f, int g_shift, const MoeGroup* grp, int64_t slots, hipStream_t st) {
+template <int REGIME, class S, int WBITS, bool CHAINS>
+static int launch_grouped_shape(const FpArgs& f, int g_shift, const G4Group& g, int64_t slots, hipStream_t st) {
   constexpr int kLds = g4_lds_bytes<S, WBITS>();
   static const hipError_t lds_optin =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, false, false, true>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, false, false, true, false, CHAINS>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   if (lds_optin != hipSuccess)
     return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin));
   const dim3 grid((unsigned)((f.NT * kTileN + S::BN - 1) / S::BN), (unsigned)slots);
-  woq_gemm_w4_kernel<REGIME, S, WBITS, false, false, true>
-      <<<grid, 256, kLds, st>>>(f, g_shift, nullptr, nullptr, (int)(f.KT / (WBITS / 4)), grp);
+  woq_gemm_w4_kernel<REGIME, S, WBITS, false, false, true, false, CHAINS>
+      <<<grid, 256, kLds, st>>>(f, g_shift, nullptr, nullptr, (int)(f.KT / (WBITS / 4)), g);
   return check_launch("woq_gemm_w4_kernel (grouped)");
 }
 
@@ -730,9 +793,15 @@ int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGrou
   }
   using S2 = G4Shape<8, 2>;
   using S42 = G4Shape<4, 2>;
-#define WOQ_GROUPED(RG, WB)                                                         \
-  (tile_rows == 64 ? launch_grouped_shape<RG, S42, WB>(f, g_shift, grp, slots, st) \
-                   : launch_grouped_shape<RG, S2, WB>(f, g_shift, grp, slots, st))
+  // Chains on 64 x 128 tiles only: a second copy of the accumulators costs a 128 x 128 tile its second workgroup on a CU (us with
+  // 64 / 128 rows a tile: 32 experts 7168 -> 2048, top-8, 1024 tokens 1228 / 1295, 16 experts 4096 -> 1536,
+  // top-4, 2048 tokens 562 / 697).
+  const int ksteps = (int)(f.KT / (wbits / 4));
+  const G4Group g{grp, split_rows(f.K, f.N, 4), split_k_steps(ksteps, 4), split_rows(f.K, f.N, 2), split_k_steps(ksteps, 2)};
+#define WOQ_GROUPED(RG, WB)                                                                  \
+  (tile_rows == 128 ? launch_grouped_shape<RG, S2, WB, false>(f, g_shift, g, slots, st)      \
+   : g.rows2 > 64   ? launch_grouped_shape<RG, S42, WB, true>(f, g_shift, g, slots, st)      \
+                    : launch_grouped_shape<RG, S42, WB, false>(f, g_shift, g, slots, st))
   if (wbits == 4) return regime == kRegimeF16 ? WOQ_GROUPED(kRegimeF16, 4) : WOQ_GROUPED(kRegimeBF16, 4);
   return regime == kRegimeF16 ? WOQ_GROUPED(kRegimeF16, 8) : WOQ_GROUPED(kRegimeBF16, 8);
 #undef WOQ_GROUPED
@@ -744,18 +813,6 @@ template <class S>
 static double shape_cost(const FpArgs& f) {
   const double wgs = (double)((f.NT * kTileN + S::BN - 1) / S::BN) * (double)((f.M + S::BM - 1) / S::BM);
   return (double)(int64_t)((wgs + 255) / 256) * (S::NTW + 1.0);
-}
-
-// K splits of the 64 x 128 shape: 4 or 2 workgroups per tile while that stays within 256 workgroups,
-// leaves each at least 16 K steps and the caller's scratch suffices (14336 -> 4096, M = 128: 64 tiles).
-static int pick_splits(const FpArgs& f, int wbits, int64_t tiles, const SplitKScratch* scratch) {
-  if (!scratch || !scratch->partial || !scratch->counters || tiles > kSplitKCounters) return 1;
-  const int64_t ksteps = f.KT / (wbits / 4);
-  for (int s = 4; s >= 2; s -= 2) {
-    const int64_t need = (int64_t)s * tiles * 64 * 128 * (int64_t)sizeof(float);
-    if (tiles * s <= 256 && ksteps / s >= 16 && scratch->bytes >= need) return s;
-  }
-  return 1;
 }
 
 // 8-bit weights of one shape: integers or float8 bytes, fp16 or bf16 compute

@@ -61,6 +61,8 @@ struct SplitKScratch {
 // Entries the caller's split-K counter array must have, and the largest number of K splits.
 constexpr int kSplitKCounters = 512;
 constexpr int kSplitKMax = 4;
+// Prefill problems that get split-K scratch by themselves (woq_hip_linear_auto_split_k_workspace_bytes).
+constexpr int64_t kSplitKPrefillMinK = 4096, kSplitKPrefillElems = 1048576;
 
 int launch_pack_weight(const void* plain, int weight_dtype, int64_t N, int64_t K, void* packed,
                        hipStream_t st);
@@ -158,6 +160,7 @@ bool gemm_w4s_applies(const FpArgs& f, int wbits, int regime);
 int launch_gemm_w4s(const FpArgs& f, int regime, hipStream_t st);
 int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int shape = 0, int splits = 0,
                    const SplitKScratch* scratch = nullptr);
+int gemm_w4_split_rows(int64_t K, int64_t N);  // most rows of an expert of a routed layer that runs K in chains, 0: none
 // The same kernel over the slots of a routed layer (at most tile_rows = 64 or 128 routed rows of one expert each)
 int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGroup* grp, int64_t slots, int tile_rows,
                            hipStream_t st);

@@ -198,8 +198,8 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const int64_t* __restric
 // flight instead of eight, an expert's slots written inside the loop over the experts before it (a wave's lanes one after the
 // other) and the unused ends of the tables by one thread.
 //   slots   [4 classes][expert, first row, rows][S]: 0: experts with fewer than split_lo rows, 1: at most split_mid, 2: at most
-//           64, one slot each; 3: the others in slots of at most tile_rows rows, an expert's slots one after the other;
-//           unused entries expert -1.
+//           64, one slot each; 3: the others in slots of at most tile_rows rows, an expert's slots one after the other,
+//           rows | the expert's rows << 16 in place of rows; unused entries expert -1.
 //   x_row, row_of, slot_of as above.
 constexpr int kMoeTilesMax = WOQ_HIP_MOE_TILES_MAX;
 constexpr int kMoeTilesExperts = WOQ_HIP_MOE_TILES_EXPERTS;
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(1024) void moe_route_tiles_kernel(const int64_t* __
       if (idx >= S) break;  // (the host gives S entries for every case)
       tab[idx] = tid;
       tab[S + idx] = before + row;
-      tab[2 * S + idx] = n - row < step ? n - row : step;
+      tab[2 * S + idx] = (n - row < step ? n - row : step) | (cls == 3 ? n << 16 : 0);
     }
   }
   __syncthreads();

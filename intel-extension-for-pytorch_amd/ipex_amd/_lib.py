@@ -54,6 +54,7 @@ EXPORTS = [
     "woq_hip_linear_grouped",
     "woq_hip_moe_route_tiles",
     "woq_hip_linear_grouped_tiles",
+    "woq_hip_moe_chained_rows",
     "woq_hip_moe_combine_rows",
 ]
 
@@ -175,6 +176,8 @@ def load():
         lib.woq_hip_moe_route_tiles.argtypes = [vp, i64, i64, i64, i64, i64, i64, i64, vp, vp, vp, vp, vp]
         lib.woq_hip_linear_grouped_tiles.restype = i32
         lib.woq_hip_linear_grouped_tiles.argtypes = [ctypes.POINTER(LinearParams), vp, i64, i32]
+        lib.woq_hip_moe_chained_rows.restype = i64
+        lib.woq_hip_moe_chained_rows.argtypes = [i64, i64]
         lib.woq_hip_moe_combine_rows.restype = i32
         lib.woq_hip_moe_combine_rows.argtypes = [vp, i32, i64, i64, vp, vp, i64, vp, vp, i32, vp]
         if lib.woq_hip_abi_version() != 3:

@@ -756,6 +756,8 @@ class _MoeGroupedPlan:
         self.tiles_ok = len(gate_ctx) <= _lib.MOE_TILES_EXPERTS and all(
             x["K"] % 128 == 0 and (x["G"] <= 0 or (x["G"] >= (32 if x["wd"] == _lib.DTYPE_INT4 else 128) and x["G"] & (x["G"] - 1) == 0))
             for x in self.shapes)
+        # experts of more than 64 and at most this many rows add K in chains, as their own launches do (64-row tiles only)
+        self.chained_rows = max(_lib.load().woq_hip_moe_chained_rows(x["K"], x["N"]) for x in self.shapes)
         self.ok = True
 
     def tile_routing(self):
@@ -911,8 +913,8 @@ def _moe_tile_rows(rows, experts):
 
 def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights):
     """The layer for prompts (more than 64 tokens): the routed rows of all experts in row tiles of the prefill kernel, one
-    launch per linear (woq_hip_linear_grouped_tiles), experts with at most 64 rows on the decode kernels as above (which are
-    the kernels that the per-expert path runs for them).  The routing is read on the host to refuse ids that name no
+    launch per linear (woq_hip_linear_grouped_tiles), with the bits of the experts' own launches; experts with at most 64
+    rows on the decode kernels as above.  The routing is read on the host to refuse ids that name no
     expert, as the per-expert path does, and says which of the size classes are empty."""
     T, H = x.shape
     topk, experts, lowp = topk_ids.shape[1], plan.S, plan.shapes[0]["lowp"]
@@ -926,7 +928,8 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights):
     if int(host_ids.min()) < 0 or int(host_ids.max()) >= experts:
         raise RuntimeError(f"torch_ipex::deepseek_moe_woq: expert ids must lie in [0, {experts})")
     counts = torch.bincount(host_ids.reshape(-1), minlength=experts).tolist()
-    rows = _moe_tile_rows(R, experts)
+    chained = any(64 < n <= plan.chained_rows for n in counts)
+    rows = 64 if chained else _moe_tile_rows(R, experts)
     used = [0, 0, 0, 0]  # slots of each size class
     for n in counts:
         if n:
