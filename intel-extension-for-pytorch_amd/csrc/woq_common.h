@@ -297,12 +297,16 @@ __device__ __forceinline__ void epilogue_store(const Epilogue& e, int64_t m, int
   store_act(e.out, e.out_dtype, idx, y);
 }
 
-// a pointer every lane of the wave loaded from the same address, moved to scalar registers
+// A pointer to global memory that every lane of the wave loaded from the same address, moved to scalar registers.  The cast
+// says which memory it is: a pointer put together from integers alone is generic, and loads through it are FLAT instructions,
+// after which no count but zero of s_waitcnt is defined (they count as memory and as LDS accesses and may return out of order
+// with both), whereas the kernels wait for their loads by counts.
 template <typename T>
 __device__ __forceinline__ T* dq_uniform(T* p) {
+  typedef __attribute__((address_space(1))) T* global_t;
   const uint64_t v = (uint64_t)p;
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return (T*)(((uint64_t)hi << 32) | lo);
+  return (T*)(global_t)(((uint64_t)hi << 32) | lo);
 }
 
 // ---- 4-bit weights as MFMA operands: one packed dword (8 weights of one row) -> 8 bf16 / fp16 ----

@@ -63,21 +63,21 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
   if constexpr (GROUPED) {
     const MoeGroup& g = *a_in.grp;
     const int slot = (int)blockIdx.z;
-    const int e = __builtin_amdgcn_readfirstlane(g.slot_expert[slot]);
+    const int e = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_expert)[slot]);
     if (e < 0) return;  // the whole workgroup, before anything is synchronized
-    const int64_t row0 = __builtin_amdgcn_readfirstlane(g.slot_row0[slot]);
-    const int rows = __builtin_amdgcn_readfirstlane(g.slot_rows[slot]);
+    const int64_t row0 = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_row0)[slot]);
+    const int rows = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_rows)[slot]);
     ag = a_in;
     ag.M = rows < MAXM ? rows : MAXM;
-    ag.qweight = dq_uniform((const uint8_t*)g.qweight[e]);
-    ag.sz = dq_uniform((const uint32_t*)g.scales[e]);
-    ag.bias = g.bias ? dq_uniform(g.bias[e]) : nullptr;
+    ag.qweight = dq_uniform((const uint8_t*)dq_uniform(g.qweight)[e]);
+    ag.sz = dq_uniform((const uint32_t*)dq_uniform(g.scales)[e]);
+    ag.bias = g.bias ? dq_uniform(dq_uniform(g.bias)[e]) : nullptr;
     ag.out = (uint8_t*)a_in.out + row0 * a_in.N * 2;
     if (a_in.other0) ag.other0 = (const uint8_t*)a_in.other0 + row0 * a_in.N * 2;
 #pragma unroll
     for (int m = 0; m < MAXM; ++m) {
       const int64_t row = row0 + (m < (int)ag.M ? m : (int)ag.M - 1);
-      xr[m] = g.x_row ? (int64_t)__builtin_amdgcn_readfirstlane((int)g.x_row[row]) : row;
+      xr[m] = g.x_row ? (int64_t)__builtin_amdgcn_readfirstlane((int)dq_uniform(g.x_row)[row]) : row;
     }
   }
   const DecodeArgs& a = GROUPED ? ag : a_in;
@@ -286,14 +286,14 @@ __global__ __launch_bounds__(KPW == 4 ? 512 : 1024, KPW == 2 ? 8 : 4) void woq_d
   if constexpr (GROUPED) {
     const MoeGroup& g = *a_in.grp;
     const int slot = (int)blockIdx.z;
-    const int e = __builtin_amdgcn_readfirstlane(g.slot_expert[slot]);
+    const int e = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_expert)[slot]);
     if (e < 0) return;  // the whole workgroup, before anything is synchronized
-    const int64_t row = __builtin_amdgcn_readfirstlane(g.slot_row0[slot]);
-    const int64_t xr = g.x_row ? (int64_t)__builtin_amdgcn_readfirstlane((int)g.x_row[row]) : row;
+    const int64_t row = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_row0)[slot]);
+    const int64_t xr = g.x_row ? (int64_t)__builtin_amdgcn_readfirstlane((int)dq_uniform(g.x_row)[row]) : row;
     ag = a_in;
-    ag.qweight = dq_uniform((const uint8_t*)g.qweight[e]);
-    ag.sz = dq_uniform((const uint32_t*)g.scales[e]);
-    ag.bias = g.bias ? dq_uniform(g.bias[e]) : nullptr;
+    ag.qweight = dq_uniform((const uint8_t*)dq_uniform(g.qweight)[e]);
+    ag.sz = dq_uniform((const uint32_t*)dq_uniform(g.scales)[e]);
+    ag.bias = g.bias ? dq_uniform(dq_uniform(g.bias)[e]) : nullptr;
     ag.x = a_in.x + xr * a_in.K;
     ag.out = (uint8_t*)a_in.out + row * a_in.N * 2;
     if (a_in.other0) ag.other0 = (const uint8_t*)a_in.other0 + row * a_in.N * 2;

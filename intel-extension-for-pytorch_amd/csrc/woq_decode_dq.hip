@@ -141,22 +141,22 @@ __global__ __launch_bounds__(512, (MT * NTW > 8 ? 2 : 4)) void woq_decode_dq_ker
     // every workgroup of a slot takes the same path, and nothing has been synchronized yet
     const MoeGroup& g = *a.grp;
     const int slot = (int)blockIdx.z;
-    const int e = __builtin_amdgcn_readfirstlane(g.slot_expert[slot]);
+    const int e = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_expert)[slot]);
     if (e < 0) return;
-    const int64_t row0 = __builtin_amdgcn_readfirstlane(g.slot_row0[slot]);
-    const int rows = __builtin_amdgcn_readfirstlane(g.slot_rows[slot]);
+    const int64_t row0 = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_row0)[slot]);
+    const int rows = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_rows)[slot]);
     fg = a.f;
     fg.M = rows < (int)fg.M ? rows : fg.M;
-    fg.qweight = dq_uniform((const uint8_t*)g.qweight[e]);
-    fg.scales = dq_uniform((const uint16_t*)g.scales[e]);
-    fg.zeros = g.zeros ? dq_uniform(g.zeros[e]) : nullptr;
-    fg.bias = g.bias ? dq_uniform(g.bias[e]) : nullptr;
+    fg.qweight = dq_uniform((const uint8_t*)dq_uniform(g.qweight)[e]);
+    fg.scales = dq_uniform((const uint16_t*)dq_uniform(g.scales)[e]);
+    fg.zeros = g.zeros ? dq_uniform(dq_uniform(g.zeros)[e]) : nullptr;
+    fg.bias = g.bias ? dq_uniform(dq_uniform(g.bias)[e]) : nullptr;
     const int64_t out_elt = fg.out_dtype == WOQ_HIP_ACT_FP32 ? 4 : 2, x_elt = 2;  // rows are 16-bit here
     fg.out = (uint8_t*)fg.out + row0 * fg.N * out_elt;
     if (fg.other0) fg.other0 = (const uint8_t*)fg.other0 + row0 * fg.N * x_elt;
     if (fg.other1) fg.other1 = (const uint8_t*)fg.other1 + row0 * fg.N * x_elt;
     if (g.x_row) {
-      xrow = g.x_row;
+      xrow = dq_uniform(g.x_row);
       xrow0 = row0;
     } else {
       fg.x = (const uint8_t*)fg.x + row0 * fg.K * x_elt;

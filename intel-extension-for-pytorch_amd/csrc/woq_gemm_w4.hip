@@ -159,23 +159,23 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
   int chain = kts;                  // CHAINS: K steps of a chain
   if constexpr (GROUPED) {
     const MoeGroup& g = *grp.tables;
-    const int e = __builtin_amdgcn_readfirstlane(g.slot_expert[by]);
+    const int e = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_expert)[by]);
     if (e < 0) return;
-    const int64_t row0 = __builtin_amdgcn_readfirstlane(g.slot_row0[by]);
-    const int packed = __builtin_amdgcn_readfirstlane(g.slot_rows[by]);
+    const int64_t row0 = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_row0)[by]);
+    const int packed = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_rows)[by]);
     const int rows = packed & 0xFFFF, expert_rows = packed >> 16;  // (0: not known, one chain)
     if constexpr (CHAINS)
       chain = expert_rows == 0 ? kts : expert_rows <= grp.rows4 ? grp.kts4 : expert_rows <= grp.rows2 ? grp.kts2 : kts;
     fg = fa;
     fg.M = rows < G4_BM ? rows : G4_BM;
-    fg.qweight = dq_uniform((const uint8_t*)g.qweight[e]);
-    fg.scales = dq_uniform((const uint16_t*)g.scales[e]);
-    fg.zeros = g.zeros ? dq_uniform(g.zeros[e]) : nullptr;
-    fg.bias = g.bias ? dq_uniform(g.bias[e]) : nullptr;
+    fg.qweight = dq_uniform((const uint8_t*)dq_uniform(g.qweight)[e]);
+    fg.scales = dq_uniform((const uint16_t*)dq_uniform(g.scales)[e]);
+    fg.zeros = g.zeros ? dq_uniform(dq_uniform(g.zeros)[e]) : nullptr;
+    fg.bias = g.bias ? dq_uniform(dq_uniform(g.bias)[e]) : nullptr;
     fg.out = (uint8_t*)fa.out + row0 * fa.N * 2;  // (16-bit rows)
     if (fa.other0) fg.other0 = (const uint8_t*)fa.other0 + row0 * fa.N * 2;
     if (g.x_row)
-      xrow = g.x_row + row0;
+      xrow = dq_uniform(g.x_row) + row0;
     else
       fg.x = (const uint8_t*)fa.x + row0 * fa.K * 2;
     by = 0;

@@ -1,0 +1,50 @@
+"""Static checks of the built library's kernels that wait for their loads by counts (no GPU): ``s_waitcnt vmcnt(n)`` with
+n > 0 rests on loads that return in the order of their requests, and on n being counted from the loads that the compiler
+really emits."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "intel-extension-for-pytorch_amd", "lib", "libwoq_hip.so")
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+pytestmark = pytest.mark.skipif(not os.path.exists(LIB) or not os.path.exists(OBJDUMP), reason="needs the built library and llvm-objdump")
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """{mangled name: [(address, instruction)]} of the prefill and decode kernels."""
+    d = tmp_path_factory.mktemp("isa")
+    shutil.copy(LIB, d / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=d, check=True, capture_output=True)
+    out = {}
+    for name in sorted(os.listdir(d)):
+        if not name.endswith("gfx950"):
+            continue
+        with open(d / name, "rb") as f:
+            code = f.read()
+        if b"woq_gemm_w4_kernel" not in code and b"woq_decode_dq_kernel" not in code and b"woq_decode_kernel" not in code:
+            continue
+        body = None
+        for line in subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", name], cwd=d, check=True, capture_output=True, text=True).stdout.split("\n"):
+            m = re.match(r"^[0-9a-f]+ <(\w+)>:", line)
+            if m:
+                body = out.setdefault(m.group(1), [])
+            else:
+                m = re.match(r"^\t(.*?)\s*// ([0-9A-F]+):", line)
+                if m:
+                    body.append((int(m.group(2), 16), m.group(1)))
+    return out
+
+
+def test_no_flat_accesses(kernels):
+    """After a FLAT load (generic address) only a wait for zero is defined: every address must be known to be global."""
+    seen = 0
+    for name, body in kernels.items():
+        if re.search("woq_gemm_w4_kernel|woq_decode_dq_kernel|woq_decode_kernel|woq_decode_m1_kernel", name):
+            seen += 1
+            assert not [t for _, t in body if t.startswith("flat_")], name
+    assert seen >= 100, seen
