@@ -246,7 +246,8 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
 
   // ---- weights of one K tile: one dwordx4 + one (scale, zero) per row-block and lane.  Symmetric
   // weights carry no zero points: scale bytes are read (and ignored) instead of branching. ----
-  const bool has_z = f.zeros != nullptr;
+  constexpr bool kZeros = !NF4 && !FP8;
+  const bool has_z = kZeros && f.zeros != nullptr;
   const uint8_t* wbase[G4_NTW];
   const uint8_t* sbase[G4_NTW];
   const uint8_t* zbase[G4_NTW];
@@ -267,8 +268,11 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
 #pragma unroll
     for (int t = 0; t < G4_NTW; ++t) {
       s[t] = *(const uint16_t*)(sbase[t] + (uint32_t)(qoff * 2u));
-      const uint8_t zb = *(zbase[t] + qoff);
-      z[t] = has_z ? zb : (uint8_t)(WBITS == 4 ? 8 : 128);  // symmetric: the stored code of zero
+      z[t] = 0;
+      if constexpr (kZeros) {
+        const uint8_t zb = *(zbase[t] + qoff);
+        z[t] = has_z ? zb : (uint8_t)(WBITS == 4 ? 8 : 128);  // symmetric: the stored code of zero
+      }
     }
   };
   auto load_m = [&](int kt, uint32_t (&p)[G4_NTW]) {
@@ -341,9 +345,9 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
   // s_waitcnt immediates (vmcnt in bits 3:0 and 15:14; expcnt 6:4 and lgkmcnt 11:8 left at maximum)
   constexpr int kVmcnt0 = 0x0F70, kLgkmcnt0 = 0xC07F;
   constexpr int kVmcntW = 0x0F70 | (G4_NTW * TPS);  // all but the last loads (one weight stage) have landed
-  // everything older than one whole step of loads (2 NTW parameter loads -- merged: NTW --, XLOADS + NTW * TPS
-  // LDS loads)
-  constexpr int kStepLoads = ((MERGED ? 1 : 2) + TPS) * G4_NTW + G4_XLOADS;
+  // everything older than one whole step of loads (2 NTW parameter loads -- one dword or no zero points: NTW --,
+  // XLOADS + NTW * TPS LDS loads)
+  constexpr int kStepLoads = ((MERGED || !kZeros ? 1 : 2) + TPS) * G4_NTW + G4_XLOADS;
   static_assert(kStepLoads < 64 && G4_NTW * TPS < 16, "s_waitcnt vmcnt is a 6-bit field");
   constexpr int kVmcntStep = 0x0F70 | (kStepLoads & 15) | ((kStepLoads >> 4) << 14);
 

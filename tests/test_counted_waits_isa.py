@@ -48,3 +48,29 @@ def test_no_flat_accesses(kernels):
             seen += 1
             assert not [t for _, t in body if t.startswith("flat_")], name
     assert seen >= 100, seen
+
+
+def test_prefill_waits_count_no_more_loads_than_a_step_has(kernels):
+    """The prefill kernel's K loop reads a step's packed tiles from LDS after vmcnt(n), n the loads of one whole step: with
+    fewer loads in the compiled loop than n, the wait would let the tiles' own loads be outstanding still."""
+    seen = 0
+    for name, body in kernels.items():
+        if "woq_gemm_w4_kernel" not in name:
+            continue
+        at = {a: i for i, (a, _) in enumerate(body)}
+        loops = []
+        for i, (a, t) in enumerate(body):
+            m = re.match(r"s_c?branch\S* (\d+)", t)
+            if m:
+                off = int(m.group(1))
+                first = at.get(a + 4 + 4 * (off - 65536 if off >= 32768 else off))
+                if first is not None and first < i:
+                    loop = [x for _, x in body[first:i]]
+                    loops.append((sum(x.startswith("v_mfma") for x in loop), -len(loop), loop))
+        mfmas, _, loop = max(loops)
+        loads = sum(x.startswith("global_load") for x in loop)
+        waits = [int(n) for x in loop for n in re.findall(r"^s_waitcnt.*vmcnt\((\d+)\)", x)]
+        assert mfmas >= 32 and waits, name
+        assert max(waits) <= loads, (name, waits, loads)
+        seen += 1
+    assert seen >= 40, seen
