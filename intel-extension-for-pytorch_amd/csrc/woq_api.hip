@@ -335,12 +335,12 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
       return launch_gemm_dense(f, p->dense_bf16, wbits, st, 0);
   }
   if (nf4) {
-    // table lookups instead of the integer decode: the dequantizing decode kernel and the two
+    // table lookups instead of the integer decode: the dequantizing decode kernel, the prefill kernel and the two
     // general kernels carry them
     if (kernel == 0) kernel = decode_dq_applies(f, wbits, regime) ? 7 : (p->M <= 64 ? 1 : 2);
     if (kernel != 1 && kernel != 2 && (kernel < 7 || kernel > 9) && kernel != 13 && kernel != 14 && kernel != 16)
       return set_error("woq_linear: NF4 weights run on kernels 1, 2, 7..9, 13, 14 and 16 only");
-    if (p->force_kernel == 0 && kernel != 7 && p->M > 64 && gemm_w4_applies(f, wbits, regime) && gemm_w4_nf4_faster(f)) kernel = 3;
+    if (p->force_kernel == 0 && kernel != 7 && p->M > 64 && gemm_w4_applies(f, wbits, regime)) kernel = 3;
   }
   if (kernel == 0 && decode_kernel_applies(f, wbits, regime, p->scale_zero_f16x2))
     return launch_decode(f, p->scale_zero_f16x2, st);

@@ -694,15 +694,16 @@ bool gemm_w4_applies(const FpArgs& f, int wbits, int regime) {
   return f.G >= (wbits == 4 ? 32 : 128) && (f.G & (f.G - 1)) == 0;
 }
 
-// NF4 weights above 32 rows: this kernel or the general tiled one.  Measured at K = 4096: 64 x 128 tiles 40 us while they fit
-// one generation (the general kernel: 98 us at M = 77, N = 11008); beyond that 83 us per 256 workgroups of 128 x 256 or 512 of
-// 128 x 128, the general kernel 105 us and 0.22 us per 128 x 128 tile: M = 2048, 4096 -> 11008 247 against 283 us, M = 1024,
-// 4096 -> 14336 165 against 230 us, but M = 1000, 4096 -> 11008 (688 tiles, two generations here) 165 against 155 us.
-bool gemm_w4_nf4_faster(const FpArgs& f) {
+// NF4: 128 x 256 tiles, or 64 x 128 ones.  Measured at K = 4096 (other K in proportion): a generation of 256 wide tiles 83 us;
+// the small tiles, three of which share a CU, 40 / 56 / 72 us up to 256 / 512 / 768, 100 just beyond, then 12 + 0.084 a tile.  Small / wide,
+// us: M = 300, N = 11008 57 / 88, M = 512, N = 14336 101 / 90, M = 1000, N = 14336 162 / 172, M = 2048, N = 4096 105 / 93, N = 28672
+// 602 / 571.  128 x 128 tiles (82 KiB of LDS with the pair table: one a CU) were never the fastest (114, 114, 221, 118, 758 us),
+// nor was the general tiled kernel (113, 113, 233, 118, 659 us).
+static bool nf4_wide_tiles(const FpArgs& f) {
   auto wgs = [&](int bm, int bn) { return ((f.NT * kTileN + bn - 1) / bn) * ((f.M + bm - 1) / bm); };
-  if (wgs(64, 128) <= 256) return true;
-  const int64_t w2 = wgs(128, 128), gens = std::min((wgs(128, 256) + 255) / 256, (w2 + 511) / 512);
-  return 83.0 * (double)gens < std::max(105.0, 0.22 * (double)w2);
+  const int64_t w = wgs(64, 128);
+  const double small = w <= 256 ? 40.0 : w <= 512 ? 56.0 : w <= 768 ? 72.0 : std::max(100.0, 12.0 + 0.084 * (double)w);
+  return 83.0 * (double)((wgs(128, 256) + 255) / 256) < small;
 }
 
 // Even, so that every split starts on buffer 0.
@@ -872,16 +873,12 @@ int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int s
   using ST = G4Shape<16, 3>;
   using S42 = G4Shape<4, 2>;
   if (f.nf4) {
-    // NF4: the 128 x 256, 128 x 128 and 64 x 128 tiles
     if (shape != 0 || splits > 1) return set_error("woq_gemm_w4_kernel: NF4 weights take the automatic shape only");
     const int64_t wgs42 = ((f.NT * kTileN + S42::BN - 1) / S42::BN) * ((f.M + S42::BM - 1) / S42::BM);
 #define WOQ_NF4(S, ...)                                                                    \
   (regime == kRegimeF16 ? launch_shape<kRegimeF16, S, 4, false, true>(f, g_shift, st, ##__VA_ARGS__) \
                         : launch_shape<kRegimeBF16, S, 4, false, true>(f, g_shift, st, ##__VA_ARGS__))
-    if (wgs42 <= 256) return WOQ_NF4(S42, pick_splits(f, 4, wgs42, scratch), scratch);
-    const int64_t wgs4 = ((f.NT * kTileN + S4::BN - 1) / S4::BN) * ((f.M + S4::BM - 1) / S4::BM);
-    const int64_t wgs2 = ((f.NT * kTileN + S2::BN - 1) / S2::BN) * ((f.M + S2::BM - 1) / S2::BM);
-    return (wgs4 + 255) / 256 < (wgs2 + 511) / 512 ? WOQ_NF4(S4) : WOQ_NF4(S2);  // (two 128 x 128 tiles share a CU)
+    return nf4_wide_tiles(f) ? WOQ_NF4(S4) : WOQ_NF4(S42, pick_splits(f, 4, wgs42, scratch), scratch);
 #undef WOQ_NF4
   }
   if (wbits == 8) {

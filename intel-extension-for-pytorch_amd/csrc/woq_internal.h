@@ -151,7 +151,6 @@ int launch_gemm(const FpArgs& a, int wbits, int regime, hipStream_t st);
 // Prefill GEMM with register-resident dequantization (woq_gemm_w4.hip): 4-bit integer weights, or
 // 8-bit weights with one scale per channel or per group of at least 128
 bool gemm_w4_applies(const FpArgs& f, int wbits, int regime);
-bool gemm_w4_nf4_faster(const FpArgs& f);  // ... than the general tiled kernel, on a problem it takes
 // shape: row-blocks per wave (7, 4 or 2: 448, 256 or 128 columns per workgroup), 163 / 42 = 256 x 192 /
 // 64 x 128 tiles, 0 = by cost model; 8-bit weights: 4, 2, 42 or 0
 // splits: workgroups that share the K steps of a tile (64 x 128 shape only; 2 or 4 need the scratch),

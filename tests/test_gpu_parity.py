@@ -1046,9 +1046,10 @@ def test_nf4_dequant_weight_bit_exact_and_pack_roundtrip(cuda, G):
     assert torch.equal(k.unpack_weight(ctx.at_weight_, 3, 80, 512).cpu(), case["qweight"])
 
 
-@pytest.mark.parametrize("M,K,N,G", [(65, 128, 80, 64), (77, 1024, 528, 32), (128, 4096, 272, -1), (129, 512, 4112, 128), (300, 256, 11008, 64)])
+@pytest.mark.parametrize("M,K,N,G", [(65, 128, 80, 64), (77, 1024, 528, 32), (128, 4096, 272, -1), (129, 512, 4112, 128), (300, 256, 11008, 64),
+                                     (1000, 256, 6288, 64), (515, 128, 13008, 32)])  # (the last two: 128 x 256 tiles)
 def test_nf4_prefill_kernel(cuda, M, K, N, G):
-    """NF4 codes through the pair table in the register-dequantizing kernel: 64 x 128 tiles (with K split), 128 x 128 tiles."""
+    """NF4 codes through the pair table in the register-dequantizing kernel: 64 x 128 tiles (with K split), 128 x 256 tiles."""
     case = _synthetic().make_nf4_case(26, M, K, N, G, bias=True)
     _check_fp(case, O.LOWP_BF16, cols=np.arange(0, N, 7) if N > 512 else None, label=f"nf4 prefill M={M} K={K} N={N} G={G}")
     assert _lib_last_kernel() == "woq_gemm_w4_kernel"
