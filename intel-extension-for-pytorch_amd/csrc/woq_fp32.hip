@@ -9,10 +9,14 @@
 //
 // y[M, N] = x[M, K] * w[N, K]^T on v_mfma_f32_32x32x2_f32: workgroup tile 128 x 128, K step 32,
 // 4 waves in a 2 x 2 grid, each owning 64 x 64 as 2 x 2 MFMA tiles (A = activations, B = weights:
-// a lane's accumulator registers hold consecutive rows of its own output column).  Weights are dequantized once per workgroup and K step into LDS.  One MFMA consumes the K pair (2t, 2t + 1),
+// a lane's accumulator registers hold consecutive rows of its own output column); up to 64 rows
+// (SMALL) the tile is 32 x 128 and a wave owns one 32 x 32 MFMA tile, a quarter of the MFMA work
+// per K step.  Weights are dequantized once per workgroup and K step into LDS.  One MFMA consumes the K pair (2t, 2t + 1),
 // lanes 0..31 the even element and lanes 32..63 the odd one; both LDS tiles keep the even elements
 // of a row in floats 0..15 and the odd ones in floats 16..31, so that a lane reads the operands of
 // four MFMAs with one 16-byte load.
+#include <algorithm>
+
 #include "woq_common.h"
 #include "woq_internal.h"
 
@@ -23,22 +27,22 @@ constexpr int F_BM = 128, F_BN = 128, F_BK = 32;
 constexpr int F_STRIDE = F_BK + 4;  // floats; keeps 16-byte alignment, spreads rows over the banks
 }  // namespace
 
-template <int WBITS, bool NF4>
+template <int WBITS, bool NF4, bool SMALL>
 __global__ __launch_bounds__(256) void woq_fp32_kernel(const Fp32Args f) {
   static_assert(!NF4 || WBITS == 4, "NF4 codes are 4 bits wide");
   constexpr int TK = WBITS == 4 ? kTileK4 : kTileK8;
-  constexpr int BM = F_BM;
+  constexpr int BM = SMALL ? 32 : F_BM;
   constexpr int XI = BM / 32;         // 16-byte activation pieces per thread and K step
-  constexpr int TM = 2;               // MFMA tiles per wave along M and N
-  constexpr int TN = 2;
+  constexpr int TM = SMALL ? 1 : 2;   // MFMA tiles per wave along M and N
+  constexpr int TN = SMALL ? 1 : 2;
   __shared__ __align__(16) float sA[BM * F_STRIDE];
   __shared__ __align__(16) float sB[F_BN * F_STRIDE];
   __shared__ float sTab[16];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const int row0 = (wave >> 1) * 64;  // first row / column of this wave
-  const int col0 = (wave & 1) * 64;
+  const int row0 = SMALL ? 0 : (wave >> 1) * 64;             // first row / column of this wave
+  const int col0 = SMALL ? wave * 32 : (wave & 1) * 64;
   const int64_t m0 = (int64_t)blockIdx.y * BM;
   const int64_t n0 = (int64_t)blockIdx.x * F_BN;
   const int64_t nt0 = n0 / kTileN;
@@ -189,12 +193,11 @@ __global__ __launch_bounds__(256) void woq_fp32_kernel(const Fp32Args f) {
 // A 16-row MFMA would spend three quarters of its time on absent rows (9 us of fp32 matrix work at 4096 -> 11008
 // against 2.3 us).
 // Bound: HBM and the launch up to four rows, the fp32 matrix pipes from 16 rows (16 rows, 4096 -> 11008: 9.2 us at 157 TFLOP/s).
-// Against the tiles of 32 / 128 x 128 outputs below, whose workgroups (86 at N = 11008) go through K alone with two barriers
-// every 32 values (us, INT8 per channel): 4096 -> 11008 M = 1 / 4 / 16 / 64 / 128: 16.4 / 17.3 / 25.5 / 64 / 123 against
-// 223 / 224 / 223 / 223 / 521; 4096 -> 28672: 32 / 33 / 51 / 153 / 297 against 225 / 226 / 226 / 254 / 570;
-// 14336 -> 1024: 18 / 29 / 34 / 107 / 108 against 665 / 691 / 700 / 712 / 1777.  128 rows (two workgroups along M) is where
-// the measurements end; beyond it the weights would be dequantized a third time.  Error against 64 bits 2e-7 .. 8e-7 in the
-// 2-norm (one chain over all of K: 1.1e-6 .. 2.2e-6).
+// Against the tiles of 32 / 128 x 128 outputs above, whose workgroups (86 at N = 11008) go through K alone with two barriers
+// every 32 values (us, INT8 per channel): 4096 -> 11008 M = 1 / 4 / 16 / 64 / 128 / 512 / 2048: 16.4 / 17.3 / 25.5 / 64 / 123 / 446 /
+// 1630 against 223 / 224 / 223 / 223 / 502 / 728 / 1868; 14336 -> 1024, M = 64 / 128 / 2048: 107 / 108 / 479 against 700 / 1761 / 1772.
+// The tiles win where K is short (fp32_few_rows).  Error against 64 bits 2e-7 .. 8e-7 in the 2-norm (one chain over all of K:
+// 1.1e-6 .. 2.2e-6).
 enum { kFmtInt8, kFmtFp8, kFmtInt4, kFmtNf4 };
 
 template <int RT, int NTW>
@@ -366,20 +369,25 @@ void woq_fp32_decode_kernel(const Fp32Args f) {
   }
 }
 
-template <int FMT, int RT>
-static void launch_fp32_decode_rows(const Fp32Args& f, unsigned gy, hipStream_t st) {
-  // row-blocks per workgroup: the shortest schedule, generations of 256 workgroups times a workgroup's length (its
-  // row-blocks and about half a one for the activations), ties to the larger count
+// Row-blocks per workgroup: the shortest schedule, generations of 256 workgroups times a workgroup's length (its
+// row-blocks and about half a one for the activations), ties to the larger count.
+static int fp32_decode_ntw(int64_t NT, int64_t gy) {
   int best = 1;
   double best_cost = 1e300;
   for (int n = 1; n <= 4; ++n) {
-    const int64_t wg = (f.NT + n - 1) / n * gy;
+    const int64_t wg = (NT + n - 1) / n * gy;
     const double cost = (double)((wg + 255) / 256) * (n + 0.5);
     if (cost <= best_cost) { best = n; best_cost = cost; }
   }
-  const dim3 grid((unsigned)((f.NT + best - 1) / best), gy);
+  return best;
+}
+
+template <int FMT, int RT>
+static void launch_fp32_decode_rows(const Fp32Args& f, unsigned gy, hipStream_t st) {
+  const int ntw = fp32_decode_ntw(f.NT, gy);
+  const dim3 grid((unsigned)((f.NT + ntw - 1) / ntw), gy);
 #define WOQ_FP32_DECODE(N) woq_fp32_decode_kernel<FMT, RT, N><<<grid, Fp32Decode<RT, N>::kWaves * 64, 0, st>>>(f)
-  switch (best) {
+  switch (ntw) {
     case 1: WOQ_FP32_DECODE(1); break;
     case 2: WOQ_FP32_DECODE(2); break;
     case 3: WOQ_FP32_DECODE(3); break;
@@ -400,23 +408,58 @@ static void launch_fp32_decode(const Fp32Args& f, hipStream_t st) {
   }
 }
 
+// The kernel for few rows or the tiles: the shorter of two estimates (us).
+// Few rows: generations of 256 workgroups, each a fixed part and its MFMAs, 0.00103 us a K value and accumulator tile (eight
+// waves), but at least one wave's way through one K tile (64 or, 4-bit, 128 K values); rows that are no multiple of 16 bytes are read value by value (1.75
+// times).  Tiles: 8 + 0.115 K while they fit the chip once (SMALL: 5 + 0.05 K up to twice), 8 + 0.08 K per 256 of them beyond;
+// 4-bit weights less.
+// Measured few rows / tiles: K = 64, N = 16384, M = 64 12 / 9; K = 128, N = 65536, M = 32 / 64 / 128 25 / 46 / 88 against 15 / 22 / 46;
+// N = 16384, M = 512: K = 256 98 / 71, 512 131 / 117, 1024 197 / 208, 2048 330 / 387; M = 4096: K = 1024 1512 / 1489, 2048 2604 / 2795;
+// INT4 K = 256, M = 64 19 / 15, K = 1024, M = 512 209 / 195; 4090 -> 11000, M = 129 / 512 / 2048: 239 / 755 / 2757 against 464 / 720 / 2022; 512 -> 32,
+// M = 8192 13 / 59; 4096 -> 11008, M = 8192 6385 / 6868.
+static bool fp32_few_rows(const Fp32Args& f, int wbits) {
+  // (its group index is 32 bits wide, its row blocks are a grid dimension)
+  if (f.KT * kTileK4 >= (1ll << 31) || f.M > 64 * 65535) return false;
+  if (f.M <= 4) return true;
+  const double K = (double)f.K, thin = wbits == 4 ? 0.85 : 1.0;
+  const int64_t tiles16 = (f.M + 15) / 16, gy = (tiles16 + 3) / 4, rt = (tiles16 + gy - 1) / gy;
+  const int64_t ntw = fp32_decode_ntw(f.NT, gy);
+  const double u = (double)(rt * ntw), gens = (double)(((f.NT + ntw - 1) / ntw * gy + 255) / 256);
+  const double few = gens * (2.7 + 0.27 * u + u * std::max(wbits == 4 ? 0.6 : 0.26, 0.00103 * K) * (f.K % 4 ? 1.75 : 1.0));
+  const int64_t columns = (f.NT * kTileN + F_BN - 1) / F_BN;
+  double tiled;
+  if (f.M <= 64) {
+    const double wgs = (double)(columns * ((f.M + 31) / 32));
+    tiled = (5.0 + 0.05 * thin * K) * std::max(1.0, wgs / 512.0);
+  } else {
+    const double wgs = (double)(columns * ((f.M + F_BM - 1) / F_BM));
+    tiled = std::max(8.0 + 0.115 * thin * K, wgs / 256.0 * (8.0 + 0.08 * thin * K));
+  }
+  return few <= tiled;
+}
+
 int launch_fp32(const Fp32Args& f, int wbits, hipStream_t st) {
   if (f.G <= 0 || f.G % F_BK != 0) return set_error("woq_linear: fp32 compute needs groups that are multiples of 32");
-  // up to 128 rows the kernel for few rows (figures there); its group index is 32 bits wide
-  if (f.M <= 128 && f.KT * kTileK4 < (1ll << 31)) {
+  if (fp32_few_rows(f, wbits)) {
     if (wbits == 8)
       f.fp8 ? launch_fp32_decode<kFmtFp8>(f, st) : launch_fp32_decode<kFmtInt8>(f, st);
     else
       f.nf4 ? launch_fp32_decode<kFmtNf4>(f, st) : launch_fp32_decode<kFmtInt4>(f, st);
     return check_launch("woq_fp32_decode_kernel");
   }
-  const dim3 grid((unsigned)((f.NT * kTileN + F_BN - 1) / F_BN), (unsigned)((f.M + F_BM - 1) / F_BM));
+  const bool small = f.M <= 64;
+  const int bm = small ? 32 : F_BM;
+  const dim3 grid((unsigned)((f.NT * kTileN + F_BN - 1) / F_BN), (unsigned)((f.M + bm - 1) / bm));
+#define WOQ_FP32(WB, NF)                                          \
+  (small ? woq_fp32_kernel<WB, NF, true><<<grid, 256, 0, st>>>(f) \
+         : woq_fp32_kernel<WB, NF, false><<<grid, 256, 0, st>>>(f))
   if (wbits == 8)
-    woq_fp32_kernel<8, false><<<grid, 256, 0, st>>>(f);
+    WOQ_FP32(8, false);
   else if (f.nf4)
-    woq_fp32_kernel<4, true><<<grid, 256, 0, st>>>(f);
+    WOQ_FP32(4, true);
   else
-    woq_fp32_kernel<4, false><<<grid, 256, 0, st>>>(f);
+    WOQ_FP32(4, false);
+#undef WOQ_FP32
   return check_launch("woq_fp32_kernel");
 }
 

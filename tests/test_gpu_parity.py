@@ -2225,12 +2225,16 @@ def test_fp32_compute(cuda, kind, M, K, N, G, bias):
         # one, two, three and four row tiles, the first and last row of each; more waves than K tiles
         ("int8", 5, 4096, 528, -1), ("int8", 16, 192, 80, -1), ("int4", 17, 1408, 96, 32), ("int8", 32, 1001, 272, -1), ("int4", 33, 512, 4112, 128),
         ("int8", 48, 640, 8224, -1), ("nf4", 49, 512, 272, 64), ("fp8", 64, 1024, 4112, 128), ("int8", 64, 512, 12304, -1),
-        # two workgroups along the rows, and the tiled kernel from 129 rows on
+        # two and more workgroups along the rows
         ("int8", 65, 640, 528, -1), ("int8", 97, 512, 4112, 64), ("int4", 128, 512, 272, 32), ("int8", 129, 512, 272, -1),
+        ("int4", 193, 1024, 528, 64), ("nf4", 321, 512, 80, 32), ("int8", 700, 1001, 272, -1),
+        # a short K on a wide layer: the tiles of 32 and of 128 rows
+        ("int8", 40, 64, 16400, -1), ("int4", 33, 128, 16384, 32), ("fp8", 64, 128, 16400, 128), ("nf4", 64, 128, 16384, 64),
+        ("int8", 300, 64, 8208, -1), ("int4", 130, 128, 16400, 64), ("int8", 257, 100, 8208, -1),
     ],
 )
 def test_fp32_few_rows(cuda, kind, M, K, N, G):
-    """The kernel for few rows against the products in 64 bits; fp32 sums of K terms in any order lie within
+    """The kernel for few rows, and the tiles where K is short, against the products in 64 bits; fp32 sums of K terms in any order lie within
     K * 2^-24 of the terms' absolute sum, and well inside 1e-5 in the 2-norm at these widths."""
     syn = _synthetic()
     if kind == "int8":
@@ -2243,7 +2247,7 @@ def test_fp32_few_rows(cuda, kind, M, K, N, G):
         case = syn.make_int4_case(430, M, K, N, G, bias=True, scale_dtype=torch.float32)
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(431))
     y = make_context(case, O.LOWP_NONE).run(x.cuda()).cpu().numpy()
-    assert _lib_last_kernel() == ("woq_fp32_decode_kernel" if M <= 128 else "woq_fp32_kernel")
+    assert _lib_last_kernel() == ("woq_fp32_kernel" if K <= 128 and N >= 8208 else "woq_fp32_decode_kernel")
     c = case_np(case)
     acc, _ = O.woq_linear_ref(x.numpy(), "fp32", c["qw"], N, K, c["scales"], c["zps"], c["bias"], case["weight_dtype"], G, "fp32")
     assert rel_l2(y, acc) <= 1e-5
