@@ -194,6 +194,13 @@ int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_
   return decode || prefill ? woq_hip_linear_split_k_workspace_bytes(M, N) : 0;
 }
 
+// Operand i of the post-op, null where the post-op has none: a caller's parameter struct may hold another call's pointers,
+// to other shapes or freed memory, and the kernels request the operands they are given before they look at the post-op.
+static const void* post_op_operand(const woq_hip_linear_params* p, int i) {
+  const bool one = p->fusion == WOQ_HIP_FUSE_ADD || p->fusion == WOQ_HIP_FUSE_MUL, two = p->fusion == WOQ_HIP_FUSE_ADD_ADD;
+  return two || (one && i == 0) ? p->others[i] : nullptr;
+}
+
 int woq_hip_linear(const woq_hip_linear_params* p) {
   if (!p) return set_error("woq_linear: null params");
   if (p->struct_size != sizeof(woq_hip_linear_params))
@@ -269,7 +276,7 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
       a.x = p->x; a.x_dtype = p->x_dtype; a.M = p->M; a.K = p->K; a.N = p->N; a.NT = NT; a.KT = KT;
       a.qweight = (const uint8_t*)p->qweight; a.wbits = wbits; a.scales = p->scales_f32;
       a.zeros = p->zeros_u8; a.G = G; a.KG = KG; a.bias = p->bias; a.act_quant_mode = p->act_quant_mode;
-      a.fusion = p->fusion; a.other0 = p->others[0]; a.other1 = p->others[1]; a.out = p->out;
+      a.fusion = p->fusion; a.other0 = post_op_operand(p, 0); a.other1 = post_op_operand(p, 1); a.out = p->out;
       a.out_dtype = p->out_dtype; a.workspace = p->workspace; a.workspace_bytes = p->workspace_bytes;
       a.split_k_counters = p->split_k_counters;
       a.debug_block_sums = p->debug_block_sums;
@@ -294,7 +301,7 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
     a.x = (const float*)p->x; a.M = p->M; a.K = p->K; a.N = p->N; a.NT = NT; a.KT = KT;
     a.qweight = (const uint8_t*)p->qweight; a.scales = p->scales_f32; a.zeros = p->zeros_u8;
     a.G = G; a.KG = KG; a.bias = p->bias; a.fusion = p->fusion;
-    a.other0 = p->others[0]; a.other1 = p->others[1]; a.out = p->out; a.nf4 = nf4 ? 1 : 0;
+    a.other0 = post_op_operand(p, 0); a.other1 = post_op_operand(p, 1); a.out = p->out; a.nf4 = nf4 ? 1 : 0;
     a.fp8 = fp8 ? 1 : 0;
     return launch_fp32(a, wbits, st);
   } else {
@@ -306,7 +313,7 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
   f.qweight = (const uint8_t*)p->qweight;
   f.scales = (const uint16_t*)(regime == kRegimeF16 ? p->scales_f16 : p->scales_bf16);
   f.zeros = p->zeros_u8; f.G = G; f.KG = KG; f.bias = p->bias; f.fusion = p->fusion;
-  f.other0 = p->others[0]; f.other1 = p->others[1]; f.out = p->out; f.out_dtype = p->out_dtype;
+  f.other0 = post_op_operand(p, 0); f.other1 = post_op_operand(p, 1); f.out = p->out; f.out_dtype = p->out_dtype;
   f.nf4 = nf4 ? 1 : 0;
   f.fp8 = fp8 ? 1 : 0;
   f.szb = (regime == kRegimeBF16 && !nf4 && !fp8) ? p->scale_zero_bf16 : nullptr;
@@ -432,7 +439,7 @@ static int grouped_problem(const woq_hip_linear_params* p, const void* group, in
   f.qweight = nullptr; f.scales = nullptr; f.zeros = nullptr;  // per expert, from the group table
   f.szb = nullptr;
   f.G = G; f.KG = KG; f.bias = nullptr; f.fusion = p->fusion;
-  f.other0 = p->others[0]; f.other1 = nullptr; f.out = p->out; f.out_dtype = p->out_dtype;
+  f.other0 = post_op_operand(p, 0); f.other1 = nullptr; f.out = p->out; f.out_dtype = p->out_dtype;
   f.nf4 = 0; f.fp8 = 0;
   return 0;
 }

@@ -1079,6 +1079,34 @@ def test_prefill_kernel_post_ops_four_columns_at_a_time(cuda, M, N, shape, dtype
         assert torch.allclose(run(fusion=fusion).float(), f(base.float()), rtol=eps, atol=1e-6)
 
 
+@pytest.mark.parametrize("M", [1, 16, 40, 200])
+@pytest.mark.parametrize("post_op", ["NONE", "GELU_ERF", "GELU_TANH", "RELU", "SILU", "ADD", "MUL"])
+def test_operands_that_a_post_op_does_not_have_are_not_read(cuda, M, post_op):
+    """A parameter struct that still holds the operands of an earlier, smaller call (here 8 bytes, which a read of M x N would
+    leave at once)."""
+    import ctypes
+
+    from ipex_amd import _lib
+
+    K, N = 256, 272
+    case = _synthetic().make_int4_case(29, M, K, N, 128, bias=True)
+    ctx = make_context(case, O.LOWP_BF16)
+    x = case["x"].cuda()
+    stale = torch.full((4,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    other = torch.randn(M, N, generator=torch.Generator().manual_seed(30)).to(torch.bfloat16).cuda()
+    code = getattr(_lib, "FUSE_" + post_op)
+    mine = (other,) if post_op in ("ADD", "MUL") else ()
+    want = ctx.run(x, fusion=code, others=mine)
+    p = ctx._tls.plan  # the context's parameter struct, as that call left it
+    out = torch.empty_like(want)
+    p.out = out.data_ptr()
+    p.others[0] = (mine or (stale,))[0].data_ptr()
+    p.others[1] = stale.data_ptr()
+    assert _lib.load().woq_hip_linear(ctypes.byref(p)) == 0
+    p.others[0] = p.others[1] = None
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("M,K,dtype", [(63, 264, torch.bfloat16), (64, 264, torch.bfloat16), (65, 4104, torch.float16), (70, 30, torch.bfloat16),
                                        (64, 32768, torch.bfloat16), (64, 32776, torch.bfloat16), (80, 1000, torch.float32), (3, 16392, torch.float32)])
 def test_shuffle_activations_rows(cuda, M, K, dtype):
