@@ -743,12 +743,11 @@ class _MoeGroupedPlan:
             col = lambda k: torch.tensor([r[k] for r in rows], dtype=torch.int64, device=device)
             self.tables.append(dict(qweight=col(0), s16=col(1), sb16=col(2), z8=col(3) if rows[0][3] else None,
                                     bias=col(4) if rows[0][4] else None, sz=col(12) if rows[0][12] else None))
-        # the single-row decode kernel serves the experts with one row where all three linears have its
-        # (scale, zero) tables: 4-bit weights in groups of 32, 64 or 128 x 2^k, K a multiple of 256
-        self.single_row = all(t["sz"] is not None for t in self.tables) and all(
-            x["wd"] == _lib.DTYPE_INT4 and x["K"] % 256 == 0 and (x["G"] in (32, 64) or (
-                x["G"] % 128 == 0 and (x["G"] // 128) & (x["G"] // 128 - 1) == 0))
-            for x in self.shapes)
+        # linears that the integer-weight decode kernels take: (scale, zero) tables, 4-bit weights in groups of 32, 64 or
+        # 128 x 2^k, K a multiple of 256; the single-row one serves the experts with one row where all three are
+        self.few_rows = [t["sz"] is not None and x["wd"] == _lib.DTYPE_INT4 and x["K"] % 256 == 0 and (x["G"] in (32, 64) or (
+            x["G"] % 128 == 0 and (x["G"] // 128) & (x["G"] // 128 - 1) == 0)) for t, x in zip(self.tables, self.shapes)]
+        self.single_row = all(self.few_rows)
         self.structs = {}
         self.device = device
         self.tiles = None
@@ -922,8 +921,10 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights):
     if f16 != (x.dtype == torch.float16):  # rows must be in the compute type
         return None
     R, N1 = T * topk, plan.shapes[0]["N"]
-    single = plan.single_row and _f16_regime(lowp, x.dtype, 1)
-    split = 5 if (lowp == 2 or single) else 0
+    # an expert of fewer than five rows takes the integer-weight decode kernel in every linear that has one, as its own launches
+    # do: its weights are exact there, and rounded to fp16 in the dequantizing kernel
+    few = [ok and _f16_regime(lowp, x.dtype, 1) for ok in plan.few_rows]
+    split = 5 if (lowp == 2 or any(few)) else 0
     host_ids = topk_ids.detach().to("cpu", torch.int64)
     if int(host_ids.min()) < 0 or int(host_ids.max()) >= experts:
         raise RuntimeError(f"torch_ipex::deepseek_moe_woq: expert ids must lie in [0, {experts})")
@@ -962,7 +963,7 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights):
                 if not used[cls]:
                     continue
                 p.M = bound
-                sz = cls == 0 and single
+                sz = cls == 0 and few[li]
                 p.scale_zero_f16x2 = plan.tables[li]["sz"].data_ptr() if sz else None
                 g = plan.group_struct(li, cls, _f16_regime(lowp, x.dtype, bound), gather, sz, tiles=True)
                 if cls == 3:

@@ -1067,6 +1067,26 @@ def test_deepseek_moe_prompts_have_the_bits_of_the_experts_own_launches(cuda, mo
     assert torch.equal(op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False), want)
 
 
+@pytest.mark.parametrize("H,I,lowp,G", [(512, 384, "BF16", 64), (384, 512, "BF16", 128), (512, 512, "BF16", 32), (512, 384, "FP16", 32)])
+def test_deepseek_moe_prompt_experts_of_two_to_four_rows(cuda, monkeypatch, H, I, lowp, G):
+    """... run the integer-weight decode kernel in the linears that have it (K a multiple of 256), as their own launches do,
+    whatever the layer's other linears have: bit for bit the per-expert path, which rounds no weight there."""
+    ipex = _ipex()
+    T, E, topk = 75, 6, 2
+    mk = lambda k, n, s: _woq_module(ipex, k, n, "INT4", G, lowp, bias=False, seed=s)._op_context
+    ctxs = [[mk(H, I, 800 + e) for e in range(E)], [mk(H, I, 810 + e) for e in range(E)], [mk(I, H, 820 + e) for e in range(E)]]
+    g = torch.Generator().manual_seed(I)
+    xdt = torch.float16 if lowp == "FP16" else torch.bfloat16
+    hidden = torch.randn(T, H, generator=g).to(xdt).to(cuda)
+    ids = torch.stack([torch.zeros(T, dtype=torch.long), torch.tensor([1] * 2 + [2] * 3 + [3] * 4 + [5] * 66)], 1).to(cuda)
+    rw = torch.softmax(torch.randn(T, topk, generator=g), -1).to(xdt).to(cuda)
+    op = torch.ops.torch_ipex.deepseek_moe_woq
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
+    want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
+    assert torch.equal(op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False), want)
+
+
 def test_deepseek_moe_threads_on_one_stream(cuda):
     """Layers called from several threads share their stream's routing buffers: every call has the bits it has alone."""
     import threading
