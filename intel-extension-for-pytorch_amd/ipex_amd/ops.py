@@ -818,7 +818,7 @@ def _f16_regime(lowp, x_dtype, rows):
     return lowp == 1 or (lowp == 0 and x_dtype == torch.float16) or (lowp == 2 and rows < _small_batch_threshold())
 
 
-def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, routing_weights):
+def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, routing_weights, host_ids):
     """The layer in five to fourteen launches and, up to 64 tokens, without reading the routing on the host: the routing is sorted on the
     device, every linear runs once per compute type over all experts that have tokens (woq_hip_linear_grouped), and
     the contributions of a token are added in ascending expert order.  Returns None when the layer does not fit
@@ -842,7 +842,7 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     if not plan.ok or plan.shapes[0]["K"] != H:
         return None
     if tiles:
-        return _deepseek_moe_tiles(plan, x, topk_ids, routing_weights) if plan.tiles_ok else None
+        return _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids) if plan.tiles_ok else None
     lowp = plan.shapes[0]["lowp"]
     # experts with fewer than five rows on the integer-weight decode kernels, as woq_hip_linear serves them, where
     # such rows compute in fp16 and the layer has the kernels' tables; those with exactly one row (most of them in a
@@ -910,11 +910,35 @@ def _moe_tile_rows(rows, experts):
     return 128 if rows >= 192 * experts else 64
 
 
-def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights):
+def _moe_expert_launches_faster(shapes, counts):
+    """Prompts for which the per-expert path is the faster one.  ``shapes``: K, N and weight dtype (wd) of the three linears,
+    ``counts``: rows of every expert.
+    One expert with tokens, long K: its own launches split K over workgroups (INT4 g128, one expert, us per expert / in tiles: 14336 -> 4096
+    with 128 / 512 tokens 223 / 277 and 368 / 386, 11008 -> 2048 193 / 240 and 261 / 247, but 8192 -> 4096 209 / 204 and 274 / 270).
+    INT8 experts of many rows: their launches have 128 x 256 tiles, the slots 128 x 128 at most (2 experts 8192 -> 8192, 2048
+    rows each 1969 / 2287, 4096 -> 14336 with 2500 rows 2728 / 2566, with 4096 3692 / 3997; INT4 with 4096 rows 4329 / 3105).
+    Estimates at K = 4096: 69.6 us for 256 tiles of 128 x 256, 0.159 us a tile of 128 x 128; 40 us and 0.015 us a row more
+    for an expert's launches."""
+    active = [n for n in counts if n]
+    if len(active) == 1 and active[0] <= 512 and shapes[0]["K"] > 8192:
+        return True
+    if any(s["wd"] != _lib.DTYPE_INT8 for s in shapes) or sum(active) < 768 * len(active):
+        return False
+    tiles = own = 0.0
+    for n in active:
+        rows = -(-n // 128)
+        own += 40.0 + 0.015 * n
+        for s in shapes:
+            tiles += 0.159 * rows * -(-s["N"] // 128) * s["K"] / 4096
+            own += 69.6 * -(-rows * -(-s["N"] // 256) // 256) * s["K"] / 4096
+    return own < tiles
+
+
+def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids):
     """The layer for prompts (more than 64 tokens): the routed rows of all experts in row tiles of the prefill kernel, one
     launch per linear (woq_hip_linear_grouped_tiles), with the bits of the experts' own launches; experts with at most 64
-    rows on the decode kernels as above.  The routing is read on the host to refuse ids that name no
-    expert, as the per-expert path does, and says which of the size classes are empty."""
+    rows on the decode kernels as above.  The routing is read on the host to refuse ids that name no expert, as the
+    per-expert path does, and says which of the size classes are empty.  None where the per-expert path is the faster one."""
     T, H = x.shape
     topk, experts, lowp = topk_ids.shape[1], plan.S, plan.shapes[0]["lowp"]
     f16 = _f16_regime(lowp, x.dtype, 64)
@@ -925,10 +949,12 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights):
     # do: its weights are exact there, and rounded to fp16 in the dequantizing kernel
     few = [ok and _f16_regime(lowp, x.dtype, 1) for ok in plan.few_rows]
     split = 5 if (lowp == 2 or any(few)) else 0
-    host_ids = topk_ids.detach().to("cpu", torch.int64)
-    if int(host_ids.min()) < 0 or int(host_ids.max()) >= experts:
+    read = host_ids()
+    if int(read.min()) < 0 or int(read.max()) >= experts:
         raise RuntimeError(f"torch_ipex::deepseek_moe_woq: expert ids must lie in [0, {experts})")
-    counts = torch.bincount(host_ids.reshape(-1), minlength=experts).tolist()
+    counts = torch.bincount(read.reshape(-1), minlength=experts).tolist()
+    if _moe_expert_launches_faster(plan.shapes, counts):
+        return None
     chained = any(64 < n <= plan.chained_rows for n in counts)
     rows = 64 if chained else _moe_tile_rows(R, experts)
     used = [0, 0, 0, 0]  # slots of each size class
@@ -987,12 +1013,19 @@ def deepseek_moe_woq(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, routin
     num_experts = len(gate_ctx)
     if len(up_ctx) != num_experts or len(down_ctx) != num_experts:
         raise RuntimeError("torch_ipex::deepseek_moe_woq: gate / up / down lists differ in length")
+    read = []
+
+    def host_ids():  # (read once, by whichever path needs them)
+        if not read:
+            read.append(topk_ids.detach().to("cpu", torch.int64))
+        return read[0]
+
     if topk_ids.numel() and os.environ.get("IPEX_AMD_MOE_GROUPED", "1") != "0":
-        grouped = _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, routing_weights)
+        grouped = _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, routing_weights, host_ids)
         if grouped is not None:
             return grouped
     output = torch.zeros_like(hidden_states)
-    ids = topk_ids.detach().to("cpu", torch.int64)
+    ids = host_ids()
     if ids.numel() == 0:
         return output
     if int(ids.min()) < 0 or int(ids.max()) >= num_experts:

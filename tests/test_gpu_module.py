@@ -1034,10 +1034,10 @@ def test_deepseek_moe_prompts_in_row_tiles(cuda, monkeypatch, T, E, topk, tile, 
 
 
 @pytest.mark.parametrize("H,I,T,weight_dtype,G", [
-    (4096, 144, 200, "INT4", 128),   # gate / up: two chains of 16 K steps
-    (4352, 272, 333, "INT4", 32),    # 34 K steps: chains of 18 and 16
-    (8192, 144, 65, "INT4", -1),     # four chains; one row in the last tile
-    (8320, 2064, 300, "INT4", 128),  # 65 K steps in two chains, 17 column tiles
+    (4096, 128, 200, "INT4", 128),   # gate / up: two chains of 16 K steps
+    (4352, 384, 333, "INT4", 32),    # 34 K steps: chains of 18 and 16
+    (8192, 128, 65, "INT4", -1),     # four chains; one row in the last tile
+    (8320, 2176, 300, "INT4", 128),  # 65 K steps in two chains, 17 column tiles
     (4096, 4352, 90, "INT8", -1),    # down split, 34 columns tiles of gate / up not
     (128, 8192, 129, "INT8", 128),   # down in four chains
     (4096, 2048, 1100, "INT4", 128),  # more rows than a split launch takes in expert 0, tiles of 64
@@ -1047,6 +1047,8 @@ def test_deepseek_moe_prompts_in_row_tiles(cuda, monkeypatch, T, E, topk, tile, 
 def test_deepseek_moe_prompts_have_the_bits_of_the_experts_own_launches(cuda, monkeypatch, H, I, T, weight_dtype, G):
     """Experts of more than 64 rows, on layers whose expert launches split K over workgroups: the grouped launch adds the same
     partial sums in the same order, so the layer gives the same bits on both paths."""
+    from ipex_amd import _lib
+
     ipex = _ipex()
     E, topk = 3, 2
     mk = lambda k, n, s: _woq_module(ipex, k, n, weight_dtype, G, "BF16", bias=True, seed=s)._op_context
@@ -1064,13 +1066,17 @@ def test_deepseek_moe_prompts_have_the_bits_of_the_experts_own_launches(cuda, mo
     monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
     want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
     monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
-    assert torch.equal(op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False), want)
+    got = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    assert _lib.last_kernel() == "moe_combine_rows"
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("H,I,lowp,G", [(512, 384, "BF16", 64), (384, 512, "BF16", 128), (512, 512, "BF16", 32), (512, 384, "FP16", 32)])
 def test_deepseek_moe_prompt_experts_of_two_to_four_rows(cuda, monkeypatch, H, I, lowp, G):
     """... run the integer-weight decode kernel in the linears that have it (K a multiple of 256), as their own launches do,
     whatever the layer's other linears have: bit for bit the per-expert path, which rounds no weight there."""
+    from ipex_amd import _lib
+
     ipex = _ipex()
     T, E, topk = 75, 6, 2
     mk = lambda k, n, s: _woq_module(ipex, k, n, "INT4", G, lowp, bias=False, seed=s)._op_context
@@ -1084,7 +1090,30 @@ def test_deepseek_moe_prompt_experts_of_two_to_four_rows(cuda, monkeypatch, H, I
     monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
     want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
     monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
-    assert torch.equal(op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False), want)
+    got = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    assert _lib.last_kernel() == "moe_combine_rows"
+    assert torch.equal(got, want)
+
+
+def test_deepseek_moe_prompt_of_one_expert_with_a_long_k(cuda):
+    """... runs the expert's own launches (which split K over workgroups); with a second expert the tiles: same bits."""
+    from ipex_amd import _lib
+
+    ipex = _ipex()
+    H, I, T = 8320, 256, 100
+    mk = lambda k, n, s: _woq_module(ipex, k, n, "INT4", 128, "BF16", bias=False, seed=s)._op_context
+    ctxs = [[mk(H, I, 830 + e) for e in range(2)], [mk(H, I, 840 + e) for e in range(2)], [mk(I, H, 850 + e) for e in range(2)]]
+    g = torch.Generator().manual_seed(1)
+    hidden = torch.randn(T, H, generator=g).to(torch.bfloat16).to(cuda)
+    one = torch.ones(T, 1, dtype=torch.long, device=cuda)
+    op = torch.ops.torch_ipex.deepseek_moe_woq
+    got = op(hidden, one, ctxs[0], ctxs[1], ctxs[2], one.to(torch.bfloat16), False)
+    assert _lib.last_kernel() != "moe_combine_rows"
+    both = torch.cat([one, one - 1], 1)
+    rw = torch.tensor([1.0, 0.0], dtype=torch.bfloat16, device=cuda).expand(T, 2).contiguous()
+    want = op(hidden, both, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    assert _lib.last_kernel() == "moe_combine_rows"
+    assert torch.equal(got, want)
 
 
 def test_deepseek_moe_threads_on_one_stream(cuda):

@@ -365,3 +365,19 @@ def test_environment_knobs_of_the_reference_are_read_by_the_library():
     assert run() == ["5", "64"]
     assert run(IPEX_WOQ_SMALL_BATCH_THRESHOLD="9", IPEX_WOQ_WEIGHT_CACHE_BATCH_THRESHOLD="256") == ["9", "256"]
     assert run(IPEX_WOQ_SMALL_BATCH_THRESHOLD="many", IPEX_WOQ_WEIGHT_CACHE_BATCH_THRESHOLD="-3") == ["5", "64"]
+
+
+def test_moe_prompts_that_stay_on_the_experts_own_launches():
+    """The rule at measured points (own launches against tiles, us)."""
+    from ipex_amd import _lib, ops
+
+    def own(H, I, wd, counts):
+        return ops._moe_expert_launches_faster([dict(K=H, N=I, wd=wd), dict(K=H, N=I, wd=wd), dict(K=I, N=H, wd=wd)], counts)
+
+    i4, i8 = _lib.DTYPE_INT4, _lib.DTYPE_INT8
+    assert own(14336, 4096, i4, [0, 128, 0]) and own(11008, 2048, i8, [256])  # 223 / 277, 193 / 240
+    assert not own(14336, 4096, i4, [768]) and not own(8192, 4096, i4, [128])  # 482 / 432, 209 / 204
+    assert not own(14336, 4096, i4, [128, 128])  # 369 / 291
+    assert own(4096, 14336, i8, [4096, 4096]) and own(8192, 8192, i8, [2048, 2048])  # 3692 / 3997, 1969 / 2287
+    assert not own(4096, 14336, i8, [2500, 2500]) and not own(4096, 4096, i8, [4096, 4096])  # 2728 / 2566, 1291 / 1264
+    assert not own(4096, 14336, i4, [4096, 4096])  # 4329 / 3105
