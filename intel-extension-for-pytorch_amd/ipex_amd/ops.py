@@ -687,8 +687,14 @@ _MOE_PLAN_LIMIT = 128
 # by all layers of those widths (calls on one stream follow each other).
 _MOE_ROWS = {}
 # Threads that share a stream share those buffers too: a layer's launches are queued as a whole, never between those of
-# another thread's layer (whose routing would name other slots and more rows than this call's buffers hold).
-_moe_launch_lock = threading.Lock()
+# another thread's layer (whose routing would name other slots and more rows than this call's buffers hold).  One lock for
+# each (device, stream): layers on other streams share nothing and do not wait.
+_moe_launch_locks = {}
+
+
+def _moe_launch_lock(device_index, stream):
+    key = (device_index, stream)
+    return _moe_launch_locks.get(key) or _moe_launch_locks.setdefault(key, threading.Lock())
 
 
 def _context_epochs():
@@ -842,7 +848,7 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     if not plan.ok or plan.shapes[0]["K"] != H:
         return None
     if tiles:
-        return _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids) if plan.tiles_ok else None
+        return _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids, raw_stream) if plan.tiles_ok else None
     lowp = plan.shapes[0]["lowp"]
     # experts with fewer than five rows on the integer-weight decode kernels, as woq_hip_linear serves them, where
     # such rows compute in fp16 and the layer has the kernels' tables; those with exactly one row (most of them in a
@@ -871,7 +877,7 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     N1 = plan.shapes[0]["N"]
     out = torch.empty_like(x)
     code = _kernels._ACT_CODE[x.dtype]
-    with _moe_launch_lock, torch.cuda.device(x.device):
+    with _moe_launch_lock(x.device.index, raw_stream), torch.cuda.device(x.device):
         act, inter, y = plan.buffers(x.dtype, raw_stream)  # calls on one stream follow each other
         stream = _kernels._stream()
         _lib.check(lib.woq_hip_moe_route(ids.data_ptr(), T, topk, len(gate_ctx), split, 16, 2 if each else int(single), plan.S,
@@ -934,7 +940,7 @@ def _moe_expert_launches_faster(shapes, counts):
     return own < tiles
 
 
-def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids):
+def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids, raw_stream):
     """The layer for prompts (more than 64 tokens): the routed rows of all experts in row tiles of the prefill kernel, one
     launch per linear (woq_hip_linear_grouped_tiles), with the bits of the experts' own launches; experts with at most 64
     rows on the decode kernels as above.  The routing is read on the host to refuse ids that name no expert, as the
@@ -965,7 +971,7 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids):
     ids = topk_ids.to(torch.int64).contiguous()
     rw = routing_weights.contiguous()
     code = _kernels._ACT_CODE[x.dtype]
-    with _moe_launch_lock, torch.cuda.device(x.device):
+    with _moe_launch_lock(x.device.index, raw_stream), torch.cuda.device(x.device):
         buf = plan.tile_routing()
         stream = _kernels._stream()
         out = torch.empty_like(x)

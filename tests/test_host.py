@@ -381,3 +381,15 @@ def test_moe_prompts_that_stay_on_the_experts_own_launches():
     assert own(4096, 14336, i8, [4096, 4096]) and own(8192, 8192, i8, [2048, 2048])  # 3692 / 3997, 1969 / 2287
     assert not own(4096, 14336, i8, [2500, 2500]) and not own(4096, 4096, i8, [4096, 4096])  # 2728 / 2566, 1291 / 1264
     assert not own(4096, 14336, i4, [4096, 4096])  # 4329 / 3105
+
+
+def test_moe_layers_on_other_devices_and_streams_do_not_wait_for_each_other():
+    from ipex_amd import ops
+
+    held = ops._moe_launch_lock(0, 1)
+    assert ops._moe_launch_lock(0, 1) is held
+    with held:
+        for other in (ops._moe_launch_lock(0, 2), ops._moe_launch_lock(1, 1)):
+            assert other.acquire(blocking=False)
+            other.release()
+        assert not ops._moe_launch_lock(0, 1).acquire(blocking=False)
