@@ -1033,35 +1033,38 @@ def test_deepseek_moe_prompts_in_row_tiles(cuda, monkeypatch, T, E, topk, tile, 
         op(hidden, bad, ctxs[0], ctxs[1], ctxs[2], rw, False)
 
 
-@pytest.mark.parametrize("H,I,T,weight_dtype,G", [
-    (4096, 128, 200, "INT4", 128),   # gate / up: two chains of 16 K steps
-    (4352, 384, 333, "INT4", 32),    # 34 K steps: chains of 18 and 16
-    (8192, 128, 65, "INT4", -1),     # four chains; one row in the last tile
-    (8320, 2176, 300, "INT4", 128),  # 65 K steps in two chains, 17 column tiles
-    (4096, 4352, 90, "INT8", -1),    # down split, 34 columns tiles of gate / up not
-    (128, 8192, 129, "INT8", 128),   # down in four chains
-    (4096, 2048, 1100, "INT4", 128),  # more rows than a split launch takes in expert 0, tiles of 64
-    (4096, 14336, 600, "INT4", 128),  # gate and up wide: one chain
-    (4096, 8192, 2500, "INT4", 64),  # every expert beyond the split: tiles of 128
+@pytest.mark.parametrize("H,I,T,weight_dtype,G,lowp", [
+    (4096, 128, 200, "INT4", 128, "BF16"),   # gate / up: two chains of 16 K steps
+    (4352, 384, 333, "INT4", 32, "BF16"),    # 34 K steps: chains of 18 and 16
+    (8192, 128, 65, "INT4", -1, "BF16"),     # four chains; one row in the last tile
+    (8320, 2176, 300, "INT4", 128, "BF16"),  # 65 K steps in two chains, 17 column tiles
+    (4096, 4352, 90, "INT8", -1, "BF16"),    # down split, 34 columns tiles of gate / up not
+    (128, 8192, 129, "INT8", 128, "BF16"),   # down in four chains
+    (4096, 2048, 1100, "INT4", 128, "BF16"),  # more rows than a split launch takes in expert 0, tiles of 64
+    (4096, 14336, 600, "INT4", 128, "BF16"),  # gate and up wide: one chain
+    (4096, 8192, 2500, "INT4", 64, "BF16"),  # every expert beyond the split: tiles of 128
+    (4096, 128, 200, "INT4", 64, "FP16"),
+    (8192, 128, 65, "INT8", -1, "FP16"),
 ])
-def test_deepseek_moe_prompts_have_the_bits_of_the_experts_own_launches(cuda, monkeypatch, H, I, T, weight_dtype, G):
+def test_deepseek_moe_prompts_have_the_bits_of_the_experts_own_launches(cuda, monkeypatch, H, I, T, weight_dtype, G, lowp):
     """Experts of more than 64 rows, on layers whose expert launches split K over workgroups: the grouped launch adds the same
     partial sums in the same order, so the layer gives the same bits on both paths."""
     from ipex_amd import _lib
 
     ipex = _ipex()
     E, topk = 3, 2
-    mk = lambda k, n, s: _woq_module(ipex, k, n, weight_dtype, G, "BF16", bias=True, seed=s)._op_context
+    mk = lambda k, n, s: _woq_module(ipex, k, n, weight_dtype, G, lowp, bias=True, seed=s)._op_context
     ctxs = [[mk(H, I, 700 + e) for e in range(E)], [mk(H, I, 710 + e) for e in range(E)], [mk(I, H, 720 + e) for e in range(E)]]
     g = torch.Generator().manual_seed(T)
-    hidden = torch.randn(T, H, generator=g).to(torch.bfloat16).to(cuda)
+    xdt = torch.float16 if lowp == "FP16" else torch.bfloat16
+    hidden = torch.randn(T, H, generator=g).to(xdt).to(cuda)
     ids = torch.tensor([0, 2]).expand(T, topk).contiguous()
     few = 65 if T < 2000 else 900
     ids[: T - few, 1] = 1  # expert 2 has `few` rows, expert 0 all, expert 1 the others (none, or more than 64)
     if T - few <= 64:
         ids[:, 1] = 2
     ids = ids.to(cuda)
-    rw = torch.softmax(torch.randn(T, topk, generator=g), -1).to(torch.bfloat16).to(cuda)
+    rw = torch.softmax(torch.randn(T, topk, generator=g), -1).to(xdt).to(cuda)
     op = torch.ops.torch_ipex.deepseek_moe_woq
     monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
     want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)

@@ -1055,6 +1055,43 @@ def test_nf4_prefill_kernel(cuda, M, K, N, G):
     assert _lib_last_kernel() == "woq_gemm_w4_kernel"
 
 
+@pytest.mark.parametrize("M,K,N,G", [(65, 128, 80, 128), (77, 1024, 528, 32), (300, 256, 1040, 64), (515, 128, 13008, 64)])
+def test_nf4_prefill_kernel_fp16_and_post_ops(cuda, M, K, N, G):
+    """Both tile shapes under fp16 compute (products and sums of 11-bit significands, rounded once more on output), and the
+    post-ops of both compute types, bit for bit those of the rounded output."""
+    from ipex_amd import _lib
+
+    cols = np.arange(0, N, 7) if N > 512 else np.arange(N)
+    g = torch.Generator().manual_seed(N)
+    for lowp, dtype in ((O.LOWP_FP16, torch.float16), (O.LOWP_BF16, torch.bfloat16)):
+        case = _synthetic().make_nf4_case(29, M, K, N, G, bias=True, scale_dtype=dtype)
+        ctx = make_context(case, lowp)
+        x = case["x"].to(dtype)
+        base = ctx.run(x.cuda())
+        assert _lib_last_kernel() == "woq_gemm_w4_kernel"
+        if dtype == torch.float16:
+            c = case_np(case)
+            _, y_ref = O.woq_linear_ref(to_np_f32(x), "fp16", c["qw"][cols], len(cols), K, c["scales"][cols], None, c["bias"][cols], 3, G, "fp16")
+            assert rel_l2(to_np_f32(base)[:, cols], y_ref) <= REL_L2_OUT
+        o1, o2 = (torch.randn(M, N, generator=g).to(dtype).cuda() for _ in range(2))
+        assert torch.equal(ctx.run(x.cuda(), fusion=_lib.FUSE_ADD, others=(o1,)), base + o1)
+        assert torch.equal(ctx.run(x.cuda(), fusion=_lib.FUSE_MUL, others=(o1,)), base * o1)
+        assert torch.equal(ctx.run(x.cuda(), fusion=_lib.FUSE_ADD_ADD, others=(o1, o2)), (base + o1) + o2)
+        assert _lib_last_kernel() == "woq_gemm_w4_kernel"
+
+
+@pytest.mark.parametrize("M,K,N,G", [(65, 128, 80, 32), (128, 512, 272, 64), (200, 1024, 528, 128), (150, 256, 144, -1), (131, 192, 144, 96)])
+def test_nf4_general_kernel(cuda, M, K, N, G):
+    """The general tiled kernel on whole K steps, which the dispatch gives to the prefill kernel now, and on groups that this
+    one does not take."""
+    case = _synthetic().make_nf4_case(30, M, K, N, G, bias=True)
+    _check_fp(case, O.LOWP_BF16, cols=np.arange(0, N, 5), force_kernel=2, label=f"nf4 general M={M} K={K} N={N} G={G}")
+    assert _lib_last_kernel() == "woq_gemm_kernel"
+    if G == 96:
+        _check_fp(case, O.LOWP_BF16, label=f"nf4 M={M} K={K} N={N} G={G}")
+        assert _lib_last_kernel() == "woq_gemm_kernel"
+
+
 @pytest.mark.parametrize("M,N,shape", [(65, 80, 12), (200, 272, 12), (200, 272, 6), (131, 272, 5), (130, 460, 4), (300, 400, 11)])  # (4: 128 x 448, one element a lane)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_prefill_kernel_post_ops_four_columns_at_a_time(cuda, M, N, shape, dtype):
