@@ -419,7 +419,8 @@ int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, in
  * split_lo and split_mid at most 64.  x_row, row_of and slot_of as from woq_hip_moe_route.
  * woq_hip_linear_grouped_tiles runs one linear over the slots of class 3 on the prefill kernel: p as for
  * woq_hip_linear_grouped (M is ignored), INT4 weights with power-of-two groups of at least 32 or INT8 weights with
- * power-of-two groups of at least 128, or per-channel; K a multiple of 128, rows in the compute type of five and more rows.
+ * power-of-two groups of at least 128, or per-channel; K a multiple of 128, rows in the compute type of five and more rows. x with
+ * x_row has at most 2^31 bytes (its row offsets are 32 bits wide; so it is for woq_hip_linear_grouped).
  * With slots of 64 rows an expert whose own launch would split K over workgroups (woq_hip_linear with the scratch that
  * woq_hip_linear_auto_split_k_workspace_bytes asks for) runs the same K ranges one after the other and adds them in that
  * launch's order, so it has that launch's bits; woq_hip_moe_chained_rows: the most rows of such an expert, 0 if there is none

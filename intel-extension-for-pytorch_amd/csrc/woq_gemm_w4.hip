@@ -127,8 +127,8 @@ __device__ __forceinline__ float post_op(float y, int fusion, int act_dtype, flo
 
 // GROUPED (mixture of experts): the row tile of a workgroup is a slot of the routing tables -- at most G4_BM routed rows of
 // one expert, whose tensors come from the group's pointer tables; a slot without an expert ends at once.
-// 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3832 us with three launches per expert (each on 32 to 192 workgroups),
-// 619 us with one launch per linear (three of about 200 us).
+// 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3738 us with three launches per expert (each on 32 to 192 workgroups),
+// 611..643 us with one launch per linear (three of about 200 us).
 // Where an expert's own launch would split K over workgroups (pick_splits), the workgroup runs the same K steps in as many
 // chains, one after the other, and adds them in the same order: the expert has the bits of its own launch.
 // NF4: a dword's eight table values come from the 256-entry table of value pairs in LDS (nf4_dequant), built before the first

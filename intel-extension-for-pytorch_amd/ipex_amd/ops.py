@@ -910,9 +910,11 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
 
 
 def _moe_tile_rows(rows, experts):
-    """Rows of a slot of the prefill kernel: 128 from 192 rows per expert on.  Tiles of 128 rows dequantize half as often, but
-    waste more of an expert's last tile (INT4 g128, us with 64 / 128 rows: 128 rows per expert 794 / 846 and 192 / 234,
-    200 rows 603 / 538, 512 rows 413 / 385; both sides before the epilogue and the routing kernel got faster: the 794 are 619)."""
+    """Rows of a slot of the prefill kernel: 128 from 192 rows per expert on, counting the rows of layers of at least 6144
+    columns only (``rows`` is 0 on the others).  Tiles of 128 rows dequantize half as often, but waste more of an expert's last
+    tile and two instead of three share a CU (8 experts, INT4 g128, us with 64 / 128 rows a tile: 4096 -> 14336 with 320 / 1000 rows per
+    expert 1408 / 1282 and 3606 / 3274, 4096 -> 6144 with 270 / 1000 588 / 568 and 1644 / 1490; 2048 -> 2048 with 200 / 1000 165 / 170
+    and 402 / 413, 3072 -> 1024 with 200 / 1000 142 / 174 and 342 / 359)."""
     return 128 if rows >= 192 * experts else 64
 
 
@@ -962,7 +964,7 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids, raw_stream
     if _moe_expert_launches_faster(plan.shapes, counts):
         return None
     chained = any(64 < n <= plan.chained_rows for n in counts)
-    rows = 64 if chained else _moe_tile_rows(R, experts)
+    rows = 64 if chained else _moe_tile_rows(R if N1 >= 6144 else 0, experts)
     used = [0, 0, 0, 0]  # slots of each size class
     for n in counts:
         if n:
