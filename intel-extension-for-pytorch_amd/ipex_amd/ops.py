@@ -944,8 +944,8 @@ def _moe_expert_launches_faster(shapes, counts):
 
 def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids, raw_stream):
     """The layer for prompts (more than 64 tokens): the routed rows of all experts in row tiles of the prefill kernel, one
-    launch per linear (woq_hip_linear_grouped_tiles), with the bits of the experts' own launches; experts with at most 64
-    rows on the decode kernels as above.  The routing is read on the host to refuse ids that name no expert, as the
+    launch per linear (woq_hip_linear_grouped_tiles), with the bits of the experts' own launches (those from the packed weight);
+    experts with at most 64 rows on the decode kernels as above.  The routing is read on the host to refuse ids that name no expert, as the
     per-expert path does, and says which of the size classes are empty.  None where the per-expert path is the faster one."""
     T, H = x.shape
     topk, experts, lowp = topk_ids.shape[1], plan.S, plan.shapes[0]["lowp"]
