@@ -251,7 +251,7 @@ typedef struct woq_hip_linear_params {
   /* force_kernel: 0 = automatic; 1 = small-M streaming kernel; 2 = tiled MFMA GEMM (any shape);
    * 3 = prefill GEMM with register-resident dequantization (4-bit integer weights, or 8-bit weights with
    * groups of at least 128; K % 128 == 0, power-of-two or per-channel groups, x in the compute dtype),
-   * workgroup shape by cost model; 4 / 5 / 6 = the same kernel with 448 / 256 / 128 columns per workgroup;
+   * workgroup shape and K splits by estimated time; 4 / 5 / 6 = the same kernel with 448 / 256 / 128 columns per workgroup;
    * 7 = dequantizing decode kernel (M <= 64, K % 128 == 0 for 4-bit and K % 64 == 0 for 8-bit weights, x in the
    * compute dtype), 8 / 9 / 10 = the same with one / two / four weight row-blocks per workgroup;
    * 11 / 12 = the same prefill GEMM with 256 rows x 192 columns / 64 rows x 128 columns per workgroup
@@ -277,13 +277,13 @@ int64_t woq_hip_linear_workspace_bytes(int64_t M, int64_t K, int32_t lowp_mode,
                                        int32_t act_quant_mode, int64_t group_size);
 
 /* Scratch bytes that let woq_hip_linear split K across workgroups for M rows and N output columns
- * in the floating-point modes (decode kernel up to 32 rows; prefill GEMM when its 64 x 128 tiles are
- * at most 128); 0 where it never does.  No counterpart in the reference. */
+ * in the floating-point modes (decode kernel up to 32 rows; prefill GEMM from 65 to 1024 rows while its tiles leave
+ * room for a second workgroup each, at most 32 MiB); 0 where it never does.  No counterpart in the reference. */
 int64_t woq_hip_linear_split_k_workspace_bytes(int64_t M, int64_t N);
 
 /* The same size for the problems on which woq_hip_linear shares K between workgroups BY ITSELF (force_kernel 0):
  * few output tiles and a long K -- 5..32 rows with K >= 8192 and N <= 4096 in the floating-point modes, more than
- * 64 rows with K >= 4096 and M * N <= 2^20 in every mode -- and 0 for every other problem, where scratch and
+ * 64 and at most 1024 rows with K >= 4096 (lowp_mode INT8: M * N <= 2^20) -- and 0 for every other problem, where scratch and
  * counters would go unused.  A caller that allocates per call asks this function; there is no second copy of the
  * rule to keep in step.  No counterpart in the reference. */
 int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t lowp_mode);

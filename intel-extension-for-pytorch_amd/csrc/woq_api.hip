@@ -175,10 +175,14 @@ int64_t woq_hip_linear_workspace_bytes(int64_t M, int64_t K, int32_t lowp_mode, 
 int64_t woq_hip_linear_split_k_workspace_bytes(int64_t M, int64_t N) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64) {
-    // prefill GEMM, 64 x 128 tiles, up to four workgroups per tile while the tiles alone fill less than
-    // half of the chip
-    const int64_t tiles = ((M + 63) / 64) * ((woq_hip_padded_n(N) + 127) / 128);
-    return tiles <= 128 ? 4 * tiles * 64 * 128 * (int64_t)sizeof(float) : 0;
+    // prefill GEMM: the most that its plans take -- 64 x 128 tiles on up to three workgroups a CU, 128 x 256 tiles on one
+    if (M > kSplitKPrefillMaxRows) return 0;
+    const int64_t np = woq_hip_padded_n(N);
+    const int64_t t42 = ((M + 63) / 64) * ((np + 127) / 128), t8 = ((M + 127) / 128) * ((np + 255) / 256);
+    const int64_t s42 = 768 / t42 < 4 ? 768 / t42 : 4, s8 = 256 / t8 < 4 ? 256 / t8 : 4;
+    const int64_t b42 = s42 > 1 ? s42 * t42 * 64 * 128 * (int64_t)sizeof(float) : 0;
+    const int64_t b8 = s8 > 1 ? s8 * t8 * 128 * 256 * (int64_t)sizeof(float) : 0;
+    return b42 > b8 ? b42 : b8;
   }
   if (M > 32) return 0;
   const int64_t NT = woq_hip_padded_n(N) / kTileN;
@@ -188,9 +192,9 @@ int64_t woq_hip_linear_split_k_workspace_bytes(int64_t M, int64_t N) {
 
 int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t lowp_mode) {
   const bool int8 = lowp_mode == WOQ_HIP_LOWP_INT8;
-  // the dequantizing decode kernel (launch_decode_dq) and the 64 x 128 tiles of the prefill GEMMs (pick_splits)
+  // the dequantizing decode kernel (launch_decode_dq) and the prefill GEMMs (plan_tiles; lowp_mode INT8: 64 x 128 tiles)
   const bool decode = !int8 && M >= 5 && M <= 32 && K >= 8192 && N <= 4096;
-  const bool prefill = M > 64 && K >= kSplitKPrefillMinK && M * N <= kSplitKPrefillElems;
+  const bool prefill = M > 64 && K >= kSplitKPrefillMinK && (int8 ? M * N <= kSplitKPrefillElems : M <= kSplitKPrefillMaxRows);
   return decode || prefill ? woq_hip_linear_split_k_workspace_bytes(M, N) : 0;
 }
 

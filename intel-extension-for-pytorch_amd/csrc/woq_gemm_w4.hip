@@ -32,24 +32,34 @@
 //     zero point of a (row, group) come as one dword, bf16 scale << 16 | fp16 (1024 + zero), and the two
 //     nibble positions are read as the fp16 numbers 1024 + q and 64 + q, so that one scale serves both:
 //     7 instead of 14 parameter requests and 21 instead of 56 vector instructions per K step and wave
-//     (M = 2048, 4096 -> 14336: 198 against 202-206 us on the same boxes; same bits out).
+//     (M = 2048, 4096 -> 14336: 198 against 202-206 us on the same boxes; same bits out);
+//   * 128 x 256 tiles have eight waves of two row-blocks each (WAVES 8), two on a SIMD: one wave alone issues a vector
+//     instruction every 8.2 clocks, two together one every 4.6 (MFMA with three vector instructions behind it: 30 clocks
+//     alone, 21.4 each with two waves), and 2.5 vector instructions stand beside each MFMA here.  The A fragments of the next
+//     sub-step are then read in all blocks of a sub-step instead of one (SPREAD: with every wave in the same block the LDS
+//     stood still in the others).  Against four waves of four row-blocks, us: INT4 M = 512, 4096 -> 14336 62 / 56, NF4
+//     M = 1000 172 / 126, FP8 M = 2048 329 / 273, INT8 M = 2048, 4096 -> 11008 199 / 180.  What bounds them now is LDS
+//     reads (256 KiB a K step).  Four waves a workgroup with SPREAD were slower (128 x 448 by 5 %, 128 x 128 by 6 %); eight
+//     waves of 128 x 512 91 us a generation but 448 workgroups where 128 x 448 makes 512 (M = 2048, N = 14336: 206 / 204).
 #include <algorithm>
+#include <type_traits>
 
 #include "woq_common.h"
 #include "woq_internal.h"
 
 namespace woq {
 
-constexpr int G4_WAVES = 4;
-template <int MT_, int NTW_>
+template <int MT_, int NTW_, int WAVES_ = 4>
 struct G4Shape {
   static constexpr int MT = MT_;                        // 16-row accumulator tiles
   static constexpr int NTW = NTW_;                      // weight row-blocks (16 columns) per wave
+  static constexpr int WAVES = WAVES_;                  // waves per workgroup
+  static constexpr bool SPLITS = MT * NTW <= 8 || WAVES == 8;  // K may be shared by several workgroups
   static constexpr int BM = 16 * MT;                    // rows per workgroup
-  static constexpr int BN = G4_WAVES * NTW * kTileN;    // columns per workgroup
+  static constexpr int BN = WAVES * NTW * kTileN;       // columns per workgroup
   static constexpr int XBYTES = BM * kTileK4 * 2;       // one activation buffer
-  static constexpr int XLOADS = XBYTES / (G4_WAVES * 1024);  // LDS loads per wave and buffer
-  static constexpr int WSTAGE = G4_WAVES * NTW * kTileBytes;  // one weight stage of 4-bit tiles (8-bit: two)
+  static constexpr int XLOADS = XBYTES / (WAVES * 1024);     // LDS loads per wave and buffer
+  static constexpr int WSTAGE = WAVES * NTW * kTileBytes;    // one weight stage of 4-bit tiles (8-bit: two)
   static constexpr int LDS_BYTES = 2 * XBYTES + 2 * WSTAGE;   // 4-bit weights; lds_bytes() below
   static constexpr int SSTRIDE = NTW * kTileN + 4;      // fp32 row stride of the epilogue staging tile
   // Row-block during whose MFMAs the A fragments of the next K sub-step are read from LDS.  One
@@ -57,6 +67,7 @@ struct G4Shape {
   // a block is long enough (256 cycles) to read them in the last block, each into the registers of
   // the fragment whose last MFMA has just been issued.
   static constexpr int XA_SETS = MT >= 16 ? 1 : 2;
+  static constexpr bool SPREAD = WAVES == 8 && XA_SETS == 2;
   static constexpr int FETCH_T = XA_SETS == 1 ? NTW - 1 : NTW - 2;
 };
 
@@ -73,10 +84,19 @@ __device__ __forceinline__ f4 g4_mfma(u4 a, u4 b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<b8>(a), bitcast<b8>(b), c, 0, 0, 0);
 }
 
+// (eight waves have 256 registers each: accumulators that need not be AGPRs leave the allocator free to place them)
+template <int WAVES>
+__device__ __forceinline__ void g4_opaque(f4& v) {
+  if constexpr (WAVES == 8)
+    asm volatile("" : "+v"(v));
+  else
+    asm volatile("" : "+a"(v));
+}
+
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* global_ptr_t;
 
-// gridDim.z > 1 (small M x N with a long K, where the tiles alone leave most CUs idle): workgroup z
+// gridDim.z > 1 (M x N that leaves CUs or their wave slots idle, see plan_tiles): workgroup z
 // of a tile takes the K steps [z * kts, (z + 1) * kts), writes its accumulators to scratch memory as they
 // lie in the registers, and the workgroup that arrives last at the tile's counter adds the partial
 // tiles in z order (its own from the registers) and runs the epilogue.  Nobody waits; the order of
@@ -129,25 +149,26 @@ __device__ __forceinline__ float post_op(float y, int fusion, int act_dtype, flo
 // one expert, whose tensors come from the group's pointer tables; a slot without an expert ends at once.
 // 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3738 us with three launches per expert (each on 32 to 192 workgroups),
 // 611..643 us with one launch per linear (three of about 200 us).
-// Where an expert's own launch would split K over workgroups (pick_splits), the workgroup runs the same K steps in as many
+// Where an expert's own launch would split K over workgroups (plan_tiles), the workgroup runs the same K steps in as many
 // chains, one after the other, and adds them in the same order: the expert has the bits of its own launch.
 // NF4: a dword's eight table values come from the 256-entry table of value pairs in LDS (nf4_dequant), built before the first
 // request; four 8-byte reads, eight products and four conversions against 17 instructions for integers.
+constexpr int kPrefillSplitMax = 4;  // workgroups that share the K steps of a tile
 struct G4Group {
   const MoeGroup* tables;
-  int rows4, kts4, rows2, kts2;  // experts of at most rows4 / rows2 rows (0: none): chains of kts4 / kts2 K steps
+  int chains[kSplitKPrefillMaxRows / 64 + 1];  // CHAINS: [rows / 64, rounded up] K steps of a chain, 0: one chain
 };
 template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false, bool NF4 = false, bool CHAINS = false>
-__global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const int g_shift, float* const sk_partial,
+__global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs fa, const int g_shift, float* const sk_partial,
                                                           int* const sk_counters, const int kts, const G4Group grp) {
   static_assert(!NF4 || (WBITS == 4 && !FP8 && !MERGED && !GROUPED), "NF4 codes have a table and a scale");
   __shared__ f2 sNf4[NF4 ? kNf4LutEntries : 1];
-  if constexpr (NF4) nf4_fill_lut(sNf4, (int)threadIdx.x, 256);  // (the barrier before the first use is the K loop's first)
+  if constexpr (NF4) nf4_fill_lut(sNf4, (int)threadIdx.x, 64 * S::WAVES);  // (the barrier before the first use is the K loop's first)
   static_assert(!GROUPED || !MERGED, "the pointer tables hold scales and zero points apart");
   static_assert(GROUPED || !CHAINS, "an ungrouped launch splits K over workgroups");
   constexpr int TPS = WBITS / 4;  // packed tiles per row-block and K step of 128
   constexpr int G4_MT = S::MT, G4_NTW = S::NTW, G4_BM = S::BM, G4_XBYTES = S::XBYTES, G4_XLOADS = S::XLOADS,
-                G4_WSTAGE = S::WSTAGE * TPS, G4_SSTRIDE = S::SSTRIDE;
+                G4_WSTAGE = S::WSTAGE * TPS, G4_SSTRIDE = S::SSTRIDE, G4_WAVES = S::WAVES;
   // two activation buffers, then two weight stages of 4 waves x NTW tiles x 1 KiB
   extern __shared__ __align__(1024) uint8_t sX[];
   uint8_t* const sW = sX + 2 * G4_XBYTES;
@@ -165,7 +186,10 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
     const int packed = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_rows)[by]);
     const int rows = packed & 0xFFFF, expert_rows = packed >> 16;  // (0: not known, one chain)
     if constexpr (CHAINS)
-      chain = expert_rows == 0 ? kts : expert_rows <= grp.rows4 ? grp.kts4 : expert_rows <= grp.rows2 ? grp.kts2 : kts;
+      if (expert_rows <= kSplitKPrefillMaxRows) {
+        const int steps = grp.chains[(expert_rows + 63) / 64];
+        chain = steps ? steps : kts;
+      }
     fg = fa;
     fg.M = rows < G4_BM ? rows : G4_BM;
     fg.qweight = dq_uniform((const uint8_t*)dq_uniform(g.qweight)[e]);
@@ -356,7 +380,7 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
   // 10 clocks alone and about 40 when the three other waves issue theirs with it.  The waves therefore meet at the
   // barrier in different blocks of the last sub-step -- wave w in block FETCH_T - w, the same moment for all -- and so
   // reach the fetching block one block apart, in every sub-step (M = 2048, 4096 -> 6144: 92 us against 99 us).
-  constexpr int STAG_MAX = S::XA_SETS == 1 ? (S::FETCH_T < 3 ? S::FETCH_T : 3) : 0;
+  constexpr int STAG_MAX = S::XA_SETS == 1 && G4_WAVES == 4 ? (S::FETCH_T < 3 ? S::FETCH_T : 3) : 0;
   const int bar_t = S::FETCH_T - (wave < STAG_MAX ? wave : STAG_MAX);
   load_x(kt_lo, 0);
   dma_w(kt_lo, 0);
@@ -380,7 +404,7 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
 #pragma unroll
   for (int mt = 0; mt < G4_MT; ++mt)
 #pragma unroll
-    for (int t = 0; t < G4_NTW; ++t) asm volatile("" : "+a"(acc[mt][t]));
+    for (int t = 0; t < G4_NTW; ++t) g4_opaque<G4_WAVES>(acc[mt][t]);
 
   // (the requests of a chain's last steps are the next chain's first ones; -0 + x is x for every x)
   f4 total[CHAINS ? G4_MT : 1][CHAINS ? G4_NTW : 1];
@@ -415,7 +439,8 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
         for (int t = 0; t < G4_NTW; ++t) {
           const int cur = (j * G4_NTW + t) & 1;
           const bool last_t = t == G4_NTW - 1;
-          const bool fetch_t = t == S::FETCH_T;
+          const bool fetch_t = S::SPREAD || t == S::FETCH_T;
+          const bool bar_here = S::SPREAD ? t == 0 : t == S::FETCH_T;
           if (j == 0 && t == 1) {
             // the LDS reads of the previous step's last blocks have returned: their stage is free
             __builtin_amdgcn_s_waitcnt(kLgkmcnt0);
@@ -424,7 +449,7 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
           }
           if (j == 3 && t == 0) __builtin_amdgcn_s_waitcnt(kVmcntStep);  // tiles of step kt + 1 are in LDS
           if constexpr (STAG_MAX == 0) {
-            if (fetch_t && j == 3) {
+            if (bar_here && j == 3) {
               // Written as an instruction, not as the barrier builtin: before that one the compiler
               // waits for every outstanding load, the tiles requested for step kt + 2 included.
               __builtin_amdgcn_s_waitcnt(kVmcntW);
@@ -449,7 +474,7 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
 #pragma unroll
           for (int mt = 0; mt < G4_MT; ++mt) {
             acc[mt][t] = g4_mfma<REGIME>(bop[cur], xa[(j & 1) % S::XA_SETS][mt], acc[mt][t]);
-            if (fetch_t)
+            if (S::SPREAD ? mt * G4_NTW / G4_MT == t : fetch_t)
               xa[((j & 1) ^ 1) % S::XA_SETS][mt] = j == 3 ? *(const u4*)(xsn + mt * 4096 + rd[0])
                                            : *(const u4*)(xs + mt * 4096 + rd[j + 1]);
           }
@@ -458,9 +483,9 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
             for (int u = 0; u < TPS; ++u) wr[t][u] = read_w((kt & 1) ^ 1, t, u);
           }
 #pragma unroll
-          for (int mt = 0; mt < G4_MT; ++mt) {
+          for (int mt = 0; mt < (NF4 && G4_WAVES == 8 ? 0 : G4_MT); ++mt) {  // (NF4 with eight waves: 126 us without, 132 with)
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (fetch_t) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (S::SPREAD ? mt < (t + 1) * G4_MT / G4_NTW - t * G4_MT / G4_NTW : fetch_t) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
           }
           __builtin_amdgcn_sched_barrier(0);
@@ -490,22 +515,25 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
 #pragma unroll
   for (int mt = 0; mt < G4_MT; ++mt)
 #pragma unroll
-    for (int t = 0; t < G4_NTW; ++t) asm volatile("" : "+a"(acc[mt][t]));
+    for (int t = 0; t < G4_NTW; ++t) g4_opaque<G4_WAVES>(acc[mt][t]);
 
-  // (built for the 64 x 128 shape only, the one that is ever launched with gridDim.z > 1: with more
-  // accumulator tiles the second copy of them would not fit the registers)
-  if constexpr (G4_MT * G4_NTW <= 8) if (gridDim.z > 1) {
+  // (built for the shapes that are launched with gridDim.z > 1)
+  if constexpr (S::SPLITS && !GROUPED) if (gridDim.z > 1) {
     const int nsplit = (int)gridDim.z, z = (int)blockIdx.z;
     const int tiles = (int)(gridDim.x * gridDim.y), tile = (int)(blockIdx.y * gridDim.x + blockIdx.x);
     constexpr int kWaveFloats = G4_MT * G4_NTW * 256;
-    float* const mine = sk_partial + ((size_t)(z * tiles + tile) * G4_WAVES + wave) * kWaveFloats + lane * 4;
+    // accumulator pair h of tile (mt, t): 64 lanes x 8 bytes side by side (an access of its four registers one by one, 16 bytes
+    // apart in memory, moved a quarter as much per instruction)
+    auto part = [&](int zz) { return (uint64_t*)(sk_partial + ((size_t)(zz * tiles + tile) * G4_WAVES + wave) * kWaveFloats) + lane; };
+    auto at = [](int mt, int t, int h) { return ((mt * G4_NTW + t) * 2 + h) * 64; };
+    uint64_t* const mine = part(z);
 #pragma unroll
     for (int mt = 0; mt < G4_MT; ++mt)
 #pragma unroll
       for (int t = 0; t < G4_NTW; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          __hip_atomic_store(mine + (mt * G4_NTW + t) * 256 + e, acc[mt][t][e], __ATOMIC_RELAXED,
+        for (int h = 0; h < 2; ++h)
+          __hip_atomic_store(mine + at(mt, t, h), bitcast<uint64_t>(f2{acc[mt][t][2 * h], acc[mt][t][2 * h + 1]}), __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
     __builtin_amdgcn_s_waitcnt(kVmcnt0);  // this thread's stores have completed
     __syncthreads();
@@ -514,41 +542,56 @@ __global__ __launch_bounds__(256) void woq_gemm_w4_kernel(const FpArgs fa, const
       s_last = __hip_atomic_fetch_add(sk_counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsplit - 1;
     __syncthreads();
     if (!s_last) return;
-    // the other workgroups' partial tiles, one after the other in z order: all loads of one in flight
-    // together, then the additions (this workgroup's own tile comes from its registers, in its turn)
-    f4 total[G4_MT][G4_NTW];
-#pragma unroll 1
-    for (int zz = 0; zz < nsplit; ++zz) {
-      f4 v[G4_MT][G4_NTW];
-      const float* const other = sk_partial + ((size_t)(zz * tiles + tile) * G4_WAVES + wave) * kWaveFloats + lane * 4;
+    // the other workgroups' partial tiles, two row tiles of all of them in flight together; added in z order, this workgroup's
+    // own from its registers in its turn
+    auto sum = [&](auto count) {
+      constexpr int N = decltype(count)::value;
+      const uint64_t* src[N - 1];
 #pragma unroll
-      for (int mt = 0; mt < G4_MT; ++mt)
+      for (int k = 0; k < N - 1; ++k) src[k] = part(k + (k >= z ? 1 : 0));
 #pragma unroll
-        for (int t = 0; t < G4_NTW; ++t) {
-          v[mt][t] = acc[mt][t];
-          if (zz != z) {
+      for (int mc = 0; mc < G4_MT; mc += 2) {
+        uint64_t v[N - 1][2][G4_NTW][2];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              v[mt][t][e] = __hip_atomic_load(other + (mt * G4_NTW + t) * 256 + e, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-          }
-        }
+        for (int k = 0; k < N - 1; ++k)
 #pragma unroll
-      for (int mt = 0; mt < G4_MT; ++mt)
+          for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int t = 0; t < G4_NTW; ++t) {
-          if (zz == 0) {
-            total[mt][t] = v[mt][t];
-          } else {
+            for (int t = 0; t < G4_NTW; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) total[mt][t][e] = total[mt][t][e] + v[mt][t][e];
-          }
-        }
-    }
+              for (int h = 0; h < 2; ++h)
+                v[k][i][t][h] = __hip_atomic_load(src[k] + at(mc + i, t, h), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int mt = 0; mt < G4_MT; ++mt)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int t = 0; t < G4_NTW; ++t) acc[mt][t] = total[mt][t];
+          for (int t = 0; t < G4_NTW; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const f2 own = {acc[mc + i][t][2 * h], acc[mc + i][t][2 * h + 1]};
+              auto value = [&](int zz) {  // partial tile zz
+                const f2 below = bitcast<f2>(v[zz < N - 1 ? zz : N - 2][i][t][h]), above = bitcast<f2>(v[zz > 0 ? zz - 1 : 0][i][t][h]);
+                return zz < z ? below : zz > z ? above : own;
+              };
+              f2 total = value(0);
+#pragma unroll
+              for (int zz = 1; zz < N; ++zz) {
+                const f2 p = value(zz);
+                total[0] = total[0] + p[0];
+                total[1] = total[1] + p[1];
+              }
+              acc[mc + i][t][2 * h] = total[0];
+              acc[mc + i][t][2 * h + 1] = total[1];
+            }
+        __builtin_amdgcn_sched_barrier(0);  // (the next row tiles' loads stay behind: their registers are these)
+      }
+    };
+    if (nsplit == 2)
+      sum(std::integral_constant<int, 2>{});
+    else if (nsplit == 3)
+      sum(std::integral_constant<int, 3>{});
+    else
+      sum(std::integral_constant<int, 4>{});
     // the counter is back at zero for the next launch that uses it
     if (tid == 0) __hip_atomic_store(sk_counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -694,42 +737,83 @@ bool gemm_w4_applies(const FpArgs& f, int wbits, int regime) {
   return f.G >= (wbits == 4 ? 32 : 128) && (f.G & (f.G - 1)) == 0;
 }
 
-// NF4: 128 x 256 tiles, or 64 x 128 ones.  Measured at K = 4096 (other K in proportion): a generation of 256 wide tiles 83 us;
-// the small tiles, three of which share a CU, 40 / 56 / 72 us up to 256 / 512 / 768, 100 just beyond, then 12 + 0.084 a tile.  Small / wide,
-// us: M = 300, N = 11008 57 / 88, M = 512, N = 14336 101 / 90, M = 1000, N = 14336 162 / 172, M = 2048, N = 4096 105 / 93, N = 28672
-// 602 / 571.  128 x 128 tiles (82 KiB of LDS with the pair table: one a CU) were never the fastest (114, 114, 221, 118, 758 us),
-// nor was the general tiled kernel (113, 113, 233, 118, 659 us).
-static bool nf4_wide_tiles(const FpArgs& f) {
-  auto wgs = [&](int bm, int bn) { return ((f.NT * kTileN + bn - 1) / bn) * ((f.M + bm - 1) / bm); };
-  const int64_t w = wgs(64, 128);
-  const double small = w <= 256 ? 40.0 : w <= 512 ? 56.0 : w <= 768 ? 72.0 : std::max(100.0, 12.0 + 0.084 * (double)w);
-  return 83.0 * (double)((wgs(128, 256) + 255) / 256) < small;
-}
-
 // Even, so that every split starts on buffer 0.
 static int split_k_steps(int ksteps, int splits) { return ((ksteps + splits - 1) / splits + 1) & ~1; }
 
-constexpr int kSplitWorkgroups = 256, kSplitMinSteps = 16;
-// K splits of the 64 x 128 shape: 4 or 2 workgroups per tile while that stays within 256 workgroups,
-// leaves each at least 16 K steps and the caller's scratch suffices (14336 -> 4096, M = 128: 64 tiles).
-static int pick_splits(const FpArgs& f, int wbits, int64_t tiles, const SplitKScratch* scratch) {
-  if (!scratch || !scratch->partial || !scratch->counters || tiles > kSplitKCounters) return 1;
-  const int64_t ksteps = f.KT / (wbits / 4);
-  for (int s = 4; s >= 2; s -= 2) {
-    const int64_t need = (int64_t)s * tiles * 64 * 128 * (int64_t)sizeof(float);
-    if (tiles * s <= kSplitWorkgroups && ksteps / s >= kSplitMinSteps && scratch->bytes >= need) return s;
-  }
-  return 1;
-}
+// ---- which tiles, and whether workgroups share K: the lowest of these estimates -----------------------------------------
+// Microseconds of a K step of 128 by the weights' kind, measured at K = 4096 .. 14336 with one, two and (48 KiB of LDS) three
+// 64 x 128 workgroups on a CU, one and two of 128 x 128, one of the others.  A workgroup alone on its CU has one wave a SIMD
+// (eight waves: two), which issues a vector instruction every eight clocks only, two or three waves together one every four:
+// that is why two tiles on a CU cost 1.6 times as much as one, and why sharing K pays until every CU has its three workgroups.
+// The shared tiles cost about 0.25 and 0.5 us a megabyte besides (64 x 128, 128 x 256), written and read once: reduction terms.
+// (INT4, M = 333, 11008 -> 4096: 72 us unsplit, 49-55 with 64 x 128 tiles in four, 46-50 with 128 x 256 in four; M = 128, 7168 ->
+// 2048 25.7 with two, 17.8 with four; NF4, M = 77, 4096 -> 11008 40 -> 26.6; FP8, M = 1000, 7168 -> 4096 95 with 128 x 128 tiles, 77 with 128 x 256 in two).
+struct StepTimes {
+  double t42[3];   // 64 x 128
+  double t2[2];    // 128 x 128 (0: not built)
+  double t8, t8f;  // 128 x 256 on at most 192 CUs, on more (the clock drops)
+  double t7, t163; // 128 x 448, 256 x 192 (0: not built)
+};
+constexpr StepTimes kSteps4 = {{0.74, 1.22, 1.66}, {1.05, 2.02}, 1.50, 1.68, 3.05, 2.75};
+constexpr StepTimes kStepsNf4 = {{1.07, 1.50, 2.05}, {0, 0}, 1.85, 1.90, 0, 0};
+constexpr StepTimes kSteps8 = {{0.73, 1.36, 0}, {1.25, 0}, 1.62, 1.80, 0, 0};
+constexpr StepTimes kStepsFp8 = {{1.04, 1.82, 0}, {1.52, 0}, 1.95, 2.02, 0, 0};
 
-// The same choice for one expert of a grouped launch, as its own launch makes it with the scratch that
-// woq_hip_linear_auto_split_k_workspace_bytes asks for: experts of at most this many rows run in `splits` chains (0: none).
-static int split_rows(int64_t K, int64_t N, int splits) {
-  if (K < kSplitKPrefillMinK || K / kTileK4 / splits < kSplitMinSteps) return 0;
-  const int64_t columns = (N + 127) / 128;
-  return (int)std::min(kSplitWorkgroups / (splits * columns) * 64, kSplitKPrefillElems / N);
+struct TilePlan {
+  int shape = 42, splits = 1;  // shape as launch_gemm_w4's argument
+  double us = 1e30;
+};
+constexpr int kSplitMinSteps = 8;
+constexpr int64_t kSplitScratchMax = 32 << 20;
+static int64_t split_bytes(int64_t M, int64_t N, int shape, int splits) {
+  const int64_t bm = shape == 5 ? 128 : 64, bn = shape == 5 ? 256 : 128;
+  return splits * ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * bm * bn * (int64_t)sizeof(float);
 }
-int gemm_w4_split_rows(int64_t K, int64_t N) { return split_rows(K, N, 2); }
+// share: K may be shared between workgroups (64 < M <= kSplitKPrefillMaxRows, K >= kSplitKPrefillMinK, at least eight steps each)
+static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t, bool share) {
+  const int64_t np = (N + kTileN - 1) / kTileN * kTileN;
+  auto wgs = [&](int bm, int bn) { return ((np + bn - 1) / bn) * ((M + bm - 1) / bm); };
+  auto gens = [](int64_t w) { return (double)((w + 255) / 256); };
+  TilePlan best;
+  auto offer = [&](int shape, int splits, double us) {
+    if (us < best.us) best.shape = shape, best.splits = splits, best.us = us;
+  };
+  share = share && M > 64 && M <= kSplitKPrefillMaxRows && (int64_t)ksteps * kTileK4 >= kSplitKPrefillMinK;
+  const int most42 = t.t42[2] > 0 ? 3 : 2, most2 = t.t2[1] > 0 ? 2 : 1;
+  for (int s = 1; s <= (share ? kPrefillSplitMax : 1); ++s) {
+    const int kts = s == 1 ? ksteps : split_k_steps(ksteps, s);
+    if (s > 1 && (kts < kSplitMinSteps || (s - 1) * kts >= ksteps)) break;
+    const int64_t w42 = wgs(64, 128) * s, w8 = wgs(128, 256) * s;
+    auto red = [&](int shape, double a, double b) { return s == 1 ? 0.0 : a + b * (double)split_bytes(M, np, shape, s) * 1e-6; };
+    if (w42 <= 256 * most42)
+      offer(42, s, kts * t.t42[(w42 + 255) / 256 - 1] + red(42, 2.0 + 0.4 * s, 0.25));
+    else if (s == 1)
+      offer(42, 1, kts * t.t42[most42 - 1] * ((double)w42 / (256 * most42) + 0.25));
+    if (s == 1 || (w8 <= 256 && split_bytes(M, np, 5, s) <= kSplitScratchMax))
+      offer(5, s, kts * gens(w8) * (w8 <= 192 ? t.t8 : t.t8f) + red(5, 2.0, 0.48));
+  }
+  const int64_t w2 = wgs(128, 128);
+  if (t.t2[0] > 0)
+    offer(2, 1, ksteps * (w2 <= 256 ? t.t2[0] : most2 == 1 ? gens(w2) * t.t2[0] : t.t2[1] * (w2 <= 512 ? 1.0 : (double)w2 / 512 + 0.1)));
+  if (t.t163 > 0 && wgs(256, 192) % 256 == 0) offer(163, 1, ksteps * gens(wgs(256, 192)) * t.t163);
+  if (t.t7 > 0) offer(7, 1, ksteps * gens(wgs(128, 448)) * t.t7);
+  best.us += 0.125 * ksteps;  // launch, first requests, stores: 4 us at K = 4096, in proportion as in gemm_dense_cost's figures
+  return best;
+}
+static const StepTimes& step_times(int wbits, int nf4, int fp8) { return wbits == 8 ? (fp8 ? kStepsFp8 : kSteps8) : nf4 ? kStepsNf4 : kSteps4; }
+
+// K steps of a chain for an expert of 64 (i - 1) < rows <= 64 i rows, i = 2 ..: as its own launch shares them with the scratch
+// that woq_hip_linear_auto_split_k_workspace_bytes asks for (0: one chain).
+static int chain_steps(int64_t K, int64_t N, int wbits, int row_tiles) {
+  const int ksteps = (int)(K / kTileK4);
+  const TilePlan p = plan_tiles(64 * row_tiles, N, ksteps, step_times(wbits, 0, 0), true);
+  return p.splits > 1 ? split_k_steps(ksteps, p.splits) : 0;
+}
+int gemm_w4_split_rows(int64_t K, int64_t N) {
+  for (int i = (int)(kSplitKPrefillMaxRows / 64); i >= 2; --i)
+    if (chain_steps(K, N, 4, i) || chain_steps(K, N, 8, i)) return 64 * i;
+  return 0;
+}
 
 template <int REGIME, class S, int WBITS = 4, bool FP8 = false, bool NF4 = false>
 static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits = 1,
@@ -747,7 +831,7 @@ static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits
   const int ksteps = (int)(f.KT / (WBITS / 4));
   int kts = ksteps;
   if (splits > 1) {
-    if (S::MT * S::NTW > 8) return set_error("woq_gemm_w4_kernel: K is split for the 64 x 128 shape only");
+    if (!S::SPLITS) return set_error("woq_gemm_w4_kernel: K is split for the 64 x 128 and 128 x 256 shapes only");
     kts = split_k_steps(ksteps, splits);
     const int64_t tiles = (int64_t)grid.x * grid.y;
     const int64_t need = (int64_t)splits * tiles * S::BM * S::BN * (int64_t)sizeof(float);
@@ -764,12 +848,12 @@ static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits
                               hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
       if (lds_optin_m != hipSuccess)
         return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin_m));
-      woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, true><<<grid, 256, kLds, st>>>(
+      woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, true><<<grid, 64 * S::WAVES, kLds, st>>>(
           f, g_shift, splits > 1 ? scratch->partial : nullptr, splits > 1 ? scratch->counters : nullptr, kts, G4Group{});
       return check_launch("woq_gemm_w4_kernel");
     }
   }
-  woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4><<<grid, 256, kLds, st>>>(f, g_shift, splits > 1 ? scratch->partial : nullptr,
+  woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4><<<grid, 64 * S::WAVES, kLds, st>>>(f, g_shift, splits > 1 ? scratch->partial : nullptr,
                                                                  splits > 1 ? scratch->counters : nullptr, kts, G4Group{});
   return check_launch("woq_gemm_w4_kernel");
 }
@@ -785,7 +869,7 @@ static int launch_grouped_shape(const FpArgs& f, int g_shift, const G4Group& g, 
     return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin));
   const dim3 grid((unsigned)((f.NT * kTileN + S::BN - 1) / S::BN), (unsigned)slots);
   woq_gemm_w4_kernel<REGIME, S, WBITS, false, false, true, false, CHAINS>
-      <<<grid, 256, kLds, st>>>(f, g_shift, nullptr, nullptr, (int)(f.KT / (WBITS / 4)), g);
+      <<<grid, 64 * S::WAVES, kLds, st>>>(f, g_shift, nullptr, nullptr, (int)(f.KT / (WBITS / 4)), g);
   return check_launch("woq_gemm_w4_kernel (grouped)");
 }
 
@@ -801,23 +885,17 @@ int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGrou
   // Chains on 64 x 128 tiles only: a second copy of the accumulators costs a 128 x 128 tile its second workgroup on a CU (us with
   // 64 / 128 rows a tile: 32 experts 7168 -> 2048, top-8, 1024 tokens 1228 / 1295, 16 experts 4096 -> 1536,
   // top-4, 2048 tokens 562 / 697).
-  const int ksteps = (int)(f.KT / (wbits / 4));
-  const G4Group g{grp, split_rows(f.K, f.N, 4), split_k_steps(ksteps, 4), split_rows(f.K, f.N, 2), split_k_steps(ksteps, 2)};
+  G4Group g{};
+  g.tables = grp;
+  bool chained = false;
+  for (int i = 2; tile_rows == 64 && i <= kSplitKPrefillMaxRows / 64; ++i) chained |= (g.chains[i] = chain_steps(f.K, f.N, wbits, i)) != 0;
 #define WOQ_GROUPED(RG, WB)                                                                  \
   (tile_rows == 128 ? launch_grouped_shape<RG, S2, WB, false>(f, g_shift, g, slots, st)      \
-   : g.rows2 > 64   ? launch_grouped_shape<RG, S42, WB, true>(f, g_shift, g, slots, st)      \
+   : chained         ? launch_grouped_shape<RG, S42, WB, true>(f, g_shift, g, slots, st)      \
                     : launch_grouped_shape<RG, S42, WB, false>(f, g_shift, g, slots, st))
   if (wbits == 4) return regime == kRegimeF16 ? WOQ_GROUPED(kRegimeF16, 4) : WOQ_GROUPED(kRegimeBF16, 4);
   return regime == kRegimeF16 ? WOQ_GROUPED(kRegimeF16, 8) : WOQ_GROUPED(kRegimeBF16, 8);
 #undef WOQ_GROUPED
-}
-
-// Relative time of a shape: generations of 256 workgroups times the length of one K step, which
-// is proportional to the row-blocks per wave plus a fixed part (requests, barrier, pipeline fill).
-template <class S>
-static double shape_cost(const FpArgs& f) {
-  const double wgs = (double)((f.NT * kTileN + S::BN - 1) / S::BN) * (double)((f.M + S::BM - 1) / S::BM);
-  return (double)(int64_t)((wgs + 255) / 256) * (S::NTW + 1.0);
 }
 
 // 8-bit weights of one shape: integers or float8 bytes, fp16 or bf16 compute
@@ -831,24 +909,9 @@ static int launch8(const FpArgs& f, int regime, int g_shift, hipStream_t st, int
                               : launch_shape<kRegimeBF16, S, 8>(f, g_shift, st, splits, scratch);
 }
 
-// Estimated time of the automatic choice below, in microseconds, for the comparison with the dense kernel
-// (gemm_dense_cost): per 4096 input channels a generation of 256 workgroups measured 92 / 58 / 37 us with 7 / 4 / 2
-// row-blocks per wave, the 64 x 128 shape 27 us while it fits one generation; the 128 x 128 shape beyond 512
-// workgroups (two share a CU) 68 us per 512 and 24-68 us for the rest; 8-bit weights a fifth more.
+// Estimated time of the automatic choice below, in microseconds, for the comparison with the dense kernel (gemm_dense_cost).
 double gemm_w4_cost(const FpArgs& f, int wbits) {
-  auto wgs = [&](int bm, int bn) { return ((f.NT * kTileN + bn - 1) / bn) * ((f.M + bm - 1) / bm); };
-  auto gens = [](int64_t w) { return (double)((w + 255) / 256); };
-  const int64_t w42 = wgs(64, 128), w2 = wgs(128, 128);
-  double c;
-  if (w42 <= 256) {
-    c = 27.0;
-  } else {
-    const int64_t rem = w2 % 512;
-    const double c2 = w2 <= 512 ? gens(w2) * 37.0 : 68.0 * (double)(w2 / 512) + (rem ? 24.0 + 44.0 * (double)rem / 512.0 : 0.0);
-    c = std::min(gens(wgs(128, 256)) * 58.0, c2);
-    if (wbits == 4) c = std::min(c, gens(wgs(128, 448)) * 92.0);
-  }
-  return c * (wbits == 8 ? 1.2 : 1.0) * (double)f.K / 4096.0;
+  return plan_tiles(f.M, f.N, (int)(f.KT / (wbits / 4)), step_times(wbits, f.nf4, f.fp8), true).us;
 }
 
 int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int shape, int splits,
@@ -858,84 +921,47 @@ int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int s
     g_shift = 0;
     while (((int64_t)1 << g_shift) < f.G) ++g_shift;
   }
-  // 128 rows x 448, 256 or 128 columns per workgroup: the widest shape does the most work per
-  // activation fragment, the narrower ones make enough workgroups to fill the chip when M * N is
-  // small (e.g. N = 4096: 10 column blocks of 448 but 16 of 256).
-  // 256 rows x 192 columns (MT 16, NTW 3: 192 accumulator registers) dequantizes half as much per
-  // MFMA but measured no faster per output (a workgroup takes 95-120 us for K = 4096 against 103 us
-  // for the 17 % larger 128 x 448 one); it is chosen only where it tiles the problem into whole
-  // generations of 256 workgroups and the others do not (N = 6144, M = 2048: 93 us against 138 us).
-  // A 256 x 256 shape would need all 256 accumulator registers; the register allocator then
-  // copies accumulators through VGPRs and scratch, it measured slower and is not built.
+  // 256 rows x 192 columns (MT 16, NTW 3: 192 accumulator registers) dequantizes half as much per MFMA but measured no faster
+  // per output (95-120 us at K = 4096 against 103 for the 17 % larger 128 x 448 one): it is offered only where it tiles the
+  // problem into whole generations of 256 workgroups.  256 x 256 would need all 256 accumulator registers; the register
+  // allocator then copies accumulators through VGPRs and scratch, it measured slower and is not built.
   using S7 = G4Shape<8, 7>;
-  using S4 = G4Shape<8, 4>;
+  using S8 = G4Shape<8, 2, 8>;
   using S2 = G4Shape<8, 2>;
   using ST = G4Shape<16, 3>;
   using S42 = G4Shape<4, 2>;
-  if (f.nf4) {
-    if (shape != 0 || splits > 1) return set_error("woq_gemm_w4_kernel: NF4 weights take the automatic shape only");
-    const int64_t wgs42 = ((f.NT * kTileN + S42::BN - 1) / S42::BN) * ((f.M + S42::BM - 1) / S42::BM);
-#define WOQ_NF4(S, ...)                                                                    \
-  (regime == kRegimeF16 ? launch_shape<kRegimeF16, S, 4, false, true>(f, g_shift, st, ##__VA_ARGS__) \
-                        : launch_shape<kRegimeBF16, S, 4, false, true>(f, g_shift, st, ##__VA_ARGS__))
-    return nf4_wide_tiles(f) ? WOQ_NF4(S4) : WOQ_NF4(S42, pick_splits(f, 4, wgs42, scratch), scratch);
-#undef WOQ_NF4
-  }
-  if (wbits == 8) {
-    // 8-bit weights: twice the tile bytes per K step, so at most four row-blocks per wave fit the LDS
-    // (128 x 256, 128 x 128 and 64 x 128 workgroup tiles), chosen like the 4-bit ones
-    if (shape != 0 && shape != 4 && shape != 2 && shape != 42)
-      return set_error("woq_gemm_w4_kernel: 8-bit weights take the 128 x 256, 128 x 128 and 64 x 128 shapes");
-    const int64_t wgs42 = ((f.NT * kTileN + S42::BN - 1) / S42::BN) * ((f.M + S42::BM - 1) / S42::BM);
-    if (shape == 0) shape = wgs42 <= 256 ? 42 : (shape_cost<S4>(f) <= shape_cost<S2>(f) ? 4 : 2);
-    if (shape == 42) {
-      if (splits == 0) splits = pick_splits(f, 8, wgs42, scratch);
-      return launch8<S42>(f, regime, g_shift, st, splits, scratch);
-    }
-    if (splits > 1) return set_error("woq_gemm_w4_kernel: K is split for the 64 x 128 shape only");
-    if (shape == 4)
-      return launch8<S4>(f, regime, g_shift, st);
-    return launch8<S2>(f, regime, g_shift, st);
-  }
+  if (shape == 4) shape = 5;  // (four row-blocks a wave in the caller's terms: 128 x 256)
+  if (f.nf4 && (shape != 0 || splits > 1)) return set_error("woq_gemm_w4_kernel: NF4 weights take the automatic shape only");
+  if (wbits == 8 && shape != 0 && shape != 5 && shape != 2 && shape != 42)
+    return set_error("woq_gemm_w4_kernel: 8-bit weights take the 128 x 256, 128 x 128 and 64 x 128 shapes");
+  if (shape != 0 && shape != 42 && splits > 1) return set_error("woq_gemm_w4_kernel: K is split for the 64 x 128 shape only");
   if (shape == 0) {
-    // Small M x N: 64 x 128 tiles at four waves per SIMD (79 + 32 registers, 48 KiB of LDS).  While
-    // every workgroup has a CU to itself the K loop is one memory round trip per step whatever the
-    // tile, and the small tile's steps are the shortest: M = 128, 4096 -> 14336 takes 27.7 us against
-    // 37.2 us with 128 x 128 tiles, 14336 -> 4096 80.8 us against 112.5 us.
-    const int64_t wgs42 = ((f.NT * kTileN + S42::BN - 1) / S42::BN) * ((f.M + S42::BM - 1) / S42::BM);
-    if (wgs42 <= 256) shape = 42;
+    const bool have = scratch && scratch->partial && scratch->counters && splits == 0;
+    const int ksteps = (int)(f.KT / (wbits / 4));
+    const StepTimes& t = step_times(wbits, f.nf4, f.fp8);
+    TilePlan p = plan_tiles(f.M, f.N, ksteps, t, have);
+    if (p.splits > 1 && scratch->bytes < split_bytes(f.M, f.NT * kTileN, p.shape, p.splits)) p = plan_tiles(f.M, f.N, ksteps, t, false);
+    shape = p.shape;
+    splits = p.splits;
   }
-  if (shape == 42) {
-    const int64_t wgs42 = ((f.NT * kTileN + S42::BN - 1) / S42::BN) * ((f.M + S42::BM - 1) / S42::BM);
-    if (splits == 0) splits = pick_splits(f, 4, wgs42, scratch);
-    return regime == kRegimeF16 ? launch_shape<kRegimeF16, S42>(f, g_shift, st, splits, scratch)
-                                : launch_shape<kRegimeBF16, S42>(f, g_shift, st, splits, scratch);
+  if (splits == 0) splits = 1;
+#define WOQ_W4(S, ...)                                                                                  \
+  (regime == kRegimeF16 ? launch_shape<kRegimeF16, S, ##__VA_ARGS__>(f, g_shift, st, splits, scratch) \
+                        : launch_shape<kRegimeBF16, S, ##__VA_ARGS__>(f, g_shift, st, splits, scratch))
+  if (f.nf4) return shape == 5 ? WOQ_W4(S8, 4, false, true) : WOQ_W4(S42, 4, false, true);
+  // 8-bit weights: twice the tile bytes per K step
+  if (wbits == 8)
+    return shape == 42 ? launch8<S42>(f, regime, g_shift, st, splits, scratch)
+           : shape == 5 ? launch8<S8>(f, regime, g_shift, st, splits, scratch)
+                        : launch8<S2>(f, regime, g_shift, st, splits, scratch);
+  switch (shape) {
+    case 42: return WOQ_W4(S42);
+    case 5: return WOQ_W4(S8);
+    case 163: return WOQ_W4(ST);
+    case 7: return WOQ_W4(S7);
+    default: return WOQ_W4(S2);
   }
-  if (splits > 1) return set_error("woq_gemm_w4_kernel: K is split for the 64 x 128 shape only");
-  const double c7 = shape_cost<S7>(f), c4 = shape_cost<S4>(f);
-  // 128 x 128 tiles of 4-bit weights: two workgroups share a CU, so beyond two generations the CUs stay
-  // evenly loaded (fractional generations), and a generation measured 0.53 of a 128 x 256 one (37 against
-  // 70 us at K = 4096).  M = 1024, 4096 -> 11008 (688 workgroups): 101 us against 124 us with 128 x 448
-  // tiles (200 workgroups); M = 1024 / 2048, 8192 -> 10240: 180 / 313 us against 207 / 329 us.
-  const double wgs2 = (double)((f.NT * kTileN + S2::BN - 1) / S2::BN) * (double)((f.M + S2::BM - 1) / S2::BM);
-  const double c2 = wgs2 <= 512 ? shape_cost<S2>(f) : wgs2 / 256.0 * 2.7;
-  if (shape == 0) {
-    shape = (c7 <= c4 && c7 <= c2) ? 7 : (c4 <= c2 ? 4 : 2);
-    const int64_t wgs_t = ((f.NT * kTileN + ST::BN - 1) / ST::BN) * ((f.M + ST::BM - 1) / ST::BM);
-    const double ct = (double)(wgs_t / 256) * 7.4;
-    if (wgs_t % 256 == 0 && ct < c7 && ct < c4 && ct < c2) shape = 163;
-  }
-  if (shape == 163)
-    return regime == kRegimeF16 ? launch_shape<kRegimeF16, ST>(f, g_shift, st)
-                                : launch_shape<kRegimeBF16, ST>(f, g_shift, st);
-  if (shape == 7)
-    return regime == kRegimeF16 ? launch_shape<kRegimeF16, S7>(f, g_shift, st)
-                                : launch_shape<kRegimeBF16, S7>(f, g_shift, st);
-  if (shape == 4)
-    return regime == kRegimeF16 ? launch_shape<kRegimeF16, S4>(f, g_shift, st)
-                                : launch_shape<kRegimeBF16, S4>(f, g_shift, st);
-  return regime == kRegimeF16 ? launch_shape<kRegimeF16, S2>(f, g_shift, st)
-                              : launch_shape<kRegimeBF16, S2>(f, g_shift, st);
+#undef WOQ_W4
 }
 
 }  // namespace woq

@@ -61,8 +61,9 @@ struct SplitKScratch {
 // Entries the caller's split-K counter array must have, and the largest number of K splits.
 constexpr int kSplitKCounters = 512;
 constexpr int kSplitKMax = 4;
-// Prefill problems that get split-K scratch by themselves (woq_hip_linear_auto_split_k_workspace_bytes).
-constexpr int64_t kSplitKPrefillMinK = 4096, kSplitKPrefillElems = 1048576;
+// Prefill problems that get split-K scratch by themselves (woq_hip_linear_auto_split_k_workspace_bytes): the least K and the most
+// rows; lowp_mode INT8: the most outputs.
+constexpr int64_t kSplitKPrefillMinK = 4096, kSplitKPrefillMaxRows = 1024, kSplitKPrefillElems = 1048576;
 
 int launch_pack_weight(const void* plain, int weight_dtype, int64_t N, int64_t K, void* packed,
                        hipStream_t st);
@@ -151,10 +152,10 @@ int launch_gemm(const FpArgs& a, int wbits, int regime, hipStream_t st);
 // Prefill GEMM with register-resident dequantization (woq_gemm_w4.hip): 4-bit integer weights, or
 // 8-bit weights with one scale per channel or per group of at least 128
 bool gemm_w4_applies(const FpArgs& f, int wbits, int regime);
-// shape: row-blocks per wave (7, 4 or 2: 448, 256 or 128 columns per workgroup), 163 / 42 = 256 x 192 /
-// 64 x 128 tiles, 0 = by cost model; 8-bit weights: 4, 2, 42 or 0
-// splits: workgroups that share the K steps of a tile (64 x 128 shape only; 2 or 4 need the scratch),
-// 0 = by problem size, 1 = none
+// shape: 7, 4, 2: 448, 256 or 128 columns of 128 rows per workgroup, 163 / 42 = 256 x 192 /
+// 64 x 128 tiles, 0 = by estimated time; 8-bit weights: 4, 2, 42 or 0
+// splits: workgroups that share the K steps of a tile (as an argument: 64 x 128 tiles only; 2 to 4 need the scratch),
+// 0 = by estimated time, 1 = none
 bool gemm_w4s_applies(const FpArgs& f, int wbits, int regime);
 int launch_gemm_w4s(const FpArgs& f, int regime, hipStream_t st);
 int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int shape = 0, int splits = 0,

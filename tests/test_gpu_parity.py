@@ -632,6 +632,39 @@ def test_prefill_kernel_split_k(cuda, kind, M, K, N, G, bias, kernel):
     assert all(int(buf.abs().sum()) == 0 for buf in kmod._counter_cache.values())
 
 
+@pytest.mark.parametrize("kind,M,K,N", [
+    ("int4", 65, 4096, 144),    # four workgroups of eight K steps each; one row in the last 64 x 128 tile
+    ("int4", 333, 4352, 4096),  # 34 K steps in parts of 10, the last shorter
+    ("int4", 1024, 4224, 1008),  # the most rows that share K, 33 K steps
+    ("int4", 1025, 4096, 256),  # one more: not shared
+    ("int4_f16", 130, 8192, 272),
+    ("nf4", 77, 4096, 3088), ("nf4", 129, 4096, 272),
+    ("int8", 600, 4096, 4112), ("int8", 1000, 4608, 4096),  # 128 x 256 tiles of eight waves, K in two
+    ("fp8", 999, 4096, 4080), ("fp8", 70, 4352, 272),
+])
+def test_prefill_kernel_by_estimated_time(cuda, kind, M, K, N):
+    """The automatic choice of tiles and K shares: against the general kernel (the same rounded weights, fp32 sums in another
+    order, then one rounding to the output's 16 bits: flips of a last bit of 2^-9 (2^-11) in few outputs, 1e-3 in the 2-norm), a
+    post-op and a bias included; repeated calls give the same bits and leave the counters at zero."""
+    from ipex_amd import _kernels as kmod
+    syn = _synthetic()
+    f16 = kind == "int4_f16"
+    case = (syn.make_int8_case(61, M, K, N) if kind == "int8" else syn.make_fp8_case(61, M, K, N, group_size=128) if kind == "fp8" else
+            syn.make_nf4_case(61, M, K, N, 64, bias=True) if kind == "nf4" else
+            syn.make_int4_case(61, M, K, N, 128, bias=True, scale_dtype=torch.float16 if f16 else torch.bfloat16))
+    x = (case["x"].half() if f16 else case["x"]).cuda()
+    ctx = make_context(case, O.LOWP_FP16 if f16 else O.LOWP_BF16)
+    other = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(x.dtype).cuda()
+    for args in ({}, {"fusion": _lib_mod().FUSE_ADD, "others": (other,)}):
+        got = ctx.run(x, **args)
+        assert _lib_last_kernel() == "woq_gemm_w4_kernel"
+        assert rel_l2(to_np_f32(got), to_np_f32(ctx.run(x, force_kernel=2, **args))) <= 1e-3
+        runs = [ctx.run(x, **args) for _ in range(20)]
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, got) for y in runs)
+    assert all(int(buf.abs().sum()) == 0 for buf in kmod._counter_cache.values())
+
+
 def test_prefill_kernel_split_k_rejections(cuda):
     case = _synthetic().make_int4_case(30, 128, 512, 256, 128)  # four K steps: too few to share
     with pytest.raises(RuntimeError, match="too few"):
