@@ -294,6 +294,13 @@ int64_t woq_hip_int8_block_k(int64_t group_size, int64_t K);
 
 int woq_hip_linear(const woq_hip_linear_params* p);
 
+/* The front half of a gated MLP in one launch: out = silu(x Wg^T + bg) * (x Wu^T + bu), rounded as woq_hip_linear on `gate` with the
+ * silu and then on `up` with the mul round it (Linear2SiluMul; with 17 to 32 rows the K sums may be added in another order).  Both parameter sets name the same x, out, sizes,
+ * modes and stream, no post-op.  For the problems of woq_hip_linear_pair_applies: INT4 and INT8 weights with their scale_zero_bf16
+ * tables (and scale_zero_f16x2 for rows that compute in fp16), bf16 rows, lowp_mode BF16 or NONE, at most 64 rows. */
+int woq_hip_linear_pair_applies(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);
+int woq_hip_linear_pair(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);
+
 /* woq_hip_linear for callers that cannot allocate and hold no workspace: code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference, whose kernels
  * take their temporaries from the CPU heap.  Same arguments and results as woq_hip_linear, except that
@@ -406,11 +413,27 @@ typedef struct woq_hip_moe_group {
   const void* const* scales;       /* [experts] scales in the compute type of the call (fp16 or bf16 layout of woq_hip_pack_qparams) */
   const uint8_t* const* zeros_u8;  /* [experts] or NULL (symmetric) */
   const float* const* bias;        /* [experts] or NULL */
+  /* read by woq_hip_moe_linear only: */
+  const uint32_t* const* szb;      /* [experts] scale_zero_bf16 tables, with WOQ_HIP_MOE_SZB */
+  const void* const* qweight_b;    /* WOQ_HIP_MOE_PAIR: the same of the up projections */
+  const void* const* scales_b;
+  const uint8_t* const* zeros_b;
+  const float* const* bias_b;
+  const uint32_t* const* szb_b;
 } woq_hip_moe_group;
 int woq_hip_moe_route(const int64_t* topk_ids, int64_t T, int64_t topk, int64_t experts, int64_t split_lo,
                       int64_t split_mid, int use_single, int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of,
                       int32_t* slot_of, void* stream);
 int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, int64_t slots);
+/* woq_hip_linear_grouped (tile_rows 0) and woq_hip_linear_grouped_tiles below (64 or 128) with two options.
+ * WOQ_HIP_MOE_SZB: the group has the experts' merged (scale, zero) tables; bf16 compute then reads those (same results).
+ * WOQ_HIP_MOE_PAIR: out = silu(gate) * up of the group's two sets of linears in one launch, rounded as the launch with the silu
+ * and the one with the mul round it; p without a post-op.  For the problems of woq_hip_moe_pair_applies(p, tile_rows) (bf16 rows;
+ * p->scale_zero_f16x2 as above), in bf16 compute with WOQ_HIP_MOE_SZB. */
+#define WOQ_HIP_MOE_PAIR 1
+#define WOQ_HIP_MOE_SZB 2
+int woq_hip_moe_pair_applies(const woq_hip_linear_params* p, int tile_rows);
+int woq_hip_moe_linear(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows, int flags);
 /*
  * The same layer for prompts: woq_hip_moe_route_tiles sorts at most WOQ_HIP_MOE_TILES_MAX entries over at most
  * WOQ_HIP_MOE_TILES_EXPERTS experts and cuts the routed rows into slots, int32 [4][3][S], S >= experts + T * topk /

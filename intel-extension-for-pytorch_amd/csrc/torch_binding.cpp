@@ -234,12 +234,13 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
   // What a grouped launch over many contexts (the experts of a mixture-of-experts layer) needs of each: the device
   // addresses of the packed weight, the fp16 and bf16 scales, the zero points and the fp32 bias (0: none), then
   // N, K, group size, weight dtype, lowp_mode, whether the input channels are permuted (g_idx), the device index,
-  // and the (fp16 scale, fp16 128 + zero) dword table of the single-row decode kernel (0: none).
+  // the (fp16 scale, fp16 128 + zero) dword table of the single-row decode kernel (0: none) and the merged table of the
+  // bf16 kernels (0: none).
   std::vector<int64_t> kernel_pointers() {
     auto addr = [](const Tensor& t) -> int64_t { return t.defined() ? (int64_t)(uintptr_t)t.data_ptr() : 0; };
     return {addr(packed_), addr(q_.s16), addr(q_.sb16), q_.z8.has_value() ? addr(*q_.z8) : 0, addr(bias_f32_),
             N_, K_, group_size_, weight_dtype_, lowp_mode_, g_src_.defined() ? 1 : 0, (int64_t)packed_.device().index(),
-            q_.sz.has_value() ? addr(*q_.sz) : 0};
+            q_.sz.has_value() ? addr(*q_.sz) : 0, q_.szb.has_value() ? addr(*q_.szb) : 0};
   }
   optional<Tensor> get_g_idx() { return g_idx_; }
   // The dequantized bf16 copy of the weight that cache_weight_for_large_batch asks for under lowp_mode BF16
@@ -305,6 +306,34 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
     Tensor x = x_in;
     if (g_src_.defined()) x = shuffle_activations(x, g_src_);
     return run_sorted(x, M, fusion, others, out_sizes);
+  }
+
+  // silu(gate(x)) * up(x), in one launch where the library has one (woq_hip_linear_pair), else in the two that the ops
+  // woq_linear_silu and woq_linear_mul make
+  static Tensor run_pair(WoqLinearOpContext& gate, WoqLinearOpContext& up, const Tensor& x_in) {
+    const int64_t M = x_in.numel() > 0 && x_in.size(-1) == gate.K_ ? x_in.numel() / gate.K_ : 0;
+    if (M >= 1 && M <= 64 && gate.K_ == up.K_ && gate.N_ == up.N_ && !gate.g_src_.defined() && !up.g_src_.defined() &&
+        gate.packed_.device() == x_in.device() && up.packed_.device() == x_in.device() && x_in.scalar_type() == at::kBFloat16) {
+      Tensor x2 = x_in.is_contiguous() ? x_in : x_in.contiguous();
+      if ((uintptr_t)x2.data_ptr() % 16) x2 = x2.clone();  // the kernels read activation rows with 16-byte loads
+      std::vector<int64_t> out_sizes = x_in.sizes().vec();
+      out_sizes.back() = gate.N_;
+      woq_hip_linear_params p[2];
+      gate.fill_params(p[0], x2, M);
+      up.fill_params(p[1], x2, M);
+      DeviceScope scope(x2);
+      Tensor out = at::empty(out_sizes, x_in.options());
+      for (auto& q : p) {
+        q.out = out.data_ptr();
+        q.out_dtype = act_code(x2.scalar_type());
+        q.stream = current_stream(x2);
+      }
+      if (woq_hip_linear_pair_applies(&p[0], &p[1])) {
+        check_rc(woq_hip_linear_pair(&p[0], &p[1]), "woq_linear_silu_mul");
+        return out;
+      }
+    }
+    return up.run(x_in, WOQ_HIP_FUSE_MUL, {gate.run(x_in, WOQ_HIP_FUSE_SILU, {})});
   }
 
   int64_t handle() const { return handle_; }
@@ -418,24 +447,8 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
     batch_size_ = o.batch_size_; cache_weight_ = o.cache_weight_;
   }
 
-  // `run` behind the act-order shuffle: the input channels of x are in the order of the stored weight
-  Tensor run_sorted(const Tensor& x, int64_t M, int64_t fusion, const std::vector<Tensor>& others,
-                    const std::vector<int64_t>& out_sizes) {
-    Tensor x2 = x.is_contiguous() ? x : x.contiguous();
-    if ((uintptr_t)x2.data_ptr() % 16) x2 = x2.clone();  // the kernels read activation rows with 16-byte loads
-    Tensor out = at::empty(out_sizes, x.options());
-    if (lowp_mode_ == WOQ_HIP_LOWP_FP16 && x.scalar_type() == at::kBFloat16 && M > 16 && fusion == WOQ_HIP_FUSE_NONE) {
-      // fp16 compute on bf16 rows beyond one row tile: the reference converts the rows to fp16 and casts
-      // the fp16 result to bf16 (csrc/cpu/aten/utils/woq.h:3076-3085).  The library converts the rows once;
-      // its fp16 kernels then write the bf16 output themselves.
-      Tensor xh = at::empty(x2.sizes(), x2.options().dtype(at::kHalf));
-      DeviceScope scope(x2);
-      check_rc(woq_hip_convert_activations(x2.data_ptr(), WOQ_HIP_ACT_BF16, xh.data_ptr(), WOQ_HIP_ACT_FP16,
-                                           x2.numel(), current_stream(x2)),
-               "woq_linear");
-      x2 = xh;
-    }
-    woq_hip_linear_params p;
+  // everything of a call's parameters that does not depend on the output, the post-op and the scratch
+  void fill_params(woq_hip_linear_params& p, const Tensor& x2, int64_t M) const {
     memset(&p, 0, sizeof(p));
     p.struct_size = sizeof(p);
     p.x = x2.data_ptr();
@@ -454,6 +467,27 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
     p.bias = bias_f32_.defined() ? bias_f32_.data_ptr<float>() : nullptr;
     p.lowp_mode = (int32_t)lowp_mode_;
     p.act_quant_mode = (int32_t)act_quant_mode_;
+  }
+
+  // `run` behind the act-order shuffle: the input channels of x are in the order of the stored weight
+  Tensor run_sorted(const Tensor& x, int64_t M, int64_t fusion, const std::vector<Tensor>& others,
+                    const std::vector<int64_t>& out_sizes) {
+    Tensor x2 = x.is_contiguous() ? x : x.contiguous();
+    if ((uintptr_t)x2.data_ptr() % 16) x2 = x2.clone();  // the kernels read activation rows with 16-byte loads
+    Tensor out = at::empty(out_sizes, x.options());
+    if (lowp_mode_ == WOQ_HIP_LOWP_FP16 && x.scalar_type() == at::kBFloat16 && M > 16 && fusion == WOQ_HIP_FUSE_NONE) {
+      // fp16 compute on bf16 rows beyond one row tile: the reference converts the rows to fp16 and casts
+      // the fp16 result to bf16 (csrc/cpu/aten/utils/woq.h:3076-3085).  The library converts the rows once;
+      // its fp16 kernels then write the bf16 output themselves.
+      Tensor xh = at::empty(x2.sizes(), x2.options().dtype(at::kHalf));
+      DeviceScope scope(x2);
+      check_rc(woq_hip_convert_activations(x2.data_ptr(), WOQ_HIP_ACT_BF16, xh.data_ptr(), WOQ_HIP_ACT_FP16,
+                                           x2.numel(), current_stream(x2)),
+               "woq_linear");
+      x2 = xh;
+    }
+    woq_hip_linear_params p;
+    fill_params(p, x2, M);
     p.fusion = (int32_t)fusion;
     std::vector<Tensor> keep;
     for (size_t i = 0; i < others.size() && i < 2; ++i) {
@@ -714,6 +748,13 @@ static Tensor woq_linear_binary(const Tensor& input, const Tensor& W_prepack, co
   return context_from_handle(W_prepack, "torch_ipex::woq_linear_<post-op>")->run(input, FUSION, o);
 }
 
+static Tensor woq_linear_silu_mul(const Tensor& input, const Tensor& W_gate, const Tensor& W_up) {
+  const char* op = "torch_ipex::woq_linear_silu_mul";
+  require_gpu_input(input, op);
+  auto gate = context_from_handle(W_gate, op), up = context_from_handle(W_up, op);
+  return WoqLinearOpContext::run_pair(*gate, *up, input);
+}
+
 // ---- mixture of experts over WOQ linears (csrc/cpu/aten/MoE.cpp:260-328) -------------------------------
 // One expert: gather its tokens, down(up(x) * silu(gate(x))), weighted accumulation into `output`
 // (mixtral_moe_woq_kernl_impl, csrc/cpu/aten/kernels/MoEKrnl.cpp:254-284).
@@ -943,6 +984,11 @@ static Tensor woq_linear_binary_autocast(const Tensor& input, const Tensor& W_pr
   return woq_linear_binary<FUSION, NOTHERS>(autocast_input(input), W_prepack, others);
 }
 
+static Tensor woq_linear_silu_mul_autocast(const Tensor& input, const Tensor& W_gate, const Tensor& W_up) {
+  c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
+  return woq_linear_silu_mul(autocast_input(input), W_gate, W_up);
+}
+
 static Tensor woq_linear_v2_autocast(const Tensor& input, const Tensor& qweight, c10::string_view weight_dtype,
                                      std::vector<int64_t> weight_shape, std::vector<Tensor> weight_scales,
                                      optional<std::vector<Tensor>> weight_zeros, optional<std::vector<Tensor>> bias,
@@ -1015,6 +1061,8 @@ TORCH_LIBRARY_FRAGMENT(torch_ipex, m) {
   m.def("woq_linear_new_gelu(Tensor input, Tensor W_prepack) -> Tensor");
   m.def("woq_linear_relu(Tensor input, Tensor W_prepack) -> Tensor");
   m.def("woq_linear_silu(Tensor input, Tensor W_prepack) -> Tensor");
+  // silu(gate(x)) * up(x) of a gated MLP (Linear2SiluMul); no counterpart among the reference's operators, which calls the two above
+  m.def("woq_linear_silu_mul(Tensor input, Tensor W_gate, Tensor W_up) -> Tensor");
   m.def("woq_linear_add(Tensor input, Tensor W_prepack, Tensor[] others) -> Tensor");
   m.def("woq_linear_add_add(Tensor input, Tensor W_prepack, Tensor[] others) -> Tensor");
   m.def("woq_linear_mul(Tensor input, Tensor W_prepack, Tensor[] others) -> Tensor");
@@ -1045,6 +1093,7 @@ TORCH_LIBRARY_IMPL(torch_ipex, CUDA, m) {
   m.impl("woq_linear_add", TORCH_FN((woq_linear_binary<WOQ_HIP_FUSE_ADD, 1>)));
   m.impl("woq_linear_add_add", TORCH_FN((woq_linear_binary<WOQ_HIP_FUSE_ADD_ADD, 2>)));
   m.impl("woq_linear_mul", TORCH_FN((woq_linear_binary<WOQ_HIP_FUSE_MUL, 1>)));
+  m.impl("woq_linear_silu_mul", TORCH_FN(woq_linear_silu_mul));
   m.impl("woq_linear", TORCH_FN(woq_linear_v2));
   m.impl("dequantize_nf4", TORCH_FN(dequantize_nf4));
   m.impl("deepseek_moe_woq", TORCH_FN(deepseek_moe_woq));
@@ -1071,6 +1120,7 @@ TORCH_LIBRARY_IMPL(torch_ipex, CPU, m) {
   for (const char* name : {"ipex_woq_linear", "woq_linear_gelu", "woq_linear_new_gelu", "woq_linear_relu", "woq_linear_silu"})
     m.impl(name, TORCH_FN(refuse_cpu_2));
   for (const char* name : {"woq_linear_add", "woq_linear_add_add", "woq_linear_mul"}) m.impl(name, TORCH_FN(refuse_cpu_3));
+  m.impl("woq_linear_silu_mul", TORCH_FN(woq_linear_silu_mul));  // raises on its CPU input
   m.impl("woq_linear", TORCH_FN(woq_linear_v2));      // raises on its CPU input
   m.impl("dequantize_nf4", TORCH_FN(dequantize_nf4));  // raises on its CPU input
 }
@@ -1084,5 +1134,6 @@ TORCH_LIBRARY_IMPL(torch_ipex, AutocastCUDA, m) {
   m.impl("woq_linear_add", TORCH_FN((woq_linear_binary_autocast<WOQ_HIP_FUSE_ADD, 1>)));
   m.impl("woq_linear_add_add", TORCH_FN((woq_linear_binary_autocast<WOQ_HIP_FUSE_ADD_ADD, 2>)));
   m.impl("woq_linear_mul", TORCH_FN((woq_linear_binary_autocast<WOQ_HIP_FUSE_MUL, 1>)));
+  m.impl("woq_linear_silu_mul", TORCH_FN(woq_linear_silu_mul_autocast));
   m.impl("woq_linear", TORCH_FN(woq_linear_v2_autocast));
 }

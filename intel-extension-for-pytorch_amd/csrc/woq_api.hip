@@ -405,9 +405,58 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
                      : launch_gemm(f, wbits, regime, st);
 }
 
+// The pair's problem in FpArgs, or false where woq_hip_linear_pair does not take it.
+static bool pair_problem(const woq_hip_linear_params* g, const woq_hip_linear_params* u, FpArgs& f, int& wbits, int& regime) {
+  if (!g || !u || g->struct_size != sizeof(*g) || u->struct_size != sizeof(*u)) return false;
+  if (g->weight_dtype != WOQ_HIP_DTYPE_INT4 && g->weight_dtype != WOQ_HIP_DTYPE_INT8) return false;
+  if (u->weight_dtype != g->weight_dtype || u->M != g->M || u->K != g->K || u->N != g->N || u->group_size != g->group_size ||
+      u->lowp_mode != g->lowp_mode || u->x != g->x || u->x_dtype != g->x_dtype || u->out != g->out || u->out_dtype != g->out_dtype ||
+      u->stream != g->stream || (u->zeros_u8 != nullptr) != (g->zeros_u8 != nullptr))
+    return false;
+  if (g->M < 1 || g->K <= 0 || g->N <= 0 || g->x_dtype != WOQ_HIP_ACT_BF16 || g->out_dtype != g->x_dtype) return false;
+  if (g->fusion != WOQ_HIP_FUSE_NONE || u->fusion != WOQ_HIP_FUSE_NONE || g->force_kernel || u->force_kernel || g->debug_block_sums ||
+      u->debug_block_sums)
+    return false;
+  if (g->lowp_mode != WOQ_HIP_LOWP_BF16 && g->lowp_mode != WOQ_HIP_LOWP_NONE) return false;
+  if (g->group_size > 0 && g->group_size % 32 != 0) return false;
+  if (!g->x || !g->out || !g->qweight || !u->qweight || !g->scale_zero_bf16 || !u->scale_zero_bf16) return false;
+  wbits = wdtype_is_8bit(g->weight_dtype) ? 8 : 4;
+  const int tk = wbits == 4 ? kTileK4 : kTileK8;
+  regime = g->lowp_mode == WOQ_HIP_LOWP_BF16 && g->M < small_batch_threshold() ? kRegimeF16 : kRegimeBF16;
+  f = FpArgs{};
+  f.x = g->x; f.x_dtype = g->x_dtype; f.M = g->M; f.K = g->K; f.N = g->N;
+  f.NT = woq_hip_padded_n(g->N) / kTileN;
+  f.KT = woq_hip_padded_k(g->weight_dtype, g->K) / tk;
+  f.qweight = (const uint8_t*)g->qweight; f.scales = (const uint16_t*)g->scales_bf16; f.zeros = g->zeros_u8; f.szb = g->scale_zero_bf16;
+  f.G = g->group_size > 0 ? g->group_size : f.KT * tk;
+  f.KG = g->group_size > 0 ? (f.K + f.G - 1) / f.G : 1;
+  f.bias = g->bias; f.fusion = WOQ_HIP_FUSE_NONE; f.out = g->out; f.out_dtype = g->out_dtype;
+  f.pair = 1;
+  f.qweight_b = (const uint8_t*)u->qweight; f.scales_b = (const uint16_t*)u->scales_bf16; f.zeros_b = u->zeros_u8;
+  f.szb_b = u->scale_zero_bf16; f.bias_b = u->bias;
+  if (regime == kRegimeF16)
+    return g->scale_zero_f16x2 && u->scale_zero_f16x2 && decode_kernel_applies(f, wbits, regime, g->scale_zero_f16x2) && decode_pair_applies(f);
+  return decode_dq_pair_applies(f, wbits, regime);
+}
+
+int woq_hip_linear_pair_applies(const woq_hip_linear_params* gate, const woq_hip_linear_params* up) {
+  FpArgs f;
+  int wbits, regime;
+  return pair_problem(gate, up, f, wbits, regime) ? 1 : 0;
+}
+
+int woq_hip_linear_pair(const woq_hip_linear_params* gate, const woq_hip_linear_params* up) {
+  FpArgs f;
+  int wbits, regime;
+  if (!pair_problem(gate, up, f, wbits, regime)) return set_error("woq_linear_pair: not a pair that woq_hip_linear_pair_applies to");
+  hipStream_t st = (hipStream_t)gate->stream;
+  return regime == kRegimeF16 ? launch_decode(f, gate->scale_zero_f16x2, st, up->scale_zero_f16x2) : launch_decode_dq_pair(f, wbits, st);
+}
+
 // The problem of one expert of a grouped launch: arguments checked, FpArgs and compute type filled in (rows: the bound on a
 // slot's rows that selects the compute type).
 static int grouped_problem(const woq_hip_linear_params* p, const void* group, int64_t rows, FpArgs& f, int& wbits, int& regime) {
+  f = FpArgs{};
   if (!p || !group) return set_error("woq_linear_grouped: null params or group table");
   if (p->struct_size != sizeof(woq_hip_linear_params))
     return set_error("woq_linear_grouped: struct_size %u does not match this library (%zu)", p->struct_size,
@@ -448,12 +497,45 @@ static int grouped_problem(const woq_hip_linear_params* p, const void* group, in
   return 0;
 }
 
-int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, int64_t slots) {
+static int linear_grouped(const woq_hip_linear_params* p, const void* group, int64_t slots, int flags);
+static int linear_grouped_tiles(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows, int flags);
+
+int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, int64_t slots) { return linear_grouped(p, group, slots, 0); }
+int woq_hip_linear_grouped_tiles(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows) {
+  return linear_grouped_tiles(p, group, slots, tile_rows, 0);
+}
+
+// Post-op and tables of a woq_hip_moe_linear call on the problem of its two predecessors.
+static int moe_flags(const woq_hip_linear_params* p, int flags, FpArgs& f, int regime) {
+  if (flags & ~(WOQ_HIP_MOE_PAIR | WOQ_HIP_MOE_SZB)) return set_error("moe_linear: unknown flags 0x%x", flags);
+  f.grp_szb = (flags & WOQ_HIP_MOE_SZB) != 0 && regime == kRegimeBF16;
+  f.pair = (flags & WOQ_HIP_MOE_PAIR) != 0;
+  if (f.pair && p->fusion != WOQ_HIP_FUSE_NONE) return set_error("moe_linear: a pair takes no post-op");
+  return 0;
+}
+
+int woq_hip_moe_linear(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows, int flags) {
+  return tile_rows ? linear_grouped_tiles(p, group, slots, tile_rows, flags) : linear_grouped(p, group, slots, flags);
+}
+
+int woq_hip_moe_pair_applies(const woq_hip_linear_params* p, int tile_rows) {
+  FpArgs f;
+  int wbits, regime;
+  const int64_t rows = tile_rows ? tile_rows : p ? p->M : 0;
+  if (rows < 1 || grouped_problem(p, p, rows, f, wbits, regime) || f.NT % 2 != 0) return 0;
+  if (tile_rows) return 0;
+  if (p->scale_zero_f16x2)
+    return p->M <= 4 && decode_kernel_applies(f, wbits, regime, (const uint32_t*)p->scale_zero_f16x2) && decode_pair_applies(f);
+  return p->M <= 64 && decode_dq_pair_applies(f, wbits, regime);
+}
+
+static int linear_grouped(const woq_hip_linear_params* p, const void* group, int64_t slots, int flags) {
   FpArgs f;
   int wbits, regime;
   if (p && p->struct_size == sizeof(woq_hip_linear_params) && (p->M < 1 || p->M > 64))
     return set_error("woq_linear_grouped: 1..64 rows per slot, got M=%lld", (long long)p->M);
   if (int rc = grouped_problem(p, group, p ? p->M : 0, f, wbits, regime)) return rc;
+  if (int rc = moe_flags(p, flags, f, regime)) return rc;
   if (p->scale_zero_f16x2) {
     // up to four routed rows per slot on the integer-weight decode kernels: the group's scales table holds the
     // experts' (fp16 scale, fp16 128 + zero) dword tables
@@ -469,12 +551,13 @@ int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, in
 
 int64_t woq_hip_moe_chained_rows(int64_t K, int64_t N) { return K > 0 && N > 0 ? gemm_w4_split_rows(K, N) : 0; }
 
-int woq_hip_linear_grouped_tiles(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows) {
+static int linear_grouped_tiles(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows, int flags) {
   FpArgs f;
   int wbits, regime;
   if (tile_rows != 64 && tile_rows != 128) return set_error("woq_linear_grouped_tiles: 64 or 128 rows per slot, got %d", tile_rows);
   if (slots < 1 || slots > 65535) return set_error("woq_linear_grouped_tiles: bad slot count %lld", (long long)slots);
   if (int rc = grouped_problem(p, group, tile_rows, f, wbits, regime)) return rc;
+  if (int rc = moe_flags(p, flags, f, regime)) return rc;
   if (!gemm_w4_applies(f, wbits, regime))
     return set_error("woq_linear_grouped_tiles: K a multiple of 128, power-of-two groups (INT4: 32 and more, INT8: 128 and "
                      "more) or per-channel, 16-byte aligned rows in the compute type");

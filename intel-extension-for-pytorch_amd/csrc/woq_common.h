@@ -297,6 +297,13 @@ __device__ __forceinline__ void epilogue_store(const Epilogue& e, int64_t m, int
   store_act(e.out, e.out_dtype, idx, y);
 }
 
+// silu(gate) * up of a pair launch (FpArgs::pair) as the two launches round it, rounded once more by the store.
+template <int REGIME>
+__device__ __forceinline__ float pair_value(float gate, bool has_bias, float bias, float up, bool has_bias_b, float bias_b, int act_dtype) {
+  const float g = round_to_act(silu(round_to_act(finalize_acc<REGIME>(gate, has_bias, bias), act_dtype)), act_dtype);
+  return round_to_act(finalize_acc<REGIME>(up, has_bias_b, bias_b), act_dtype) * g;
+}
+
 // A pointer to global memory that every lane of the wave loaded from the same address, moved to scalar registers.  The cast
 // says which memory it is: a pointer put together from integers alone is generic, and loads through it are FLAT instructions,
 // after which no count but zero of s_waitcnt is defined (they count as memory and as LDS accesses and may return out of order

@@ -55,9 +55,13 @@ __device__ __forceinline__ f4 mfma16(u4 a, u4 b, f4 c) {
 // group's (scale, zero) dword; the lane columns are added at the end.
 // GROUPED (mixture of experts): the workgroups with blockIdx.z = s serve slot s, up to four routed rows of one expert,
 // whose packed weight, (scale, zero) table and bias come from pointer tables in device memory; an empty slot exits.
-template <bool XF16, int NTW, int MAXM, bool ONE_ROUND, int GPT, bool GROUPED, int KPW = kDecodeKPW>
+// PAIR (the front half of a gated MLP, FpArgs::pair): the two tiles of a workgroup are the same row-block of two weights, and the
+// tail stores silu(first) * second: one launch, its ramp and its activations instead of two, and no intermediate tensor
+// (one row, 4096 -> 2 x 14336 and back with a residual: 24.4 us in three launches, 19.7 in two).
+template <bool XF16, int NTW, int MAXM, bool ONE_ROUND, int GPT, bool GROUPED, int KPW = kDecodeKPW, bool PAIR = false>
 __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(const DecodeArgs a_in) {
   static_assert(GPT == 1 || GPT == 2 || GPT == 4, "groups of 128 x 2^k, 64 or 32");
+  static_assert(!PAIR || NTW == 2, "a row-block of each weight");
   DecodeArgs ag;
   int64_t xr[MAXM];  // GROUPED: the rows of x that the slot's rows read
   if constexpr (GROUPED) {
@@ -72,6 +76,11 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
     ag.qweight = dq_uniform((const uint8_t*)dq_uniform(g.qweight)[e]);
     ag.sz = dq_uniform((const uint32_t*)dq_uniform(g.scales)[e]);
     ag.bias = g.bias ? dq_uniform(dq_uniform(g.bias)[e]) : nullptr;
+    if constexpr (PAIR) {
+      ag.qweight_b = dq_uniform((const uint8_t*)dq_uniform(g.qweight_b)[e]);
+      ag.sz_b = dq_uniform((const uint32_t*)dq_uniform(g.scales_b)[e]);
+      ag.bias_b = g.bias_b ? dq_uniform(dq_uniform(g.bias_b)[e]) : nullptr;
+    }
     ag.out = (uint8_t*)a_in.out + row0 * a_in.N * 2;
     if (a_in.other0) ag.other0 = (const uint8_t*)a_in.other0 + row0 * a_in.N * 2;
 #pragma unroll
@@ -94,7 +103,7 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
   // the scalar unit and leaves one VGPR offset per stream
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int r = lane & 15, c = lane >> 4;
-  const int64_t nt0 = (int64_t)blockIdx.x * NTW;
+  const int64_t nt0 = (int64_t)blockIdx.x * (PAIR ? 1 : NTW);
 
   uint16_t* sx = (uint16_t*)smem + (size_t)wave * XROWS * SLICE;           // private [MAXM][SLICE] (+ zeros)
   f4* red = (f4*)(smem + (size_t)W * XROWS * SLICE * sizeof(uint16_t));    // [NTW][W][16]
@@ -125,6 +134,8 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
   const int xrow = G32 ? ((r >> 2) < GPT && (c >> (GPT == 2 ? 1 : 0)) == (r >> 2) ? (r & 3) : MAXM) : (r < MAXM ? r : 0);
   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void*)a.qweight, 0, (int)a.wbytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc((void*)a.sz, 0, (int)a.szbytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wrs_b = __builtin_amdgcn_make_buffer_rsrc((void*)(PAIR ? a.qweight_b : a.qweight), 0, (int)a.wbytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t srs_b = __builtin_amdgcn_make_buffer_rsrc((void*)(PAIR ? a.sz_b : a.sz), 0, (int)a.szbytes, 0x00020000);
 
   // 32-bit offsets from uniform base pointers keep the per-lane address state in one VGPR each
   // (the packed weight, its parameters and the activations are each far below 4 GiB)
@@ -160,12 +171,12 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
     for (int i = 0; i < KPW; ++i) {
 #pragma unroll
       for (int t = 0; t < NTW; ++t) {
-        const uint32_t nt = (uint32_t)nt0 + t;
+        const uint32_t nt = (uint32_t)nt0 + (PAIR ? 0 : t);
         const int woff = (int)((nt * (uint32_t)KT + (uint32_t)(ktw + i)) * (uint32_t)kTileBytes);
         const uint32_t grp = G32 ? (uint32_t)(ktw + i) * (uint32_t)GPT : (uint32_t)(ktw + i) >> tpg_shift;
         const int soff = (int)((nt * (uint32_t)KG + grp) * (uint32_t)(kTileN * sizeof(uint32_t)));
-        wreg[t][i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, woff, 2);  // non-temporal
-        szreg[t][i] = __builtin_amdgcn_raw_buffer_load_b32(srs, r4, soff, 0);
+        wreg[t][i] = __builtin_amdgcn_raw_buffer_load_b128(PAIR && t ? wrs_b : wrs, lane16, woff, 2);  // non-temporal
+        szreg[t][i] = __builtin_amdgcn_raw_buffer_load_b32(PAIR && t ? srs_b : srs, r4, soff, 0);
       }
     }
 
@@ -234,6 +245,26 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
 
   Epilogue ep{a.bias, a.fusion, a.other0, a.other1, a.out, a.out_dtype, a.x_dtype, a.N};
   const float* redf = (const float*)red;
+  if constexpr (PAIR) {
+    if (threadIdx.x < 64) {
+      const int e = threadIdx.x & 3, col = threadIdx.x >> 2;
+      const int64_t n = nt0 * kTileN + col;
+      if (e >= M || n >= a.N) return;
+      float s[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float part[16];
+#pragma unroll
+        for (int w = 0; w < 16; ++w) part[w] = w < W ? redf[((t * W + w) * 16 + col) * 4 + e] : 0.0f;
+        s[t] = part[0];
+#pragma unroll
+        for (int w = 1; w < 16; ++w) s[t] += part[w];
+      }
+      store_act(a.out, a.out_dtype, (int64_t)e * a.N + n,
+                pair_value<kRegimeF16>(s[0], a.bias != nullptr, a.bias ? a.bias[n] : 0.f, s[1], a.bias_b != nullptr, a.bias_b ? a.bias_b[n] : 0.f, a.x_dtype));
+    }
+    return;
+  }
   // one thread per output element (tile, column, row); its W <= 16 partial sums are fetched with
   // independent LDS reads (a rolled loop would pay one LDS round trip per wave) and added in wave
   // order
@@ -277,9 +308,10 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
 // elsewhere (read from a zeroed LDS slice, no instruction more), so D[4 c][n] -- the accumulator register the kernel
 // uses anyway -- is the sum over the group of lane column c alone, and that lane column applies the group's
 // (scale, zero) dword; one lane column per group is added at the end.
-template <bool XBF16, int NTW, int KPW, bool ONE_ROUND, bool GROUPED, int GPT>
+template <bool XBF16, int NTW, int KPW, bool ONE_ROUND, bool GROUPED, int GPT, bool PAIR = false>
 __global__ __launch_bounds__(KPW == 4 ? 512 : 1024, KPW == 2 ? 8 : 4) void woq_decode_m1_kernel(const DecodeArgs a_in) {
   static_assert(GPT == 1 || GPT == 2 || GPT == 4, "groups of 128 x 2^k, 64 or 32");
+  static_assert(!PAIR || NTW == 2, "a row-block of each weight");
   constexpr bool G32 = GPT > 1;       // the groups of a tile are kept apart
   constexpr int CS = GPT == 2 ? 1 : 0;  // lane columns per group, as a shift
   DecodeArgs ag;
@@ -294,6 +326,11 @@ __global__ __launch_bounds__(KPW == 4 ? 512 : 1024, KPW == 2 ? 8 : 4) void woq_d
     ag.qweight = dq_uniform((const uint8_t*)dq_uniform(g.qweight)[e]);
     ag.sz = dq_uniform((const uint32_t*)dq_uniform(g.scales)[e]);
     ag.bias = g.bias ? dq_uniform(dq_uniform(g.bias)[e]) : nullptr;
+    if constexpr (PAIR) {
+      ag.qweight_b = dq_uniform((const uint8_t*)dq_uniform(g.qweight_b)[e]);
+      ag.sz_b = dq_uniform((const uint32_t*)dq_uniform(g.scales_b)[e]);
+      ag.bias_b = g.bias_b ? dq_uniform(dq_uniform(g.bias_b)[e]) : nullptr;
+    }
     ag.x = a_in.x + xr * a_in.K;
     ag.out = (uint8_t*)a_in.out + row * a_in.N * 2;
     if (a_in.other0) ag.other0 = (const uint8_t*)a_in.other0 + row * a_in.N * 2;
@@ -305,7 +342,7 @@ __global__ __launch_bounds__(KPW == 4 ? 512 : 1024, KPW == 2 ? 8 : 4) void woq_d
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int r = lane & 15, c = lane >> 4;
-  const int64_t nt0 = (int64_t)blockIdx.x * NTW;
+  const int64_t nt0 = (int64_t)blockIdx.x * (PAIR ? 1 : NTW);
 
   // this wave's fp16 slice of the row (G32: followed by a slice of zeros)
   uint16_t* sx = (uint16_t*)smem + (size_t)wave * SLICE * (G32 ? 2 : 1);
@@ -322,6 +359,8 @@ __global__ __launch_bounds__(KPW == 4 ? 512 : 1024, KPW == 2 ? 8 : 4) void woq_d
   // launcher sends larger weights elsewhere); reads past the end return zero
   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void*)a.qweight, 0, (int)a.wbytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc((void*)a.sz, 0, (int)a.szbytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wrs_b = __builtin_amdgcn_make_buffer_rsrc((void*)(PAIR ? a.qweight_b : a.qweight), 0, (int)a.wbytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t srs_b = __builtin_amdgcn_make_buffer_rsrc((void*)(PAIR ? a.sz_b : a.sz), 0, (int)a.szbytes, 0x00020000);
 
   uint32_t mask_lo, mask_hi, magic_a, magic_b;
   asm volatile("s_mov_b32 %0, 0x000F000F" : "=s"(mask_lo));
@@ -370,12 +409,12 @@ __global__ __launch_bounds__(KPW == 4 ? 512 : 1024, KPW == 2 ? 8 : 4) void woq_d
     for (int i = 0; i < KPW; ++i) {
 #pragma unroll
       for (int t = 0; t < NTW; ++t) {
-        const uint32_t nt = (uint32_t)nt0 + t;
+        const uint32_t nt = (uint32_t)nt0 + (PAIR ? 0 : t);
         const int woff = (int)((nt * (uint32_t)KT + (uint32_t)(ktw + i)) * (uint32_t)kTileBytes);
         const uint32_t grp = G32 ? (uint32_t)(ktw + i) * (uint32_t)GPT : (uint32_t)(ktw + i) >> tpg_shift;
         const int soff = (int)((nt * (uint32_t)KG + grp) * (uint32_t)(kTileN * sizeof(uint32_t)));
-        wreg[t][i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, woff, 2);  // non-temporal
-        szreg[t][i] = __builtin_amdgcn_raw_buffer_load_b32(srs, r4, soff, 0);
+        wreg[t][i] = __builtin_amdgcn_raw_buffer_load_b128(PAIR && t ? wrs_b : wrs, lane16, woff, 2);  // non-temporal
+        szreg[t][i] = __builtin_amdgcn_raw_buffer_load_b32(PAIR && t ? srs_b : srs, r4, soff, 0);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -457,6 +496,23 @@ __global__ __launch_bounds__(KPW == 4 ? 512 : 1024, KPW == 2 ? 8 : 4) void woq_d
   }
   __syncthreads();
 
+  if constexpr (PAIR) {
+    if (threadIdx.x < 16) {
+      const int64_t n = nt0 * kTileN + (int)threadIdx.x;
+      float s[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const f4* mine = (const f4*)(red + (t * 16 + (int)threadIdx.x) * 16);
+        const f4 p0 = mine[0], p1 = mine[1], p2 = mine[2], p3 = mine[3];
+        s[t] = (((p0[0] + p0[1]) + (p0[2] + p0[3])) + ((p1[0] + p1[1]) + (p1[2] + p1[3]))) +
+               (((p2[0] + p2[1]) + (p2[2] + p2[3])) + ((p3[0] + p3[1]) + (p3[2] + p3[3])));
+      }
+      if (n < n_cols)
+        store_act(a.out, a.out_dtype, n,
+                  pair_value<kRegimeF16>(s[0], a.bias != nullptr, a.bias ? a.bias[n] : 0.f, s[1], a.bias_b != nullptr, a.bias_b ? a.bias_b[n] : 0.f, a.x_dtype));
+    }
+    return;
+  }
   if (threadIdx.x < NTW * 16) {
     const int col = threadIdx.x & 15, t = threadIdx.x >> 4;
     const int n = ((int)nt0 + t) * kTileN + col;
@@ -476,6 +532,42 @@ __global__ __launch_bounds__(KPW == 4 ? 512 : 1024, KPW == 2 ? 8 : 4) void woq_d
       }
     }
   }
+}
+
+// Pair launches (bf16 rows): the instances of two row-blocks, one of each weight, a workgroup for every row-block.
+template <int KPW, bool ONE_ROUND>
+static int launch_decode_m1_pair(const DecodeArgs& a, hipStream_t st, int slots) {
+  const bool apart = a.G == 32 || a.G == 64;
+  const size_t smem = (size_t)2 * 16 * 16 * sizeof(float) + (size_t)a.W * KPW * kTileK4 * sizeof(uint16_t) * (apart ? 2 : 1);
+  const dim3 grid((unsigned)a.NT, 1, (unsigned)(slots > 0 ? slots : 1));
+#define WOQ_M1_PAIR(GR, GPT) woq_decode_m1_kernel<true, 2, KPW, ONE_ROUND, GR, GPT, true><<<grid, a.W * 64, smem, st>>>(a)
+  if (slots > 0)
+    a.G == 32 ? WOQ_M1_PAIR(true, 4) : a.G == 64 ? WOQ_M1_PAIR(true, 2) : WOQ_M1_PAIR(true, 1);
+  else
+    a.G == 32 ? WOQ_M1_PAIR(false, 4) : a.G == 64 ? WOQ_M1_PAIR(false, 2) : WOQ_M1_PAIR(false, 1);
+#undef WOQ_M1_PAIR
+  return check_launch("woq_decode_m1_kernel");
+}
+template <bool ONE_ROUND, int GPT, bool GROUPED>
+static int launch_decode_pair_g(const DecodeArgs& a, hipStream_t st, int slots) {
+  const size_t smem = (size_t)2 * a.W * 16 * sizeof(f4) + (size_t)a.W * (4 + (GPT > 1 ? 1 : 0)) * kDecodeKPW * kTileK4 * sizeof(uint16_t);
+  auto kern = woq_decode_kernel<false, 2, 4, ONE_ROUND, GPT, GROUPED, kDecodeKPW, true>;
+  if (smem > 64 * 1024) {
+    hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (err != hipSuccess) return set_error("hipFuncSetAttribute: %s", hipGetErrorString(err));
+  }
+  kern<<<dim3((unsigned)a.NT, 1, (unsigned)(GROUPED ? slots : 1)), a.W * 64, smem, st>>>(a);
+  return check_launch("woq_decode_kernel");
+}
+template <bool ONE_ROUND>
+static int launch_decode_pair(const DecodeArgs& a, hipStream_t st, int slots) {
+  if (slots > 0)
+    return a.G == 32   ? launch_decode_pair_g<ONE_ROUND, 4, true>(a, st, slots)
+           : a.G == 64 ? launch_decode_pair_g<ONE_ROUND, 2, true>(a, st, slots)
+                       : launch_decode_pair_g<ONE_ROUND, 1, true>(a, st, slots);
+  return a.G == 32   ? launch_decode_pair_g<ONE_ROUND, 4, false>(a, st, 0)
+         : a.G == 64 ? launch_decode_pair_g<ONE_ROUND, 2, false>(a, st, 0)
+                     : launch_decode_pair_g<ONE_ROUND, 1, false>(a, st, 0);
 }
 
 template <bool XBF16, int NTW, int KPW, bool ONE_ROUND>
@@ -534,9 +626,30 @@ bool decode_kernel_applies(const FpArgs& f, int wbits, int regime, const uint32_
          (f.K % (kDecodeKPW * kTileK4)) == 0 && (f.x_dtype == WOQ_HIP_ACT_BF16 || f.x_dtype == WOQ_HIP_ACT_FP16);
 }
 
-static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t st, const MoeGroup* grp, int slots);
+// Two to four rows of a long K run eight K tiles a wave in one round: no pair instance (its registers would not hold both tiles).
+static bool eight_tiles(const FpArgs& f, bool one_round) {
+  return !one_round && f.KT % 8 == 0 && f.KT / 8 <= 16 && f.G != 32 && f.G != 64;
+}
+// waves per workgroup: cover K in as few equal rounds as possible, at most 16 waves
+static int decode_waves(const FpArgs& f) {
+  int64_t w = (f.KT + kDecodeKPW - 1) / kDecodeKPW;
+  if (w > 16) {
+    const int64_t rounds = (w + 15) / 16;
+    w = (w + rounds - 1) / rounds;
+  }
+  return (int)w;
+}
+bool decode_pair_applies(const FpArgs& f) {
+  return f.x_dtype == WOQ_HIP_ACT_BF16 && f.out_dtype == WOQ_HIP_ACT_BF16 &&
+         (f.M == 1 || !eight_tiles(f, f.KT == (int64_t)decode_waves(f) * kDecodeKPW));
+}
 
-int launch_decode(const FpArgs& f, const uint32_t* sz, hipStream_t st) { return launch_decode_impl(f, sz, st, nullptr, 0); }
+static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t st, const MoeGroup* grp, int slots,
+                              const uint32_t* sz_b = nullptr);
+
+int launch_decode(const FpArgs& f, const uint32_t* sz, hipStream_t st, const uint32_t* sz_b) {
+  return launch_decode_impl(f, sz, st, nullptr, 0, sz_b);
+}
 
 int launch_decode_grouped(const FpArgs& f, const MoeGroup* grp, int64_t slots, hipStream_t st) {
   if (!grp || slots < 1 || slots > 65535) return set_error("woq_linear_grouped: 1..65535 slots and a group table");
@@ -544,9 +657,11 @@ int launch_decode_grouped(const FpArgs& f, const MoeGroup* grp, int64_t slots, h
   return launch_decode_impl(f, nullptr, st, grp, (int)slots);
 }
 
-static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t st, const MoeGroup* grp, int slots) {
+static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t st, const MoeGroup* grp, int slots, const uint32_t* sz_b) {
+  if (f.pair && !decode_pair_applies(f)) return set_error("woq_decode_kernel: no pair launch for this problem");
   DecodeArgs a;
   a.grp = grp;
+  a.qweight_b = f.qweight_b; a.sz_b = sz_b; a.bias_b = f.bias_b;
   a.x = (const uint16_t*)f.x;
   a.x_dtype = f.x_dtype;
   a.M = f.M; a.K = f.K; a.N = f.N; a.NT = f.NT; a.KT = f.KT;
@@ -558,13 +673,7 @@ static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t s
   a.Kpad = f.KT * kTileK4;
   a.tpg_shift = 0;
   while ((int64_t)kTileK4 << (a.tpg_shift + 1) <= f.G && a.tpg_shift < 30) ++a.tpg_shift;
-  // waves per workgroup: cover K in as few equal rounds as possible, at most 16 waves
-  int64_t w = (f.KT + kDecodeKPW - 1) / kDecodeKPW;
-  if (w > 16) {
-    const int64_t rounds = (w + 15) / 16;
-    w = (w + rounds - 1) / rounds;
-  }
-  a.W = (int)w;
+  a.W = decode_waves(f);
   const bool xf16 = f.x_dtype == WOQ_HIP_ACT_FP16;
   // Two row-blocks per workgroup from 512 row-blocks on; a single row only above 768: up to there one
   // row-block per workgroup spreads more evenly over the 256 CUs (M = 1: 8192 -> 10240 9.6 us against
@@ -575,11 +684,12 @@ static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t s
   a.szbytes = (uint32_t)(f.NT * f.KG * kTileN * (int64_t)sizeof(uint32_t));
   const bool one_row = f.M == 1;
   const bool one_round = f.KT == (int64_t)a.W * kDecodeKPW;
-  if (one_row && !one_round && f.KT % 8 == 0 && f.KT / 8 <= 16 && f.G != 32 && f.G != 64) {
+  if (one_row && eight_tiles(f, one_round)) {
     // A long K in one round: eight K tiles per wave (8 KiB in flight per wave, a budget of 128 registers) instead of
     // several rounds of two, each of which waits for its own requests (M = 1, 14336 -> 4096: 7.48 against 7.71 us,
     // 8192 -> 8192 8.04 against 8.39 us; with groups of 32 the larger zeroed slice makes it a loss, 8.6 against 8.2 us).
     a.W = (int)(f.KT / 8);
+    if (f.pair) return launch_decode_m1_pair<8, true>(a, st, slots);
     if (xf16) return two ? launch_decode_m1_cfg<false, 2, 8, true>(a, st, slots) : launch_decode_m1_cfg<false, 1, 8, true>(a, st, slots);
     return two ? launch_decode_m1_cfg<true, 2, 8, true>(a, st, slots) : launch_decode_m1_cfg<true, 1, 8, true>(a, st, slots);
   }
@@ -591,16 +701,19 @@ static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t s
     const int64_t waves2 = (f.NT / (two ? 2 : 1)) * ((f.KT + 1) / 2);
     if (waves2 <= 2048 && f.KT % 4 == 0 && f.KT / 4 <= 8) {
       a.W = (int)(f.KT / 4);
+      if (f.pair) return launch_decode_m1_pair<4, true>(a, st, slots);
       if (xf16) return two ? launch_decode_m1_cfg<false, 2, 4, true>(a, st, slots) : launch_decode_m1_cfg<false, 1, 4, true>(a, st, slots);
       return two ? launch_decode_m1_cfg<true, 2, 4, true>(a, st, slots) : launch_decode_m1_cfg<true, 1, 4, true>(a, st, slots);
     }
+    if (f.pair) return one_round ? launch_decode_m1_pair<2, true>(a, st, slots) : launch_decode_m1_pair<2, false>(a, st, slots);
 #define WOQ_DECODE_M1(XB, NTW) \
   (one_round ? launch_decode_m1_cfg<XB, NTW, 2, true>(a, st, slots) : launch_decode_m1_cfg<XB, NTW, 2, false>(a, st, slots))
     if (xf16) return two ? WOQ_DECODE_M1(false, 2) : WOQ_DECODE_M1(false, 1);
     return two ? WOQ_DECODE_M1(true, 2) : WOQ_DECODE_M1(true, 1);
 #undef WOQ_DECODE_M1
   }
-  if (!one_round && f.KT % 8 == 0 && f.KT / 8 <= 16 && f.G != 32 && f.G != 64 && !two) {
+  if (f.pair) return one_round ? launch_decode_pair<true>(a, st, slots) : launch_decode_pair<false>(a, st, slots);
+  if (eight_tiles(f, one_round) && !two) {
     // a long K in one round of eight K tiles per wave, as for one row above (M = 4, 14336 -> 4096: 8.9 against 9.2 us)
     a.W = (int)(f.KT / 8);
     if (slots > 0)

@@ -118,12 +118,17 @@ __device__ __forceinline__ u4 dq_dequant_m(uint32_t d, const G4Masks& k, uint32_
   return r;
 }
 
-// SZB (bf16 compute, integer weights, not GROUPED): scale and zero point of a (row, group) come as one dword
+// SZB (bf16 compute, integer weights; GROUPED: with the group's szb tables): scale and zero point of a (row, group) come as one dword
 // (f.szb): one request and three vector instructions per row-block and round instead of two and eight.
-template <int REGIME, int WBITS, int MT, int NTW, bool NF4, bool XCONV, bool FP8, bool GROUPED, bool SZB = false>
+// PAIR (the front half of a gated MLP, FpArgs::pair; SZB instances): the first half of a workgroup's row-blocks are the gate
+// projection's, the second half the same row-blocks of the up projection; the tail stores silu(gate) * up
+// (16 rows, 4096 -> 2 x 14336: 25 us in two launches, 20 in one).
+template <int REGIME, int WBITS, int MT, int NTW, bool NF4, bool XCONV, bool FP8, bool GROUPED, bool SZB = false, bool PAIR = false>
 __global__ __launch_bounds__(512, (MT * NTW > 8 ? 2 : 4)) void woq_decode_dq_kernel(const DecodeDqArgs a) {
   static_assert(!XCONV || (REGIME == kRegimeF16 && MT == 1), "bf16 -> fp16 rows: fp16 regime, one row tile");
-  static_assert(!SZB || (REGIME == kRegimeBF16 && !NF4 && !FP8 && !GROUPED), "merged parameters: bf16 compute, integer weights");
+  static_assert(!SZB || (REGIME == kRegimeBF16 && !NF4 && !FP8), "merged parameters: bf16 compute, integer weights");
+  static_assert(!PAIR || (SZB && NTW % 2 == 0), "pairs: merged parameters, as many row-blocks of each weight");
+  constexpr int NTO = PAIR ? NTW / 2 : NTW;  // row-blocks of the output
   using Geo = DqGeom<WBITS, MT>;
   constexpr int TK = Geo::TK, NJ = Geo::NJ, NX = Geo::NX, SLICE = Geo::SLICE;
   static_assert(!NF4 || WBITS == 4, "NF4 codes are 4 bits wide");
@@ -151,6 +156,12 @@ __global__ __launch_bounds__(512, (MT * NTW > 8 ? 2 : 4)) void woq_decode_dq_ker
     fg.scales = dq_uniform((const uint16_t*)dq_uniform(g.scales)[e]);
     fg.zeros = g.zeros ? dq_uniform(dq_uniform(g.zeros)[e]) : nullptr;
     fg.bias = g.bias ? dq_uniform(dq_uniform(g.bias)[e]) : nullptr;
+    if constexpr (SZB) fg.szb = dq_uniform(dq_uniform(g.szb)[e]);
+    if constexpr (PAIR) {
+      fg.qweight_b = dq_uniform((const uint8_t*)dq_uniform(g.qweight_b)[e]);
+      fg.szb_b = dq_uniform(dq_uniform(g.szb_b)[e]);
+      fg.bias_b = g.bias_b ? dq_uniform(dq_uniform(g.bias_b)[e]) : nullptr;
+    }
     const int64_t out_elt = fg.out_dtype == WOQ_HIP_ACT_FP32 ? 4 : 2, x_elt = 2;  // rows are 16-bit here
     fg.out = (uint8_t*)fg.out + row0 * fg.N * out_elt;
     if (fg.other0) fg.other0 = (const uint8_t*)fg.other0 + row0 * fg.N * x_elt;
@@ -168,7 +179,7 @@ __global__ __launch_bounds__(512, (MT * NTW > 8 ? 2 : 4)) void woq_decode_dq_ker
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int r = lane & 15, c = lane >> 4;
   const int M = (int)f.M, K = (int)f.K, KT = (int)f.KT, KG = (int)f.KG;
-  const int64_t nt0 = (int64_t)blockIdx.x * NTW;
+  const int64_t nt0 = (int64_t)blockIdx.x * NTO;
   uint8_t* const sx = smem + wave * (2 * SLICE);  // this wave's two activation buffers
   f4* const red = (f4*)smem;                      // [NTW * MT][W][64], after the K loop
 
@@ -211,10 +222,10 @@ __global__ __launch_bounds__(512, (MT * NTW > 8 ? 2 : 4)) void woq_decode_dq_ker
   for (int t = 0; t < NTW; ++t) {
     // the row-blocks per workgroup need not divide the row-blocks: the last workgroup reads its
     // missing ones from the last real row-block, and the store below drops their columns (n >= N)
-    const int64_t nt = nt0 + t < f.NT ? nt0 + t : f.NT - 1;
-    wbase[t] = f.qweight + (size_t)nt * KT * kTileBytes;
+    const int64_t nt = nt0 + t % NTO < f.NT ? nt0 + t % NTO : f.NT - 1;
+    wbase[t] = (t < NTO ? f.qweight : f.qweight_b) + (size_t)nt * KT * kTileBytes;
     if constexpr (SZB) {
-      sbase[t] = (const uint8_t*)f.szb + (size_t)nt * KG * (kTileN * 4);
+      sbase[t] = (const uint8_t*)(t < NTO ? f.szb : f.szb_b) + (size_t)nt * KG * (kTileN * 4);
       zbase[t] = sbase[t];
     } else {
       sbase[t] = (const uint8_t*)(f.scales + (size_t)nt * KG * kTileN);
@@ -383,6 +394,17 @@ __global__ __launch_bounds__(512, (MT * NTW > 8 ? 2 : 4)) void woq_decode_dq_ker
     else
       epilogue_store<REGIME>(ep, m, n, s);
   };
+  if constexpr (PAIR) {
+    for (int idx = threadIdx.x; idx < kTileElems / 2; idx += blockDim.x) {
+      const int col = idx & 15, tm = idx >> 8, t = tm / MT, m = (tm - t * MT) * 16 + ((idx >> 4) & 15);
+      const int64_t n = (nt0 + t) * kTileN + col;
+      if (m >= M || n >= f.N) continue;
+      store_act(f.out, f.out_dtype, (int64_t)m * f.N + n,
+                pair_value<REGIME>(wave_sum(idx), f.bias != nullptr, f.bias ? f.bias[n] : 0.f, wave_sum(idx + kTileElems / 2), f.bias_b != nullptr,
+                                   f.bias_b ? f.bias_b[n] : 0.f, f.x_dtype));
+    }
+    return;
+  }
   const int S = (int)gridDim.y;
   if (S == 1) {
     for (int idx = threadIdx.x; idx < kTileElems; idx += blockDim.x) store(idx, wave_sum(idx));
@@ -416,7 +438,7 @@ __global__ __launch_bounds__(512, (MT * NTW > 8 ? 2 : 4)) void woq_decode_dq_ker
   if (threadIdx.x == 0) __hip_atomic_store(a.counters + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int REGIME, int WBITS, int MT, int NTW, bool NF4, bool XCONV, bool FP8, bool GROUPED, bool SZB>
+template <int REGIME, int WBITS, int MT, int NTW, bool NF4, bool XCONV, bool FP8, bool GROUPED, bool SZB, bool PAIR = false>
 static int launch_dq_cfg_impl(DecodeDqArgs a, int splits, hipStream_t st, int slots) {
   using Geo = DqGeom<WBITS, MT>;
   if (MT > 2 && splits > 1) return set_error("woq_decode_dq_kernel: split K takes at most 32 rows");
@@ -427,7 +449,8 @@ static int launch_dq_cfg_impl(DecodeDqArgs a, int splits, hipStream_t st, int sl
   // four row tiles (33..64 rows) a wave's two buffers are 32 KiB and one workgroup of four waves takes
   // 128 KiB.  Sixteen waves of one row tile measured no faster than eight.
   constexpr int kLdsMax = 131072;
-  const dim3 grid((unsigned)((a.f.NT + NTW - 1) / NTW), (unsigned)splits, (unsigned)slots);
+  constexpr int NTO = PAIR ? NTW / 2 : NTW;
+  const dim3 grid((unsigned)((a.f.NT + NTO - 1) / NTO), (unsigned)splits, (unsigned)slots);
   const bool alone = MT == 2 && grid.x * grid.y <= 256;
   const int lds_cap = (MT > 2 || alone) ? kLdsMax : 65536;
   const int max_w = lds_cap / (2 * Geo::SLICE);
@@ -437,7 +460,7 @@ static int launch_dq_cfg_impl(DecodeDqArgs a, int splits, hipStream_t st, int sl
   size_t smem = (size_t)a.W * 2 * Geo::SLICE;
   const size_t red = (size_t)NTW * MT * a.W * 64 * sizeof(f4);
   if (red > smem) smem = red;
-  auto kern = woq_decode_dq_kernel<REGIME, WBITS, MT, NTW, NF4, XCONV, FP8, GROUPED, SZB>;
+  auto kern = woq_decode_dq_kernel<REGIME, WBITS, MT, NTW, NF4, XCONV, FP8, GROUPED, SZB, PAIR>;
   if (MT >= 2) {
     // more than 64 KiB of LDS per workgroup needs an opt-in (once per kernel and process)
     static const hipError_t lds_optin =
@@ -451,6 +474,10 @@ static int launch_dq_cfg_impl(DecodeDqArgs a, int splits, hipStream_t st, int sl
 
 template <int REGIME, int WBITS, int MT, int NTW, bool NF4 = false, bool XCONV = false, bool FP8 = false, bool GROUPED = false>
 static int launch_dq_cfg(DecodeDqArgs a, int splits, hipStream_t st, int slots = 1) {
+  if constexpr (REGIME == kRegimeBF16 && !NF4 && !FP8 && GROUPED && !XCONV) {
+    if (a.f.pair) return launch_dq_cfg_impl<REGIME, WBITS, MT, NTW, NF4, XCONV, FP8, GROUPED, true, true>(a, splits, st, slots);
+    if (a.f.grp_szb) return launch_dq_cfg_impl<REGIME, WBITS, MT, NTW, NF4, XCONV, FP8, GROUPED, true>(a, splits, st, slots);
+  }
   if constexpr (REGIME == kRegimeBF16 && !NF4 && !FP8 && !GROUPED && !XCONV) {
     // the caller's merged (scale, zero) dword table: one parameter request per row-block and round
     if (a.f.szb) return launch_dq_cfg_impl<REGIME, WBITS, MT, NTW, NF4, XCONV, FP8, GROUPED, true>(a, splits, st, slots);
@@ -469,6 +496,11 @@ bool decode_dq_applies(const FpArgs& f, int wbits, int regime) {
   if (f.K % tk != 0 || f.M * f.K * 2 >= (int64_t)1 << 31) return false;
   if (f.G >= f.KT * tk) return true;
   return f.G >= (wbits == 4 ? 32 : 16) && (f.G & (f.G - 1)) == 0;
+}
+
+bool decode_dq_pair_applies(const FpArgs& f, int wbits, int regime) {
+  return regime == kRegimeBF16 && !f.nf4 && !f.fp8 && f.x_dtype == WOQ_HIP_ACT_BF16 && f.out_dtype == WOQ_HIP_ACT_BF16 &&
+         decode_dq_applies(f, wbits, regime);
 }
 
 template <int REGIME, int WBITS, bool FP8 = false>
@@ -543,6 +575,7 @@ static int launch_dq_grouped_regime(const DecodeDqArgs& a, int slots, hipStream_
 int launch_decode_dq_grouped(const FpArgs& f, int wbits, int regime, const MoeGroup* grp, int64_t slots, hipStream_t st) {
   if (!grp || slots < 1 || slots > 65535) return set_error("woq_linear_grouped: 1..65535 slots and a group table");
   if (f.nf4 || f.fp8) return set_error("woq_linear_grouped: INT4 and INT8 weights");
+  if (f.pair && (!decode_dq_pair_applies(f, wbits, regime) || !f.grp_szb)) return set_error("woq_decode_dq_kernel: no pair launch for this problem");
   if (f.NT % 2 != 0) return set_error("woq_linear_grouped: an even number of row-blocks (N a multiple of 32 after padding)");
   if (!decode_dq_applies(f, wbits, regime))
     return set_error("woq_linear_grouped: at most 64 rows per slot, K a multiple of the weight tile, a power-of-two or "
@@ -564,6 +597,34 @@ int launch_decode_dq_grouped(const FpArgs& f, int wbits, int regime, const MoeGr
                                 : launch_dq_grouped_regime<kRegimeBF16, 4>(a, (int)slots, st);
   return regime == kRegimeF16 ? launch_dq_grouped_regime<kRegimeF16, 8>(a, (int)slots, st)
                               : launch_dq_grouped_regime<kRegimeBF16, 8>(a, (int)slots, st);
+}
+
+// One or two row-blocks of each weight per workgroup, by the rule of launch_decode_dq with the two weights' row-blocks; K is
+// never shared.
+int launch_decode_dq_pair(const FpArgs& f, int wbits, hipStream_t st) {
+  if (!decode_dq_pair_applies(f, wbits, kRegimeBF16) || !f.szb || !f.szb_b)
+    return set_error("woq_decode_dq_kernel: no pair launch for this problem");
+  DecodeDqArgs a;
+  a.f = f;
+  a.partial = nullptr;
+  a.counters = nullptr;
+  a.grp = nullptr;
+  a.W = 1;
+  a.KTs = (int)f.KT;
+  a.g_shift = 30;
+  if (f.G < f.KT * (wbits == 4 ? kTileK4 : kTileK8)) {
+    a.g_shift = 0;
+    while (((int64_t)1 << a.g_shift) < f.G) ++a.g_shift;
+  }
+  const double per = f.M > 32 ? 2.5 : 1.9, fixed = f.M > 32 ? 7.0 : 1.0;
+  auto cost = [&](int blocks) { return (double)(((f.NT + blocks / 2 - 1) / (blocks / 2) + 255) / 256) * (blocks * per + fixed); };
+  const bool four = cost(4) <= cost(2);
+#define WOQ_DQ_PAIR(WB, MT) (four ? launch_dq_cfg_impl<kRegimeBF16, WB, MT, 4, false, false, false, false, true, true>(a, 1, st, 1) \
+                                  : launch_dq_cfg_impl<kRegimeBF16, WB, MT, 2, false, false, false, false, true, true>(a, 1, st, 1))
+#define WOQ_DQ_PAIR_ROWS(WB) (f.M > 32 ? WOQ_DQ_PAIR(WB, 4) : f.M > 16 ? WOQ_DQ_PAIR(WB, 2) : WOQ_DQ_PAIR(WB, 1))
+  return wbits == 4 ? WOQ_DQ_PAIR_ROWS(4) : WOQ_DQ_PAIR_ROWS(8);
+#undef WOQ_DQ_PAIR_ROWS
+#undef WOQ_DQ_PAIR
 }
 
 int64_t decode_dq_splitk_bytes(int64_t M, int64_t NT, int splits) {

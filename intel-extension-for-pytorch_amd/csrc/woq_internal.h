@@ -26,6 +26,14 @@ struct MoeGroup {
   const void* const* scales;   // [experts] scales in the regime's dtype
   const uint8_t* const* zeros; // [experts] or null
   const float* const* bias;    // [experts] or null
+  // read by launches that are told of them only:
+  const uint32_t* const* szb;  // [experts] merged (scale, zero) dword tables (FpArgs::szb)
+  // pair launches: the up projections (qweight .. szb are the gate projections then)
+  const void* const* qweight_b;
+  const void* const* scales_b;
+  const uint8_t* const* zeros_b;
+  const float* const* bias_b;
+  const uint32_t* const* szb_b;
 };
 
 struct FpArgs {
@@ -49,6 +57,16 @@ struct FpArgs {
   int out_dtype;
   int nf4;  // 4-bit codes index the NF4 table instead of standing for integers (zeros == nullptr)
   int fp8;  // 8-bit weights are float8 e4m3fn bytes, not offset-binary integers (zeros == nullptr)
+  // Pair launch: out = silu(x W^T + bias) * (x Wb^T + bias_b), the front half of a gated MLP; the second weight has the first
+  // one's shape, type and groups.  The rounding is that of the two launches: every value goes through the activation type
+  // where a launch would have stored it.
+  int pair = 0;
+  const uint8_t* qweight_b = nullptr;
+  const uint16_t* scales_b = nullptr;
+  const uint8_t* zeros_b = nullptr;
+  const uint32_t* szb_b = nullptr;
+  const float* bias_b = nullptr;
+  int grp_szb = 0;  // grouped launches: the group's szb tables (and szb_b) are there
 };
 
 // Split-K scratch of the dequantizing decode kernel: fp32 partial tiles, and one counter per
@@ -110,9 +128,14 @@ struct DecodeArgs {
   int tpg_shift;  // log2(G / 128)
   uint32_t wbytes, szbytes;  // extents of qweight and sz: the single-row kernel addresses them with 32-bit offsets
   const MoeGroup* grp;       // GROUPED instances of the single-row kernel: one routed row per slot (blockIdx.z)
+  const uint8_t* qweight_b;  // PAIR instances: the second weight, its (scale, zero) table and bias
+  const uint32_t* sz_b;
+  const float* bias_b;
 };
 bool decode_kernel_applies(const FpArgs& f, int wbits, int regime, const uint32_t* sz);
-int launch_decode(const FpArgs& f, const uint32_t* sz, hipStream_t st);
+int launch_decode(const FpArgs& f, const uint32_t* sz, hipStream_t st, const uint32_t* sz_b = nullptr);
+// whether launch_decode / launch_decode_grouped take the pair (f.pair) of a problem that decode_kernel_applies to
+bool decode_pair_applies(const FpArgs& f);
 // One routed row per slot, the experts' (scale, zero) dword tables in grp->scales.
 int launch_decode_grouped(const FpArgs& f, const MoeGroup* grp, int64_t slots, hipStream_t st);
 
@@ -140,6 +163,8 @@ int launch_fp32(const Fp32Args& f, int wbits, hipStream_t st);
 // splits: workgroups that share the K tiles of a row-block set (1, 2 or 4; more than 1 needs the
 // scratch and at most 32 rows), 0 = automatic (only together with ntw = 0)
 bool decode_dq_applies(const FpArgs& f, int wbits, int regime);
+bool decode_dq_pair_applies(const FpArgs& f, int wbits, int regime);  // launch_decode_dq_pair / the grouped launch with f.pair
+int launch_decode_dq_pair(const FpArgs& f, int wbits, hipStream_t st);
 int launch_decode_dq_grouped(const FpArgs& f, int wbits, int regime, const MoeGroup* grp, int64_t slots, hipStream_t st);
 int launch_decode_dq(const FpArgs& f, int wbits, int regime, hipStream_t st, int ntw = 0, int splits = 1,
                      const SplitKScratch* scratch = nullptr);

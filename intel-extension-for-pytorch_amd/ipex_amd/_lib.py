@@ -20,6 +20,7 @@ LOWP_NONE, LOWP_FP16, LOWP_BF16, LOWP_INT8 = 0, 1, 2, 3
 ACT_FP32, ACT_FP16, ACT_BF16 = 0, 1, 2
 FUSE_NONE, FUSE_GELU_ERF, FUSE_GELU_TANH, FUSE_RELU, FUSE_SILU = 0x0, 0x1, 0x2, 0x3, 0x4
 FUSE_ADD, FUSE_ADD_ADD, FUSE_MUL = 0x10, 0x20, 0x30
+MOE_PAIR, MOE_SZB = 1, 2
 TILE_N, TILE_BYTES, TILE_K_INT4, TILE_K_INT8 = 16, 1024, 128, 64
 
 EXPORTS = [
@@ -55,6 +56,10 @@ EXPORTS = [
     "woq_hip_moe_route_tiles",
     "woq_hip_linear_grouped_tiles",
     "woq_hip_moe_chained_rows",
+    "woq_hip_linear_pair_applies",
+    "woq_hip_linear_pair",
+    "woq_hip_moe_pair_applies",
+    "woq_hip_moe_linear",
     "woq_hip_moe_combine_rows",
 ]
 
@@ -176,6 +181,14 @@ def load():
         lib.woq_hip_moe_route_tiles.argtypes = [vp, i64, i64, i64, i64, i64, i64, i64, vp, vp, vp, vp, vp]
         lib.woq_hip_linear_grouped_tiles.restype = i32
         lib.woq_hip_linear_grouped_tiles.argtypes = [ctypes.POINTER(LinearParams), vp, i64, i32]
+        lib.woq_hip_linear_pair_applies.restype = i32
+        lib.woq_hip_linear_pair_applies.argtypes = [ctypes.POINTER(LinearParams), ctypes.POINTER(LinearParams)]
+        lib.woq_hip_linear_pair.restype = i32
+        lib.woq_hip_linear_pair.argtypes = [ctypes.POINTER(LinearParams), ctypes.POINTER(LinearParams)]
+        lib.woq_hip_moe_pair_applies.restype = i32
+        lib.woq_hip_moe_pair_applies.argtypes = [ctypes.POINTER(LinearParams), i32]
+        lib.woq_hip_moe_linear.restype = i32
+        lib.woq_hip_moe_linear.argtypes = [ctypes.POINTER(LinearParams), vp, i64, i32, i32]
         lib.woq_hip_moe_chained_rows.restype = i64
         lib.woq_hip_moe_chained_rows.argtypes = [i64, i64]
         lib.woq_hip_moe_combine_rows.restype = i32

@@ -113,7 +113,7 @@ class LinearSiluMul(_LinearFusion):
 class Linear2SiluMul(nn.Module):
     r"""``silu(linear_s(x)) * linear_m(x)``, the gated-MLP front half (linear_fusion.py:93-132):
     ``woq_linear_silu`` on the gate, then ``woq_linear_mul`` on the up projection with the gate as
-    its multiplicand (fusions/linear_fusion.py:475-490)."""
+    its multiplicand (fusions/linear_fusion.py:475-490), or both in one launch."""
 
     def __init__(self, linear_s, linear_m):
         super().__init__()
@@ -123,8 +123,7 @@ class Linear2SiluMul(nn.Module):
     def forward(self, x):
         hs, hm = _woq_handle(self.linear_s), _woq_handle(self.linear_m)
         if hs is not None and hm is not None:
-            y = torch.ops.torch_ipex.woq_linear_silu(x, hs)
-            return torch.ops.torch_ipex.woq_linear_mul(x, hm, [y])
+            return torch.ops.torch_ipex.woq_linear_silu_mul(x, hs, hm)
         return nn.functional.silu(self.linear_s(x)) * self.linear_m(x)
 
 

@@ -704,13 +704,14 @@ def _context_epochs():
 
 def _context_pointers(ctx):
     """[qweight, fp16 scales, bf16 scales, zero points or 0, fp32 bias or 0, N, K, group size, weight dtype,
-    lowp_mode, has g_idx, device index, (scale, zero) dword table or 0] of a context of either binding."""
+    lowp_mode, has g_idx, device index, (scale, zero) dword table or 0, merged bf16 table or 0] of a context of either binding."""
     if _is_python_context(ctx):
         ptr = lambda t: 0 if t is None else t.data_ptr()
         N, K = ctx.weight_shape_
         return [ctx.at_weight_.data_ptr(), ctx.scales_list_[1].data_ptr(), ctx.scales_list_[2].data_ptr(),
                 ptr(ctx.zeros_u8_), ptr(ctx.bias_f32_), N, K, ctx.group_size_, ctx.weight_dtype_, ctx.lowp_mode_,
-                0 if ctx.g_idx_ is None else 1, ctx.at_weight_.device.index, ptr(ctx.scale_zero_f16x2_)]
+                0 if ctx.g_idx_ is None else 1, ctx.at_weight_.device.index, ptr(ctx.scale_zero_f16x2_),
+                ptr(ctx.scale_zero_bf16_)]
     return list(ctx.kernel_pointers())
 
 
@@ -728,7 +729,7 @@ class _MoeGroupedPlan:
         for rows in infos:
             first = rows[0]
             same = all(r[5:11] == first[5:11] and (r[3] == 0) == (first[3] == 0) and (r[4] == 0) == (first[4] == 0)
-                       and (r[12] == 0) == (first[12] == 0) and r[11] == device.index for r in rows)
+                       and (r[12] == 0) == (first[12] == 0) and (r[13] == 0) == (first[13] == 0) and r[11] == device.index for r in rows)
             if not same or first[10] or first[8] not in (_lib.DTYPE_INT4, _lib.DTYPE_INT8) or first[9] not in (0, 1, 2):
                 return
             self.shapes.append(dict(N=first[5], K=first[6], G=first[7], wd=first[8], lowp=first[9]))
@@ -748,12 +749,15 @@ class _MoeGroupedPlan:
         for rows in infos:
             col = lambda k: torch.tensor([r[k] for r in rows], dtype=torch.int64, device=device)
             self.tables.append(dict(qweight=col(0), s16=col(1), sb16=col(2), z8=col(3) if rows[0][3] else None,
-                                    bias=col(4) if rows[0][4] else None, sz=col(12) if rows[0][12] else None))
+                                    bias=col(4) if rows[0][4] else None, sz=col(12) if rows[0][12] else None,
+                                    szb=col(13) if rows[0][13] else None))
         # linears that the integer-weight decode kernels take: (scale, zero) tables, 4-bit weights in groups of 32, 64 or
         # 128 x 2^k, K a multiple of 256; the single-row one serves the experts with one row where all three are
         self.few_rows = [t["sz"] is not None and x["wd"] == _lib.DTYPE_INT4 and x["K"] % 256 == 0 and (x["G"] in (32, 64) or (
             x["G"] % 128 == 0 and (x["G"] // 128) & (x["G"] // 128 - 1) == 0)) for t, x in zip(self.tables, self.shapes)]
         self.single_row = all(self.few_rows)
+        # gate and up in one launch: the same weight type, groups and tables
+        self.pair_ok = all(g[k] == u[k] for k in ("G", "wd")) and all((self.tables[0][k] is None) == (self.tables[1][k] is None) for k in ("z8", "sz", "szb"))
         self.structs = {}
         self.device = device
         self.tiles = None
@@ -782,24 +786,56 @@ class _MoeGroupedPlan:
             have = _MOE_ROWS[key] = (mk(N1), mk(N1), mk(H))
         return have
 
-    def group_struct(self, linear, cls, f16_scales, gather, sz=False, tiles=False):
+    def group_struct(self, linear, cls, f16_scales, gather, sz=False, tiles=False, pair=False):
         """Device copy of the woq_hip_moe_group of one launch (built once).  ``sz``: for the integer-weight decode
         kernels, with the (scale, zero) dword tables in place of the scales.  ``tiles``: over the slots of
-        woq_hip_moe_route_tiles."""
-        key = (linear, cls, f16_scales, gather, sz, tiles)
+        woq_hip_moe_route_tiles.  ``pair``: with the next linear's tables as the second set."""
+        key = (linear, cls, f16_scales, gather, sz, tiles, pair)
         st = self.structs.get(key)
         if st is None:
-            t = self.tables[linear]
             ptr = lambda x: 0 if x is None else x.data_ptr()
             slots, x_row = (self.tiles["slots"], self.tiles["x_row"]) if tiles else (self.slots, self.x_row)
-            tab = [ptr(slots[cls, i]) for i in range(3)] + [ptr(x_row) if gather else 0]
-            if sz:
-                fields = tab + [ptr(t["qweight"]), ptr(t["sz"]), 0, ptr(t["bias"])]
-            else:
-                fields = tab + [ptr(t["qweight"]), ptr(t["s16"] if f16_scales else t["sb16"]), ptr(t["z8"]), ptr(t["bias"])]
+            fields = [ptr(slots[cls, i]) for i in range(3)] + [ptr(x_row) if gather else 0]
+            for t in (self.tables[linear], self.tables[linear + 1] if pair else None):
+                if t is None:
+                    fields += [0] * 5
+                elif sz:
+                    fields += [ptr(t["qweight"]), ptr(t["sz"]), 0, ptr(t["bias"]), 0]
+                else:
+                    fields += [ptr(t["qweight"]), ptr(t["s16"] if f16_scales else t["sb16"]), ptr(t["z8"]), ptr(t["bias"]), ptr(t["szb"])]
             st = torch.tensor(fields, dtype=torch.int64, device=self.device)
             self.structs[key] = st
         return st
+
+    def launch(self, lib, p, linear, src, dst, cls, bound, slots, x_dtype, sz, tiles, tile_rows=0, fusion=_lib.FUSE_NONE, other=None, pair=False):
+        """One linear over the slots of a size class (``pair``: gate and up as one).  ``p`` has the call's constant fields, ``sz`` per
+        linear whether it runs on the integer-weight decode kernels; ``tiles``: the slots are those of woq_hip_moe_route_tiles (all
+        its classes, those with ``tile_rows`` on the prefill kernel)."""
+        sh, sz = self.shapes[linear], sz[linear]
+        p.K, p.N, p.weight_dtype, p.group_size, p.M = sh["K"], sh["N"], sh["wd"], sh["G"], bound
+        p.x, p.out, p.fusion, p.others[0] = src.data_ptr(), dst.data_ptr(), fusion, other.data_ptr() if other is not None else None
+        # (a non-null value tells the entry point that the group's scales are (scale, zero) dword tables)
+        p.scale_zero_f16x2 = self.tables[linear]["sz"].data_ptr() if sz else None
+        f16 = _f16_regime(sh["lowp"], x_dtype, bound)
+        flags = _lib.MOE_SZB if self.tables[linear]["szb"] is not None and not f16 and not sz else 0
+        if pair:
+            if not f16 and not flags or not lib.woq_hip_moe_pair_applies(ctypes.byref(p), tile_rows):
+                return False
+            flags |= _lib.MOE_PAIR
+        g = self.group_struct(linear, cls, f16, linear < 2, sz, tiles, pair)
+        _lib.check(lib.woq_hip_moe_linear(ctypes.byref(p), g.data_ptr(), slots, tile_rows, flags), "woq_linear_grouped")
+        return True
+
+    def gate_up(self, lib, p, x, act, inter, cls, bound, slots, sz, tiles, tile_rows=0):
+        """silu(gate(x)) * up(x) of a size class: in one launch where there is one, else in two."""
+        args = (cls, bound, slots, x.dtype, sz, tiles, tile_rows)
+        key = ("pair", bound, tile_rows, x.dtype, sz[0])
+        pair = self.pair_ok and sz[0] == sz[1] and self.structs.get(key, True)
+        if pair and self.launch(lib, p, 0, x, inter, *args, pair=True):
+            return
+        self.structs[key] = False  # (asked once)
+        self.launch(lib, p, 0, x, act, *args, fusion=_lib.FUSE_SILU)
+        self.launch(lib, p, 1, x, inter, *args, fusion=_lib.FUSE_MUL, other=act)
 
 
 def _moe_plan(gate_ctx, up_ctx, down_ctx, device, stream):
@@ -890,20 +926,10 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
         p.stream = torch.cuda.current_stream().cuda_stream
         p.lowp_mode = lowp
         p.act_quant_mode = -1
-        steps = ((0, x, act, _lib.FUSE_SILU, None, True), (1, x, inter, _lib.FUSE_MUL, act, True),
-                 (2, inter, y, _lib.FUSE_NONE, None, False))
-        for li, src, dst, fusion, other, gather in steps:
-            sh = plan.shapes[li]
-            p.K, p.N, p.weight_dtype, p.group_size = sh["K"], sh["N"], sh["wd"], sh["G"]
-            p.x, p.out, p.fusion = src.data_ptr(), dst.data_ptr(), fusion
-            p.others[0] = other.data_ptr() if other is not None else None
-            for cls, bound in launches:
-                p.M = bound
-                # (a non-null value tells the entry point that the group's scales are (scale, zero) dword tables)
-                sz = cls == 3 or (cls == 0 and single)
-                p.scale_zero_f16x2 = plan.tables[li]["sz"].data_ptr() if sz else None
-                g = plan.group_struct(li, cls, _f16_regime(lowp, x.dtype, bound), gather, sz)
-                _lib.check(lib.woq_hip_linear_grouped(ctypes.byref(p), g.data_ptr(), nslots), "woq_linear_grouped")
+        for cls, bound in launches:
+            plan.gate_up(lib, p, x, act, inter, cls, bound, nslots, [cls == 3 or (cls == 0 and single)] * 3, False)
+        for cls, bound in launches:
+            plan.launch(lib, p, 2, inter, y, cls, bound, nslots, x.dtype, [cls == 3 or (cls == 0 and single)] * 3, False)
         _lib.check(lib.woq_hip_moe_combine_rows(out.data_ptr(), code, T, H, y.data_ptr(), rw.data_ptr(), topk,
                                                 plan.row_of.data_ptr(), plan.slot_of.data_ptr(), 0, stream), "moe_combine_rows")
     return out
@@ -987,23 +1013,11 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids, raw_stream
         p.stream = torch.cuda.current_stream().cuda_stream
         p.lowp_mode = lowp
         p.act_quant_mode = -1
-        for li, src, dst, fusion, other, gather in ((0, x, act, _lib.FUSE_SILU, None, True), (1, x, inter, _lib.FUSE_MUL, act, True),
-                                                    (2, inter, y, _lib.FUSE_NONE, None, False)):
-            sh = plan.shapes[li]
-            p.K, p.N, p.weight_dtype, p.group_size = sh["K"], sh["N"], sh["wd"], sh["G"]
-            p.x, p.out, p.fusion = src.data_ptr(), dst.data_ptr(), fusion
-            p.others[0] = other.data_ptr() if other is not None else None
-            for cls, bound in ((0, 4), (1, 16), (2, 64), (3, rows)):
-                if not used[cls]:
-                    continue
-                p.M = bound
-                sz = cls == 0 and few[li]
-                p.scale_zero_f16x2 = plan.tables[li]["sz"].data_ptr() if sz else None
-                g = plan.group_struct(li, cls, _f16_regime(lowp, x.dtype, bound), gather, sz, tiles=True)
-                if cls == 3:
-                    _lib.check(lib.woq_hip_linear_grouped_tiles(ctypes.byref(p), g.data_ptr(), used[cls], rows), "woq_linear_grouped_tiles")
-                else:
-                    _lib.check(lib.woq_hip_linear_grouped(ctypes.byref(p), g.data_ptr(), used[cls]), "woq_linear_grouped")
+        classes = [(cls, bound, [cls == 0 and ok for ok in few], rows if cls == 3 else 0) for cls, bound in ((0, 4), (1, 16), (2, 64), (3, rows)) if used[cls]]
+        for cls, bound, sz, tile in classes:
+            plan.gate_up(lib, p, x, act, inter, cls, bound, used[cls], sz, True, tile)
+        for cls, bound, sz, tile in classes:
+            plan.launch(lib, p, 2, inter, y, cls, bound, used[cls], x.dtype, sz, True, tile)
         _lib.check(lib.woq_hip_moe_combine_rows(out.data_ptr(), code, T, H, y.data_ptr(), rw.data_ptr(), topk,
                                                 buf["row_of"].data_ptr(), buf["slot_of"].data_ptr(), 0, stream), "moe_combine_rows")
     return out

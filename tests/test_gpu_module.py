@@ -714,6 +714,36 @@ def test_moe_operators_of_the_binding_without_the_python_package(cuda, tmp_path,
     assert torch.equal(alone["layer"], want.cpu())
 
 
+@pytest.mark.parametrize("weight_dtype,G,lowp,K,N", [
+    ("INT4", 128, "BF16", 512, 272), ("INT4", 64, "BF16", 256, 31), ("INT4", 32, "BF16", 768, 1040), ("INT4", -1, "BF16", 384, 64),
+    ("INT4", 128, "BF16", 4352, 48), ("INT8", -1, "BF16", 320, 100), ("INT4", 128, "NONE", 256, 80), ("INT4", 128, "BF16", 256, 8240),
+])
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 16, 17, 33, 64, 65])
+def test_gate_and_up_in_one_launch(cuda, weight_dtype, G, lowp, K, N, M):
+    """woq_linear_silu_mul against woq_linear_silu and woq_linear_mul: the same bits where the sums have the same order; with 17 to 32
+    rows the waves that share K can differ (fp32 sums in another order, flips of a last bf16 bit in few outputs: 2e-3 in the 2-norm)."""
+    from ipex_amd import _lib
+
+    ipex = _ipex()
+    gate, up = (_woq_module(ipex, K, N, weight_dtype, G, lowp, bias=True, seed=s) for s in (41, 42))
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(cuda)
+    ops = torch.ops.torch_ipex
+    hg, hu = gate._op_context.get_data_handle(), up._op_context.get_data_handle()
+    want = ops.woq_linear_mul(x, hu, [ops.woq_linear_silu(x, hg)])
+    got = ops.woq_linear_silu_mul(x, hg, hu)
+    if M in range(17, 33):
+        assert float((got.double() - want.double()).norm() / want.double().norm()) < 2e-3
+    else:
+        assert torch.equal(got, want)
+    assert torch.equal(ipex.llm.modules.Linear2SiluMul(gate, up)(x), got)
+    if M <= 64:  # (views whose rows are no 16-byte pieces, three dimensions)
+        odd = torch.cat([x.new_zeros(1), x.flatten()])[1:].view(1, M, K)
+        assert torch.equal(ops.woq_linear_silu_mul(odd, hg, hu), got.view(1, M, N))
+    other = _woq_module(ipex, K, N + 16, weight_dtype, G, lowp, bias=True, seed=43)._op_context.get_data_handle()
+    with pytest.raises(RuntimeError):
+        ops.woq_linear_silu_mul(x, hg, other)
+
+
 def test_moe_route_against_the_oracle_token_lists(cuda):
     """woq_hip_moe_route: sorted positions, slots per compute type and per-token contribution order against the
     oracle's per-expert token lists (get_expert_topx_idx, MoE.cpp:64-81); ids outside the expert range drop out."""
