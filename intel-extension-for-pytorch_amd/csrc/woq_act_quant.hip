@@ -13,6 +13,7 @@
 // two-kernel form, so the bytes and the scales are identical.
 #include "woq_common.h"
 #include "woq_internal.h"
+#include "woq_int8_common.h"
 
 // every rounding of the reference's expressions is kept: no multiply-add contraction in this file
 #pragma clang fp contract(off)
@@ -20,43 +21,6 @@
 namespace woq {
 
 namespace {
-
-// lane's eight values of one chunk
-__device__ __forceinline__ void aq_unpack(u4 raw, bool bf16, float (&v)[8]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint16_t lo = (uint16_t)(raw[i] & 0xFFFFu), hi = (uint16_t)(raw[i] >> 16);
-    v[2 * i] = bf16 ? bf16_bits_to_f32(lo) : f16_bits_to_f32(lo);
-    v[2 * i + 1] = bf16 ? bf16_bits_to_f32(hi) : f16_bits_to_f32(hi);
-  }
-}
-
-struct AqParams {
-  float s, zp;
-};
-
-__device__ __forceinline__ AqParams aq_params(float mn, float mx, bool sym, int32_t* zp_out) {
-  AqParams p;
-  if (sym) {
-    p.s = __fdiv_rn(fmaxf(fabsf(mx), fabsf(mn)), 127.0f);
-    p.zp = 0.0f;
-  } else {
-    p.s = __fdiv_rn(__fsub_rn(mx, mn), 255.0f);
-    const int32_t z = (int32_t)(-rintf(__fdiv_rn(mn, p.s)));
-    p.zp = (float)z;
-    if (zp_out) *zp_out = z;
-  }
-  return p;
-}
-
-__device__ __forceinline__ uint8_t aq_quant(float v, AqParams p, bool sym, bool offset128) {
-  float t = __fadd_rn(__fdiv_rn(v, p.s), p.zp);
-  t = rintf(t);
-  const float lo = sym ? -128.0f : 0.0f, hi = sym ? 127.0f : 255.0f;
-  t = fminf(fmaxf(t, lo), hi);
-  if (p.s == 0.0f || t != t) t = sym ? 0.0f : p.zp;  // all-zero group: the reference divides 0 by 0
-  return sym ? (uint8_t)(int8_t)(int)t : (uint8_t)((int)t ^ (offset128 ? 0x80 : 0));
-}
 
 struct AqArgs {
   const uint16_t* x;

@@ -21,6 +21,7 @@
 // step all sat exposed between its VALU work (452 us for M = 2048, 4096 -> 14336, against 245 us).
 #include "woq_common.h"
 #include "woq_internal.h"
+#include "woq_int8_common.h"
 
 // the three roundings of the epilogue stay separate (see woq_int8.hip)
 #pragma clang fp contract(off)
@@ -62,36 +63,6 @@ struct W4I8Args {
 
 typedef __attribute__((address_space(3))) void* w8_lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* w8_global_ptr_t;
-
-// Four bytes at once: ((b | 0x80808080) - z4) ^ 0x80808080 never borrows across bytes for
-// |q - z| < 128 and leaves q - z in two's complement.
-__device__ __forceinline__ uint32_t w8_sub_bytes(uint32_t b, uint32_t z4) {
-  return ((b | 0x80808080u) - z4) ^ 0x80808080u;
-}
-// sixteen K values of one lane from two packed dwords, in the order [e0 e4 e1 e5][e2 e6 e3 e7] per dword
-__device__ __forceinline__ i4 w8_decode16(uint32_t d0, uint32_t d1, uint32_t z4) {
-  i4 r;
-  r[0] = (int)w8_sub_bytes(d0 & 0x0F0F0F0Fu, z4);
-  r[1] = (int)w8_sub_bytes((d0 >> 4) & 0x0F0F0F0Fu, z4);
-  r[2] = (int)w8_sub_bytes(d1 & 0x0F0F0F0Fu, z4);
-  r[3] = (int)w8_sub_bytes((d1 >> 4) & 0x0F0F0F0Fu, z4);
-  return r;
-}
-
-// One K block's int32 sum into the fp32 accumulator.  The reference computes
-// C += (float(sum) * s_a) * s_w per block (csrc/cpu/aten/utils/woq.h:2172-2186; its compiler is free to
-// contract the last multiply and the addition).  PER_K: exactly that, with the contraction: convert,
-// multiply, fused multiply-add.  Otherwise s_a is the same for every block of a row and is applied
-// once after the K loop, C = (sum over blocks of float(sum) * s_w) * s_a: convert and one fused
-// multiply-add per block, a third fewer VALU instructions in a loop that they bound; the results
-// differ from the per-block order by fp32 rounding only (~1e-7 relative).
-template <bool PER_K>
-__device__ __forceinline__ float w8_accumulate(int sum, float s_a, float s_w, float acc) {
-  if constexpr (PER_K)
-    return __builtin_fmaf((float)sum * s_a, s_w, acc);
-  else
-    return __builtin_fmaf((float)sum, s_w, acc);
-}
 
 // Asymmetric activations (uint8 q_a with zero point z_a; csrc/cpu/aten/utils/woq.h:2172-2186): the
 // reference's block integer is sum q_a B - z_a sum B.  The activations arrive as the int8 numbers

@@ -770,13 +770,15 @@ int launch_int8_linear(const Int8Args& a, hipStream_t st) {
   p.sa = sa;
   p.za = za;
   const int64_t qbk_quant = per_k ? (per_channel ? p.block_k : G) : a.K;
+  const bool direct = gemm_w4i8_applies(a, p.block_k, qbk_quant, per_k, asym);
+  if (direct && decode_i8_rows_applies(a, qbk_quant, per_m, per_k, asym)) return launch_decode_i8_rows(a, qbk_quant, per_k, st);
   if (int rc = launch_quant_impl(a.x, a.x_dtype, a.M, a.K, p.ldq, qbk_quant, mode, xq, sa, za,
                                  a.wbits == 4 ? 1 : 0, asym ? 1 : 0, st))
     return rc;
 
   // Large M, 4-bit weights, one activation scale per row or tensor: the kernel that feeds the
   // decoded dwords straight to the MFMA
-  if (gemm_w4i8_applies(a, p.block_k, qbk_quant, per_k, asym)) {
+  if (direct) {
     // what the caller gave beyond the quantized activations and their parameters serves as scratch for
     // sharing K between workgroups (with the caller's counters)
     SplitKScratch scratch;

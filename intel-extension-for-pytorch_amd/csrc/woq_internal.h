@@ -232,6 +232,9 @@ bool gemm_w4i8_applies(const Int8Args& a, int64_t block_k, int64_t qbk, bool per
 int launch_gemm_w4i8(const Int8Args& a, const uint8_t* xq, int64_t ldq, const float* sa, int64_t sa_m_stride,
                      int64_t sa_k_stride, int64_t qbk, hipStream_t st, const SplitKScratch* scratch = nullptr,
                      const int32_t* za = nullptr);
+// The same for up to four rows with their quantization in the kernel (woq_decode_i8.hip); qbk: K block of the activation scales.
+bool decode_i8_rows_applies(const Int8Args& a, int64_t qbk, bool per_m, bool per_k, bool asym);
+int launch_decode_i8_rows(const Int8Args& a, int64_t qbk, bool per_k, hipStream_t st);
 // Quantization of whole rows from registers (woq_act_quant.hip): 16-bit activations, padded rows of at
 // most 16384 elements.  per_m (one scale per row or per (row, K block)): one pass; scales shared by all
 // rows: a statistics pass, then the same kernel with the scales given.  Same bytes and scales as the

@@ -2439,3 +2439,39 @@ def test_decode_kernels_with_groups_of_32_and_64(cuda, K, N, bias, G):
     five = syn.make_int4_case(85, 5, K, N, G, bias=bias)
     make_context(five, O.LOWP_BF16).run(five["x"].cuda())
     assert _lib.last_kernel() == "woq_decode_dq_kernel"
+
+
+@pytest.mark.parametrize("M,K,N,G,weight,mode", [
+    (1, 128, 16, 128, "INT4", 6),        # one wave, one round
+    (3, 640, 272, 128, "INT4", 6),       # five waves; a row's last piece is a quarter
+    (4, 384, 48, 32, "INT4", 7),         # three waves, two pieces a wave at most
+    (1, 4224, 4100, 128, "INT4", 6),     # 33 rounds: one more than the ring's; columns past N
+    (1, 16384, 272, 64, "INT4", 7),      # four pieces a wave
+    (2, 8192, 512, 256, "INT4", 7),      # activation blocks of two rounds
+    (4, 4096, 4096, -1, "INT4", 6),      # 1024 rows x workgroups
+    (4, 4096, 4112, 128, "INT4", 6),     # past it: two launches
+    (1, 4096, 12320, 64, "INT4", 6),     # two row-blocks a workgroup
+    (1, 2048, 12320, -1, "INT8", 6),
+    (3, 5376, 80, 128, "INT8", 7),       # more pieces than four a wave: two launches
+    (1, 1152, 272, 128, "INT4", 4),      # one row: the tensor's scale is its own
+])
+def test_int8_rows_quantized_in_the_gemm_have_the_bits_of_two_launches(cuda, M, K, N, G, weight, mode):
+    """Up to four rows are quantized by the workgroups that multiply them; five rows take the quantization launch.  The same
+    rows give the same bits on both, with rows of zeros, of tiny and of large values, an infinity and a NaN among them."""
+    s = _synthetic()
+    case = s.make_int4_case(53, M, K, N, G if G > 0 else K, outliers=True) if weight == "INT4" else s.make_int8_case(53, M, K, N, group_size=G)
+    ctx = make_context(case, O.LOWP_INT8, mode)
+    per_row = 6 if mode == 4 else mode  # (five rows' tensor has another scale than one row's)
+    many = make_context(case, O.LOWP_INT8, per_row)
+    x = case["x"]
+    variants = [x, torch.zeros_like(x), x * 2.0 ** -110, x * 2.0 ** 104, x.to(torch.float16)]
+    for value in (float("inf"), float("nan")):
+        v = x.clone()
+        v[0, K // 2 + 1] = value
+        variants.append(v)
+    for v in variants:
+        v = v.cuda()
+        got = ctx.run(v)
+        want = many.run(torch.cat([v, v[:1].expand(5 - M, K)]))[:M]
+        as_bits = lambda t: torch.where(t.isnan(), torch.full_like(t, 12345.0), t)
+        assert torch.equal(as_bits(got), as_bits(want)), (M, K, N, G, weight, mode, v.dtype)
