@@ -428,8 +428,8 @@ int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, in
 /* woq_hip_linear_grouped (tile_rows 0) and woq_hip_linear_grouped_tiles below (64 or 128) with two options.
  * WOQ_HIP_MOE_SZB: the group has the experts' merged (scale, zero) tables; bf16 compute then reads those (same results).
  * WOQ_HIP_MOE_PAIR: out = silu(gate) * up of the group's two sets of linears in one launch, rounded as the launch with the silu
- * and the one with the mul round it; p without a post-op.  For the problems of woq_hip_moe_pair_applies(p, tile_rows) (bf16 rows;
- * p->scale_zero_f16x2 as above), in bf16 compute with WOQ_HIP_MOE_SZB. */
+ * and the one with the mul round it; p without a post-op.  For the problems of woq_hip_moe_pair_applies(p, tile_rows) (with
+ * tile_rows 0: bf16 rows, p->scale_zero_f16x2 as above, in bf16 compute with WOQ_HIP_MOE_SZB). */
 #define WOQ_HIP_MOE_PAIR 1
 #define WOQ_HIP_MOE_SZB 2
 int woq_hip_moe_pair_applies(const woq_hip_linear_params* p, int tile_rows);
@@ -444,11 +444,14 @@ int woq_hip_moe_linear(const woq_hip_linear_params* p, const void* group, int64_
  * woq_hip_linear_grouped (M is ignored), INT4 weights with power-of-two groups of at least 32 or INT8 weights with
  * power-of-two groups of at least 128, or per-channel; K a multiple of 128, rows in the compute type of five and more rows. x with
  * x_row has at most 2^31 bytes (its row offsets are 32 bits wide; so it is for woq_hip_linear_grouped).
- * With slots of 64 rows an expert whose own launch would split K over workgroups (woq_hip_linear with the scratch that
+ * An expert whose own launch would split K over workgroups (woq_hip_linear with the scratch that
  * woq_hip_linear_auto_split_k_workspace_bytes asks for) runs the same K ranges one after the other and adds them in that
  * launch's order, so it has that launch's bits; woq_hip_moe_chained_rows: the most rows of such an expert, 0 if there is none
- * at this K and N.  Slots of 128 rows run K in one chain, as do slots whose table does not say the expert's rows.
+ * at this K and N.  Slots whose table does not say the expert's rows run K in one chain.
+ * woq_hip_moe_tile_rows: the tile_rows (64 or 128) with the lower estimated time for a gated layer H -> I -> H whose experts
+ * have counts[e] rows (on the host).
  */
+int woq_hip_moe_tile_rows(const int64_t* counts, int64_t experts, int64_t H, int64_t I, int gate_dtype, int down_dtype);
 int64_t woq_hip_moe_chained_rows(int64_t K, int64_t N);
 int woq_hip_moe_route_tiles(const int64_t* topk_ids, int64_t T, int64_t topk, int64_t experts, int64_t split_lo,
                             int64_t split_mid, int64_t tile_rows, int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of,

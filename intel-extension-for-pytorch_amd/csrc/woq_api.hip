@@ -522,8 +522,9 @@ int woq_hip_moe_pair_applies(const woq_hip_linear_params* p, int tile_rows) {
   FpArgs f;
   int wbits, regime;
   const int64_t rows = tile_rows ? tile_rows : p ? p->M : 0;
-  if (rows < 1 || grouped_problem(p, p, rows, f, wbits, regime) || f.NT % 2 != 0) return 0;
-  if (tile_rows) return 0;
+  if (rows < 1 || grouped_problem(p, p, rows, f, wbits, regime)) return 0;
+  if (tile_rows) return (tile_rows == 64 || tile_rows == 128) && gemm_w4_applies(f, wbits, regime);
+  if (f.NT % 2 != 0) return 0;
   if (p->scale_zero_f16x2)
     return p->M <= 4 && decode_kernel_applies(f, wbits, regime, (const uint32_t*)p->scale_zero_f16x2) && decode_pair_applies(f);
   return p->M <= 64 && decode_dq_pair_applies(f, wbits, regime);
@@ -547,6 +548,13 @@ static int linear_grouped(const woq_hip_linear_params* p, const void* group, int
     return launch_decode_grouped(f, (const MoeGroup*)group, slots, (hipStream_t)p->stream);
   }
   return launch_decode_dq_grouped(f, wbits, regime, (const MoeGroup*)group, slots, (hipStream_t)p->stream);
+}
+
+int woq_hip_moe_tile_rows(const int64_t* counts, int64_t experts, int64_t H, int64_t I, int gate_dtype, int down_dtype) {
+  if (!counts || experts <= 0 || H <= 0 || I <= 0) return 64;
+  const int64_t K[2] = {H, I}, N[2] = {2 * I, H};
+  const int wbits[2] = {gate_dtype == WOQ_HIP_DTYPE_INT8 ? 8 : 4, down_dtype == WOQ_HIP_DTYPE_INT8 ? 8 : 4};
+  return gemm_w4_tile_rows(counts, experts, K, N, wbits);
 }
 
 int64_t woq_hip_moe_chained_rows(int64_t K, int64_t N) { return K > 0 && N > 0 ? gemm_w4_split_rows(K, N) : 0; }

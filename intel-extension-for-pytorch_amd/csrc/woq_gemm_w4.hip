@@ -42,6 +42,7 @@
 //     reads (256 KiB a K step).  Four waves a workgroup with SPREAD were slower (128 x 448 by 5 %, 128 x 128 by 6 %); eight
 //     waves of 128 x 512 91 us a generation but 448 workgroups where 128 x 448 makes 512 (M = 2048, N = 14336: 206 / 204).
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "woq_common.h"
@@ -148,7 +149,10 @@ __device__ __forceinline__ float post_op(float y, int fusion, int act_dtype, flo
 // GROUPED (mixture of experts): the row tile of a workgroup is a slot of the routing tables -- at most G4_BM routed rows of
 // one expert, whose tensors come from the group's pointer tables; a slot without an expert ends at once.
 // 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3738 us with three launches per expert (each on 32 to 192 workgroups),
-// 611..643 us with one launch per linear (three of about 200 us).
+// 640..670 us with one launch per linear (three of about 200 us, 64-row tiles), 543 with 128 x 256 tiles, merged parameter tables and
+// gate and up in one launch.
+// PAIR: half of a wave's row-blocks are the gate projection's, half the up projection's, of the same columns: a lane has both values
+// and stores silu(gate) * up, rounded as two launches round it.
 // Where an expert's own launch would split K over workgroups (plan_tiles), the workgroup runs the same K steps in as many
 // chains, one after the other, and adds them in the same order: the expert has the bits of its own launch.
 // NF4: a dword's eight table values come from the 256-entry table of value pairs in LDS (nf4_dequant), built before the first
@@ -158,20 +162,23 @@ struct G4Group {
   const MoeGroup* tables;
   int chains[kSplitKPrefillMaxRows / 64 + 1];  // CHAINS: [rows / 64, rounded up] K steps of a chain, 0: one chain
 };
-template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false, bool NF4 = false, bool CHAINS = false>
-__global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs fa, const int g_shift, float* const sk_partial,
-                                                          int* const sk_counters, const int kts, const G4Group grp) {
+template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false, bool NF4 = false, bool CHAINS = false, bool PAIR = false>
+__device__ __forceinline__ void g4_tile(const FpArgs& fa, const int g_shift, float* const sk_partial, int* const sk_counters, const int kts,
+                                        const G4Group& grp) {
   static_assert(!NF4 || (WBITS == 4 && !FP8 && !MERGED && !GROUPED), "NF4 codes have a table and a scale");
   __shared__ f2 sNf4[NF4 ? kNf4LutEntries : 1];
   if constexpr (NF4) nf4_fill_lut(sNf4, (int)threadIdx.x, 64 * S::WAVES);  // (the barrier before the first use is the K loop's first)
-  static_assert(!GROUPED || !MERGED, "the pointer tables hold scales and zero points apart");
   static_assert(GROUPED || !CHAINS, "an ungrouped launch splits K over workgroups");
+  static_assert(!PAIR || (GROUPED && S::NTW % 2 == 0), "pairs: routed rows, as many row-blocks of each weight");
   constexpr int TPS = WBITS / 4;  // packed tiles per row-block and K step of 128
   constexpr int G4_MT = S::MT, G4_NTW = S::NTW, G4_BM = S::BM, G4_XBYTES = S::XBYTES, G4_XLOADS = S::XLOADS,
                 G4_WSTAGE = S::WSTAGE * TPS, G4_SSTRIDE = S::SSTRIDE, G4_WAVES = S::WAVES;
-  // two activation buffers, then two weight stages of 4 waves x NTW tiles x 1 KiB
+  // two activation buffers, then two weight stages of WAVES x NTW tiles x 1 KiB
   extern __shared__ __align__(1024) uint8_t sX[];
-  uint8_t* const sW = sX + 2 * G4_XBYTES;
+  // (the epilogue's stage of one row tile of all waves lies in front of the weight stages)
+  constexpr int kStageBytes = G4_WAVES * 16 * G4_SSTRIDE * (int)sizeof(float);
+  constexpr int kXArea = 2 * G4_XBYTES > kStageBytes ? 2 * G4_XBYTES : (kStageBytes + 1023) & ~1023;
+  uint8_t* const sW = sX + kXArea;
 
   int bx, by;  // this workgroup's tile, by XCD (xcd_tile)
   xcd_tile(bx, by);
@@ -196,6 +203,14 @@ __global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs
     fg.scales = dq_uniform((const uint16_t*)dq_uniform(g.scales)[e]);
     fg.zeros = g.zeros ? dq_uniform(dq_uniform(g.zeros)[e]) : nullptr;
     fg.bias = g.bias ? dq_uniform(dq_uniform(g.bias)[e]) : nullptr;
+    if constexpr (MERGED) fg.szb = dq_uniform(dq_uniform(g.szb)[e]);
+    if constexpr (PAIR) {
+      fg.qweight_b = dq_uniform((const uint8_t*)dq_uniform(g.qweight_b)[e]);
+      fg.scales_b = dq_uniform((const uint16_t*)dq_uniform(g.scales_b)[e]);
+      fg.zeros_b = g.zeros_b ? dq_uniform(dq_uniform(g.zeros_b)[e]) : nullptr;
+      fg.bias_b = g.bias_b ? dq_uniform(dq_uniform(g.bias_b)[e]) : nullptr;
+      if constexpr (MERGED) fg.szb_b = dq_uniform(dq_uniform(g.szb_b)[e]);
+    }
     fg.out = (uint8_t*)fa.out + row0 * fa.N * 2;  // (16-bit rows)
     if (fa.other0) fg.other0 = (const uint8_t*)fa.other0 + row0 * fa.N * 2;
     if (g.x_row)
@@ -216,7 +231,8 @@ __global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs
   const int kt_lo = (int)blockIdx.z * kts;
   const int KT = KTW / TPS < kt_lo + kts ? KTW / TPS : kt_lo + kts;
   const int m0 = by * G4_BM;
-  const int nt0 = (bx * G4_WAVES + wave) * G4_NTW;  // first row-block of this wave
+  constexpr int G4_NTO = PAIR ? G4_NTW / 2 : G4_NTW;  // row-blocks of the output
+  const int nt0 = (bx * G4_WAVES + wave) * G4_NTO;    // first row-block of this wave
 
   G4Masks km;
   asm volatile("s_mov_b32 %0, 0x000F000F" : "=s"(km.lo));
@@ -278,11 +294,13 @@ __global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs
   const uint8_t* mbase[G4_NTW];
 #pragma unroll
   for (int t = 0; t < G4_NTW; ++t) {
-    const int nt = nt0 + t < NT ? nt0 + t : NT - 1;
-    wbase[t] = f.qweight + (size_t)nt * KTW * kTileBytes;
-    sbase[t] = (const uint8_t*)(f.scales + (size_t)nt * KG * kTileN);
-    zbase[t] = has_z ? f.zeros + (size_t)nt * KG * kTileN : sbase[t];
-    mbase[t] = (const uint8_t*)f.szb + (size_t)nt * KG * (kTileN * 4);
+    const bool second = t >= G4_NTO;  // PAIR: the up projection's row-blocks after the gate's
+    const int nto = nt0 + (second ? t - G4_NTO : t);
+    const int nt = nto < NT ? nto : NT - 1;
+    wbase[t] = (second ? f.qweight_b : f.qweight) + (size_t)nt * KTW * kTileBytes;
+    sbase[t] = (const uint8_t*)((second ? f.scales_b : f.scales) + (size_t)nt * KG * kTileN);
+    zbase[t] = has_z ? (second ? f.zeros_b : f.zeros) + (size_t)nt * KG * kTileN : sbase[t];
+    mbase[t] = (const uint8_t*)(second ? f.szb_b : f.szb) + (size_t)nt * KG * (kTileN * 4);
   }
   const uint32_t woff = (uint32_t)lane * 16u;
   auto load_q = [&](int kt, uint16_t (&s)[G4_NTW], uint8_t (&z)[G4_NTW]) {
@@ -609,6 +627,40 @@ __global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs
   const bool fast = f.fusion == WOQ_HIP_FUSE_NONE && (out_f16 || f.out_dtype == WOQ_HIP_ACT_BF16) && (f.N % 4) == 0 &&
                     (((uintptr_t)f.out & 7) | ((uintptr_t)f.bias & 15)) == 0;
   const bool hb = f.bias != nullptr;
+  if constexpr (PAIR) {
+    // a lane has the gate's and the up projection's values of the same four columns
+    const bool hb2 = f.bias_b != nullptr, wide = (f.N % 4) == 0 && ((uintptr_t)f.out & 7) == 0;
+#pragma unroll
+    for (int t = 0; t < G4_NTO; ++t) {
+      const int64_t n = ncol0 + t * kTileN + 4 * c;
+      f4 b0 = f4{0.f, 0.f, 0.f, 0.f}, b1 = b0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (hb && n + e < f.N) b0[e] = f.bias[n + e];
+        if (hb2 && n + e < f.N) b1[e] = f.bias_b[n + e];
+      }
+#pragma unroll
+      for (int mt = 0; mt < G4_MT; ++mt) {
+        const int m = m0 + mt * 16 + r;
+        if (m >= M || n >= f.N) continue;
+        uint16_t bits[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float y = pair_value<REGIME>(acc[mt][t][e], hb, b0[e], acc[mt][t + G4_NTO][e], hb2, b1[e], f.x_dtype);
+          bits[e] = out_f16 ? f32_to_f16_bits(y) : f32_to_bf16_bits(y);
+        }
+        uint16_t* const at = (uint16_t*)f.out + (int64_t)m * f.N + n;
+        if (wide) {
+          *(u2*)at = u2{(uint32_t)bits[0] | ((uint32_t)bits[1] << 16), (uint32_t)bits[2] | ((uint32_t)bits[3] << 16)};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < f.N) at[e] = bits[e];
+        }
+      }
+    }
+    return;
+  }
   if (fast) {
     f4 bias4[G4_NTW];
 #pragma unroll
@@ -644,7 +696,6 @@ __global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs
   // the activation buffers: the weight stages can still be written by the other waves' last requests), four columns a lane,
   // the operands of the next pair of pieces requested before the current pair is worked on.  One element a lane and
   // iteration, each waiting for its operand, took 20 us of a 88 us launch (M = 333, 11008 -> 4096 with a residual).
-  constexpr int kStageBytes = G4_WAVES * 16 * G4_SSTRIDE * (int)sizeof(float);  // one row tile of all waves
   constexpr int ECH = G4_MT % 8 == 0 && 8 * kStageBytes <= 2 * G4_XBYTES   ? 8
                       : G4_MT % 4 == 0 && 4 * kStageBytes <= 2 * G4_XBYTES ? 4
                       : 2 * kStageBytes <= 2 * G4_XBYTES                   ? 2
@@ -726,6 +777,22 @@ __global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs
   }
 }
 
+// GROUPED with 128-row slots: a slot of few rows runs the same columns with 32 or 64 rows' MFMAs and activations (every weight is
+// dequantized as before; same bits).  Of 512 tokens on 32 experts, top-8, half of the experts have a second slot of about ten rows:
+// gate + up 7168 -> 2048 350 -> 320 us, down 212 -> 175.
+template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false, bool NF4 = false, bool CHAINS = false, bool PAIR = false>
+__global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs fa, const int g_shift, float* const sk_partial,
+                                                          int* const sk_counters, const int kts, const G4Group grp) {
+  if constexpr (GROUPED && S::MT == 8) {
+    int bx, by;
+    xcd_tile(bx, by);
+    const int rows = __builtin_amdgcn_readfirstlane(dq_uniform(dq_uniform(grp.tables)->slot_rows)[by]) & 0xFFFF;
+    if (rows <= 32) return g4_tile<REGIME, G4Shape<2, S::NTW, S::WAVES>, WBITS, FP8, MERGED, GROUPED, NF4, CHAINS, PAIR>(fa, g_shift, sk_partial, sk_counters, kts, grp);
+    if (rows <= 64) return g4_tile<REGIME, G4Shape<4, S::NTW, S::WAVES>, WBITS, FP8, MERGED, GROUPED, NF4, CHAINS, PAIR>(fa, g_shift, sk_partial, sk_counters, kts, grp);
+  }
+  g4_tile<REGIME, S, WBITS, FP8, MERGED, GROUPED, NF4, CHAINS, PAIR>(fa, g_shift, sk_partial, sk_counters, kts, grp);
+}
+
 // The kernel needs whole K steps of 128, activations already in the regime's dtype, and a group size
 // whose boundaries never split a lane's 32 consecutive K values (8-bit weights: a K step, so groups of
 // at least 128 or one scale per channel).  NF4 codes like the 4-bit integers.
@@ -769,6 +836,11 @@ static int64_t split_bytes(int64_t M, int64_t N, int shape, int splits) {
   const int64_t bm = shape == 5 ? 128 : 64, bn = shape == 5 ? 256 : 128;
   return splits * ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * bm * bn * (int64_t)sizeof(float);
 }
+// Routed slots: a 128 x 256 tile of at most 64 rows as a part of a full one (its K steps wait for the requests of the step before),
+// and what a tile costs besides its K steps: the tables, the first requests, the stores (one 128 x 256 workgroup a CU: nothing
+// hides them).  Drawn from INT4 g128 and g32, us of gate + up / down with 64 and 128 rows a slot: 32 experts 7168 -> 2048, 128 rows
+// each 400 / 200 and 320 / 175; 3072 -> 1024 91 / 51 and 96 / 53; 5120 -> 1536, 100 rows each 158 / 88 with 128.
+constexpr double kLowSlot = 0.7, kSlotUs8 = 6.0, kSlotUs42 = 5.0;
 // share: K may be shared between workgroups (64 < M <= kSplitKPrefillMaxRows, K >= kSplitKPrefillMinK, at least eight steps each)
 static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t, bool share) {
   const int64_t np = (N + kTileN - 1) / kTileN * kTileN;
@@ -808,6 +880,35 @@ static int chain_steps(int64_t K, int64_t N, int wbits, int row_tiles) {
   const int ksteps = (int)(K / kTileK4);
   const TilePlan p = plan_tiles(64 * row_tiles, N, ksteps, step_times(wbits, 0, 0), true);
   return p.splits > 1 ? split_k_steps(ksteps, p.splits) : 0;
+}
+// Estimated microseconds of a grouped launch: `tall` slots of 64 rows (64 x 128 tiles), or of 128 (128 x 256) and `low` ones of at most 64.
+static double grouped_us(int64_t K, int64_t N, int wbits, int tile_rows, int64_t tall, int64_t low) {
+  const StepTimes& t = step_times(wbits, 0, 0);
+  const double steps = (double)((K + kTileK4 - 1) / kTileK4);
+  if (tile_rows == 128) {
+    const double w = (double)((N + 255) / 256) * ((double)tall + kLowSlot * (double)low);
+    return (steps * (w <= 192 ? t.t8 : t.t8f) * 1.05 + kSlotUs8) * std::ceil(w / 256);
+  }
+  const int most = t.t42[2] > 0 ? 3 : 2;
+  const int64_t w = (N + 127) / 128 * (tall + low);
+  if (w <= 256 * most) return steps * t.t42[(w + 255) / 256 - 1] + kSlotUs42;
+  return (steps * t.t42[most - 1] + kSlotUs42) * ((double)w / (256 * most) + 0.25);
+}
+int gemm_w4_tile_rows(const int64_t* counts, int64_t experts, const int64_t* K, const int64_t* N, const int* wbits) {
+  int64_t rows64 = 0, tall = 0, low = 0;
+  for (int64_t e = 0; e < experts; ++e)
+    if (counts[e] > 64) {
+      rows64 += (counts[e] + 63) / 64;
+      tall += (counts[e] + 63) / 128;
+      low += (counts[e] + 127) / 128 - (counts[e] + 63) / 128;
+    }
+  if (rows64 == 0) return 64;
+  double us64 = 0, us128 = 0;
+  for (int i = 0; i < 2; ++i) {
+    us64 += grouped_us(K[i], N[i], wbits[i], 64, rows64, 0);
+    us128 += grouped_us(K[i], N[i], wbits[i], 128, tall, low);
+  }
+  return us128 < us64 ? 128 : 64;
 }
 int gemm_w4_split_rows(int64_t K, int64_t N) {
   for (int i = (int)(kSplitKPrefillMaxRows / 64); i >= 2; --i)
@@ -858,19 +959,31 @@ static int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits
   return check_launch("woq_gemm_w4_kernel");
 }
 
-// Row tiles of the routed rows of all experts in one launch (woq_hip_linear_grouped_tiles).
-template <int REGIME, class S, int WBITS, bool CHAINS>
+// Row tiles of the routed rows of all experts in one launch (woq_hip_moe_linear).
+template <int REGIME, class S, int WBITS, bool MERGED, bool PAIR>
 static int launch_grouped_shape(const FpArgs& f, int g_shift, const G4Group& g, int64_t slots, hipStream_t st) {
   constexpr int kLds = g4_lds_bytes<S, WBITS>();
+  static_assert(kLds <= 160 * 1024, "a workgroup's LDS");
+  const auto kernel = &woq_gemm_w4_kernel<REGIME, S, WBITS, false, MERGED, true, false, true, PAIR>;
   static const hipError_t lds_optin =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, false, false, true, false, CHAINS>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   if (lds_optin != hipSuccess)
     return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin));
-  const dim3 grid((unsigned)((f.NT * kTileN + S::BN - 1) / S::BN), (unsigned)slots);
-  woq_gemm_w4_kernel<REGIME, S, WBITS, false, false, true, false, CHAINS>
-      <<<grid, 64 * S::WAVES, kLds, st>>>(f, g_shift, nullptr, nullptr, (int)(f.KT / (WBITS / 4)), g);
+  constexpr int kColumns = PAIR ? S::BN / 2 : S::BN;
+  const dim3 grid((unsigned)((f.NT * kTileN + kColumns - 1) / kColumns), (unsigned)slots);
+  kernel<<<grid, 64 * S::WAVES, kLds, st>>>(f, g_shift, nullptr, nullptr, (int)(f.KT / (WBITS / 4)), g);
   return check_launch("woq_gemm_w4_kernel (grouped)");
+}
+
+template <int REGIME, int WBITS, bool MERGED>
+static int launch_grouped_type(const FpArgs& f, int g_shift, const G4Group& g, int64_t slots, int tile_rows, hipStream_t st) {
+  using S8 = G4Shape<8, 2, 8>;
+  using S42 = G4Shape<4, 2>;
+  if (f.pair)
+    return tile_rows == 128 ? launch_grouped_shape<REGIME, S8, WBITS, MERGED, true>(f, g_shift, g, slots, st)
+                            : launch_grouped_shape<REGIME, S42, WBITS, MERGED, true>(f, g_shift, g, slots, st);
+  return tile_rows == 128 ? launch_grouped_shape<REGIME, S8, WBITS, MERGED, false>(f, g_shift, g, slots, st)
+                          : launch_grouped_shape<REGIME, S42, WBITS, MERGED, false>(f, g_shift, g, slots, st);
 }
 
 int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGroup* grp, int64_t slots, int tile_rows,
@@ -880,22 +993,15 @@ int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGrou
     g_shift = 0;
     while (((int64_t)1 << g_shift) < f.G) ++g_shift;
   }
-  using S2 = G4Shape<8, 2>;
-  using S42 = G4Shape<4, 2>;
-  // Chains on 64 x 128 tiles only: a second copy of the accumulators costs a 128 x 128 tile its second workgroup on a CU (us with
-  // 64 / 128 rows a tile: 32 experts 7168 -> 2048, top-8, 1024 tokens 1228 / 1295, 16 experts 4096 -> 1536,
-  // top-4, 2048 tokens 562 / 697).
   G4Group g{};
   g.tables = grp;
-  bool chained = false;
-  for (int i = 2; tile_rows == 64 && i <= kSplitKPrefillMaxRows / 64; ++i) chained |= (g.chains[i] = chain_steps(f.K, f.N, wbits, i)) != 0;
-#define WOQ_GROUPED(RG, WB)                                                                  \
-  (tile_rows == 128 ? launch_grouped_shape<RG, S2, WB, false>(f, g_shift, g, slots, st)      \
-   : chained         ? launch_grouped_shape<RG, S42, WB, true>(f, g_shift, g, slots, st)      \
-                    : launch_grouped_shape<RG, S42, WB, false>(f, g_shift, g, slots, st))
-  if (wbits == 4) return regime == kRegimeF16 ? WOQ_GROUPED(kRegimeF16, 4) : WOQ_GROUPED(kRegimeBF16, 4);
-  return regime == kRegimeF16 ? WOQ_GROUPED(kRegimeF16, 8) : WOQ_GROUPED(kRegimeBF16, 8);
-#undef WOQ_GROUPED
+  for (int i = 2; i <= kSplitKPrefillMaxRows / 64; ++i) g.chains[i] = chain_steps(f.K, f.N, wbits, i);
+  if (wbits == 8)
+    return regime == kRegimeF16 ? launch_grouped_type<kRegimeF16, 8, false>(f, g_shift, g, slots, tile_rows, st)
+                                : launch_grouped_type<kRegimeBF16, 8, false>(f, g_shift, g, slots, tile_rows, st);
+  if (regime == kRegimeF16) return launch_grouped_type<kRegimeF16, 4, false>(f, g_shift, g, slots, tile_rows, st);
+  return f.grp_szb ? launch_grouped_type<kRegimeBF16, 4, true>(f, g_shift, g, slots, tile_rows, st)
+                   : launch_grouped_type<kRegimeBF16, 4, false>(f, g_shift, g, slots, tile_rows, st);
 }
 
 // 8-bit weights of one shape: integers or float8 bytes, fp16 or bf16 compute

@@ -56,6 +56,7 @@ EXPORTS = [
     "woq_hip_moe_route_tiles",
     "woq_hip_linear_grouped_tiles",
     "woq_hip_moe_chained_rows",
+    "woq_hip_moe_tile_rows",
     "woq_hip_linear_pair_applies",
     "woq_hip_linear_pair",
     "woq_hip_moe_pair_applies",
@@ -185,6 +186,8 @@ def load():
         lib.woq_hip_linear_pair_applies.argtypes = [ctypes.POINTER(LinearParams), ctypes.POINTER(LinearParams)]
         lib.woq_hip_linear_pair.restype = i32
         lib.woq_hip_linear_pair.argtypes = [ctypes.POINTER(LinearParams), ctypes.POINTER(LinearParams)]
+        lib.woq_hip_moe_tile_rows.restype = i32
+        lib.woq_hip_moe_tile_rows.argtypes = [vp, i64, i64, i64, i32, i32]
         lib.woq_hip_moe_pair_applies.restype = i32
         lib.woq_hip_moe_pair_applies.argtypes = [ctypes.POINTER(LinearParams), i32]
         lib.woq_hip_moe_linear.restype = i32

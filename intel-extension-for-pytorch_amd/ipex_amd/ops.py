@@ -765,8 +765,6 @@ class _MoeGroupedPlan:
         self.tiles_ok = len(gate_ctx) <= _lib.MOE_TILES_EXPERTS and all(
             x["K"] % 128 == 0 and (x["G"] <= 0 or (x["G"] >= (32 if x["wd"] == _lib.DTYPE_INT4 else 128) and x["G"] & (x["G"] - 1) == 0))
             for x in self.shapes)
-        # experts of more than 64 and at most this many rows add K in chains, as their own launches do (64-row tiles only)
-        self.chained_rows = max(_lib.load().woq_hip_moe_chained_rows(x["K"], x["N"]) for x in self.shapes)
         self.ok = True
 
     def tile_routing(self):
@@ -819,7 +817,7 @@ class _MoeGroupedPlan:
         f16 = _f16_regime(sh["lowp"], x_dtype, bound)
         flags = _lib.MOE_SZB if self.tables[linear]["szb"] is not None and not f16 and not sz else 0
         if pair:
-            if not f16 and not flags or not lib.woq_hip_moe_pair_applies(ctypes.byref(p), tile_rows):
+            if not f16 and not flags and not tile_rows or not lib.woq_hip_moe_pair_applies(ctypes.byref(p), tile_rows):
                 return False
             flags |= _lib.MOE_PAIR
         g = self.group_struct(linear, cls, f16, linear < 2, sz, tiles, pair)
@@ -935,13 +933,11 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     return out
 
 
-def _moe_tile_rows(rows, experts):
-    """Rows of a slot of the prefill kernel: 128 from 192 rows per expert on, counting the rows of layers of at least 6144
-    columns only (``rows`` is 0 on the others).  Tiles of 128 rows dequantize half as often, but waste more of an expert's last
-    tile and two instead of three share a CU (8 experts, INT4 g128, us with 64 / 128 rows a tile: 4096 -> 14336 with 320 / 1000 rows per
-    expert 1408 / 1282 and 3606 / 3274, 4096 -> 6144 with 270 / 1000 588 / 568 and 1644 / 1490; 2048 -> 2048 with 200 / 1000 165 / 170
-    and 402 / 413, 3072 -> 1024 with 200 / 1000 142 / 174 and 342 / 359)."""
-    return 128 if rows >= 192 * experts else 64
+def _moe_tile_rows(shapes, counts):
+    """Rows of a slot of the prefill kernel, 64 or 128, by the lower estimated time.  ``shapes``: K, N and weight dtype (wd) of the
+    three linears, ``counts``: rows of every expert."""
+    gate, down = shapes[0], shapes[2]
+    return _lib.load().woq_hip_moe_tile_rows((ctypes.c_int64 * len(counts))(*counts), len(counts), gate["K"], gate["N"], gate["wd"], down["wd"])
 
 
 def _moe_expert_launches_faster(shapes, counts):
@@ -949,8 +945,8 @@ def _moe_expert_launches_faster(shapes, counts):
     ``counts``: rows of every expert.
     One expert with tokens, long K: its own launches split K over workgroups (INT4 g128, one expert, us per expert / in tiles: 14336 -> 4096
     with 128 / 512 tokens 223 / 277 and 368 / 386, 11008 -> 2048 193 / 240 and 261 / 247, but 8192 -> 4096 209 / 204 and 274 / 270).
-    INT8 experts of many rows: their launches have 128 x 256 tiles, the slots 128 x 128 at most (2 experts 8192 -> 8192, 2048
-    rows each 1969 / 2287, 4096 -> 14336 with 2500 rows 2728 / 2566, with 4096 3692 / 3997; INT4 with 4096 rows 4329 / 3105).
+    INT8 experts of many rows: drawn while the slots had 128 x 128 tiles at most (2 experts 8192 -> 8192, 2048
+    rows each 1969 / 2287; with the 128 x 256 tiles that they have now 1890..1980 / 1660..1690, 4096 -> 14336 with 2500 rows 2728 / 2566, with 4096 3692 / 3997; INT4 with 4096 rows 4329 / 3105).
     Estimates at K = 4096: 69.6 us for 256 tiles of 128 x 256, 0.159 us a tile of 128 x 128; 40 us and 0.015 us a row more
     for an expert's launches."""
     active = [n for n in counts if n]
@@ -989,8 +985,7 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids, raw_stream
     counts = torch.bincount(read.reshape(-1), minlength=experts).tolist()
     if _moe_expert_launches_faster(plan.shapes, counts):
         return None
-    chained = any(64 < n <= plan.chained_rows for n in counts)
-    rows = 64 if chained else _moe_tile_rows(R if N1 >= 6144 else 0, experts)
+    rows = _moe_tile_rows(plan.shapes, counts)
     used = [0, 0, 0, 0]  # slots of each size class
     for n in counts:
         if n:

@@ -1336,3 +1336,31 @@ def test_moe_over_registered_contexts(cuda):
     want = torch.ops.torch_ipex.deepseek_moe_woq(hidden, ids, py[0], py[1], py[2], rw, False)
     got = torch.ops.torch_ipex.deepseek_moe_woq(hidden, ids, cc[0], cc[1], cc[2], rw, False)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("H,I,weight_dtype,G,lowp", [(256, 384, "INT4", 32, "BF16"), (4096, 256, "INT4", 128, "BF16"), (4352, 128, "INT4", 128, "FP16"),
+                                                     (4096, 384, "INT8", -1, "BF16")])
+def test_deepseek_moe_prompt_slots_of_few_rows(cuda, monkeypatch, tile, H, I, weight_dtype, G, lowp):
+    """Slots of 1, 32, 33, 64, 65 and 128 rows, gate and up in one launch: bit for bit the experts' own launches."""
+    from ipex_amd import _lib, ops
+
+    ipex = _ipex()
+    rows = [129, 160, 161, 0, 192, 193, 65, 256]
+    mk = lambda k, n, s: _woq_module(ipex, k, n, weight_dtype, G, lowp, bias=True, seed=s)._op_context
+    E = len(rows)
+    ctxs = [[mk(H, I, 900 + e) for e in range(E)], [mk(H, I, 920 + e) for e in range(E)], [mk(I, H, 940 + e) for e in range(E)]]
+    g = torch.Generator().manual_seed(9)
+    xdt = torch.float16 if lowp == "FP16" else torch.bfloat16
+    T = sum(rows)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(T, generator=g)].view(T, 1).to(cuda)
+    hidden = torch.randn(T, H, generator=g).to(xdt).to(cuda)
+    rw = torch.rand(T, 1, generator=g).to(xdt).to(cuda)
+    op = torch.ops.torch_ipex.deepseek_moe_woq
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
+    want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
+    monkeypatch.setattr(ops, "_moe_tile_rows", lambda shapes, counts: tile)
+    got = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    assert _lib.last_kernel() == "moe_combine_rows"
+    assert torch.equal(got, want)
