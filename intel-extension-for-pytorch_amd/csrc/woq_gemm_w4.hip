@@ -399,6 +399,12 @@ __device__ __forceinline__ void g4_tile(const FpArgs& fa, const int g_shift, flo
   // barrier in different blocks of the last sub-step -- wave w in block FETCH_T - w, the same moment for all -- and so
   // reach the fetching block one block apart, in every sub-step (M = 2048, 4096 -> 6144: 92 us against 99 us).
   constexpr int STAG_MAX = S::XA_SETS == 1 && G4_WAVES == 4 ? (S::FETCH_T < 3 ? S::FETCH_T : 3) : 0;
+  auto wait_met = [](bool reads_too) {
+    if (reads_too)
+      __builtin_amdgcn_s_waitcnt(kVmcntW & kLgkmcnt0);
+    else
+      __builtin_amdgcn_s_waitcnt(kVmcntW);
+  };
   const int bar_t = S::FETCH_T - (wave < STAG_MAX ? wave : STAG_MAX);
   load_x(kt_lo, 0);
   dma_w(kt_lo, 0);
@@ -466,17 +472,19 @@ __device__ __forceinline__ void g4_tile(const FpArgs& fa, const int g_shift, flo
             __builtin_amdgcn_sched_barrier(0);
           }
           if (j == 3 && t == 0) __builtin_amdgcn_s_waitcnt(kVmcntStep);  // tiles of step kt + 1 are in LDS
+          // Behind the barrier the other waves refill the buffer of this step.  In the first block the barrier stands before
+          // the first use of the last sub-step's fragments: their reads must have returned (before a later block they have).
           if constexpr (STAG_MAX == 0) {
             if (bar_here && j == 3) {
               // Written as an instruction, not as the barrier builtin: before that one the compiler
               // waits for every outstanding load, the tiles requested for step kt + 2 included.
-              __builtin_amdgcn_s_waitcnt(kVmcntW);
+              wait_met(t == 0);
               asm volatile("s_barrier" ::: "memory");
             }
           } else {
             // this wave's meeting block (see bar_t)
             if (j == 3 && t <= S::FETCH_T && t >= S::FETCH_T - STAG_MAX && bar_t == t) {
-              __builtin_amdgcn_s_waitcnt(kVmcntW);
+              wait_met(t == 0);
               __builtin_amdgcn_s_barrier();
             }
           }

@@ -74,3 +74,46 @@ def test_prefill_waits_count_no_more_loads_than_a_step_has(kernels):
         assert max(waits) <= loads, (name, waits, loads)
         seen += 1
     assert seen >= 40, seen
+
+
+def _loops(body):
+    """Instruction ranges of the backward branches of a kernel that hold an MFMA and no smaller such range."""
+    at = {a: i for i, (a, _) in enumerate(body)}
+    ranges = []
+    for i, (a, t) in enumerate(body):
+        m = re.match(r"s_c?branch\S* (\d+)", t)
+        if m:
+            off = int(m.group(1))
+            first = at.get(a + 4 + 4 * (off - 65536 if off >= 32768 else off))
+            if first is not None and first < i and any(x.startswith("v_mfma") for _, x in body[first:i]):
+                ranges.append((first, i))
+    return [[x for _, x in body[f:l + 1]] for f, l in ranges if not any(f <= f2 and l2 <= l and (f, l) != (f2, l2) for f2, l2 in ranges)]
+
+
+def test_every_prefill_loop_has_its_reads_back_at_the_barrier(kernels):
+    """Behind the barrier of a K step the other waves refill the activation buffer that the step has read, so no read of it may
+    be outstanding there.  Outstanding may be the packed tiles that a wave alone reads (8-bit weights: two) in the blocks of
+    the last sub-step before the one with the barrier, number NTW - 2 (16 row tiles: NTW - 1) at most.  All loops of a kernel:
+    the grouped ones have a body each for 32, 64 and 128 rows."""
+    seen = 0
+    for name, body in kernels.items():
+        shape = re.search(r"woq_gemm_w4_kernel.*G4ShapeILi(\d+)ELi(\d+)ELi(\d+)EEELi(\d)E", name)
+        if not shape:
+            continue
+        mt, ntw, tps = int(shape.group(1)), int(shape.group(2)), int(shape.group(4)) // 4
+        for loop in _loops(body):
+            reads = []  # outstanding, oldest first; NF4's table reads are of eight bytes and of a table that stays
+            for _ in range(2):  # (the second time with those of the step before)
+                for t in loop:
+                    if t.startswith(("ds_read", "ds_write")):
+                        reads.append(t.startswith("ds_read_b128"))
+                    m = re.match(r"s_waitcnt\b.*lgkmcnt\((\d+)\)", t)
+                    if m:
+                        reads = reads[max(0, len(reads) - int(m.group(1))):]
+                    if t.startswith("s_barrier"):
+                        assert sum(reads) <= (ntw - (1 if mt >= 16 else 2)) * tps, (name, sum(reads))
+                        seen += 1
+            loads = sum(x.startswith("global_load") for x in loop)
+            waits = [int(n) for x in loop for n in re.findall(r"^s_waitcnt.*vmcnt\((\d+)\)", x)]
+            assert waits and max(waits) <= loads, (name, waits, loads)
+    assert seen >= 100, seen
