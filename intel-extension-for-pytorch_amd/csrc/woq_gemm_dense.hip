@@ -211,7 +211,12 @@ __global__ __launch_bounds__(256) void woq_gemm_dense_kernel(const GdArgs a) {
         constexpr int kLastJ = 3, kLastT = NTW - 1;
         const bool fetch_t = t == S::FETCH_T;
         if (fetch_t && j == 3) {
-          __builtin_amdgcn_s_waitcnt(kVmcntBar);
+          // (in the first block this stands before the first use of the fragments of this sub-step: behind the barrier the
+          // buffer that they are read from is refilled, so they must have returned)
+          if (t == 0)
+            __builtin_amdgcn_s_waitcnt(kVmcntBar & 0xC07F);
+          else
+            __builtin_amdgcn_s_waitcnt(kVmcntBar);
           asm volatile("s_barrier" ::: "memory");
         }
         // refill the registers of the block just finished with its fragment of the next step (block 0: the last

@@ -26,7 +26,7 @@ def kernels(tmp_path_factory):
             continue
         with open(d / name, "rb") as f:
             code = f.read()
-        if b"woq_gemm_w4_kernel" not in code and b"woq_decode_dq_kernel" not in code and b"woq_decode_kernel" not in code:
+        if b"woq_gemm_w4_kernel" not in code and b"woq_decode_dq_kernel" not in code and b"woq_decode_kernel" not in code and b"woq_gemm_dense_kernel" not in code:
             continue
         body = None
         for line in subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", name], cwd=d, check=True, capture_output=True, text=True).stdout.split("\n"):
@@ -117,3 +117,22 @@ def test_every_prefill_loop_has_its_reads_back_at_the_barrier(kernels):
             waits = [int(n) for x in loop for n in re.findall(r"^s_waitcnt.*vmcnt\((\d+)\)", x)]
             assert waits and max(waits) <= loads, (name, waits, loads)
     assert seen >= 100, seen
+
+
+def test_every_loop_of_the_dense_kernel_has_its_reads_back_at_the_barrier(kernels):
+    """As above; this kernel reads nothing but activations from LDS."""
+    seen = 0
+    for name, body in kernels.items():
+        if "woq_gemm_dense_kernel" not in name:
+            continue
+        for loop in _loops(body):
+            reads = 0
+            for t in loop + loop:
+                reads += t.startswith("ds_read")
+                m = re.match(r"s_waitcnt\b.*lgkmcnt\((\d+)\)", t)
+                if m:
+                    reads = min(reads, int(m.group(1)))
+                if t.startswith("s_barrier"):
+                    assert reads == 0, (name, reads)
+                    seen += 1
+    assert seen >= 6, seen
