@@ -19,8 +19,10 @@
 #include "woq_internal.h"
 #include "woq_int8_common.h"
 
-namespace woq {
+// the roundings of the epilogue (activation scale, bias) stay separate, as in the two launches' kernel (woq_gemm_w4i8.hip)
+#pragma clang fp contract(off)
 
+namespace woq {
 
 struct DecodeI8Args {
   const uint16_t* x;

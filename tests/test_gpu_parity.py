@@ -2475,3 +2475,14 @@ def test_int8_rows_quantized_in_the_gemm_have_the_bits_of_two_launches(cuda, M, 
         want = many.run(torch.cat([v, v[:1].expand(5 - M, K)]))[:M]
         as_bits = lambda t: torch.where(t.isnan(), torch.full_like(t, 12345.0), t)
         assert torch.equal(as_bits(got), as_bits(want)), (M, K, N, G, weight, mode, v.dtype)
+
+
+@pytest.mark.parametrize("M,K,N,G,weight,mode", [(1, 1024, 272, 128, "INT4", 6), (4, 512, 144, 32, "INT4", 6), (2, 1152, 80, 64, "INT4", 7),
+                                                 (3, 4224, 272, -1, "INT8", 6), (1, 2048, 12320, 128, "INT4", 6), (1, 1024, 272, 128, "INT4", 4)])
+def test_int8_rows_quantized_in_the_gemm_round_scale_and_bias_apart(cuda, M, K, N, G, weight, mode):
+    """The fp32 results with a bias: activation scale and bias are two roundings there as in the two launches' kernel."""
+    s = _synthetic()
+    case = s.make_int4_case(54, M, K, N, G, bias=True) if weight == "INT4" else s.make_int8_case(54, M, K, N, group_size=G)
+    x = case["x"].cuda()
+    want = make_context(case, O.LOWP_INT8, 6 if mode == 4 else mode).run(torch.cat([x, x[:1].expand(5 - M, K)]), out_fp32=True)[:M]
+    assert torch.equal(make_context(case, O.LOWP_INT8, mode).run(x, out_fp32=True), want)
