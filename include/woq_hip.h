@@ -277,13 +277,13 @@ int64_t woq_hip_linear_workspace_bytes(int64_t M, int64_t K, int32_t lowp_mode,
                                        int32_t act_quant_mode, int64_t group_size);
 
 /* Scratch bytes that let woq_hip_linear split K across workgroups for M rows and N output columns
- * in the floating-point modes (decode kernel up to 32 rows; prefill GEMM from 65 to 1024 rows while its tiles leave
- * room for a second workgroup each, at most 32 MiB); 0 where it never does.  No counterpart in the reference. */
+ * in the floating-point modes (decode kernel up to 32 rows; prefill GEMM from 65 to 1024 rows, or of any number of rows in at most 128
+ * tiles of 64 x 128, while its tiles leave room for a second workgroup each, at most 32 MiB); 0 where it never does.  No counterpart in the reference. */
 int64_t woq_hip_linear_split_k_workspace_bytes(int64_t M, int64_t N);
 
 /* The same size for the problems on which woq_hip_linear shares K between workgroups BY ITSELF (force_kernel 0):
  * few output tiles and a long K -- 5..32 rows with K >= 8192 and N <= 4096 in the floating-point modes, more than
- * 64 and at most 1024 rows with K >= 4096 (lowp_mode INT8: M * N <= 2^20) -- and 0 for every other problem, where scratch and
+ * 64 rows with K >= 4096, either at most 1024 rows or at most 128 tiles of 64 rows x 128 columns (lowp_mode INT8: the latter) -- and 0 for every other problem, where scratch and
  * counters would go unused.  A caller that allocates per call asks this function; there is no second copy of the
  * rule to keep in step.  No counterpart in the reference. */
 int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t lowp_mode);

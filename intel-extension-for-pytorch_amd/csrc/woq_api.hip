@@ -176,9 +176,9 @@ int64_t woq_hip_linear_split_k_workspace_bytes(int64_t M, int64_t N) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64) {
     // prefill GEMM: the most that its plans take -- 64 x 128 tiles on up to three workgroups a CU, 128 x 256 tiles on one
-    if (M > kSplitKPrefillMaxRows) return 0;
+    if (!split_k_prefill_rows(M, N)) return 0;
     const int64_t np = woq_hip_padded_n(N);
-    const int64_t t42 = ((M + 63) / 64) * ((np + 127) / 128), t8 = ((M + 127) / 128) * ((np + 255) / 256);
+    const int64_t t42 = split_k_tiles(M, np), t8 = ((M + 127) / 128) * ((np + 255) / 256);
     const int64_t s42 = 768 / t42 < 4 ? 768 / t42 : 4, s8 = 256 / t8 < 4 ? 256 / t8 : 4;
     const int64_t b42 = s42 > 1 ? s42 * t42 * 64 * 128 * (int64_t)sizeof(float) : 0;
     const int64_t b8 = s8 > 1 ? s8 * t8 * 128 * 256 * (int64_t)sizeof(float) : 0;
@@ -194,7 +194,7 @@ int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_
   const bool int8 = lowp_mode == WOQ_HIP_LOWP_INT8;
   // the dequantizing decode kernel (launch_decode_dq) and the prefill GEMMs (plan_tiles; lowp_mode INT8: 64 x 128 tiles)
   const bool decode = !int8 && M >= 5 && M <= 32 && K >= 8192 && N <= 4096;
-  const bool prefill = M > 64 && K >= kSplitKPrefillMinK && (int8 ? M * N <= kSplitKPrefillElems : M <= kSplitKPrefillMaxRows);
+  const bool prefill = K >= kSplitKPrefillMinK && split_k_prefill_rows(M, N) && (!int8 || split_k_tiles(M, N) <= kSplitKPrefillTiles);
   return decode || prefill ? woq_hip_linear_split_k_workspace_bytes(M, N) : 0;
 }
 

@@ -158,9 +158,10 @@ __device__ __forceinline__ float post_op(float y, int fusion, int act_dtype, flo
 // NF4: a dword's eight table values come from the 256-entry table of value pairs in LDS (nf4_dequant), built before the first
 // request; four 8-byte reads, eight products and four conversions against 17 instructions for integers.
 constexpr int kPrefillSplitMax = 4;  // workgroups that share the K steps of a tile
+constexpr int kChainRowTiles = (int)(kSplitKPrefillTiles > kSplitKPrefillMaxRows / 64 ? kSplitKPrefillTiles : kSplitKPrefillMaxRows / 64);
 struct G4Group {
   const MoeGroup* tables;
-  int chains[kSplitKPrefillMaxRows / 64 + 1];  // CHAINS: [rows / 64, rounded up] K steps of a chain, 0: one chain
+  int chains[kChainRowTiles + 1];  // CHAINS: [rows / 64, rounded up] K steps of a chain, 0: one chain
 };
 template <int REGIME, class S, int WBITS, bool FP8, bool MERGED = false, bool GROUPED = false, bool NF4 = false, bool CHAINS = false, bool PAIR = false>
 __device__ __forceinline__ void g4_tile(const FpArgs& fa, const int g_shift, float* const sk_partial, int* const sk_counters, const int kts,
@@ -193,7 +194,7 @@ __device__ __forceinline__ void g4_tile(const FpArgs& fa, const int g_shift, flo
     const int packed = __builtin_amdgcn_readfirstlane(dq_uniform(g.slot_rows)[by]);
     const int rows = packed & 0xFFFF, expert_rows = packed >> 16;  // (0: not known, one chain)
     if constexpr (CHAINS)
-      if (expert_rows <= kSplitKPrefillMaxRows) {
+      if (expert_rows <= 64 * kChainRowTiles) {
         const int steps = grp.chains[(expert_rows + 63) / 64];
         chain = steps ? steps : kts;
       }
@@ -849,7 +850,7 @@ static int64_t split_bytes(int64_t M, int64_t N, int shape, int splits) {
 // hides them).  Drawn from INT4 g128 and g32, us of gate + up / down with 64 and 128 rows a slot: 32 experts 7168 -> 2048, 128 rows
 // each 400 / 200 and 320 / 175; 3072 -> 1024 91 / 51 and 96 / 53; 5120 -> 1536, 100 rows each 158 / 88 with 128.
 constexpr double kLowSlot = 0.7, kSlotUs8 = 6.0, kSlotUs42 = 5.0;
-// share: K may be shared between workgroups (64 < M <= kSplitKPrefillMaxRows, K >= kSplitKPrefillMinK, at least eight steps each)
+// share: K may be shared between workgroups (split_k_prefill_rows, K >= kSplitKPrefillMinK, at least eight steps each)
 static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t, bool share) {
   const int64_t np = (N + kTileN - 1) / kTileN * kTileN;
   auto wgs = [&](int bm, int bn) { return ((np + bn - 1) / bn) * ((M + bm - 1) / bm); };
@@ -858,7 +859,7 @@ static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t,
   auto offer = [&](int shape, int splits, double us) {
     if (us < best.us) best.shape = shape, best.splits = splits, best.us = us;
   };
-  share = share && M > 64 && M <= kSplitKPrefillMaxRows && (int64_t)ksteps * kTileK4 >= kSplitKPrefillMinK;
+  share = share && split_k_prefill_rows(M, np) && (int64_t)ksteps * kTileK4 >= kSplitKPrefillMinK;
   const int most42 = t.t42[2] > 0 ? 3 : 2, most2 = t.t2[1] > 0 ? 2 : 1;
   for (int s = 1; s <= (share ? kPrefillSplitMax : 1); ++s) {
     const int kts = s == 1 ? ksteps : split_k_steps(ksteps, s);
@@ -918,8 +919,12 @@ int gemm_w4_tile_rows(const int64_t* counts, int64_t experts, const int64_t* K, 
   }
   return us128 < us64 ? 128 : 64;
 }
+// The largest [rows / 64, rounded up] that split_k_prefill_rows holds for.
+static int chain_row_tiles(int64_t N) {
+  return (int)std::max(kSplitKPrefillMaxRows / 64, kSplitKPrefillTiles / ((N + 127) / 128));
+}
 int gemm_w4_split_rows(int64_t K, int64_t N) {
-  for (int i = (int)(kSplitKPrefillMaxRows / 64); i >= 2; --i)
+  for (int i = chain_row_tiles(N); i >= 2; --i)
     if (chain_steps(K, N, 4, i) || chain_steps(K, N, 8, i)) return 64 * i;
   return 0;
 }
@@ -1003,7 +1008,7 @@ int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGrou
   }
   G4Group g{};
   g.tables = grp;
-  for (int i = 2; i <= kSplitKPrefillMaxRows / 64; ++i) g.chains[i] = chain_steps(f.K, f.N, wbits, i);
+  for (int i = 2, n = chain_row_tiles(f.N); i <= n; ++i) g.chains[i] = chain_steps(f.K, f.N, wbits, i);
   if (wbits == 8)
     return regime == kRegimeF16 ? launch_grouped_type<kRegimeF16, 8, false>(f, g_shift, g, slots, tile_rows, st)
                                 : launch_grouped_type<kRegimeBF16, 8, false>(f, g_shift, g, slots, tile_rows, st);

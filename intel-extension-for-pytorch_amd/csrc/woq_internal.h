@@ -79,9 +79,14 @@ struct SplitKScratch {
 // Entries the caller's split-K counter array must have, and the largest number of K splits.
 constexpr int kSplitKCounters = 512;
 constexpr int kSplitKMax = 4;
-// Prefill problems that get split-K scratch by themselves (woq_hip_linear_auto_split_k_workspace_bytes): the least K and the most
-// rows; lowp_mode INT8: the most outputs.
-constexpr int64_t kSplitKPrefillMinK = 4096, kSplitKPrefillMaxRows = 1024, kSplitKPrefillElems = 1048576;
+// Prefill problems that get split-K scratch by themselves (woq_hip_linear_auto_split_k_workspace_bytes): K of at least
+// kSplitKPrefillMinK and at most kSplitKPrefillMaxRows rows, or any number of rows in at most kSplitKPrefillTiles tiles of
+// 64 x 128, which leave half of the chip idle (the one condition of lowp_mode INT8).
+constexpr int64_t kSplitKPrefillMinK = 4096, kSplitKPrefillMaxRows = 1024, kSplitKPrefillTiles = 128;
+inline int64_t split_k_tiles(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 127) / 128); }
+inline bool split_k_prefill_rows(int64_t M, int64_t N) {
+  return M > 64 && (M <= kSplitKPrefillMaxRows || split_k_tiles(M, N) <= kSplitKPrefillTiles);
+}
 
 int launch_pack_weight(const void* plain, int weight_dtype, int64_t N, int64_t K, void* packed,
                        hipStream_t st);

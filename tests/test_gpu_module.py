@@ -1073,6 +1073,8 @@ def test_deepseek_moe_prompts_in_row_tiles(cuda, monkeypatch, T, E, topk, tile, 
     (4096, 2048, 1100, "INT4", 128, "BF16"),  # more rows than a split launch takes in expert 0, tiles of 64
     (4096, 14336, 600, "INT4", 128, "BF16"),  # gate and up wide: one chain
     (4096, 8192, 2500, "INT4", 64, "BF16"),  # every expert beyond the split: tiles of 128
+    (4096, 512, 1500, "INT4", 128, "BF16"),  # more than 1024 rows on narrow gate and up projections: split all the same
+    (4352, 256, 2600, "INT4", 32, "BF16"),
     (4096, 128, 200, "INT4", 64, "FP16"),
     (8192, 128, 65, "INT8", -1, "FP16"),
 ])

@@ -635,8 +635,11 @@ def test_prefill_kernel_split_k(cuda, kind, M, K, N, G, bias, kernel):
 @pytest.mark.parametrize("kind,M,K,N", [
     ("int4", 65, 4096, 144),    # four workgroups of eight K steps each; one row in the last 64 x 128 tile
     ("int4", 333, 4352, 4096),  # 34 K steps in parts of 10, the last shorter
-    ("int4", 1024, 4224, 1008),  # the most rows that share K, 33 K steps
-    ("int4", 1025, 4096, 256),  # one more: not shared
+    ("int4", 1024, 4224, 1008),  # the most rows that share K on any number of tiles, 33 K steps
+    ("int4", 1025, 4096, 256),  # more: 34 tiles of 64 x 128, shared
+    ("int4", 2048, 4096, 512),  # 128 tiles, shared
+    ("int4", 2049, 4096, 512),  # 132 tiles, not shared
+    ("int8", 1500, 7168, 576), ("nf4", 1500, 4096, 576),
     ("int4_f16", 130, 8192, 272),
     ("nf4", 77, 4096, 3088), ("nf4", 129, 4096, 272),
     ("int8", 600, 4096, 4112), ("int8", 1000, 4608, 4096),  # 128 x 256 tiles of eight waves, K in two

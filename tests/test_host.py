@@ -343,6 +343,26 @@ def test_auto_split_k_predicate_is_the_library_s():
     assert f(128, 2048, 4096, BF16) == 0
 
 
+@pytest.mark.parametrize("M,N,tiles", [(65, 4096, 64), (1024, 4096, 512), (1025, 256, 34), (1500, 576, 120), (2048, 512, 128), (2049, 512, 132), (8192, 128, 128),
+                                       (8193, 16, 129), (1025, 1024, 136)])
+@pytest.mark.parametrize("lowp", [1, 2, 3])
+def test_which_prompts_get_scratch_for_sharing_k(M, N, tiles, lowp):
+    """Floating-point compute: up to 1024 rows, or at most 128 tiles of 64 x 128; lowp_mode INT8: the latter.  A long prompt on a
+    narrow layer leaves half of the chip idle however many rows it has.  The scratch holds two workgroups' tiles at least."""
+    from ipex_amd import _lib
+
+    lib = _lib.load()
+    got = lib.woq_hip_linear_auto_split_k_workspace_bytes(M, 4096, N, lowp)
+    shared = tiles <= 128 or (lowp != 3 and M <= 1024 and tiles <= 384)
+    wide = ((M + 127) // 128) * ((N + 255) // 256)
+    assert (got > 0) == (shared or (lowp != 3 and M <= 1024 and wide <= 128)), got
+    if tiles <= 128:
+        assert got >= 4 * tiles * 64 * 128 * 4
+    assert lib.woq_hip_linear_auto_split_k_workspace_bytes(M, 4095, N, lowp) == 0
+    if tiles > 128 and M > 1024:
+        assert lib.woq_hip_linear_split_k_workspace_bytes(M, N) == 0
+
+
 def test_environment_knobs_of_the_reference_are_read_by_the_library():
     """IPEX_WOQ_SMALL_BATCH_THRESHOLD (csrc/cpu/aten/utils/woq.h:24) and IPEX_WOQ_WEIGHT_CACHE_BATCH_THRESHOLD
     (csrc/cpu/jit/cpu/kernels/LinearWoqPacked.cpp:17-18) are read once per process by the library; values that are
