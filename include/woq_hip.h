@@ -308,7 +308,9 @@ int woq_hip_linear_pair(const woq_hip_linear_params* gate, const woq_hip_linear_
  * lowp_mode INT8 and the split-K scratch live in an array that the library keeps resident on every GPU it
  * runs on (WOQ_HIP_NOALLOC_MAX_WORKSPACE_BYTES plus 2 KiB of counters, until the process ends).  A call
  * whose workspace need (woq_hip_linear_workspace_bytes) exceeds that maximum is rejected with an error
- * before anything is launched; K is shared between workgroups only while that scratch fits as well.
+ * before anything is launched.  K is shared between workgroups by the best plan whose scratch fits beside it: where
+ * woq_hip_linear with the scratch of woq_hip_linear_auto_split_k_workspace_bytes takes a larger one, the fp32 sums are
+ * added in another order.
  * Allocates nothing, on the device or through any library.  All calls on one GPU share the array: calls
  * that may overlap in time on one GPU (different streams, concurrent graph launches) race and must be
  * serialised by the caller.  The first call on a device that needs the array looks up its address, which cannot

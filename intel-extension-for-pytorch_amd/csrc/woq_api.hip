@@ -726,13 +726,15 @@ int woq_hip_linear_noalloc(const woq_hip_linear_params* p) {
                      "resident scratch holds %lld; use woq_hip_linear with a workspace of your own",
                      (long long)p->M, (long long)p->K, (long long)need, (long long)kNoAllocWorkspaceBytes);
   // Sharing K between workgroups is an option, not a need: offered for the problems it pays for (few
-  // output tiles and a long K) while its scratch fits behind the quantized activations.
+  // output tiles and a long K) with what is left behind the quantized activations.  The kernels take the best plan that fits;
+  // the smallest of a prompt shares 64 x 128 tiles between two workgroups.
   bool split = false;
   {
     const int64_t extra = woq_hip_linear_auto_split_k_workspace_bytes(p->M, p->K, p->N, p->lowp_mode);
-    const int64_t base = (need + 255) / 256 * 256;
-    if (extra > 0 && base + extra <= kNoAllocWorkspaceBytes) {
-      need = base + extra;
+    const int64_t base = (need + 255) / 256 * 256, left = kNoAllocWorkspaceBytes - base;
+    const int64_t least = p->M > 64 ? 2 * split_k_tiles(p->M, p->N) * 64 * 128 * (int64_t)sizeof(float) : extra;
+    if (extra > 0 && left >= least) {
+      need = base + (extra < left ? extra : left);
       split = true;
     }
   }

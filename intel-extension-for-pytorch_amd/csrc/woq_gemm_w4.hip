@@ -850,8 +850,9 @@ static int64_t split_bytes(int64_t M, int64_t N, int shape, int splits) {
 // hides them).  Drawn from INT4 g128 and g32, us of gate + up / down with 64 and 128 rows a slot: 32 experts 7168 -> 2048, 128 rows
 // each 400 / 200 and 320 / 175; 3072 -> 1024 91 / 51 and 96 / 53; 5120 -> 1536, 100 rows each 158 / 88 with 128.
 constexpr double kLowSlot = 0.7, kSlotUs8 = 6.0, kSlotUs42 = 5.0;
-// share: K may be shared between workgroups (split_k_prefill_rows, K >= kSplitKPrefillMinK, at least eight steps each)
-static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t, bool share) {
+// scratch: bytes with which K may be shared between workgroups (split_k_prefill_rows, K >= kSplitKPrefillMinK, at least eight
+// steps each), 0: not
+static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t, int64_t scratch) {
   const int64_t np = (N + kTileN - 1) / kTileN * kTileN;
   auto wgs = [&](int bm, int bn) { return ((np + bn - 1) / bn) * ((M + bm - 1) / bm); };
   auto gens = [](int64_t w) { return (double)((w + 255) / 256); };
@@ -859,18 +860,20 @@ static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t,
   auto offer = [&](int shape, int splits, double us) {
     if (us < best.us) best.shape = shape, best.splits = splits, best.us = us;
   };
-  share = share && split_k_prefill_rows(M, np) && (int64_t)ksteps * kTileK4 >= kSplitKPrefillMinK;
+  scratch = std::min(scratch, kSplitScratchMax);
+  const bool share = scratch > 0 && split_k_prefill_rows(M, np) && (int64_t)ksteps * kTileK4 >= kSplitKPrefillMinK;
   const int most42 = t.t42[2] > 0 ? 3 : 2, most2 = t.t2[1] > 0 ? 2 : 1;
   for (int s = 1; s <= (share ? kPrefillSplitMax : 1); ++s) {
     const int kts = s == 1 ? ksteps : split_k_steps(ksteps, s);
     if (s > 1 && (kts < kSplitMinSteps || (s - 1) * kts >= ksteps)) break;
     const int64_t w42 = wgs(64, 128) * s, w8 = wgs(128, 256) * s;
     auto red = [&](int shape, double a, double b) { return s == 1 ? 0.0 : a + b * (double)split_bytes(M, np, shape, s) * 1e-6; };
-    if (w42 <= 256 * most42)
+    const bool fits42 = s == 1 || split_bytes(M, np, 42, s) <= scratch, fits8 = s == 1 || split_bytes(M, np, 5, s) <= scratch;
+    if (w42 <= 256 * most42 && fits42)
       offer(42, s, kts * t.t42[(w42 + 255) / 256 - 1] + red(42, 2.0 + 0.4 * s, 0.25));
     else if (s == 1)
       offer(42, 1, kts * t.t42[most42 - 1] * ((double)w42 / (256 * most42) + 0.25));
-    if (s == 1 || (w8 <= 256 && split_bytes(M, np, 5, s) <= kSplitScratchMax))
+    if (s == 1 || (w8 <= 256 && fits8))
       offer(5, s, kts * gens(w8) * (w8 <= 192 ? t.t8 : t.t8f) + red(5, 2.0, 0.48));
   }
   const int64_t w2 = wgs(128, 128);
@@ -887,7 +890,7 @@ static const StepTimes& step_times(int wbits, int nf4, int fp8) { return wbits =
 // that woq_hip_linear_auto_split_k_workspace_bytes asks for (0: one chain).
 static int chain_steps(int64_t K, int64_t N, int wbits, int row_tiles) {
   const int ksteps = (int)(K / kTileK4);
-  const TilePlan p = plan_tiles(64 * row_tiles, N, ksteps, step_times(wbits, 0, 0), true);
+  const TilePlan p = plan_tiles(64 * row_tiles, N, ksteps, step_times(wbits, 0, 0), kSplitScratchMax);
   return p.splits > 1 ? split_k_steps(ksteps, p.splits) : 0;
 }
 // Estimated microseconds of a grouped launch: `tall` slots of 64 rows (64 x 128 tiles), or of 128 (128 x 256) and `low` ones of at most 64.
@@ -1030,7 +1033,7 @@ static int launch8(const FpArgs& f, int regime, int g_shift, hipStream_t st, int
 
 // Estimated time of the automatic choice below, in microseconds, for the comparison with the dense kernel (gemm_dense_cost).
 double gemm_w4_cost(const FpArgs& f, int wbits) {
-  return plan_tiles(f.M, f.N, (int)(f.KT / (wbits / 4)), step_times(wbits, f.nf4, f.fp8), true).us;
+  return plan_tiles(f.M, f.N, (int)(f.KT / (wbits / 4)), step_times(wbits, f.nf4, f.fp8), kSplitScratchMax).us;
 }
 
 int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int shape, int splits,
@@ -1056,10 +1059,7 @@ int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int s
   if (shape != 0 && shape != 42 && splits > 1) return set_error("woq_gemm_w4_kernel: K is split for the 64 x 128 shape only");
   if (shape == 0) {
     const bool have = scratch && scratch->partial && scratch->counters && splits == 0;
-    const int ksteps = (int)(f.KT / (wbits / 4));
-    const StepTimes& t = step_times(wbits, f.nf4, f.fp8);
-    TilePlan p = plan_tiles(f.M, f.N, ksteps, t, have);
-    if (p.splits > 1 && scratch->bytes < split_bytes(f.M, f.NT * kTileN, p.shape, p.splits)) p = plan_tiles(f.M, f.N, ksteps, t, false);
+    const TilePlan p = plan_tiles(f.M, f.N, (int)(f.KT / (wbits / 4)), step_times(wbits, f.nf4, f.fp8), have ? scratch->bytes : 0);
     shape = p.shape;
     splits = p.splits;
   }

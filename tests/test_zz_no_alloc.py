@@ -62,6 +62,33 @@ def test_noalloc_split_k_decode_and_prefill(cuda):
     assert _run_both(ctx8, case["x"][:70].cuda()) == "woq_gemm_w4i8_kernel"
 
 
+@pytest.mark.parametrize("kind,M,K,N", [("int4", 192, 8192, 4096), ("int4", 333, 11008, 4096), ("int4", 1024, 4096, 1024),
+                                        ("int4", 2048, 4096, 512), ("int8", 400, 8192, 2048), ("nf4", 129, 4096, 4096)])
+def test_noalloc_prompts_share_k_in_what_the_resident_scratch_holds(cuda, monkeypatch, kind, M, K, N):
+    """Prompts whose best plan takes more scratch than is resident: a smaller plan, not none.  Against woq_hip_linear with and
+    without scratch: fp32 sums in another order (K products of one rounding each and K additions: 1e-5 in the 2-norm), and not
+    the sums of one chain."""
+    from ipex_amd import _kernels
+
+    s = _synthetic()
+    case = (s.make_int8_case(55, M, K, N) if kind == "int8" else s.make_nf4_case(55, M, K, N, 64, bias=True) if kind == "nf4" else
+            s.make_int4_case(55, M, K, N, 128, bias=True))
+    ctx = make_context(case, O.LOWP_BF16)
+    x = case["x"].cuda()
+    args = (x, ctx.at_weight_, ctx.weight_dtype_, N, K, *ctx.scales_list_, ctx.zeros_u8_, ctx.group_size_, ctx.bias_f32_, ctx.lowp_mode_,
+            ctx.act_quant_mode_)
+    got = _kernels.linear(*args, noalloc=True, out_fp32=True)
+    shared = _kernels.linear(*args, out_fp32=True)
+    monkeypatch.setattr(_kernels, "_split_k_counters", lambda device: None)
+    alone = _kernels.linear(*args, out_fp32=True)
+    monkeypatch.undo()
+    assert float((got - shared).norm() / shared.norm()) <= 1e-5
+    assert not torch.equal(got, alone)
+    for _ in range(20):
+        again = _kernels.linear(*args, noalloc=True, out_fp32=True)
+        assert torch.equal(again, got)
+
+
 def test_noalloc_plain_calls_and_rejections(cuda):
     from ipex_amd import _kernels
 
