@@ -295,8 +295,9 @@ int64_t woq_hip_int8_block_k(int64_t group_size, int64_t K);
 int woq_hip_linear(const woq_hip_linear_params* p);
 
 /* The front half of a gated MLP in one launch: out = silu(x Wg^T + bg) * (x Wu^T + bu), rounded as woq_hip_linear on `gate` with the
- * silu and then on `up` with the mul round it (Linear2SiluMul; with 17 to 32 rows the K sums may be added in another order).  Both parameter sets name the same x, out, sizes,
- * modes and stream, no post-op.  For the problems of woq_hip_linear_pair_applies: INT4 and INT8 weights with their scale_zero_bf16
+ * silu and then on `up` with the mul round it (Linear2SiluMul).  The K sums may be added in another order with 17 to 32 rows, with 5
+ * to 16 rows where woq_hip_linear shares K (woq_hip_linear_auto_split_k_workspace_bytes), and with 33 to 64 rows and more than
+ * 16384 columns, where it takes the prefill kernel.  Both parameter sets name the same x, out, sizes, modes and stream, no post-op.  For the problems of woq_hip_linear_pair_applies: INT4 and INT8 weights with their scale_zero_bf16
  * tables (and scale_zero_f16x2 for rows that compute in fp16), bf16 rows, lowp_mode BF16 or NONE, at most 64 rows. */
 int woq_hip_linear_pair_applies(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);
 int woq_hip_linear_pair(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);

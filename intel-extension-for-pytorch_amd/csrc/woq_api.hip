@@ -406,6 +406,11 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
 }
 
 // The pair's problem in FpArgs, or false where woq_hip_linear_pair does not take it.
+// 33..64 rows: up to 24576 columns of each weight, three generations of 256 workgroups.  Beyond, two launches of the prefill
+// kernel's 64 x 128 tiles are faster (two launches / the pair, us, INT4: 64 rows 4096 -> 24576 68 / 61, 24608 68 / 78, 28672
+// 70 / 79, 2048 -> 65536 66 / 111; 33 rows 4096 -> 24576 63 / 52, 24608 63 / 66, 28672 63 / 67).  Up to there the pair is, also
+// where two launches would share K or take those tiles (16 rows 8192 -> 4096 17.6 / 10.5, 64 rows 4096 -> 22016 68 / 60).
+constexpr int64_t kPairWideN = 24576;
 static bool pair_problem(const woq_hip_linear_params* g, const woq_hip_linear_params* u, FpArgs& f, int& wbits, int& regime) {
   if (!g || !u || g->struct_size != sizeof(*g) || u->struct_size != sizeof(*u)) return false;
   if (g->weight_dtype != WOQ_HIP_DTYPE_INT4 && g->weight_dtype != WOQ_HIP_DTYPE_INT8) return false;
@@ -436,6 +441,7 @@ static bool pair_problem(const woq_hip_linear_params* g, const woq_hip_linear_pa
   f.szb_b = u->scale_zero_bf16; f.bias_b = u->bias;
   if (regime == kRegimeF16)
     return g->scale_zero_f16x2 && u->scale_zero_f16x2 && decode_kernel_applies(f, wbits, regime, g->scale_zero_f16x2) && decode_pair_applies(f);
+  if (f.M > 32 && f.N > kPairWideN && gemm_w4_applies(f, wbits, regime)) return false;
   return decode_dq_pair_applies(f, wbits, regime);
 }
 

@@ -744,6 +744,34 @@ def test_gate_and_up_in_one_launch(cuda, weight_dtype, G, lowp, K, N, M):
         ops.woq_linear_silu_mul(x, hg, other)
 
 
+@pytest.mark.parametrize("M,K,N,weight_dtype,one", [
+    (64, 256, 24576, "INT4", True), (64, 256, 24592, "INT4", False), (33, 256, 24592, "INT8", False), (32, 256, 24592, "INT4", True),
+    (48, 320, 24592, "INT8", True),  # (K no multiple of 128: not on the prefill kernel)
+    (33, 4096, 17408, "INT4", True), (5, 8192, 272, "INT4", True), (16, 8192, 1040, "INT4", True), (16, 8192, 48, "INT8", True),
+    (1, 8192, 272, "INT4", True), (2, 8192, 272, "INT4", False),  # two to four rows of a long K
+    (65, 256, 272, "INT4", False),
+])
+def test_gate_and_up_in_one_launch_or_two(cuda, M, K, N, weight_dtype, one):
+    """Which problems run in one launch -- it makes one tensor, two launches make two -- and what it computes where its sums have
+    another order than two launches': flips of a last bf16 bit in few outputs (2e-3 in the 2-norm)."""
+    from helpers import rel_l2, to_np_f32
+
+    ipex = _ipex()
+    gate, up = (_woq_module(ipex, K, N, weight_dtype, 128 if weight_dtype == "INT4" else -1, "BF16", bias=True, seed=s) for s in (44, 45))
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(cuda)
+    ops = torch.ops.torch_ipex
+    hg, hu = gate._op_context.get_data_handle(), up._op_context.get_data_handle()
+    want = ops.woq_linear_mul(x, hu, [ops.woq_linear_silu(x, hg)])
+    made = torch.cuda.memory_stats()["allocation.all.allocated"]
+    got = ops.woq_linear_silu_mul(x, hg, hu)
+    made = torch.cuda.memory_stats()["allocation.all.allocated"] - made
+    assert (made == 1) == one, made
+    if one:
+        assert rel_l2(to_np_f32(got), to_np_f32(want)) < 2e-3
+    else:
+        assert torch.equal(got, want)
+
+
 def test_moe_route_against_the_oracle_token_lists(cuda):
     """woq_hip_moe_route: sorted positions, slots per compute type and per-token contribution order against the
     oracle's per-expert token lists (get_expert_topx_idx, MoE.cpp:64-81); ids outside the expert range drop out."""
