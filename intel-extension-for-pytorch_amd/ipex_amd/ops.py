@@ -758,7 +758,7 @@ class _MoeGroupedPlan:
         self.single_row = all(self.few_rows)
         # gate and up in one launch: the same weight type, groups and tables
         self.pair_ok = all(g[k] == u[k] for k in ("G", "wd")) and all((self.tables[0][k] is None) == (self.tables[1][k] is None) for k in ("z8", "sz", "szb"))
-        self.structs = {}
+        self.structs, self.calls, self.unpaired = {}, {}, set()
         self.device = device
         self.tiles = None
         # the prefill kernel over row tiles of the routed rows: whole K steps of 128, power-of-two or per-channel groups
@@ -809,31 +809,36 @@ class _MoeGroupedPlan:
         """One linear over the slots of a size class (``pair``: gate and up as one).  ``p`` has the call's constant fields, ``sz`` per
         linear whether it runs on the integer-weight decode kernels; ``tiles``: the slots are those of woq_hip_moe_route_tiles (all
         its classes, those with ``tile_rows`` on the prefill kernel)."""
-        sh, sz = self.shapes[linear], sz[linear]
-        p.K, p.N, p.weight_dtype, p.group_size, p.M = sh["K"], sh["N"], sh["wd"], sh["G"], bound
-        p.x, p.out, p.fusion, p.others[0] = src.data_ptr(), dst.data_ptr(), fusion, other.data_ptr() if other is not None else None
-        # (a non-null value tells the entry point that the group's scales are (scale, zero) dword tables)
-        p.scale_zero_f16x2 = self.tables[linear]["sz"].data_ptr() if sz else None
-        f16 = _f16_regime(sh["lowp"], x_dtype, bound)
-        flags = _lib.MOE_SZB if self.tables[linear]["szb"] is not None and not f16 and not sz else 0
+        key = (linear, cls, bound, x_dtype, sz[linear], tiles, tile_rows, pair)
+        call = self.calls.get(key)
+        if call is None:  # what a launch of these has in every call
+            sh, t, f16 = self.shapes[linear], self.tables[linear], _f16_regime(self.shapes[linear]["lowp"], x_dtype, bound)
+            flags = _lib.MOE_SZB if t["szb"] is not None and not f16 and not sz[linear] else 0
+            # (a non-null value tells the entry point that the group's scales are (scale, zero) dword tables)
+            call = self.calls[key] = [sh["K"], sh["N"], sh["wd"], sh["G"], t["sz"].data_ptr() if sz[linear] else None, flags, f16, None]
+        p.K, p.N, p.weight_dtype, p.group_size, p.scale_zero_f16x2, flags, f16, group = call
+        p.M, p.x, p.out, p.fusion, p.others[0] = bound, src.data_ptr(), dst.data_ptr(), fusion, other.data_ptr() if other is not None else None
         if pair:
-            if not f16 and not flags and not tile_rows or not lib.woq_hip_moe_pair_applies(ctypes.byref(p), tile_rows):
+            if not f16 and not flags and not tile_rows or not lib.woq_hip_moe_pair_applies(p, tile_rows):
                 return False
             flags |= _lib.MOE_PAIR
-        g = self.group_struct(linear, cls, f16, linear < 2, sz, tiles, pair)
-        _lib.check(lib.woq_hip_moe_linear(ctypes.byref(p), g.data_ptr(), slots, tile_rows, flags), "woq_linear_grouped")
+        if group is None:
+            group = call[-1] = self.group_struct(linear, cls, f16, linear < 2, sz[linear], tiles, pair).data_ptr()
+        rc = lib.woq_hip_moe_linear(p, group, slots, tile_rows, flags)
+        if rc != 0:
+            _lib.check(rc, "woq_linear_grouped")
         return True
 
     def gate_up(self, lib, p, x, act, inter, cls, bound, slots, sz, tiles, tile_rows=0):
         """silu(gate(x)) * up(x) of a size class: in one launch where there is one, else in two."""
-        args = (cls, bound, slots, x.dtype, sz, tiles, tile_rows)
-        key = ("pair", bound, tile_rows, x.dtype, sz[0])
-        pair = self.pair_ok and sz[0] == sz[1] and self.structs.get(key, True)
-        if pair and self.launch(lib, p, 0, x, inter, *args, pair=True):
-            return
-        self.structs[key] = False  # (asked once)
-        self.launch(lib, p, 0, x, act, *args, fusion=_lib.FUSE_SILU)
-        self.launch(lib, p, 1, x, inter, *args, fusion=_lib.FUSE_MUL, other=act)
+        x_dtype = x.dtype
+        key = (bound, tile_rows, x_dtype, sz[0])
+        if self.pair_ok and sz[0] == sz[1] and key not in self.unpaired:
+            if self.launch(lib, p, 0, x, inter, cls, bound, slots, x_dtype, sz, tiles, tile_rows, pair=True):
+                return
+            self.unpaired.add(key)  # (asked once)
+        self.launch(lib, p, 0, x, act, cls, bound, slots, x_dtype, sz, tiles, tile_rows, _lib.FUSE_SILU)
+        self.launch(lib, p, 1, x, inter, cls, bound, slots, x_dtype, sz, tiles, tile_rows, _lib.FUSE_MUL, act)
 
 
 def _moe_plan(gate_ctx, up_ctx, down_ctx, device, stream):
