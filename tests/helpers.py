@@ -79,3 +79,34 @@ def make_torch_context(case, lowp_mode, act_quant_mode=-1, device="cuda", cache=
         act_quant_mode,
         cache,
     )
+
+
+def scratch_written(ctx, x):
+    """Whether woq_hip_linear, called with the scratch that the library asks for, writes any of it: the quantized activations of
+    lowp_mode INT8, the partial tiles of workgroups that share K.  ``ctx``: a context of make_context."""
+    import ctypes
+
+    from ipex_amd import _kernels, _lib
+
+    lib = _lib.load()
+    (N, K), M = ctx.weight_shape_, x.shape[0]
+    ptr = lambda t: None if t is None else t.data_ptr()
+    need = lib.woq_hip_linear_workspace_bytes(M, K, ctx.lowp_mode_, ctx.act_quant_mode_, ctx.group_size_)
+    need = (need + 255) // 256 * 256 + lib.woq_hip_linear_auto_split_k_workspace_bytes(M, K, N, ctx.lowp_mode_)
+    scratch = torch.full((max(need, 1),), 0xA5, dtype=torch.uint8, device=x.device)
+    counters = torch.zeros(512, dtype=torch.int32, device=x.device)
+    out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    p = _lib.LinearParams()
+    p.struct_size = ctypes.sizeof(_lib.LinearParams)
+    p.x, p.x_dtype, p.out, p.out_dtype = ptr(x), _kernels._ACT_CODE[x.dtype], ptr(out), _kernels._ACT_CODE[x.dtype]
+    p.M, p.K, p.N = M, K, N
+    p.qweight, p.weight_dtype, p.group_size = ptr(ctx.at_weight_), ctx.weight_dtype_, ctx.group_size_
+    p.scales_f32, p.scales_f16, p.scales_bf16 = (ptr(t) for t in ctx.scales_list_)
+    p.zeros_u8, p.bias = ptr(ctx.zeros_u8_), ptr(ctx.bias_f32_)
+    p.scale_zero_f16x2, p.scale_zero_bf16 = ptr(ctx.scale_zero_f16x2_), ptr(ctx.scale_zero_bf16_)
+    p.lowp_mode, p.act_quant_mode = ctx.lowp_mode_, ctx.act_quant_mode_
+    p.workspace, p.workspace_bytes, p.split_k_counters = (ptr(scratch), need, ptr(counters)) if need else (None, 0, None)
+    p.stream = torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.woq_hip_linear(ctypes.byref(p)), "woq_linear")
+    torch.cuda.synchronize()
+    return bool((scratch != 0xA5).any())

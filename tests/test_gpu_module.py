@@ -1391,6 +1391,15 @@ def test_deepseek_moe_prompt_slots_of_few_rows(cuda, monkeypatch, tile, H, I, we
     want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
     monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
     monkeypatch.setattr(ops, "_moe_tile_rows", lambda shapes, counts: tile)
+    launches, launch = [], ops._MoeGroupedPlan.launch
+
+    def record(self, lib, p, linear, *args, **kw):
+        done = launch(self, lib, p, linear, *args, **kw)
+        launches.append((linear, kw.get("pair", False), done))
+        return done
+
+    monkeypatch.setattr(ops._MoeGroupedPlan, "launch", record)
     got = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    assert launches == [(0, True, True), (2, False, True)]  # every expert has more than 64 rows: one class, gate and up in one launch
     assert _lib.last_kernel() == "moe_combine_rows"
     assert torch.equal(got, want)

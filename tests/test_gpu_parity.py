@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import bf16_ulp_diff, case_np, make_context, make_torch_context, max_abs, rel_l2, to_np_f32
+from helpers import bf16_ulp_diff, case_np, make_context, make_torch_context, max_abs, rel_l2, scratch_written, to_np_f32
 from oracle import woq_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -632,20 +632,22 @@ def test_prefill_kernel_split_k(cuda, kind, M, K, N, G, bias, kernel):
     assert all(int(buf.abs().sum()) == 0 for buf in kmod._counter_cache.values())
 
 
-@pytest.mark.parametrize("kind,M,K,N", [
-    ("int4", 65, 4096, 144),    # four workgroups of eight K steps each; one row in the last 64 x 128 tile
-    ("int4", 333, 4352, 4096),  # 34 K steps in parts of 10, the last shorter
-    ("int4", 1024, 4224, 1008),  # the most rows that share K on any number of tiles, 33 K steps
-    ("int4", 1025, 4096, 256),  # more: 34 tiles of 64 x 128, shared
-    ("int4", 2048, 4096, 512),  # 128 tiles, shared
-    ("int4", 2049, 4096, 512),  # 132 tiles, not shared
-    ("int8", 1500, 7168, 576), ("nf4", 1500, 4096, 576),
-    ("int4_f16", 130, 8192, 272),
-    ("nf4", 77, 4096, 3088), ("nf4", 129, 4096, 272),
-    ("int8", 600, 4096, 4112), ("int8", 1000, 4608, 4096),  # 128 x 256 tiles of eight waves, K in two
-    ("fp8", 999, 4096, 4080), ("fp8", 70, 4352, 272),
+@pytest.mark.parametrize("kind,M,K,N,shared", [
+    ("int4", 65, 4096, 144, True),    # four workgroups of eight K steps each; one row in the last 64 x 128 tile
+    ("int4", 333, 4352, 4096, False),  # 34 K steps: sharing them costs more than it gives
+    ("int4", 333, 8448, 4096, True),  # 66 K steps in parts of 18, the last shorter
+    ("int4", 1024, 4224, 1008, True),  # the most rows that share K on any number of tiles, 33 K steps
+    ("int4", 1025, 4096, 256, True),  # more: 34 tiles of 64 x 128
+    ("int4", 2048, 4096, 512, True),  # 128 tiles
+    ("int4", 2049, 4096, 512, False),  # 132 tiles
+    ("int8", 1500, 7168, 576, True), ("nf4", 1500, 4096, 576, True),
+    ("int4_f16", 130, 8192, 272, True),
+    ("nf4", 77, 4096, 3088, True), ("nf4", 129, 4096, 272, True),
+    ("int8", 600, 4096, 4112, True), ("int8", 1000, 7168, 4096, True), ("fp8", 999, 7168, 4080, True),  # 128 x 256 tiles of eight waves, K in two
+    ("int8", 1000, 4608, 4096, False), ("fp8", 999, 4096, 4080, False),  # 128 x 128 tiles
+    ("fp8", 70, 4352, 272, True),
 ])
-def test_prefill_kernel_by_estimated_time(cuda, kind, M, K, N):
+def test_prefill_kernel_by_estimated_time(cuda, kind, M, K, N, shared):
     """The automatic choice of tiles and K shares: against the general kernel (the same rounded weights, fp32 sums in another
     order, then one rounding to the output's 16 bits: flips of a last bit of 2^-9 (2^-11) in few outputs, 1e-3 in the 2-norm), a
     post-op and a bias included; repeated calls give the same bits and leave the counters at zero."""
@@ -657,6 +659,7 @@ def test_prefill_kernel_by_estimated_time(cuda, kind, M, K, N):
             syn.make_int4_case(61, M, K, N, 128, bias=True, scale_dtype=torch.float16 if f16 else torch.bfloat16))
     x = (case["x"].half() if f16 else case["x"]).cuda()
     ctx = make_context(case, O.LOWP_FP16 if f16 else O.LOWP_BF16)
+    assert scratch_written(ctx, x) == shared
     other = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(x.dtype).cuda()
     for args in ({}, {"fusion": _lib_mod().FUSE_ADD, "others": (other,)}):
         got = ctx.run(x, **args)
@@ -2467,6 +2470,8 @@ def test_int8_rows_quantized_in_the_gemm_have_the_bits_of_two_launches(cuda, M, 
     per_row = 6 if mode == 4 else mode  # (five rows' tensor has another scale than one row's)
     many = make_context(case, O.LOWP_INT8, per_row)
     x = case["x"]
+    two = (M, K, N) in ((4, 4096, 4112), (3, 5376, 80))
+    assert scratch_written(ctx, x.cuda()) == two  # (the quantized rows stay in LDS, or go through memory)
     variants = [x, torch.zeros_like(x), x * 2.0 ** -110, x * 2.0 ** 104, x.to(torch.float16)]
     for value in (float("inf"), float("nan")):
         v = x.clone()
