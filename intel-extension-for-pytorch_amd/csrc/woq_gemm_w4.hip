@@ -8,7 +8,7 @@
 //   * v_mfma_f32_16x16x32 with A = activations and B = weights, as in the decode kernel: the
 //     dequantized registers of one packed dword ARE the B operand, so weights never touch LDS
 //     in dequantized form and every weight is dequantized by exactly one wave;
-//   * a workgroup is 4 waves, one per SIMD with the whole 512-entry register file; wave w owns NTW
+//   * a workgroup is four waves (128 x 256 tiles: eight, see below), one per SIMD with the whole 512-entry register file; wave w owns NTW
 //     weight row-blocks (16 columns each) for all 16 * MT rows of the workgroup, i.e. MT x NTW
 //     accumulator tiles.  The shape built is 128 x 448 (MT 8, NTW 7: 224 accumulator registers;
 //     14336 / 448 = 32 and 2048 / 128 = 16 give 512 workgroups = two full generations on 256 CUs).
@@ -475,6 +475,7 @@ __device__ __forceinline__ void g4_tile(const FpArgs& fa, const int g_shift, flo
           if (j == 3 && t == 0) __builtin_amdgcn_s_waitcnt(kVmcntStep);  // tiles of step kt + 1 are in LDS
           // Behind the barrier the other waves refill the buffer of this step.  In the first block the barrier stands before
           // the first use of the last sub-step's fragments: their reads must have returned (before a later block they have).
+          // (What this wait costs: at most 2 %, M = 1000, 7168 -> 4096 FP8 72.0 -> 73.6 us; the other prompts 0 to 1 %.)
           if constexpr (STAG_MAX == 0) {
             if (bar_here && j == 3) {
               // Written as an instruction, not as the barrier builtin: before that one the compiler
@@ -840,7 +841,7 @@ struct TilePlan {
   double us = 1e30;
 };
 constexpr int kSplitMinSteps = 8;
-constexpr int64_t kSplitScratchMax = 32 << 20;
+constexpr int64_t kSplitScratchMax = 32 << 20;  // partial tiles of 256 workgroups of 128 x 256, the most that a plan has (64 x 128: 768, 24 MiB)
 static int64_t split_bytes(int64_t M, int64_t N, int shape, int splits) {
   const int64_t bm = shape == 5 ? 128 : 64, bn = shape == 5 ? 256 : 128;
   return splits * ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * bm * bn * (int64_t)sizeof(float);

@@ -81,7 +81,10 @@ constexpr int kSplitKCounters = 512;
 constexpr int kSplitKMax = 4;
 // Prefill problems that get split-K scratch by themselves (woq_hip_linear_auto_split_k_workspace_bytes): K of at least
 // kSplitKPrefillMinK and at most kSplitKPrefillMaxRows rows, or any number of rows in at most kSplitKPrefillTiles tiles of
-// 64 x 128, which leave half of the chip idle (the one condition of lowp_mode INT8).
+// 64 x 128, which leave half of the chip idle (the one condition of lowp_mode INT8).  Neither bound lies where sharing stops
+// paying: 1024 rows are the longest prompts that it was timed on with more tiles than that, and a shorter K gains in the kernel
+// as well (INT4, 64 x 128 tiles of one / two / four workgroups, us: M = 128, 2048 -> 1024 14.2 / 11.5 / 10.1, 3072 -> 4096
+// 19.6 / 14.6 / 12.7, M = 1000, 2048 -> 1024 15.3 / 13.4 / 14.2; not M = 333, 3072 -> 4096 21.4 / 22.3 / 21.4).
 constexpr int64_t kSplitKPrefillMinK = 4096, kSplitKPrefillMaxRows = 1024, kSplitKPrefillTiles = 128;
 inline int64_t split_k_tiles(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 127) / 128); }
 inline bool split_k_prefill_rows(int64_t M, int64_t N) {

@@ -865,7 +865,7 @@ def _f16_regime(lowp, x_dtype, rows):
 
 def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, routing_weights, host_ids):
     """The layer in five to fourteen launches and, up to 64 tokens, without reading the routing on the host: the routing is sorted on the
-    device, every linear runs once per compute type over all experts that have tokens (woq_hip_linear_grouped), and
+    device, every linear runs once per compute type over all experts that have tokens (woq_hip_moe_linear), and
     the contributions of a token are added in ascending expert order.  Returns None when the layer does not fit
     (more than 8192 routed rows, mixed experts, act-order, NF4 / FP8 / lowp INT8 ...): the caller then takes the per-expert path."""
     x = hidden_states
@@ -950,8 +950,9 @@ def _moe_expert_launches_faster(shapes, counts):
     ``counts``: rows of every expert.
     One expert with tokens, long K: its own launches split K over workgroups (INT4 g128, one expert, us per expert / in tiles: 14336 -> 4096
     with 128 / 512 tokens 223 / 277 and 368 / 386, 11008 -> 2048 193 / 240 and 261 / 247, but 8192 -> 4096 209 / 204 and 274 / 270).
-    INT8 experts of many rows: drawn while the slots had 128 x 128 tiles at most (2 experts 8192 -> 8192, 2048
-    rows each 1969 / 2287; with the 128 x 256 tiles that they have now 1890..1980 / 1660..1690, 4096 -> 14336 with 2500 rows 2728 / 2566, with 4096 3692 / 3997; INT4 with 4096 rows 4329 / 3105).
+    INT8 experts of many rows: drawn while the slots had 128 x 128 tiles at most, and not drawn again: it still sends layers to
+    the experts' launches that the slots' 128 x 256 tiles now serve faster (2 experts 8192 -> 8192, 2048
+    rows each 1969 / 2287 then, 1890..1980 / 1660..1690 now, 4096 -> 14336 with 2500 rows 2728 / 2566, with 4096 3692 / 3997; INT4 with 4096 rows 4329 / 3105).
     Estimates at K = 4096: 69.6 us for 256 tiles of 128 x 256, 0.159 us a tile of 128 x 128; 40 us and 0.015 us a row more
     for an expert's launches."""
     active = [n for n in counts if n]
@@ -971,7 +972,7 @@ def _moe_expert_launches_faster(shapes, counts):
 
 def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids, raw_stream):
     """The layer for prompts (more than 64 tokens): the routed rows of all experts in row tiles of the prefill kernel, one
-    launch per linear (woq_hip_linear_grouped_tiles), with the bits of the experts' own launches (those from the packed weight);
+    launch per linear (woq_hip_moe_linear), with the bits of the experts' own launches (those from the packed weight);
     experts with at most 64 rows on the decode kernels as above.  The routing is read on the host to refuse ids that name no expert, as the
     per-expert path does, and says which of the size classes are empty.  None where the per-expert path is the faster one."""
     T, H = x.shape
