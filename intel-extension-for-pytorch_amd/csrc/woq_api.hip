@@ -655,8 +655,8 @@ int woq_hip_moe_route_tiles(const int64_t* topk_ids, int64_t T, int64_t topk, in
                             int64_t split_mid, int64_t tile_rows, int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of,
                             int32_t* slot_of, void* stream) {
   if (T < 0 || topk <= 0 || experts <= 0) return set_error("moe_route_tiles: bad size");
-  if (split_lo < 0 || split_lo > 64 || split_mid < 0 || split_mid > 64 || (tile_rows != 64 && tile_rows != 128))
-    return set_error("moe_route_tiles: split_lo and split_mid are 0..64, tile_rows 64 or 128");
+  if (split_lo < 0 || split_lo > 64 || split_mid < 0 || split_mid > 64 || (tile_rows != 64 && tile_rows != 128 && tile_rows != 160))
+    return set_error("moe_route_tiles: split_lo and split_mid are 0..64, tile_rows 64, 128 or 160");
   if (T > 0 && (!topk_ids || !x_row || !slots || !row_of || !slot_of)) return set_error("moe_route_tiles: null pointer");
   return launch_moe_route_tiles(topk_ids, T, topk, experts, split_lo, split_mid, tile_rows, S, x_row, slots, row_of, slot_of,
                                 (hipStream_t)stream);

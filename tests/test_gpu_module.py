@@ -1403,3 +1403,47 @@ def test_deepseek_moe_prompt_slots_of_few_rows(cuda, monkeypatch, tile, H, I, we
     assert launches == [(0, True, True), (2, False, True)]  # every expert has more than 64 rows: one class, gate and up in one launch
     assert _lib.last_kernel() == "moe_combine_rows"
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("T,topk,E,rows", [(65, 1, 1, 64), (512, 8, 32, 160), (1024, 8, 1024, 128), (1023, 8, 67, 160), (777, 3, 5, 160), (4097, 1, 2, 128)])
+def test_moe_route_tiles_against_sorted_lists(cuda, T, topk, E, rows):
+    """Places, slots and the order of a token's contributions, at one and at 1024 experts, at remainders of the 64 entries that a wave
+    numbers at a time, with ids that name no expert."""
+    from ipex_amd import _lib
+
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(T)
+    ids = torch.randint(0, E, (T, topk), generator=g)
+    ids[T // 2, 0], ids[T - 1, topk - 1] = -1, E
+    R, S = T * topk, E + T * topk // 64
+    i32 = lambda *n: torch.full(n, -7, dtype=torch.int32, device=cuda)
+    x_row, slots, row_of, slot_of = torch.full((R,), -7, dtype=torch.int64, device=cuda), i32(4, 3, S), i32(R), i32(R)
+    dev = ids.to(cuda)
+    rc = lib.woq_hip_moe_route_tiles(dev.data_ptr(), T, topk, E, 5, 16, rows, S, x_row.data_ptr(), slots.data_ptr(), row_of.data_ptr(),
+                                     slot_of.data_ptr(), None)
+    assert rc == 0, lib.woq_hip_last_error()
+    torch.cuda.synchronize()
+    flat = ids.flatten().tolist()
+    order = sorted((i for i in range(R) if 0 <= flat[i] < E), key=lambda i: (flat[i], i))
+    place = {i: p for p, i in enumerate(order)}
+    assert x_row.cpu().tolist()[:len(order)] == [i // topk for i in order]
+    want = [[], [], [], []]
+    first = 0
+    for e in range(E):
+        n = flat.count(e)
+        cls = 0 if n < 5 else 1 if n <= 16 else 2 if n <= 64 else 3
+        count = 1 if cls < 3 else -(-n // rows)
+        step = 64 if cls < 3 else -(-n // count) if rows == 160 else rows
+        step = -(-step // 16) * 16
+        want[cls] += [(e, first + r, min(step, n - r) | (n << 16 if cls == 3 else 0)) for r in range(0, n, step)]
+        first += n
+    got = slots.cpu()
+    for cls in range(4):
+        n = len(want[cls])
+        assert list(zip(*(got[cls, q, :n].tolist() for q in range(3)))) == want[cls]
+        assert got[cls, 0, n:].eq(-1).all()
+    ro, so = row_of.cpu().view(T, topk).tolist(), slot_of.cpu().view(T, topk).tolist()
+    for t in range(T):
+        mine = sorted((j for j in range(topk) if t * topk + j in place), key=lambda j: (flat[t * topk + j], j))
+        assert ro[t][:len(mine)] == [place[t * topk + j] for j in mine] and so[t][:len(mine)] == mine
+        assert all(r == -1 for r in ro[t][len(mine):])
