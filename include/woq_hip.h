@@ -428,7 +428,7 @@ int woq_hip_moe_route(const int64_t* topk_ids, int64_t T, int64_t topk, int64_t 
                       int64_t split_mid, int use_single, int64_t S, int64_t* x_row, int32_t* slots, int32_t* row_of,
                       int32_t* slot_of, void* stream);
 int woq_hip_linear_grouped(const woq_hip_linear_params* p, const void* group, int64_t slots);
-/* woq_hip_linear_grouped (tile_rows 0) and woq_hip_linear_grouped_tiles below (64 or 128) with two options.
+/* woq_hip_linear_grouped (tile_rows 0) and woq_hip_linear_grouped_tiles below (64, 128 or, with 4-bit weights, 160) with two options.
  * WOQ_HIP_MOE_SZB: the group has the experts' merged (scale, zero) tables; bf16 compute then reads those (same results).
  * WOQ_HIP_MOE_PAIR: out = silu(gate) * up of the group's two sets of linears in one launch, rounded as the launch with the silu
  * and the one with the mul round it; p without a post-op.  For the problems of woq_hip_moe_pair_applies(p, tile_rows) (with
@@ -441,7 +441,8 @@ int woq_hip_moe_linear(const woq_hip_linear_params* p, const void* group, int64_
  * The same layer for prompts: woq_hip_moe_route_tiles sorts at most WOQ_HIP_MOE_TILES_MAX entries over at most
  * WOQ_HIP_MOE_TILES_EXPERTS experts and cuts the routed rows into slots, int32 [4][3][S], S >= experts + T * topk /
  * tile_rows: class 0 the experts with fewer than split_lo rows, 1 at most split_mid, 2 at most 64, one slot each; class 3
- * the others, in slots of at most tile_rows (64 or 128) rows, each slot's rows plus the expert's rows << 16;
+ * the others, in slots of at most tile_rows (64 or 128; 160: an expert's rows evenly over its slots) rows, each slot's rows plus the
+ * expert's rows << 16;
  * split_lo and split_mid at most 64.  x_row, row_of and slot_of as from woq_hip_moe_route.
  * woq_hip_linear_grouped_tiles runs one linear over the slots of class 3 on the prefill kernel: p as for
  * woq_hip_linear_grouped (M is ignored), INT4 weights with power-of-two groups of at least 32 or INT8 weights with
@@ -451,7 +452,7 @@ int woq_hip_moe_linear(const woq_hip_linear_params* p, const void* group, int64_
  * woq_hip_linear_auto_split_k_workspace_bytes asks for) runs the same K ranges one after the other and adds them in that
  * launch's order, so it has that launch's bits; woq_hip_moe_chained_rows: the most rows of such an expert, 0 if there is none
  * at this K and N.  Slots whose table does not say the expert's rows run K in one chain.
- * woq_hip_moe_tile_rows: the tile_rows (64 or 128) with the lower estimated time for a gated layer H -> I -> H whose experts
+ * woq_hip_moe_tile_rows: the tile_rows (64, 128 or 160) with the lower estimated time for a gated layer H -> I -> H whose experts
  * have counts[e] rows (on the host).
  */
 int woq_hip_moe_tile_rows(const int64_t* counts, int64_t experts, int64_t H, int64_t I, int gate_dtype, int down_dtype);

@@ -529,7 +529,7 @@ int woq_hip_moe_pair_applies(const woq_hip_linear_params* p, int tile_rows) {
   int wbits, regime;
   const int64_t rows = tile_rows ? tile_rows : p ? p->M : 0;
   if (rows < 1 || grouped_problem(p, p, rows, f, wbits, regime)) return 0;
-  if (tile_rows) return (tile_rows == 64 || tile_rows == 128) && gemm_w4_applies(f, wbits, regime);
+  if (tile_rows) return (tile_rows == 64 || tile_rows == 128 || (tile_rows == 160 && wbits == 4)) && gemm_w4_applies(f, wbits, regime);
   if (f.NT % 2 != 0) return 0;
   if (p->scale_zero_f16x2)
     return p->M <= 4 && decode_kernel_applies(f, wbits, regime, (const uint32_t*)p->scale_zero_f16x2) && decode_pair_applies(f);
@@ -568,9 +568,11 @@ int64_t woq_hip_moe_chained_rows(int64_t K, int64_t N) { return K > 0 && N > 0 ?
 static int linear_grouped_tiles(const woq_hip_linear_params* p, const void* group, int64_t slots, int tile_rows, int flags) {
   FpArgs f;
   int wbits, regime;
-  if (tile_rows != 64 && tile_rows != 128) return set_error("woq_linear_grouped_tiles: 64 or 128 rows per slot, got %d", tile_rows);
+  if (tile_rows != 64 && tile_rows != 128 && tile_rows != 160)
+    return set_error("woq_linear_grouped_tiles: 64, 128 or 160 rows per slot, got %d", tile_rows);
   if (slots < 1 || slots > 65535) return set_error("woq_linear_grouped_tiles: bad slot count %lld", (long long)slots);
   if (int rc = grouped_problem(p, group, tile_rows, f, wbits, regime)) return rc;
+  if (tile_rows == 160 && wbits != 4) return set_error("woq_linear_grouped_tiles: slots of 160 rows go with 4-bit weights");
   if (int rc = moe_flags(p, flags, f, regime)) return rc;
   if (!gemm_w4_applies(f, wbits, regime))
     return set_error("woq_linear_grouped_tiles: K a multiple of 128, power-of-two groups (INT4: 32 and more, INT8: 128 and "

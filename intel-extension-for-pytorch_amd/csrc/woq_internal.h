@@ -193,10 +193,10 @@ bool gemm_w4s_applies(const FpArgs& f, int wbits, int regime);
 int launch_gemm_w4s(const FpArgs& f, int regime, hipStream_t st);
 int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int shape = 0, int splits = 0,
                    const SplitKScratch* scratch = nullptr);
-// 64 or 128: rows of a slot with the lower estimated time of a routed layer's two launches (gate and up as one of twice the columns)
+// 64, 128 or 160: rows of a slot with the lower estimated time of a routed layer's two launches (gate and up as one of twice the columns)
 int gemm_w4_tile_rows(const int64_t* counts, int64_t experts, const int64_t* K, const int64_t* N, const int* wbits);
 int gemm_w4_split_rows(int64_t K, int64_t N);  // most rows of an expert of a routed layer that runs K in chains, 0: none
-// The same kernel over the slots of a routed layer (at most tile_rows = 64 or 128 routed rows of one expert each)
+// The same kernel over the slots of a routed layer (at most tile_rows = 64, 128 or, with 4-bit weights, 160 routed rows of one expert each)
 int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGroup* grp, int64_t slots, int tile_rows,
                            hipStream_t st);
 // Dense bf16 GEMM on the fragment-laid copy that launch_dense_weight writes (woq_gemm_dense.hip): bf16 activations,

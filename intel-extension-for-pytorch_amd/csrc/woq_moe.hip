@@ -195,8 +195,8 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const int64_t* __restric
 // token gives every entry a slot of its own.  A wave numbers the entries of its part of the table, 64 at a time: the lanes that name
 // the same expert are found with one ballot per bit of an expert's number, and a count per (wave, expert) in LDS carries over from one
 // 64 to the next.  A scan over the experts and their waves' counts then gives every entry its place.
-// Bound: latencies -- the read of the ids, some LDS round trips, the stores.  4096 entries over 32 experts 24 -> 9 us, 128 entries
-// 9.9 -> 5.5 us (the walk of a wave over all entries for each of its experts, or every entry compared with every other).
+// Bound: latencies -- the read of the ids, some LDS round trips, the stores.  4096 entries over 32 experts 24 -> 15 us, 128 entries
+// 9.9 -> 5.3 us (the walk of a wave over all entries for each of its experts, or every entry compared with every other).
 //   slots   [4 classes][expert, first row, rows][S].  TILES: 0: experts with fewer than split_lo rows, 1: at most split_mid, 2: at most
 //           64, one slot each; 3: the others in slots of at most tile_rows rows (160: the expert's rows evenly, in whole row tiles
 //           of 16), an expert's slots one after the other, rows | the expert's rows << 16 in place of rows; else the classes of

@@ -939,7 +939,7 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
 
 
 def _moe_tile_rows(shapes, counts):
-    """Rows of a slot of the prefill kernel, 64 or 128, by the lower estimated time.  ``shapes``: K, N and weight dtype (wd) of the
+    """Rows of a slot of the prefill kernel, 64, 128 or 160, by the lower estimated time.  ``shapes``: K, N and weight dtype (wd) of the
     three linears, ``counts``: rows of every expert."""
     gate, down = shapes[0], shapes[2]
     return _lib.load().woq_hip_moe_tile_rows((ctypes.c_int64 * len(counts))(*counts), len(counts), gate["K"], gate["N"], gate["wd"], down["wd"])

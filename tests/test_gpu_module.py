@@ -1405,6 +1405,36 @@ def test_deepseek_moe_prompt_slots_of_few_rows(cuda, monkeypatch, tile, H, I, we
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("H,I,G,lowp", [(256, 384, 32, "BF16"), (4096, 256, 128, "BF16"), (8192, 128, 64, "BF16"), (4352, 128, 128, "FP16")])
+def test_deepseek_moe_prompt_slots_of_160_rows(cuda, monkeypatch, H, I, G, lowp):
+    """Experts at the edges of 32, 64, 96, 128 and 160 rows a slot and of two and three slots, with K in one chain and in several: bit for
+    bit the experts' own launches.  Slots of 160 rows go with 4-bit weights."""
+    from ipex_amd import _lib, ops
+
+    ipex = _ipex()
+    rows = [65, 96, 97, 128, 129, 144, 160, 161, 0, 320, 321]
+    mk = lambda k, n, s: _woq_module(ipex, k, n, "INT4", G, lowp, bias=True, seed=s)._op_context
+    E = len(rows)
+    ctxs = [[mk(H, I, 900 + e) for e in range(E)], [mk(H, I, 920 + e) for e in range(E)], [mk(I, H, 940 + e) for e in range(E)]]
+    g = torch.Generator().manual_seed(9)
+    xdt = torch.float16 if lowp == "FP16" else torch.bfloat16
+    T = sum(rows)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(T, generator=g)].view(T, 1).to(cuda)
+    hidden = torch.randn(T, H, generator=g).to(xdt).to(cuda)
+    rw = torch.rand(T, 1, generator=g).to(xdt).to(cuda)
+    op = torch.ops.torch_ipex.deepseek_moe_woq
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
+    want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
+    monkeypatch.setattr(ops, "_moe_tile_rows", lambda shapes, counts: 160)
+    got = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    assert _lib.last_kernel() == "moe_combine_rows"
+    assert torch.equal(got, want)
+    mk8 = lambda k, n, s: _woq_module(ipex, k, n, "INT8", -1, lowp, seed=s)._op_context
+    with pytest.raises(RuntimeError, match="4-bit weights"):
+        op(hidden, ids, [mk8(H, I, e) for e in range(E)], [mk8(H, I, e) for e in range(E)], [mk8(I, H, e) for e in range(E)], rw, False)
+
+
 @pytest.mark.parametrize("T,topk,E,rows", [(65, 1, 1, 64), (512, 8, 32, 160), (1024, 8, 1024, 128), (1023, 8, 67, 160), (777, 3, 5, 160), (4097, 1, 2, 128)])
 def test_moe_route_tiles_against_sorted_lists(cuda, T, topk, E, rows):
     """Places, slots and the order of a token's contributions, at one and at 1024 experts, at remainders of the 64 entries that a wave
