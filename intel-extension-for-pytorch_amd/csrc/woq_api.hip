@@ -440,7 +440,7 @@ static bool pair_problem(const woq_hip_linear_params* g, const woq_hip_linear_pa
   f.qweight_b = (const uint8_t*)u->qweight; f.scales_b = (const uint16_t*)u->scales_bf16; f.zeros_b = u->zeros_u8;
   f.szb_b = u->scale_zero_bf16; f.bias_b = u->bias;
   if (regime == kRegimeF16)
-    return g->scale_zero_f16x2 && u->scale_zero_f16x2 && decode_kernel_applies(f, wbits, regime, g->scale_zero_f16x2) && decode_pair_applies(f);
+    return g->scale_zero_f16x2 && u->scale_zero_f16x2 && decode_kernel_applies(f, wbits, regime, g->scale_zero_f16x2) && decode_pair_applies(f, false);
   if (f.M > 32 && f.N > kPairWideN && gemm_w4_applies(f, wbits, regime)) return false;
   return decode_dq_pair_applies(f, wbits, regime);
 }
@@ -532,7 +532,7 @@ int woq_hip_moe_pair_applies(const woq_hip_linear_params* p, int tile_rows) {
   if (tile_rows) return (tile_rows == 64 || tile_rows == 128 || (tile_rows == 160 && wbits == 4)) && gemm_w4_applies(f, wbits, regime);
   if (f.NT % 2 != 0) return 0;
   if (p->scale_zero_f16x2)
-    return p->M <= 4 && decode_kernel_applies(f, wbits, regime, (const uint32_t*)p->scale_zero_f16x2) && decode_pair_applies(f);
+    return p->M <= 4 && decode_kernel_applies(f, wbits, regime, (const uint32_t*)p->scale_zero_f16x2) && decode_pair_applies(f, true);
   return p->M <= 64 && decode_dq_pair_applies(f, wbits, regime);
 }
 

@@ -58,6 +58,9 @@ __device__ __forceinline__ f4 mfma16(u4 a, u4 b, f4 c) {
 // PAIR (the front half of a gated MLP, FpArgs::pair): the two tiles of a workgroup are the same row-block of two weights, and the
 // tail stores silu(first) * second: one launch, its ramp and its activations instead of two, and no intermediate tensor
 // (one row, 4096 -> 2 x 14336 and back with a residual: 24.4 us in three launches, 19.7 in two).
+// With eight K tiles a wave (routed slots; K = 7168 in one round) the second weight's tiles take over the registers of the first one's as
+// these are consumed: eight tiles in flight all the time, 84 registers.  17 slots of two to four rows, 7168 -> 2 x 2048: 59 us against
+// 73 us in two launches, each of which reads four rows of activations with every row-block.
 template <bool XF16, int NTW, int MAXM, bool ONE_ROUND, int GPT, bool GROUPED, int KPW = kDecodeKPW, bool PAIR = false>
 __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(const DecodeArgs a_in) {
   static_assert(GPT == 1 || GPT == 2 || GPT == 4, "groups of 128 x 2^k, 64 or 32");
@@ -90,6 +93,8 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
     }
   }
   const DecodeArgs& a = GROUPED ? ag : a_in;
+  // eight tiles of each of two weights: the second weight's are requested as the first one's are consumed
+  constexpr bool LATE = PAIR && KPW == 8;
   constexpr bool G32 = GPT > 1;  // the groups of a tile are kept apart
   static_assert(!G32 || MAXM == 4, "four activation rows times up to four groups fill the 16 rows of the A operand");
   static_assert(KPW == 2 || KPW == 8, "two K tiles per wave and round, or eight in one round");
@@ -163,22 +168,23 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
     // all in flight together.  Buffer loads: the resource, one VGPR offset shared by every load and a
     // wave-uniform 32-bit offset in a scalar register, so the address arithmetic runs on the scalar
     // unit (decode_kernel_applies keeps weights of 4 GiB and more away) ----
-    u4 wreg[NTW][KPW];
-    uint32_t szreg[NTW][KPW];
+    constexpr int SETS = LATE ? 1 : NTW;  // tile registers: LATE, the second weight's tiles take over the first one's as it is consumed
+    u4 wreg[SETS][KPW];
+    uint32_t szreg[SETS][KPW];
     // (several groups per tile: lane column c takes the dword of group GPT kt + c % GPT, 64 bytes per group)
     const int lane16 = lane * 16, r4 = ((c & (GPT - 1)) * 16 + r) * 4;
+    auto request = [&](int i, int t) {
+      const uint32_t nt = (uint32_t)nt0 + (PAIR ? 0 : t);
+      const int woff = (int)((nt * (uint32_t)KT + (uint32_t)(ktw + i)) * (uint32_t)kTileBytes);
+      const uint32_t grp = G32 ? (uint32_t)(ktw + i) * (uint32_t)GPT : (uint32_t)(ktw + i) >> tpg_shift;
+      const int soff = (int)((nt * (uint32_t)KG + grp) * (uint32_t)(kTileN * sizeof(uint32_t)));
+      wreg[t % SETS][i] = __builtin_amdgcn_raw_buffer_load_b128(PAIR && t ? wrs_b : wrs, lane16, woff, 2);  // non-temporal
+      szreg[t % SETS][i] = __builtin_amdgcn_raw_buffer_load_b32(PAIR && t ? srs_b : srs, r4, soff, 0);
+    };
 #pragma unroll
-    for (int i = 0; i < KPW; ++i) {
+    for (int i = 0; i < KPW; ++i)
 #pragma unroll
-      for (int t = 0; t < NTW; ++t) {
-        const uint32_t nt = (uint32_t)nt0 + (PAIR ? 0 : t);
-        const int woff = (int)((nt * (uint32_t)KT + (uint32_t)(ktw + i)) * (uint32_t)kTileBytes);
-        const uint32_t grp = G32 ? (uint32_t)(ktw + i) * (uint32_t)GPT : (uint32_t)(ktw + i) >> tpg_shift;
-        const int soff = (int)((nt * (uint32_t)KG + grp) * (uint32_t)(kTileN * sizeof(uint32_t)));
-        wreg[t][i] = __builtin_amdgcn_raw_buffer_load_b128(PAIR && t ? wrs_b : wrs, lane16, woff, 2);  // non-temporal
-        szreg[t][i] = __builtin_amdgcn_raw_buffer_load_b32(PAIR && t ? srs_b : srs, r4, soff, 0);
-      }
-    }
+      for (int t = 0; t < SETS; ++t) request(i, t);
 
     // Every load of the round stays ahead of the first use: the scheduler would otherwise sink
     // some of them below the first s_waitcnt to save registers, exposing a full memory round
@@ -188,38 +194,57 @@ __global__ __launch_bounds__(1024, KPW == 2 ? 8 : 4) void woq_decode_kernel(cons
     for (int m = 0; m < MAXM; ++m)
 #pragma unroll
       for (int l = 0; l < XL; ++l) *(u4*)(sx + m * SLICE + (xlane + 64 * l) * 8) = xs[m][l];
-
-#pragma unroll
-    for (int i = 0; i < KPW; ++i) {
-      // -sum_k x of this K tile (shared by the NTW weight tiles)
+    uint32_t xfirst = (uint32_t)(xrow * SLICE + c * 32);
+    // -sum_k x of K tile i (shared by the NTW weight tiles, LATE: once for each)
+    auto minus_sum = [&](int i) {
       f4 d1 = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const u4 xa = *(const u4*)(sx + xrow * SLICE + i * kTileK4 + c * 32 + j * 8);
+        const u4 xa = *(const u4*)(sx + xfirst + i * kTileK4 + j * 8);
         d1 = mfma16<XF16>(xa, neg1, d1);
       }
+      return d1;
+    };
+    auto add_tile = [&](int i, int t, f4 d1) {
+      f4 dw = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const u4 xa = *(const u4*)(sx + xfirst + i * kTileK4 + j * 8);
+        const uint32_t d = wreg[t % SETS][i][j];
+        u4 bop;
+        bop[0] = v_and_or(d, mask, magic);
+        bop[1] = v_and_or(d >> 4, mask, magic);
+        bop[2] = v_and_or(d >> 8, mask, magic);
+        bop[3] = v_and_or(d >> 12, mask, magic);
+        dw = mfma16<XF16>(xa, bop, dw);
+      }
+      // dw = sum x (c + q), d1 = -sum x;  group term = s * (dw + (128 + z) * d1 [+ 896 * d1])
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float base = dw[e];
+        if (XF16) base = __builtin_fmaf(d1[e], 896.0f, base);
+        const float tsum = fma_f16hi(d1[e], szreg[t % SETS][i], base);
+        acc[t][e] = fma_f16lo(tsum, szreg[t % SETS][i], acc[t][e]);
+      }
+    };
+    if constexpr (LATE) {
 #pragma unroll
       for (int t = 0; t < NTW; ++t) {
-        f4 dw = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const u4 xa = *(const u4*)(sx + xrow * SLICE + i * kTileK4 + c * 32 + j * 8);
-          const uint32_t d = wreg[t][i][j];
-          u4 bop;
-          bop[0] = v_and_or(d, mask, magic);
-          bop[1] = v_and_or(d >> 4, mask, magic);
-          bop[2] = v_and_or(d >> 8, mask, magic);
-          bop[3] = v_and_or(d >> 12, mask, magic);
-          dw = mfma16<XF16>(xa, bop, dw);
+        for (int i = 0; i < KPW; ++i) {
+          add_tile(i, t, minus_sum(i));
+          asm volatile("" : "+v"(acc[t]));  // (else the scaling sinks into the branch of the lanes that publish it, and sixteen sums wait for it)
+          if (t == 0) request(i, 1);
+          __builtin_amdgcn_sched_barrier(0);  // (the requests stay where they are)
         }
-        // dw = sum x (c + q), d1 = -sum x;  group term = s * (dw + (128 + z) * d1 [+ 896 * d1])
+        asm volatile("" : "+v"(xfirst));  // (no fragment or sum is kept in registers for the second weight)
+      }
+    } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float base = dw[e];
-          if (XF16) base = __builtin_fmaf(d1[e], 896.0f, base);
-          const float tsum = fma_f16hi(d1[e], szreg[t][i], base);
-          acc[t][e] = fma_f16lo(tsum, szreg[t][i], acc[t][e]);
-        }
+      for (int i = 0; i < KPW; ++i) {
+        const f4 d1 = minus_sum(i);
+#pragma unroll
+        for (int t = 0; t < NTW; ++t) add_tile(i, t, d1);
       }
     }
   }
@@ -548,10 +573,10 @@ static int launch_decode_m1_pair(const DecodeArgs& a, hipStream_t st, int slots)
 #undef WOQ_M1_PAIR
   return check_launch("woq_decode_m1_kernel");
 }
-template <bool ONE_ROUND, int GPT, bool GROUPED>
+template <bool ONE_ROUND, int GPT, bool GROUPED, int KPW = kDecodeKPW>
 static int launch_decode_pair_g(const DecodeArgs& a, hipStream_t st, int slots) {
-  const size_t smem = (size_t)2 * a.W * 16 * sizeof(f4) + (size_t)a.W * (4 + (GPT > 1 ? 1 : 0)) * kDecodeKPW * kTileK4 * sizeof(uint16_t);
-  auto kern = woq_decode_kernel<false, 2, 4, ONE_ROUND, GPT, GROUPED, kDecodeKPW, true>;
+  const size_t smem = (size_t)2 * a.W * 16 * sizeof(f4) + (size_t)a.W * (4 + (GPT > 1 ? 1 : 0)) * KPW * kTileK4 * sizeof(uint16_t);
+  auto kern = woq_decode_kernel<false, 2, 4, ONE_ROUND, GPT, GROUPED, KPW, true>;
   if (smem > 64 * 1024) {
     hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (err != hipSuccess) return set_error("hipFuncSetAttribute: %s", hipGetErrorString(err));
@@ -626,7 +651,7 @@ bool decode_kernel_applies(const FpArgs& f, int wbits, int regime, const uint32_
          (f.K % (kDecodeKPW * kTileK4)) == 0 && (f.x_dtype == WOQ_HIP_ACT_BF16 || f.x_dtype == WOQ_HIP_ACT_FP16);
 }
 
-// Two to four rows of a long K run eight K tiles a wave in one round: no pair instance (its registers would not hold both tiles).
+// One to four rows of a long K run eight K tiles a wave in one round.
 static bool eight_tiles(const FpArgs& f, bool one_round) {
   return !one_round && f.KT % 8 == 0 && f.KT / 8 <= 16 && f.G != 32 && f.G != 64;
 }
@@ -639,9 +664,9 @@ static int decode_waves(const FpArgs& f) {
   }
   return (int)w;
 }
-bool decode_pair_applies(const FpArgs& f) {
+bool decode_pair_applies(const FpArgs& f, bool grouped) {
   return f.x_dtype == WOQ_HIP_ACT_BF16 && f.out_dtype == WOQ_HIP_ACT_BF16 &&
-         (f.M == 1 || !eight_tiles(f, f.KT == (int64_t)decode_waves(f) * kDecodeKPW));
+         (f.M == 1 || grouped || !eight_tiles(f, f.KT == (int64_t)decode_waves(f) * kDecodeKPW));
 }
 
 static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t st, const MoeGroup* grp, int slots,
@@ -658,7 +683,7 @@ int launch_decode_grouped(const FpArgs& f, const MoeGroup* grp, int64_t slots, h
 }
 
 static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t st, const MoeGroup* grp, int slots, const uint32_t* sz_b) {
-  if (f.pair && !decode_pair_applies(f)) return set_error("woq_decode_kernel: no pair launch for this problem");
+  if (f.pair && !decode_pair_applies(f, slots > 0)) return set_error("woq_decode_kernel: no pair launch for this problem");
   DecodeArgs a;
   a.grp = grp;
   a.qweight_b = f.qweight_b; a.sz_b = sz_b; a.bias_b = f.bias_b;
@@ -679,11 +704,15 @@ static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t s
   // row-block per workgroup spreads more evenly over the 256 CUs (M = 1: 8192 -> 10240 9.6 us against
   // 11.7 us, 4096 -> 8192 5.2 against 5.4 us, 4096 -> 11008 6.5 against 6.7 us; 4096 -> 14336 the other
   // way round, 7.1 against 7.8 us; M = 4, 4096 -> 11008: 7.4 us with two against 7.7 us).
-  const bool two = f.NT % 2 == 0 && (f.M == 1 ? f.NT > 768 : f.NT >= 512);
+  // Routed slots of two to four rows fill the chip with fewer row-blocks: a workgroup of two reads the rows of activations -- as many
+  // bytes as the weights of one row-block -- half as often (17 slots, 2048 -> 7168: 27 us against 36 us; the bits are the same,
+  // so only where one round of two K tiles a wave is what the expert's own launch runs, too).
+  const bool one_round = f.KT == (int64_t)decode_waves(f) * kDecodeKPW;
+  const bool many_slots = slots > 0 && f.M > 1 && !eight_tiles(f, one_round) && f.NT / 2 * slots >= 2048;
+  const bool two = f.NT % 2 == 0 && (f.M == 1 ? f.NT > 768 : f.NT >= 512 || many_slots);
   a.wbytes = (uint32_t)(f.NT * f.KT * kTileBytes);  // below 4 GiB (decode_kernel_applies)
   a.szbytes = (uint32_t)(f.NT * f.KG * kTileN * (int64_t)sizeof(uint32_t));
   const bool one_row = f.M == 1;
-  const bool one_round = f.KT == (int64_t)a.W * kDecodeKPW;
   if (one_row && eight_tiles(f, one_round)) {
     // A long K in one round: eight K tiles per wave (8 KiB in flight per wave, a budget of 128 registers) instead of
     // several rounds of two, each of which waits for its own requests (M = 1, 14336 -> 4096: 7.48 against 7.71 us,
@@ -712,8 +741,13 @@ static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t s
     return two ? WOQ_DECODE_M1(true, 2) : WOQ_DECODE_M1(true, 1);
 #undef WOQ_DECODE_M1
   }
+  const bool eight = eight_tiles(f, one_round);
+  if (f.pair && eight) {
+    a.W = (int)(f.KT / 8);
+    return launch_decode_pair_g<true, 1, true, 8>(a, st, slots);
+  }
   if (f.pair) return one_round ? launch_decode_pair<true>(a, st, slots) : launch_decode_pair<false>(a, st, slots);
-  if (eight_tiles(f, one_round) && !two) {
+  if (eight && !two) {
     // a long K in one round of eight K tiles per wave, as for one row above (M = 4, 14336 -> 4096: 8.9 against 9.2 us)
     a.W = (int)(f.KT / 8);
     if (slots > 0)

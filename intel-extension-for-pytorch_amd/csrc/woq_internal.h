@@ -143,7 +143,7 @@ struct DecodeArgs {
 bool decode_kernel_applies(const FpArgs& f, int wbits, int regime, const uint32_t* sz);
 int launch_decode(const FpArgs& f, const uint32_t* sz, hipStream_t st, const uint32_t* sz_b = nullptr);
 // whether launch_decode / launch_decode_grouped take the pair (f.pair) of a problem that decode_kernel_applies to
-bool decode_pair_applies(const FpArgs& f);
+bool decode_pair_applies(const FpArgs& f, bool grouped);
 // One routed row per slot, the experts' (scale, zero) dword tables in grp->scales.
 int launch_decode_grouped(const FpArgs& f, const MoeGroup* grp, int64_t slots, hipStream_t st);
 

@@ -1477,3 +1477,26 @@ def test_moe_route_tiles_against_sorted_lists(cuda, T, topk, E, rows):
         mine = sorted((j for j in range(topk) if t * topk + j in place), key=lambda j: (flat[t * topk + j], j))
         assert ro[t][:len(mine)] == [place[t * topk + j] for j in mine] and so[t][:len(mine)] == mine
         assert all(r == -1 for r in ro[t][len(mine):])
+
+
+@pytest.mark.parametrize("H,I", [(7168, 256), (4352, 512), (16384, 256), (256, 8192)])
+def test_deepseek_moe_of_two_to_four_rows_an_expert_with_long_k(cuda, monkeypatch, H, I):
+    """Gate and up of slots of two to four rows with eight K tiles a wave in one launch, and two row-blocks a workgroup where many slots
+    share the launch: bit for bit the experts' own launches."""
+    from ipex_amd import _lib
+
+    ipex = _ipex()
+    E, T, topk = 24, 24, 3
+    mk = lambda k, n, s: _woq_module(ipex, k, n, "INT4", 128, "BF16", bias=True, seed=s)._op_context
+    ctxs = [[mk(H, I, 600 + e % 3) for e in range(E)], [mk(H, I, 610 + e % 3) for e in range(E)], [mk(I, H, 620 + e % 3) for e in range(E)]]
+    g = torch.Generator().manual_seed(H)
+    hidden = torch.randn(T, H, generator=g).bfloat16().to(cuda)
+    ids = torch.stack([(t * 3 + torch.arange(3)) % (E - 4) for t in range(T)]).to(cuda)  # three or four rows each
+    rw = torch.softmax(torch.randn(T, topk, generator=g), -1).bfloat16().to(cuda)
+    op = torch.ops.torch_ipex.deepseek_moe_woq
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
+    want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
+    got = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    assert _lib.last_kernel() == "moe_combine_rows"
+    assert torch.equal(got, want)
