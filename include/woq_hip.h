@@ -384,6 +384,9 @@ int woq_hip_moe_scale_add_rows(void* out, int dtype, int64_t T, int64_t H, const
  *   expert id (-1: unused entry), first sorted position, number of rows (at most 64).  Classes: 0 fewer than split_lo
  *   rows, 1 at most split_mid, 2 more, 3 (use_single = 1) exactly one row, taken out of class 0.  use_single = 2:
  *   every sorted position is a slot of one row in class 3, at its own index (S >= T * topk; for a single token).
+ *   use_single | WOQ_HIP_MOE_CUT (0 or 1 with it, at most WOQ_HIP_MOE_TILES_EXPERTS experts): no class 2, experts with more than
+ *   split_mid rows stand in class 1 with as many slots of split_mid rows as they need (S larger by T * topk / split_mid); none of
+ *   their entries is left out.
  *   row_of[t, i] / slot_of[t, i] = sorted position and top-k slot of token t's i-th contribution in ascending expert
  *   order (row_of -1: none).  An expert id outside [0, experts) contributes nothing, and neither do an expert's entries
  *   beyond its first 64 (a slot holds at most 64 rows).
@@ -407,6 +410,7 @@ int woq_hip_moe_scale_add_rows(void* out, int dtype, int64_t T, int64_t H, const
 #define WOQ_HIP_MOE_ROUTE_MAX 2048
 #define WOQ_HIP_MOE_TILES_MAX 8192
 #define WOQ_HIP_MOE_TILES_EXPERTS 1024
+#define WOQ_HIP_MOE_CUT 4
 typedef struct woq_hip_moe_group {
   const int32_t* slot_expert;      /* [slots] expert of the slot or -1 */
   const int32_t* slot_row0;        /* [slots] */

@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const int64_t* __restric
 //   slots   [4 classes][expert, first row, rows][S].  TILES: 0: experts with fewer than split_lo rows, 1: at most split_mid, 2: at most
 //           64, one slot each; 3: the others in slots of at most tile_rows rows (160: the expert's rows evenly, in whole row tiles
 //           of 16), an expert's slots one after the other, rows | the expert's rows << 16 in place of rows; else the classes of
-//           moe_route_kernel.  Unused entries: expert -1.
+//           moe_route_kernel (WOQ_HIP_MOE_CUT: no class 2, the rows of its experts in class 1 in slots of split_mid).  Unused entries: expert -1.
 //   x_row, row_of, slot_of as above.
 constexpr int kMoeTilesMax = WOQ_HIP_MOE_TILES_MAX;
 constexpr int kMoeTilesExperts = WOQ_HIP_MOE_TILES_EXPERTS;
@@ -271,9 +271,10 @@ __global__ __launch_bounds__(64 * W) void moe_route_sort_kernel(const int64_t* _
       step = cls != 3 ? kMoeSlotRowsMax : tile_rows == 160 ? ((n + count - 1) / count + 15) & ~15 : tile_rows;
       add = n == 0 ? 0 : cls != 3 ? 1 : count;
     } else {
-      cls = single && n == 1 ? 3 : n < split_lo ? 0 : n <= split_mid ? 1 : 2;
-      step = kMoeSlotRowsMax;
-      add = n > 0;
+      const bool cut = single & WOQ_HIP_MOE_CUT;
+      cls = (single & 1) && n == 1 ? 3 : n < split_lo ? 0 : cut || n <= split_mid ? 1 : 2;
+      step = cut ? split_mid : kMoeSlotRowsMax;
+      add = cut ? (n + step - 1) / step : n > 0;
     }
     int v[5] = {n, cls == 0 ? add : 0, cls == 1 ? add : 0, cls == 2 ? add : 0, cls == 3 ? add : 0}, own[5];
 #pragma unroll
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(64 * W) void moe_route_sort_kernel(const int64_t* _
       int idx = cls == 0 ? v[1] : cls == 1 ? v[2] : cls == 2 ? v[3] : v[4];
       int32_t* const tab = slots + cls * 3 * S;
       for (int row = 0; row < n; row += step, ++idx) {
-        if (idx >= S || (!TILES && row > 0)) break;  // (the host gives S entries for every case)
+        if (idx >= S || (!TILES && !(single & WOQ_HIP_MOE_CUT) && row > 0)) break;  // (the host gives S entries for every case)
         tab[idx] = e;
         tab[S + idx] = v[0] + row;
         tab[2 * S + idx] = (n - row < step ? n - row : step) | (TILES && cls == 3 ? n << 16 : 0);
@@ -328,8 +329,8 @@ __global__ __launch_bounds__(64 * W) void moe_route_sort_kernel(const int64_t* _
       place[g] += hist[wave][e];
       p = off[e] + place[g];
       x_row[p] = t;
-      // !TILES: a slot holds at most 64 rows (an expert gets more only if a token names it twice): the rest contribute nothing
-      if (!TILES && place[g] >= kMoeSlotRowsMax) p = -1;
+      // one slot an expert holds at most 64 rows (it gets more only if a token names it twice): the rest contribute nothing
+      if (!TILES && !(single & WOQ_HIP_MOE_CUT) && place[g] >= kMoeSlotRowsMax) p = -1;
     }
     row_of[t * topk + ord] = p;
     slot_of[t * topk + ord] = p >= 0 || TILES ? j : 0;
@@ -441,7 +442,7 @@ int launch_moe_route(const int64_t* ids, int64_t T, int64_t topk, int64_t expert
   const int64_t R = T * topk;
   if (R == 0) return 0;
   if (R > kMoeRouteMax) return set_error("moe_route: at most %d (token, slot) entries, got %lld", kMoeRouteMax, (long long)R);
-  if (use_single != 2 && experts <= kMoeTilesExperts)
+  if (use_single != 2 && (experts <= kMoeTilesExperts || (use_single & WOQ_HIP_MOE_CUT)))
     moe_route_sort_kernel<4, false><<<1, 256, 0, st>>>(ids, (int)R, (int)topk, (int)experts, (int)split_lo, (int)split_mid, 0, use_single, (int)S,
                                                        x_row, slots, row_of, slot_of);
   else

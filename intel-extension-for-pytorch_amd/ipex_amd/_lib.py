@@ -21,6 +21,7 @@ ACT_FP32, ACT_FP16, ACT_BF16 = 0, 1, 2
 FUSE_NONE, FUSE_GELU_ERF, FUSE_GELU_TANH, FUSE_RELU, FUSE_SILU = 0x0, 0x1, 0x2, 0x3, 0x4
 FUSE_ADD, FUSE_ADD_ADD, FUSE_MUL = 0x10, 0x20, 0x30
 MOE_PAIR, MOE_SZB = 1, 2
+MOE_CUT = 4  # woq_hip_moe_route: use_single flag WOQ_HIP_MOE_CUT
 TILE_N, TILE_BYTES, TILE_K_INT4, TILE_K_INT8 = 16, 1024, 128, 64
 
 EXPORTS = [

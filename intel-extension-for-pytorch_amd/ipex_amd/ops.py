@@ -743,7 +743,8 @@ class _MoeGroupedPlan:
         self.x_row = torch.empty(R, dtype=torch.int64, device=device)
         # slot tables [class][expert, first row, rows][S]: experts with few / up to 16 / up to 64 rows / exactly one row
         self.S = len(gate_ctx)
-        self.slots = torch.empty((4, 3, self.S), dtype=torch.int32, device=device)
+        # (and slots for the rows of experts that are cut into several)
+        self.slots = torch.empty((4, 3, self.S + R // 16), dtype=torch.int32, device=device)
         self.row_of, self.slot_of = i32(), i32()
         self.tables = []
         for rows in infos:
@@ -909,6 +910,11 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
             return None
         if not f16 and x.dtype == torch.float16:
             return None
+    # up to 16 tokens an expert has more than 16 rows only where a token names it twice: its rows are cut into slots of 16, which spares
+    # the launches for more (4.7 us each, though nearly always empty)
+    cut = T <= 16 < most and plan.S <= _lib.MOE_TILES_EXPERTS
+    if cut:
+        launches = [c for c in launches if c[0] != 2]
     lib = _lib.load()
     ids = topk_ids.to(torch.int64).contiguous()
     rw = routing_weights.contiguous()
@@ -919,10 +925,12 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     with _moe_launch_lock(x.device.index, raw_stream), torch.cuda.device(x.device):
         act, inter, y = plan.buffers(x.dtype, raw_stream)  # calls on one stream follow each other
         stream = _kernels._stream()
-        _lib.check(lib.woq_hip_moe_route(ids.data_ptr(), T, topk, len(gate_ctx), split, 16, 2 if each else int(single), plan.S,
+        _lib.check(lib.woq_hip_moe_route(ids.data_ptr(), T, topk, len(gate_ctx), split, 16, 2 if each else int(single) + (_lib.MOE_CUT if cut else 0),
+                                         plan.slots.shape[2],
                                          plan.x_row.data_ptr(), plan.slots.data_ptr(), plan.row_of.data_ptr(),
                                          plan.slot_of.data_ptr(), stream), "moe_route")
         nslots = R if each else min(R, plan.S)  # experts that can have tokens: the tables are dense
+        slots_of = lambda cls: nslots + R // 16 if cut and cls == 1 else nslots
         p = _lib.LinearParams()
         p.struct_size = ctypes.sizeof(_lib.LinearParams)
         p.x_dtype = p.out_dtype = code
@@ -930,9 +938,9 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
         p.lowp_mode = lowp
         p.act_quant_mode = -1
         for cls, bound in launches:
-            plan.gate_up(lib, p, x, act, inter, cls, bound, nslots, [cls == 3 or (cls == 0 and single)] * 3, False)
+            plan.gate_up(lib, p, x, act, inter, cls, bound, slots_of(cls), [cls == 3 or (cls == 0 and single)] * 3, False)
         for cls, bound in launches:
-            plan.launch(lib, p, 2, inter, y, cls, bound, nslots, x.dtype, [cls == 3 or (cls == 0 and single)] * 3, False)
+            plan.launch(lib, p, 2, inter, y, cls, bound, slots_of(cls), x.dtype, [cls == 3 or (cls == 0 and single)] * 3, False)
         _lib.check(lib.woq_hip_moe_combine_rows(out.data_ptr(), code, T, H, y.data_ptr(), rw.data_ptr(), topk,
                                                 plan.row_of.data_ptr(), plan.slot_of.data_ptr(), 0, stream), "moe_combine_rows")
     return out

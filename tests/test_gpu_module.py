@@ -1479,6 +1479,44 @@ def test_moe_route_tiles_against_sorted_lists(cuda, T, topk, E, rows):
         assert all(r == -1 for r in ro[t][len(mine):])
 
 
+@pytest.mark.parametrize("T,topk", [(16, 4), (9, 8), (16, 2)])
+def test_deepseek_moe_of_few_tokens_that_name_an_expert_often(cuda, monkeypatch, T, topk):
+    """Up to 16 tokens: an expert with more than 16 rows (tokens name it twice and more) is cut into slots of 16 rows.  The per-expert path runs
+    the k-th mentions of all tokens in one go: the same rows in other batches, so other fp32 sums and bf16 (2^-9) flips of
+    single values, each well below 4e-3 in the 2-norm."""
+    from ipex_amd import _lib
+
+    ipex = _ipex()
+    E, H, I = 5, 512, 256
+    mk = lambda k, n, s: _woq_module(ipex, k, n, "INT4", 128, "BF16", bias=True, seed=s)._op_context
+    ctxs = [[mk(H, I, 600 + e) for e in range(E)], [mk(H, I, 610 + e) for e in range(E)], [mk(I, H, 620 + e) for e in range(E)]]
+    g = torch.Generator().manual_seed(T)
+    hidden = torch.randn(T, H, generator=g).bfloat16().to(cuda)
+    ids = torch.full((T, topk), 3)
+    ids[0, 0], ids[T - 1, topk - 1] = 1, 4
+    ids = ids.to(cuda)
+    rw = torch.softmax(torch.randn(T, topk, generator=g), -1).bfloat16().to(cuda)
+    op = torch.ops.torch_ipex.deepseek_moe_woq
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
+    want = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False).double()
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
+    got = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
+    assert _lib.last_kernel() == "moe_combine_rows"
+    assert float((got.double() - want).norm() / want.norm()) < 4e-3
+    R, S = T * topk, E + T * topk // 16
+    i32 = lambda *n: torch.full(n, -7, dtype=torch.int32, device=cuda)
+    x_row, slots, row_of, slot_of = torch.empty(R, dtype=torch.int64, device=cuda), i32(4, 3, S), i32(R), i32(R)
+    lib = _lib.load()
+    tables = (x_row.data_ptr(), slots.data_ptr(), row_of.data_ptr(), slot_of.data_ptr(), None)
+    assert lib.woq_hip_moe_route(ids.data_ptr(), T, topk, E, 5, 16, 1 + _lib.MOE_CUT, S - R // 16 - 1, *tables) != 0
+    assert lib.woq_hip_moe_route(ids.data_ptr(), T, topk, E, 5, 16, 1 + _lib.MOE_CUT, S, *tables) == 0
+    n = R - 2
+    got = slots.cpu()
+    assert [tuple(got[1, :, k].tolist()) for k in range(-(-n // 16))] == [(3, 1 + r, min(16, n - r)) for r in range(0, n, 16)]
+    assert got[1, 0, -(-n // 16):].eq(-1).all() and got[2, 0].eq(-1).all() and got[3, 0].tolist()[:3] == [1, 4, -1]
+    assert sorted(row_of.cpu().tolist()) == list(range(R))
+
+
 @pytest.mark.parametrize("H,I", [(7168, 256), (4352, 512), (16384, 256), (256, 8192)])
 def test_deepseek_moe_of_two_to_four_rows_an_expert_with_long_k(cuda, monkeypatch, H, I):
     """Gate and up of slots of two to four rows with eight K tiles a wave in one launch, and two row-blocks a workgroup where many slots
