@@ -7,8 +7,8 @@
 //
 // The two-kernel form (one workgroup per quantization group for the statistics, then one thread per
 // 8 elements) reads the activations twice and, for per-(row, K block) scales, starts one workgroup
-// per 128 elements.  Here a wave owns a row: it loads the row once (16 bytes per lane and 512-element
-// chunk, kept as the raw 16-bit values), reduces min / max over the wave (or over the lanes of a K
+// per 128 elements.  Here a workgroup owns a row: it loads the row once (16 bytes per lane and 512-element
+// chunk, kept as the raw 16-bit values), reduces min / max over its waves (or over the lanes of a K
 // block), and quantizes from the registers.  Same arithmetic, expression by expression, as the
 // two-kernel form, so the bytes and the scales are identical.
 #include "woq_common.h"
@@ -37,17 +37,17 @@ struct AqArgs {
   int given;  // the scales (and zero points) are inputs, shared by all rows: one per tensor or per K block
 };
 
-// NCH: 512-element chunks of a (padded) row that one wave holds.  SPLIT: the four waves of a
-// workgroup share one row (wave w takes chunks w, w + 4, ...), for the few rows of a decode step,
-// where a single wave per row would be one long dependent chain (M = 1, K = 4096: 6.5 us).
-template <int NCH, bool SPLIT>
+// NCH: 512-element chunks of a (padded) row that one wave holds; the four waves of a workgroup share one row (wave w takes chunks w,
+// w + 4, ...).  A wave with a whole row is one long dependent chain -- loads, extremes, an IEEE division for every element -- that
+// few other waves of its SIMD hide at any number of rows (M = 1, K = 4096: 6.5 us; M = 180, K = 7040, a scale per K block: 17.6 us, now 6.8; M = 2048, K = 4096:
+// 14.7, now 12.6).
+template <int NCH>
 __global__ __launch_bounds__(256) void act_quant_rows_kernel(const AqArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int64_t m = SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
-  if (m >= a.M) return;
+  const int64_t m = (int64_t)blockIdx.x;
   // chunk held in register slot c
-  auto chunk_of = [&](int c) { return SPLIT ? wave + 4 * c : c; };
+  auto chunk_of = [&](int c) { return wave + 4 * c; };
   const uint16_t* const row = a.x + m * a.K;
   const bool bf16 = a.bf16 != 0, sym = a.sym != 0, per_k = a.block_lanes_log2 >= 0;
 
@@ -88,19 +88,17 @@ __global__ __launch_bounds__(256) void act_quant_rows_kernel(const AqArgs a) {
       mn[0] = fminf(mn[0], __shfl_xor(mn[0], off));
       mx[0] = fmaxf(mx[0], __shfl_xor(mx[0], off));
     }
-    if constexpr (SPLIT) {
-      // the four waves' extremes meet in LDS (every wave of the workgroup is here: same row)
-      __shared__ float smn[4], smx[4];
-      if (lane == 0) {
-        smn[wave] = mn[0];
-        smx[wave] = mx[0];
-      }
-      __syncthreads();
+    // the four waves' extremes meet in LDS (every wave of the workgroup is here: same row)
+    __shared__ float smn[4], smx[4];
+    if (lane == 0) {
+      smn[wave] = mn[0];
+      smx[wave] = mx[0];
+    }
+    __syncthreads();
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        mn[0] = fminf(mn[0], smn[w]);
-        mx[0] = fmaxf(mx[0], smx[w]);
-      }
+    for (int w = 0; w < 4; ++w) {
+      mn[0] = fminf(mn[0], smn[w]);
+      mx[0] = fmaxf(mx[0], smx[w]);
     }
   } else {
     // the lanes of one K block are 2^block_lanes_log2 consecutive lanes, aligned
@@ -119,7 +117,7 @@ __global__ __launch_bounds__(256) void act_quant_rows_kernel(const AqArgs a) {
   } else if (!per_k) {
     int32_t z = 0;
     row_p = aq_params(mn[0], mx[0], sym, &z);
-    if (lane == 0 && (!SPLIT || wave == 0)) {
+    if (lane == 0 && wave == 0) {
       a.scales[m] = row_p.s;
       if (!sym) a.zps[m] = z;
     }
@@ -281,31 +279,16 @@ __global__ void aq_shared_finalize_kernel(int groups, int sym, float* scales, in
   if (!sym) zps[i] = z;
 }
 
-template <int NCH, bool SPLIT>
-void aq_launch_rows(const AqArgs& a, unsigned grid, hipStream_t st) {
-  act_quant_rows_kernel<NCH, SPLIT><<<grid, 256, 0, st>>>(a);
-}
-
 // the quantization pass over whole rows, for scales computed here or given
 void aq_launch_quant(const AqArgs& a, hipStream_t st) {
   const int64_t chunks = (a.ldq + 511) / 512;
-  if (a.M <= 64) {
-    // few rows: a workgroup per row, a quarter of the chunks per wave
-    if (chunks <= 8)
-      aq_launch_rows<2, true>(a, (unsigned)a.M, st);
-    else if (chunks <= 16)
-      aq_launch_rows<4, true>(a, (unsigned)a.M, st);
-    else
-      aq_launch_rows<8, true>(a, (unsigned)a.M, st);
-    return;
-  }
-  const unsigned grid = (unsigned)((a.M + 3) / 4);
+  const unsigned grid = (unsigned)a.M;
   if (chunks <= 8)
-    aq_launch_rows<8, false>(a, grid, st);
+    act_quant_rows_kernel<2><<<grid, 256, 0, st>>>(a);
   else if (chunks <= 16)
-    aq_launch_rows<16, false>(a, grid, st);
+    act_quant_rows_kernel<4><<<grid, 256, 0, st>>>(a);
   else
-    aq_launch_rows<32, false>(a, grid, st);
+    act_quant_rows_kernel<8><<<grid, 256, 0, st>>>(a);
 }
 
 }  // namespace
