@@ -288,6 +288,13 @@ int64_t woq_hip_linear_split_k_workspace_bytes(int64_t M, int64_t N);
  * rule to keep in step.  No counterpart in the reference. */
 int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t lowp_mode);
 
+/* The scratch of one call, M of p included: woq_hip_linear_auto_split_k_workspace_bytes where that is not 0, else what the plan of a
+ * prompt of more than 64 rows takes at any K -- a K below 4096 in the floating-point modes, any number of tiles under lowp_mode INT8 --, 0 where K is
+ * not shared.  (A linear of a routed layer's expert asks the older function: woq_hip_linear_grouped_tiles has the bits of those
+ * launches.)  woq_hip_linear_pair_scratch_bytes: of a woq_hip_linear_pair call, given in the workspace and counters of `gate`.  No counterpart in the reference. */
+int64_t woq_hip_linear_scratch_bytes(const woq_hip_linear_params* p);
+int64_t woq_hip_linear_pair_scratch_bytes(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);
+
 /* K-block of the int8 path: min(group_size, 128), per-channel -> 128
  * (get_block_k, csrc/cpu/aten/Linear.cpp:362-376). */
 int64_t woq_hip_int8_block_k(int64_t group_size, int64_t K);
@@ -298,7 +305,8 @@ int woq_hip_linear(const woq_hip_linear_params* p);
  * silu and then on `up` with the mul round it (Linear2SiluMul).  The K sums may be added in another order with 17 to 32 rows, with 5
  * to 16 rows where woq_hip_linear shares K (woq_hip_linear_auto_split_k_workspace_bytes), and with 33 to 64 rows and more than
  * 16384 columns, where it takes the prefill kernel.  Both parameter sets name the same x, out, sizes, modes and stream, no post-op.  For the problems of woq_hip_linear_pair_applies: INT4 and INT8 weights with their scale_zero_bf16
- * tables (and scale_zero_f16x2 for rows that compute in fp16), bf16 rows, lowp_mode BF16 or NONE, at most 64 rows. */
+ * tables (and scale_zero_f16x2 for rows that compute in fp16), bf16 rows, lowp_mode BF16 or NONE; beyond 64 rows INT4 weights without a dense copy, K of at least
+ * 1024 and a multiple of 128, at least 512 columns, where the estimated time is the lower one (K may be shared otherwise than in two launches). */
 int woq_hip_linear_pair_applies(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);
 int woq_hip_linear_pair(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);
 
@@ -310,8 +318,8 @@ int woq_hip_linear_pair(const woq_hip_linear_params* gate, const woq_hip_linear_
  * runs on (WOQ_HIP_NOALLOC_MAX_WORKSPACE_BYTES plus 2 KiB of counters, until the process ends).  A call
  * whose workspace need (woq_hip_linear_workspace_bytes) exceeds that maximum is rejected with an error
  * before anything is launched.  K is shared between workgroups by the best plan whose scratch fits beside it: where
- * woq_hip_linear with the scratch of woq_hip_linear_auto_split_k_workspace_bytes takes a larger one, the fp32 sums are
- * added in another order.
+ * woq_hip_linear with the scratch of woq_hip_linear_scratch_bytes takes a larger one, the fp32 sums are added in
+ * another order.
  * Allocates nothing, on the device or through any library.  All calls on one GPU share the array: calls
  * that may overlap in time on one GPU (different streams, concurrent graph launches) race and must be
  * serialised by the caller.  The first call on a device that needs the array looks up its address, which cannot

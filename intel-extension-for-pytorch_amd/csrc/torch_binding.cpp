@@ -296,7 +296,9 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
   }
 
   // ---- execution ----
-  Tensor run(const Tensor& x_in, int64_t fusion, const std::vector<Tensor>& others) {
+  // expert: a linear of a routed layer's expert, whose K is shared between workgroups on the problems only that the layer's own launches
+  // run in as many chains (woq_hip_linear_auto_split_k_workspace_bytes)
+  Tensor run(const Tensor& x_in, int64_t fusion, const std::vector<Tensor>& others, bool expert = false) {
     TORCH_CHECK(x_in.size(-1) == K_, "WOQ linear: input and weight shapes do not match, got k = ", x_in.size(-1),
                 " and ", K_, " respectively.");
     const int64_t M = x_in.numel() > 0 ? x_in.numel() / K_ : 0;
@@ -305,14 +307,14 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
     if (M == 0) return at::empty(out_sizes, x_in.options());
     Tensor x = x_in;
     if (g_src_.defined()) x = shuffle_activations(x, g_src_);
-    return run_sorted(x, M, fusion, others, out_sizes);
+    return run_sorted(x, M, fusion, others, out_sizes, expert);
   }
 
   // silu(gate(x)) * up(x), in one launch where the library has one (woq_hip_linear_pair), else in the two that the ops
   // woq_linear_silu and woq_linear_mul make
   static Tensor run_pair(WoqLinearOpContext& gate, WoqLinearOpContext& up, const Tensor& x_in) {
     const int64_t M = x_in.numel() > 0 && x_in.size(-1) == gate.K_ ? x_in.numel() / gate.K_ : 0;
-    if (M >= 1 && M <= 64 && gate.K_ == up.K_ && gate.N_ == up.N_ && !gate.g_src_.defined() && !up.g_src_.defined() &&
+    if (M >= 1 && gate.K_ == up.K_ && gate.N_ == up.N_ && !gate.g_src_.defined() && !up.g_src_.defined() &&
         gate.packed_.device() == x_in.device() && up.packed_.device() == x_in.device() && x_in.scalar_type() == at::kBFloat16) {
       Tensor x2 = x_in.is_contiguous() ? x_in : x_in.contiguous();
       if ((uintptr_t)x2.data_ptr() % 16) x2 = x2.clone();  // the kernels read activation rows with 16-byte loads
@@ -322,13 +324,26 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
       gate.fill_params(p[0], x2, M);
       up.fill_params(p[1], x2, M);
       DeviceScope scope(x2);
-      Tensor out = at::empty(out_sizes, x_in.options());
+      Tensor out;
       for (auto& q : p) {
-        q.out = out.data_ptr();
+        q.out = x2.data_ptr();  // (any address: what applies does not depend on it)
         q.out_dtype = act_code(x2.scalar_type());
         q.stream = current_stream(x2);
       }
       if (woq_hip_linear_pair_applies(&p[0], &p[1])) {
+        out = at::empty(out_sizes, x_in.options());
+        p[0].out = p[1].out = out.data_ptr();
+        Tensor ws;
+        optional<Tensor> counters;
+        if (const int64_t bytes = woq_hip_linear_pair_scratch_bytes(&p[0], &p[1])) {  // with which workgroups share K
+          counters = split_k_counters(x2);
+          if (counters.has_value()) {
+            ws = at::empty({bytes}, x_in.options().dtype(at::kByte));
+            p[0].workspace = ws.data_ptr();
+            p[0].workspace_bytes = bytes;
+            p[0].split_k_counters = counters->data_ptr<int32_t>();
+          }
+        }
         check_rc(woq_hip_linear_pair(&p[0], &p[1]), "woq_linear_silu_mul");
         return out;
       }
@@ -471,7 +486,7 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
 
   // `run` behind the act-order shuffle: the input channels of x are in the order of the stored weight
   Tensor run_sorted(const Tensor& x, int64_t M, int64_t fusion, const std::vector<Tensor>& others,
-                    const std::vector<int64_t>& out_sizes) {
+                    const std::vector<int64_t>& out_sizes, bool expert) {
     Tensor x2 = x.is_contiguous() ? x : x.contiguous();
     if ((uintptr_t)x2.data_ptr() % 16) x2 = x2.clone();  // the kernels read activation rows with 16-byte loads
     Tensor out = at::empty(out_sizes, x.options());
@@ -505,9 +520,10 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
     const bool int8 = lowp_mode_ == WOQ_HIP_LOWP_INT8;
     int64_t wbytes = int8 ? woq_hip_linear_workspace_bytes(M, K_, WOQ_HIP_LOWP_INT8, (int32_t)act_quant_mode_, group_size_) : 0;
     optional<Tensor> counters;
-    // long K and few output tiles: scratch with which the kernels share K between workgroups, and the zeroed
+    // few output tiles: scratch with which the kernels share K between workgroups, and the zeroed
     // counters of this stream (the library says for which problems it would use them)
-    if (const int64_t extra = woq_hip_linear_auto_split_k_workspace_bytes(M, K_, N_, (int32_t)lowp_mode_)) {
+    if (const int64_t extra = expert ? woq_hip_linear_auto_split_k_workspace_bytes(M, K_, N_, (int32_t)lowp_mode_)
+                                     : woq_hip_linear_scratch_bytes(&p)) {
       counters = split_k_counters(x2);
       if (counters.has_value()) wbytes = (wbytes + 255) / 256 * 256 + extra;
     }
@@ -748,6 +764,15 @@ static Tensor woq_linear_binary(const Tensor& input, const Tensor& W_prepack, co
   return context_from_handle(W_prepack, "torch_ipex::woq_linear_<post-op>")->run(input, FUSION, o);
 }
 
+// woq_linear_silu, woq_linear_mul or ipex_woq_linear as a routed layer's expert runs it (WoqLinearOpContext::run)
+static Tensor woq_linear_expert(const Tensor& input, const Tensor& W_prepack, int64_t fusion, const std::vector<Tensor>& others) {
+  const char* op = "torch_ipex::woq_linear_expert";
+  require_gpu_input(input, op);
+  TORCH_CHECK(fusion == WOQ_HIP_FUSE_NONE || fusion == WOQ_HIP_FUSE_SILU || (fusion == WOQ_HIP_FUSE_MUL && others.size() == 1), op,
+              ": unexpected post-op ", fusion);
+  return context_from_handle(W_prepack, op)->run(input, fusion, others, true);
+}
+
 static Tensor woq_linear_silu_mul(const Tensor& input, const Tensor& W_gate, const Tensor& W_up) {
   const char* op = "torch_ipex::woq_linear_silu_mul";
   require_gpu_input(input, op);
@@ -776,8 +801,8 @@ static Tensor moe_expert(const Tensor& hidden, const Tensor& top_x_in, const Ten
   DeviceScope scope(x);
   check_rc(woq_hip_moe_gather_rows(x.data_ptr(), act_code(x.scalar_type()), T, H, top_x.data_ptr<int64_t>(), n,
                                    cur.data_ptr(), current_stream(x)), op);
-  const Tensor act = gate.run(cur, WOQ_HIP_FUSE_SILU, {});
-  const Tensor out = down.run(up.run(cur, WOQ_HIP_FUSE_MUL, {act}), WOQ_HIP_FUSE_NONE, {}).contiguous();
+  const Tensor act = gate.run(cur, WOQ_HIP_FUSE_SILU, {}, true);
+  const Tensor out = down.run(up.run(cur, WOQ_HIP_FUSE_MUL, {act}, true), WOQ_HIP_FUSE_NONE, {}, true).contiguous();
   TORCH_CHECK(out.dim() == 2 && out.size(0) == n && out.size(1) == H, op, ": the down projection must return to the hidden width");
   check_rc(woq_hip_moe_scale_add_rows(output.data_ptr(), act_code(output.scalar_type()), T, H, out.data_ptr(), rw.data_ptr(),
                                       rw.size(1), top_x.data_ptr<int64_t>(), idx.data_ptr<int64_t>(), n, current_stream(x)),
@@ -1063,6 +1088,7 @@ TORCH_LIBRARY_FRAGMENT(torch_ipex, m) {
   m.def("woq_linear_silu(Tensor input, Tensor W_prepack) -> Tensor");
   // silu(gate(x)) * up(x) of a gated MLP (Linear2SiluMul); no counterpart among the reference's operators, which calls the two above
   m.def("woq_linear_silu_mul(Tensor input, Tensor W_gate, Tensor W_up) -> Tensor");
+  m.def("woq_linear_expert(Tensor input, Tensor W_prepack, int fusion, Tensor[] others) -> Tensor");
   m.def("woq_linear_add(Tensor input, Tensor W_prepack, Tensor[] others) -> Tensor");
   m.def("woq_linear_add_add(Tensor input, Tensor W_prepack, Tensor[] others) -> Tensor");
   m.def("woq_linear_mul(Tensor input, Tensor W_prepack, Tensor[] others) -> Tensor");
@@ -1094,6 +1120,7 @@ TORCH_LIBRARY_IMPL(torch_ipex, CUDA, m) {
   m.impl("woq_linear_add_add", TORCH_FN((woq_linear_binary<WOQ_HIP_FUSE_ADD_ADD, 2>)));
   m.impl("woq_linear_mul", TORCH_FN((woq_linear_binary<WOQ_HIP_FUSE_MUL, 1>)));
   m.impl("woq_linear_silu_mul", TORCH_FN(woq_linear_silu_mul));
+  m.impl("woq_linear_expert", TORCH_FN(woq_linear_expert));
   m.impl("woq_linear", TORCH_FN(woq_linear_v2));
   m.impl("dequantize_nf4", TORCH_FN(dequantize_nf4));
   m.impl("deepseek_moe_woq", TORCH_FN(deepseek_moe_woq));

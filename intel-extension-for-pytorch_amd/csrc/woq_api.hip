@@ -198,6 +198,17 @@ int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_
   return decode || prefill ? woq_hip_linear_split_k_workspace_bytes(M, N) : 0;
 }
 
+int64_t woq_hip_linear_scratch_bytes(const woq_hip_linear_params* p) {
+  if (!p || p->struct_size != sizeof(*p) || !valid_wdtype(p->weight_dtype) || p->M <= 0 || p->K <= 0 || p->N <= 0) return 0;
+  if (const int64_t bytes = woq_hip_linear_auto_split_k_workspace_bytes(p->M, p->K, p->N, p->lowp_mode)) return bytes;
+  if (p->M <= 64) return 0;
+  const int wbits = wdtype_is_8bit(p->weight_dtype) ? 8 : 4;
+  if (p->lowp_mode == WOQ_HIP_LOWP_INT8 && p->x_dtype != WOQ_HIP_ACT_FP32)
+    return gemm_w4i8_scratch_bytes(p->M, p->N, p->K, wbits, p->group_size);
+  if (p->K % kTileK4 != 0 || p->x_dtype == WOQ_HIP_ACT_FP32) return 0;
+  return gemm_w4_scratch_bytes(p->M, p->N, p->K / kTileK4, wbits, p->weight_dtype == WOQ_HIP_DTYPE_NF4, p->weight_dtype == WOQ_HIP_DTYPE_FP8, false);
+}
+
 // Operand i of the post-op, null where the post-op has none: a caller's parameter struct may hold another call's pointers,
 // to other shapes or freed memory, and the kernels request the operands they are given before they look at the post-op.
 static const void* post_op_operand(const woq_hip_linear_params* p, int i) {
@@ -441,6 +452,7 @@ static bool pair_problem(const woq_hip_linear_params* g, const woq_hip_linear_pa
   f.szb_b = u->scale_zero_bf16; f.bias_b = u->bias;
   if (regime == kRegimeF16)
     return g->scale_zero_f16x2 && u->scale_zero_f16x2 && decode_kernel_applies(f, wbits, regime, g->scale_zero_f16x2) && decode_pair_applies(f, false);
+  if (f.M > 64) return !g->dense_bf16 && !u->dense_bf16 && gemm_w4_pair_applies(f, wbits, regime);
   if (f.M > 32 && f.N > kPairWideN && gemm_w4_applies(f, wbits, regime)) return false;
   return decode_dq_pair_applies(f, wbits, regime);
 }
@@ -451,11 +463,26 @@ int woq_hip_linear_pair_applies(const woq_hip_linear_params* gate, const woq_hip
   return pair_problem(gate, up, f, wbits, regime) ? 1 : 0;
 }
 
+int64_t woq_hip_linear_pair_scratch_bytes(const woq_hip_linear_params* gate, const woq_hip_linear_params* up) {
+  FpArgs f;
+  int wbits, regime;
+  return pair_problem(gate, up, f, wbits, regime) && f.M > 64 ? gemm_w4_scratch_bytes(f.M, f.N, f.KT, 4, 0, 0, true) : 0;
+}
+
 int woq_hip_linear_pair(const woq_hip_linear_params* gate, const woq_hip_linear_params* up) {
   FpArgs f;
   int wbits, regime;
   if (!pair_problem(gate, up, f, wbits, regime)) return set_error("woq_linear_pair: not a pair that woq_hip_linear_pair_applies to");
   hipStream_t st = (hipStream_t)gate->stream;
+  if (f.M > 64) {
+    SplitKScratch scratch;
+    if (gate->split_k_counters && gate->workspace && gate->workspace_bytes > 0) {
+      scratch.partial = (float*)gate->workspace;
+      scratch.bytes = gate->workspace_bytes;
+      scratch.counters = gate->split_k_counters;
+    }
+    return launch_gemm_w4_pair(f, st, &scratch);
+  }
   return regime == kRegimeF16 ? launch_decode(f, gate->scale_zero_f16x2, st, up->scale_zero_f16x2) : launch_decode_dq_pair(f, wbits, st);
 }
 
@@ -737,14 +764,14 @@ int woq_hip_linear_noalloc(const woq_hip_linear_params* p) {
                      "resident scratch holds %lld; use woq_hip_linear with a workspace of your own",
                      (long long)p->M, (long long)p->K, (long long)need, (long long)kNoAllocWorkspaceBytes);
   // Sharing K between workgroups is an option, not a need: offered for the problems it pays for (few
-  // output tiles and a long K) with what is left behind the quantized activations.  The kernels take the best plan that fits;
+  // output tiles) with what is left behind the quantized activations.  The kernels take the best plan that fits;
   // the smallest of a prompt shares 64 x 128 tiles between two workgroups.
   bool split = false;
   {
-    const int64_t extra = woq_hip_linear_auto_split_k_workspace_bytes(p->M, p->K, p->N, p->lowp_mode);
+    const int64_t extra = woq_hip_linear_scratch_bytes(p);
     const int64_t base = (need + 255) / 256 * 256, left = kNoAllocWorkspaceBytes - base;
     const int64_t least = p->M > 64 ? 2 * split_k_tiles(p->M, p->N) * 64 * 128 * (int64_t)sizeof(float) : extra;
-    if (extra > 0 && left >= least) {
+    if (extra > 0 && (left >= extra || left >= least)) {
       need = base + (extra < left ? extra : left);
       split = true;
     }

@@ -167,7 +167,7 @@ __device__ __forceinline__ void g4_tile(const FpArgs& fa, const int g_shift, flo
   __shared__ f2 sNf4[NF4 ? kNf4LutEntries : 1];
   if constexpr (NF4) nf4_fill_lut(sNf4, (int)threadIdx.x, 64 * S::WAVES);  // (the barrier before the first use is the K loop's first)
   static_assert(GROUPED || !CHAINS, "an ungrouped launch splits K over workgroups");
-  static_assert(!PAIR || (GROUPED && S::NTW % 2 == 0), "pairs: routed rows, as many row-blocks of each weight");
+  static_assert(!PAIR || S::NTW % 2 == 0, "pairs: as many row-blocks of each weight");
   constexpr int TPS = WBITS / 4;  // packed tiles per row-block and K step of 128
   // (ten row tiles on eight waves: one set of fragments only where a chain's sum needs the other's registers)
   constexpr int XA_SETS = S::WAVES == 8 && !CHAINS ? 2 : S::XA_SETS;
@@ -817,18 +817,13 @@ __global__ __launch_bounds__(64 * S::WAVES) void woq_gemm_w4_kernel(const FpArgs
 // Even, so that every split starts on buffer 0.
 inline int split_k_steps(int ksteps, int splits) { return ((ksteps + splits - 1) / splits + 1) & ~1; }
 
-template <int REGIME, class S, int WBITS = 4, bool FP8 = false, bool NF4 = false>
+template <int REGIME, class S, int WBITS = 4, bool FP8 = false, bool NF4 = false, bool PAIR = false>
 int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits = 1,
                         const SplitKScratch* scratch = nullptr) {
   constexpr int kLds = g4_lds_bytes<S, WBITS>();
   static_assert(kLds <= 160 * 1024, "a workgroup's LDS");
-  // more than 64 KiB of LDS per workgroup needs an opt-in (once per kernel and process)
-  static const hipError_t lds_optin =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-  if (lds_optin != hipSuccess)
-    return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin));
-  dim3 grid((unsigned)((f.NT * kTileN + S::BN - 1) / S::BN), (unsigned)((f.M + S::BM - 1) / S::BM),
+  constexpr int kColumns = PAIR ? S::BN / 2 : S::BN;
+  dim3 grid((unsigned)((f.NT * kTileN + kColumns - 1) / kColumns), (unsigned)((f.M + S::BM - 1) / S::BM),
             (unsigned)splits);
   const int ksteps = (int)(f.KT / (WBITS / 4));
   int kts = ksteps;
@@ -846,18 +841,27 @@ int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits = 1,
   if constexpr (REGIME == kRegimeBF16 && WBITS == 4 && !NF4) {
     if (f.szb) {  // scale and zero point of a (row, group) in one dword
       static const hipError_t lds_optin_m =
-          hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, true>),
+          hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, true, false, false, false, PAIR>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
       if (lds_optin_m != hipSuccess)
         return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin_m));
-      woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, true><<<grid, 64 * S::WAVES, kLds, st>>>(
+      woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, true, false, false, false, PAIR><<<grid, 64 * S::WAVES, kLds, st>>>(
           f, g_shift, splits > 1 ? scratch->partial : nullptr, splits > 1 ? scratch->counters : nullptr, kts, G4Group{});
       return check_launch("woq_gemm_w4_kernel");
     }
   }
+  if constexpr (PAIR) return set_error("woq_gemm_w4_kernel: a pair needs the merged parameter tables");
+  else {
+  // more than 64 KiB of LDS per workgroup needs an opt-in (once per kernel and process)
+  static const hipError_t lds_optin =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+  if (lds_optin != hipSuccess)
+    return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin));
   woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4><<<grid, 64 * S::WAVES, kLds, st>>>(f, g_shift, splits > 1 ? scratch->partial : nullptr,
                                                                  splits > 1 ? scratch->counters : nullptr, kts, G4Group{});
   return check_launch("woq_gemm_w4_kernel");
+  }
 }
 
 // 4-bit weights in one of the shapes (launch_gemm_w4's argument).

@@ -40,7 +40,7 @@ struct TilePlan {
   int shape = 42, splits = 1;  // shape as launch_gemm_w4's argument
   double us = 1e30;
 };
-constexpr int kSplitMinSteps = 8;
+constexpr int kSplitMinSteps = 4;
 constexpr int64_t kSplitScratchMax = 32 << 20;  // partial tiles of 256 workgroups of 128 x 256, the most that a plan has (64 x 128: 768, 24 MiB)
 static int64_t split_bytes(int64_t M, int64_t N, int shape, int splits) {
   const int64_t bm = shape == 5 ? 128 : 64, bn = shape == 5 ? 256 : 128;
@@ -48,9 +48,9 @@ static int64_t split_bytes(int64_t M, int64_t N, int shape, int splits) {
 }
 // What a tile costs besides its K steps: the tables, the first requests, the stores (one 128 x 256 workgroup a CU: nothing hides them).
 constexpr double kSlotUs8 = 6.0, kSlotUs42 = 5.0;
-// scratch: bytes with which K may be shared between workgroups (split_k_prefill_rows, K >= kSplitKPrefillMinK, at least eight
-// steps each), 0: not
-static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t, int64_t scratch) {
+// scratch: bytes with which K may be shared between workgroups (split_k_prefill_rows, at least four steps each), 0: not; pair: gate and
+// up as one problem of twice the columns, in the shapes whose waves have an even number of row-blocks
+static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t, int64_t scratch, bool pair = false) {
   const int64_t np = (N + kTileN - 1) / kTileN * kTileN;
   auto wgs = [&](int bm, int bn) { return ((np + bn - 1) / bn) * ((M + bm - 1) / bm); };
   auto gens = [](int64_t w) { return (double)((w + 255) / 256); };
@@ -59,7 +59,7 @@ static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t,
     if (us < best.us) best.shape = shape, best.splits = splits, best.us = us;
   };
   scratch = std::min(scratch, kSplitScratchMax);
-  const bool share = scratch > 0 && split_k_prefill_rows(M, np) && (int64_t)ksteps * kTileK4 >= kSplitKPrefillMinK;
+  const bool share = scratch > 0 && split_k_prefill_rows(M, np);
   const int most42 = t.t42[2] > 0 ? 3 : 2, most2 = t.t2[1] > 0 ? 2 : 1;
   for (int s = 1; s <= (share ? kPrefillSplitMax : 1); ++s) {
     const int kts = s == 1 ? ksteps : split_k_steps(ksteps, s);
@@ -75,20 +75,20 @@ static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t,
       offer(5, s, kts * gens(w8) * (w8 <= 192 ? t.t8 : t.t8f) + red(5, 2.0, 0.48));
   }
   const int64_t w2 = wgs(128, 128);
-  if (t.t2[0] > 0)
+  if (t.t2[0] > 0 && !pair)
     offer(2, 1, ksteps * (w2 <= 256 ? t.t2[0] : most2 == 1 ? gens(w2) * t.t2[0] : t.t2[1] * (w2 <= 512 ? 1.0 : (double)w2 / 512 + 0.1)));
-  if (t.t163 > 0 && wgs(256, 192) % 256 == 0) offer(163, 1, ksteps * gens(wgs(256, 192)) * t.t163);
-  if (t.t7 > 0) offer(7, 1, ksteps * gens(wgs(128, 448)) * t.t7);
+  if (t.t163 > 0 && !pair && wgs(256, 192) % 256 == 0) offer(163, 1, ksteps * gens(wgs(256, 192)) * t.t163);
+  if (t.t7 > 0 && !pair) offer(7, 1, ksteps * gens(wgs(128, 448)) * t.t7);
   best.us += 0.125 * ksteps;  // launch, first requests, stores: 4 us at K = 4096, in proportion as in gemm_dense_cost's figures
   return best;
 }
 static const StepTimes& step_times(int wbits, int nf4, int fp8) { return wbits == 8 ? (fp8 ? kStepsFp8 : kSteps8) : nf4 ? kStepsNf4 : kSteps4; }
 
-// K steps of a chain for an expert of 64 (i - 1) < rows <= 64 i rows, i = 2 ..: as its own launch shares them with the scratch
+// K steps of a chain for an expert (whose own launch has scratch from kSplitKPrefillMinK on) of 64 (i - 1) < rows <= 64 i rows, i = 2 ..: as its own launch shares them with the scratch
 // that woq_hip_linear_auto_split_k_workspace_bytes asks for (0: one chain).
 static int chain_steps(int64_t K, int64_t N, int wbits, int row_tiles) {
   const int ksteps = (int)(K / kTileK4);
-  const TilePlan p = plan_tiles(64 * row_tiles, N, ksteps, step_times(wbits, 0, 0), kSplitScratchMax);
+  const TilePlan p = plan_tiles(64 * row_tiles, N, ksteps, step_times(wbits, 0, 0), K >= kSplitKPrefillMinK ? kSplitScratchMax : 0);
   return p.splits > 1 ? split_k_steps(ksteps, p.splits) : 0;
 }
 // The largest [rows / 64, rounded up] that split_k_prefill_rows holds for.
@@ -155,6 +155,35 @@ int gemm_w4_chain_steps(const FpArgs& f, int wbits, int row_tiles) { return row_
 // Estimated time of the automatic choice below, in microseconds, for the comparison with the dense kernel (gemm_dense_cost).
 double gemm_w4_cost(const FpArgs& f, int wbits) {
   return plan_tiles(f.M, f.N, (int)(f.KT / (wbits / 4)), step_times(wbits, f.nf4, f.fp8), kSplitScratchMax).us;
+}
+
+int64_t gemm_w4_scratch_bytes(int64_t M, int64_t N, int64_t ksteps, int wbits, int nf4, int fp8, bool pair) {
+  const TilePlan p = plan_tiles(M, pair ? 2 * N : N, (int)ksteps, step_times(wbits, nf4, fp8), kSplitScratchMax, pair);
+  return p.splits > 1 ? split_bytes(M, (pair ? 2 * N : N) + 2 * kTileN - 1, p.shape, p.splits) : 0;
+}
+
+// Gate and up of a gated MLP as one launch, from kPairMinK input channels and kPairMinN columns of each on: it has twice the workgroups
+// where one of them leaves the chip idle, and the gate's rows stay in registers.  MLP of three linears, us, before / now (with K shared
+// below 4096 as well): M = 196, 3072 -> 3200 82.9 / 45.5, M = 363, 1536 -> 3456 68.4 / 39.7, M = 121, 1408 -> 5504 59.3 / 36.6, M = 180,
+// 2304 -> 12928 103.7 / 68.3; blocks M = 396, 3840 -> 6528 210 / 172, M = 101, 7168 -> 13056 200 / 164.  (Smaller layers keep two
+// launches, whose bits they have.)
+constexpr int64_t kPairMinK = 1024, kPairMinN = 512;
+bool gemm_w4_pair_applies(const FpArgs& f, int wbits, int regime) {
+  if (wbits != 4 || regime != kRegimeBF16 || f.nf4 || !f.szb || !f.szb_b || f.M <= 64 || f.K < kPairMinK || f.N < kPairMinN) return false;
+  if (!gemm_w4_applies(f, wbits, regime)) return false;
+  const int ksteps = (int)f.KT;
+  return plan_tiles(f.M, 2 * f.N, ksteps, kSteps4, kSplitScratchMax, true).us < 2 * plan_tiles(f.M, f.N, ksteps, kSteps4, kSplitScratchMax).us;
+}
+int launch_gemm_w4_pair(const FpArgs& f, hipStream_t st, const SplitKScratch* scratch) {
+  int g_shift = 30;
+  if (f.G < f.KT * kTileK4) {
+    g_shift = 0;
+    while (((int64_t)1 << g_shift) < f.G) ++g_shift;
+  }
+  const bool have = scratch && scratch->partial && scratch->counters;
+  const TilePlan p = plan_tiles(f.M, 2 * f.N, (int)f.KT, kSteps4, have ? scratch->bytes : 0, true);
+  return p.shape == 5 ? launch_shape<kRegimeBF16, G4Shape<8, 2, 8>, 4, false, false, true>(f, g_shift, st, p.splits, scratch)
+                      : launch_shape<kRegimeBF16, G4Shape<4, 2>, 4, false, false, true>(f, g_shift, st, p.splits, scratch);
 }
 
 int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int shape, int splits,

@@ -19,6 +19,8 @@
 // bounds the kernel.  A workgroup is 64 rows x 128 columns so that three fit on a CU (152 registers,
 // 48 KiB of LDS): with 128 rows and one wave per SIMD the LDS reads, the barrier and the MFMAs of a
 // step all sat exposed between its VALU work (452 us for M = 2048, 4096 -> 14336, against 245 us).
+#include <type_traits>
+
 #include "woq_common.h"
 #include "woq_internal.h"
 #include "woq_int8_common.h"
@@ -454,14 +456,19 @@ __global__ __launch_bounds__(256, (GSUB > 1 ? 2 : 3)) void woq_gemm_w4i8_kernel(
     const int nsplit = (int)gridDim.z, z = (int)blockIdx.z;
     const int tiles = (int)(gridDim.x * gridDim.y), tile = (int)(blockIdx.y * gridDim.x + blockIdx.x);
     constexpr int kWaveFloats = W8_MT * W8_NTW * 256;
-    float* const mine = a.sk_partial + ((size_t)(z * tiles + tile) * W8_WAVES + wave) * kWaveFloats + lane * 4;
+    // accumulator pair h of tile (mt, t): 64 lanes x 8 bytes side by side, the other workgroups' partial tiles two row tiles of all of them
+    // in flight together, as in the bf16 prefill kernel (one register an access, 16 bytes apart, and one partial tile after the other:
+    // M = 180, 7040 -> 5244 in four 45.7 us, now 33)
+    auto part = [&](int zz) { return (uint64_t*)(a.sk_partial + ((size_t)(zz * tiles + tile) * W8_WAVES + wave) * kWaveFloats) + lane; };
+    auto at = [](int mt, int t, int h) { return ((mt * W8_NTW + t) * 2 + h) * 64; };
+    uint64_t* const mine = part(z);
 #pragma unroll
     for (int mt = 0; mt < W8_MT; ++mt)
 #pragma unroll
       for (int t = 0; t < W8_NTW; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          __hip_atomic_store(mine + (mt * W8_NTW + t) * 256 + e, acc[mt][t][e], __ATOMIC_RELAXED,
+        for (int h = 0; h < 2; ++h)
+          __hip_atomic_store(mine + at(mt, t, h), bitcast<uint64_t>(f2{acc[mt][t][2 * h], acc[mt][t][2 * h + 1]}), __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
     __builtin_amdgcn_s_waitcnt(kVmcnt0);  // this thread's stores have completed
     __syncthreads();
@@ -470,41 +477,55 @@ __global__ __launch_bounds__(256, (GSUB > 1 ? 2 : 3)) void woq_gemm_w4i8_kernel(
       s_last = __hip_atomic_fetch_add(a.sk_counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsplit - 1;
     __syncthreads();
     if (!s_last) return;
-    // the other workgroups' partial tiles, one after the other in z order: all loads of one in flight
-    // together, then the additions (this workgroup's own tile comes from its registers, in its turn)
-    f4 total[W8_MT][W8_NTW];
-#pragma unroll 1
-    for (int zz = 0; zz < nsplit; ++zz) {
-      f4 v[W8_MT][W8_NTW];
-      const float* const other = a.sk_partial + ((size_t)(zz * tiles + tile) * W8_WAVES + wave) * kWaveFloats + lane * 4;
+    // added in z order, this workgroup's own from its registers in its turn
+    auto sum = [&](auto count) {
+      constexpr int N = decltype(count)::value;
+      const uint64_t* src[N - 1];
 #pragma unroll
-      for (int mt = 0; mt < W8_MT; ++mt)
+      for (int k = 0; k < N - 1; ++k) src[k] = part(k + (k >= z ? 1 : 0));
 #pragma unroll
-        for (int t = 0; t < W8_NTW; ++t) {
-          v[mt][t] = acc[mt][t];
-          if (zz != z) {
+      for (int mc = 0; mc < W8_MT; mc += 2) {
+        uint64_t v[N - 1][2][W8_NTW][2];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              v[mt][t][e] = __hip_atomic_load(other + (mt * W8_NTW + t) * 256 + e, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-          }
-        }
+        for (int k = 0; k < N - 1; ++k)
 #pragma unroll
-      for (int mt = 0; mt < W8_MT; ++mt)
+          for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int t = 0; t < W8_NTW; ++t) {
-          if (zz == 0) {
-            total[mt][t] = v[mt][t];
-          } else {
+            for (int t = 0; t < W8_NTW; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) total[mt][t][e] = total[mt][t][e] + v[mt][t][e];
-          }
-        }
-    }
+              for (int h = 0; h < 2; ++h)
+                v[k][i][t][h] = __hip_atomic_load(src[k] + at(mc + i, t, h), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int mt = 0; mt < W8_MT; ++mt)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int t = 0; t < W8_NTW; ++t) acc[mt][t] = total[mt][t];
+          for (int t = 0; t < W8_NTW; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const f2 own = {acc[mc + i][t][2 * h], acc[mc + i][t][2 * h + 1]};
+              auto value = [&](int zz) {  // partial tile zz
+                const f2 below = bitcast<f2>(v[zz < N - 1 ? zz : N - 2][i][t][h]), above = bitcast<f2>(v[zz > 0 ? zz - 1 : 0][i][t][h]);
+                return zz < z ? below : zz > z ? above : own;
+              };
+              f2 total = value(0);
+#pragma unroll
+              for (int zz = 1; zz < N; ++zz) {
+                const f2 p = value(zz);
+                total[0] = total[0] + p[0];
+                total[1] = total[1] + p[1];
+              }
+              acc[mc + i][t][2 * h] = total[0];
+              acc[mc + i][t][2 * h + 1] = total[1];
+            }
+        __builtin_amdgcn_sched_barrier(0);  // (the next row tiles' loads stay behind: their registers are these)
+      }
+    };
+    if (nsplit == 2)
+      sum(std::integral_constant<int, 2>{});
+    else if (nsplit == 3)
+      sum(std::integral_constant<int, 3>{});
+    else
+      sum(std::integral_constant<int, 4>{});
     // the counter is back at zero for the next launch that uses it
     if (tid == 0) __hip_atomic_store(a.sk_counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -802,6 +823,30 @@ bool gemm_w4i8_applies(const Int8Args& a, int64_t block_k, int64_t qbk, bool per
   return a.M * a.K < ((int64_t)1 << 31);
 }
 
+// Workgroups that share the K steps of a tile: the lowest of the estimates.  A K step takes about 1.25 us whether a CU has one workgroup or
+// all that fit (three; two with 8-bit weights or K blocks inside a tile): what it waits for are its own requests and sums, so sharing K pays until
+// the chip is full, whatever K is.  The partial tiles cost 3 us and 0.4 us a megabyte.
+static int64_t w4i8_split_bytes(int64_t tiles, int splits) { return splits * tiles * W8_BM * W8_BN * (int64_t)sizeof(float); }
+static int w4i8_splits(int64_t tiles, int64_t ksteps, int wbits, int64_t group_size, int64_t scratch) {
+  const int64_t room = 256 * (wbits == 8 || group_size == 32 || group_size == 64 ? 2 : 3);
+  int best = 1;
+  double us = 1e30;
+  for (int s = 1; s <= 4; ++s) {
+    const int64_t kts = (ksteps + s - 1) / s;
+    if (s > 1 && (tiles > kSplitKCounters || kts < 4 || (s - 1) * kts >= ksteps || w4i8_split_bytes(tiles, s) > scratch)) continue;
+    const double gens = tiles * s <= room ? 1.0 : (double)(tiles * s) / (double)room + 0.25;
+    const double here = (double)kts * 1.25 * gens + (s > 1 ? 3.0 + 0.4e-6 * (double)w4i8_split_bytes(tiles, s) : 0.0);
+    if (here < us) best = s, us = here;
+  }
+  return best;
+}
+int64_t gemm_w4i8_scratch_bytes(int64_t M, int64_t N, int64_t K, int wbits, int64_t group_size) {
+  const int64_t tiles = split_k_tiles(M, N);
+  if (K % 128 != 0 || M <= 64) return 0;
+  const int s = w4i8_splits(tiles, K / 128, wbits, group_size, (int64_t)32 << 20);
+  return s > 1 ? w4i8_split_bytes(tiles, s) : 0;
+}
+
 int launch_gemm_w4i8(const Int8Args& a, const uint8_t* xq, int64_t ldq, const float* sa, int64_t sa_m_stride,
                      int64_t sa_k_stride, int64_t qbk, hipStream_t st, const SplitKScratch* scratch,
                      const int32_t* za) {
@@ -958,20 +1003,14 @@ int launch_gemm_w4i8(const Int8Args& a, const uint8_t* xq, int64_t ldq, const fl
     return check_launch("woq_decode_w4i8_kernel");
   }
   dim3 grid((unsigned)((a.NT * kTileN + W8_BN - 1) / W8_BN), (unsigned)((a.M + W8_BM - 1) / W8_BM));
-  // few tiles and a long K: 4 or 2 workgroups per tile while that stays within 256 workgroups, leaves
-  // each at least 16 K steps and the caller's scratch suffices
   const int64_t tiles = (int64_t)grid.x * grid.y;
-  if (scratch && scratch->partial && scratch->counters && tiles <= kSplitKCounters) {
-    for (int s = 4; s >= 2; s -= 2) {
-      const int64_t need = (int64_t)s * tiles * W8_BM * W8_BN * (int64_t)sizeof(float);
-      const int kts = (int)((ksteps + s - 1) / s);
-      if (tiles * s <= 256 && ksteps / s >= 16 && scratch->bytes >= need && (int64_t)(s - 1) * kts < ksteps) {
-        grid.z = (unsigned)s;
-        k.kts = kts;
-        k.sk_partial = scratch->partial;
-        k.sk_counters = scratch->counters;
-        break;
-      }
+  if (scratch && scratch->partial && scratch->counters) {
+    const int s = w4i8_splits(tiles, ksteps, a.wbits, a.group_size, scratch->bytes);
+    if (s > 1) {
+      grid.z = (unsigned)s;
+      k.kts = (int)((ksteps + s - 1) / s);
+      k.sk_partial = scratch->partial;
+      k.sk_counters = scratch->counters;
     }
   }
   if (a.group_size == 64 && sa_k_stride != 0)

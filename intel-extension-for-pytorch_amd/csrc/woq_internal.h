@@ -81,10 +81,12 @@ constexpr int kSplitKCounters = 512;
 constexpr int kSplitKMax = 4;
 // Prefill problems that get split-K scratch by themselves (woq_hip_linear_auto_split_k_workspace_bytes): K of at least
 // kSplitKPrefillMinK and at most kSplitKPrefillMaxRows rows, or any number of rows in at most kSplitKPrefillTiles tiles of
-// 64 x 128, which leave half of the chip idle (the one condition of lowp_mode INT8).  Neither bound lies where sharing stops
-// paying: 1024 rows are the longest prompts that it was timed on with more tiles than that, and a shorter K gains in the kernel
-// as well (INT4, 64 x 128 tiles of one / two / four workgroups, us: M = 128, 2048 -> 1024 14.2 / 11.5 / 10.1, 3072 -> 4096
-// 19.6 / 14.6 / 12.7, M = 1000, 2048 -> 1024 15.3 / 13.4 / 14.2; not M = 333, 3072 -> 4096 21.4 / 22.3 / 21.4).
+// 64 x 128, which leave half of the chip idle (the one condition of lowp_mode INT8).  Neither bound lies where sharing stops paying: 1024 rows
+// are the longest prompts that it was timed on with more tiles than that, and a shorter K gains as well (INT4, 64 x 128 tiles of one / two / four
+// workgroups, us: M = 128, 2048 -> 1024 14.2 / 11.5 / 10.1, 3072 -> 4096 19.6 / 14.6 / 12.7, M = 1000, 2048 -> 1024 15.3 / 13.4 / 14.2; not
+// M = 333, 3072 -> 4096 21.4 / 22.3 / 21.4): woq_hip_linear_scratch_bytes asks for scratch there too, by the plan's estimate.  The bounds
+// are those of callers of the older function and of the experts of a routed layer, whose grouped launch runs in chains where K is shared
+// (10 % slower than in one chain).
 constexpr int64_t kSplitKPrefillMinK = 4096, kSplitKPrefillMaxRows = 1024, kSplitKPrefillTiles = 128;
 inline int64_t split_k_tiles(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 127) / 128); }
 inline bool split_k_prefill_rows(int64_t M, int64_t N) {
@@ -193,6 +195,11 @@ bool gemm_w4s_applies(const FpArgs& f, int wbits, int regime);
 int launch_gemm_w4s(const FpArgs& f, int regime, hipStream_t st);
 int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int shape = 0, int splits = 0,
                    const SplitKScratch* scratch = nullptr);
+// scratch with which the plan of a problem shares K between workgroups (pair: of gate and up together), 0 where it does not
+int64_t gemm_w4_scratch_bytes(int64_t M, int64_t N, int64_t ksteps, int wbits, int nf4, int fp8, bool pair);
+// f.pair for more than 64 rows: silu(gate) * up in one launch
+bool gemm_w4_pair_applies(const FpArgs& f, int wbits, int regime);
+int launch_gemm_w4_pair(const FpArgs& f, hipStream_t st, const SplitKScratch* scratch);
 // 64, 128 or 160: rows of a slot with the lower estimated time of a routed layer's two launches (gate and up as one of twice the columns)
 int gemm_w4_tile_rows(const int64_t* counts, int64_t experts, const int64_t* K, const int64_t* N, const int* wbits);
 int gemm_w4_split_rows(int64_t K, int64_t N);  // most rows of an expert of a routed layer that runs K in chains, 0: none
@@ -239,6 +246,7 @@ struct Int8Args {
 // sa[m * sa_m_stride + (k / qbk) * sa_k_stride] is the activation scale of row m at k, za (asymmetric
 // modes, else nullptr) the zero point at the same index, the quantized activations then being q_a - 128.
 bool gemm_w4i8_applies(const Int8Args& a, int64_t block_k, int64_t qbk, bool per_k, bool asym);
+int64_t gemm_w4i8_scratch_bytes(int64_t M, int64_t N, int64_t K, int wbits, int64_t group_size);  // beyond its workspace
 int launch_gemm_w4i8(const Int8Args& a, const uint8_t* xq, int64_t ldq, const float* sa, int64_t sa_m_stride,
                      int64_t sa_k_stride, int64_t qbk, hipStream_t st, const SplitKScratch* scratch = nullptr,
                      const int32_t* za = nullptr);

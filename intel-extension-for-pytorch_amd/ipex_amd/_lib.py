@@ -43,6 +43,8 @@ EXPORTS = [
     "woq_hip_linear_workspace_bytes",
     "woq_hip_linear_split_k_workspace_bytes",
     "woq_hip_linear_auto_split_k_workspace_bytes",
+    "woq_hip_linear_scratch_bytes",
+    "woq_hip_linear_pair_scratch_bytes",
     "woq_hip_int8_block_k",
     "woq_hip_linear",
     "woq_hip_linear_noalloc",
@@ -157,6 +159,10 @@ def load():
         lib.woq_hip_linear_split_k_workspace_bytes.argtypes = [i64, i64]
         lib.woq_hip_linear_auto_split_k_workspace_bytes.restype = i64
         lib.woq_hip_linear_auto_split_k_workspace_bytes.argtypes = [i64, i64, i64, i32]
+        lib.woq_hip_linear_scratch_bytes.restype = i64
+        lib.woq_hip_linear_scratch_bytes.argtypes = [vp]
+        lib.woq_hip_linear_pair_scratch_bytes.restype = i64
+        lib.woq_hip_linear_pair_scratch_bytes.argtypes = [vp, vp]
         lib.woq_hip_int8_block_k.restype = i64
         lib.woq_hip_int8_block_k.argtypes = [i64, i64]
         lib.woq_hip_linear.restype = i32

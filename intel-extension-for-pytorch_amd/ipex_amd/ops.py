@@ -276,7 +276,7 @@ class WoqLinearOpContext:
         self.__init__(*state)
 
     # ---- execution ----
-    def _run_planned(self, x, M, fusion, others):
+    def _run_planned(self, x, M, fusion, others, expert=False):
         """The common call (no debugging options) through a parameter block that is filled once per
         context and thread: per call only the activation / output pointers, M, the post-op, the
         workspace and the stream change."""
@@ -338,9 +338,11 @@ class WoqLinearOpContext:
             int8 = self.lowp_mode_ == _lib.LOWP_INT8
             if int8:  # the quantized activations and their scales
                 wbytes = lib.woq_hip_linear_workspace_bytes(M, K, _lib.LOWP_INT8, self.act_quant_mode_, self.group_size_)
-            # long K and few output tiles: scratch with which the decode kernel or the prefill GEMMs share K
-            # between workgroups, and the zeroed counters of this stream (the library says for which problems)
-            extra = lib.woq_hip_linear_auto_split_k_workspace_bytes(M, K, N, self.lowp_mode_)
+            # few output tiles: scratch with which the decode kernel or the prefill GEMMs share K
+            # between workgroups, and the zeroed counters of this stream (the library says for which problems; expert: those that a
+            # routed layer's own launches run in as many chains)
+            extra = (lib.woq_hip_linear_auto_split_k_workspace_bytes(M, K, N, self.lowp_mode_) if expert
+                     else lib.woq_hip_linear_scratch_bytes(tl.plan_ref))
             if extra > 0:
                 counters = _kernels._split_k_counters(x.device)
                 if counters is not None:
@@ -358,7 +360,7 @@ class WoqLinearOpContext:
             _lib.check(rc, "woq_linear")
         return out
 
-    def run(self, x, fusion=_lib.FUSE_NONE, others=(), **kw):
+    def run(self, x, fusion=_lib.FUSE_NONE, others=(), expert=False, **kw):
         N, K = self.weight_shape_
         if x.shape[-1] != K:
             raise RuntimeError(
@@ -369,9 +371,9 @@ class WoqLinearOpContext:
             return x.new_empty(*x.shape[:-1], N)
         if self.g_src_ is not None:
             x = _kernels.shuffle_activations(x, self.g_src_)
-        return self._run_sorted(x, M, fusion, others, kw)
+        return self._run_sorted(x, M, fusion, others, kw, expert)
 
-    def _run_sorted(self, x, M, fusion, others, kw):
+    def _run_sorted(self, x, M, fusion, others, kw, expert=False):
         """``run`` behind the act-order shuffle: the input channels of ``x`` are already in the order of
         the stored weight."""
         N, K = self.weight_shape_
@@ -389,7 +391,7 @@ class WoqLinearOpContext:
             x = _kernels.convert_activations(x, torch.float16)
             kw = {"out_dtype": torch.bfloat16}
         if not kw and x.dtype in _kernels._ACT_CODE and x.is_cuda:
-            return self._run_planned(x, M, fusion, others)
+            return self._run_planned(x, M, fusion, others, expert)
         return _kernels.linear(
             x,
             self.at_weight_,
@@ -638,15 +640,9 @@ def _run_context(ctx, x, fusion=_lib.FUSE_NONE, others=()):
     if isinstance(ctx, torch.Tensor) and ctx.numel() == 1 and ctx.dtype == torch.int64 and ctx.item() < 0:
         ctx = _context_from_handle(ctx)  # a handle of the ctypes twin (negative), resolved here
     if _is_python_context(ctx):
-        return ctx.run(x, fusion=fusion, others=others)
+        return ctx.run(x, fusion=fusion, others=others, expert=True)
     h = ctx if isinstance(ctx, torch.Tensor) else ctx.get_data_handle()
-    if fusion == _lib.FUSE_NONE:
-        return torch.ops.torch_ipex.ipex_woq_linear(x, h)
-    if fusion == _lib.FUSE_SILU:
-        return torch.ops.torch_ipex.woq_linear_silu(x, h)
-    if fusion == _lib.FUSE_MUL:
-        return torch.ops.torch_ipex.woq_linear_mul(x, h, list(others))
-    raise RuntimeError(f"unexpected post-op 0x{fusion:x} in an expert")
+    return torch.ops.torch_ipex.woq_linear_expert(x, h, fusion, list(others))
 
 
 def _moe_expert(hidden_states, top_x, idx, gate, up, down, routing_weights, output):

@@ -1538,3 +1538,50 @@ def test_deepseek_moe_of_two_to_four_rows_an_expert_with_long_k(cuda, monkeypatc
     got = op(hidden, ids, ctxs[0], ctxs[1], ctxs[2], rw, False)
     assert _lib.last_kernel() == "moe_combine_rows"
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,K,N,weight_dtype,G,lowp", [
+    (128, 2048, 1024, "INT4", 128, "BF16"), (65, 1024, 512, "INT4", 32, "BF16"), (333, 3200, 1040, "INT4", 64, "BF16"), (129, 1152, 272, "INT4", 128, "FP16"),
+    (200, 3968, 528, "INT8", -1, "BF16"), (1100, 2048, 256, "INT4", 128, "BF16"), (70, 2048, 100, "NF4", 64, "BF16"),
+    (128, 2048, 1024, "INT4", 128, "INT8"), (129, 1152, 272, "INT4", 32, "INT8"), (333, 3200, 1040, "INT4", 64, "INT8"), (200, 3968, 528, "INT8", -1, "INT8"),
+    (500, 4096, 4096, "INT4", 128, "INT8"),
+])
+def test_prompts_share_k_whatever_its_length(cuda, M, K, N, weight_dtype, G, lowp):
+    """Shapes whose tiles leave CUs idle, with K below 4096 and, under lowp_mode INT8, any number of tiles: against the same call of an
+    expert, which does not share K there.  The same products in another order of fp32 sums: flips of a last 16-bit digit in few outputs
+    (2e-3 in the 2-norm).  The sums have one order: every call has the same bits."""
+    from helpers import rel_l2, to_np_f32
+
+    ipex = _ipex()
+    mod = _woq_module(ipex, K, N, weight_dtype, G, lowp, bias=True, seed=7)
+    xdt = torch.float16 if lowp == "FP16" else torch.bfloat16
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(xdt).to(cuda)
+    handle = mod._op_context.get_data_handle()
+    alone = torch.ops.torch_ipex.woq_linear_expert(x, handle, 0, [])
+    first = torch.cuda.memory_stats()["allocation.all.allocated"]
+    got = torch.ops.torch_ipex.ipex_woq_linear(x, handle)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - first == 2  # the output; scratch (lowp_mode INT8: with its workspace)
+    assert rel_l2(to_np_f32(got), to_np_f32(alone)) < 2e-3
+    for _ in range(5):
+        assert torch.equal(torch.ops.torch_ipex.ipex_woq_linear(x, handle), got)
+
+
+@pytest.mark.parametrize("M,K,N,G", [(65, 1024, 512, 128), (128, 1152, 528, 32), (129, 4096, 1040, 64), (200, 2048, 3000, 128), (64 * 5, 1024, 8208, -1),
+                                     (512, 4096, 11008, 128)])
+def test_gate_and_up_of_prompts_in_one_launch(cuda, M, K, N, G):
+    """Beyond 64 rows: one launch over both weights, with or without shared K, against two launches (fp32 sums in another order at most:
+    flips of a last bf16 bit, 2e-3 in the 2-norm); every call has the same bits."""
+    from helpers import rel_l2, to_np_f32
+
+    ipex = _ipex()
+    gate, up = (_woq_module(ipex, K, N, "INT4", G, "BF16", bias=True, seed=s) for s in (44, 45))
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(cuda)
+    ops = torch.ops.torch_ipex
+    hg, hu = gate._op_context.get_data_handle(), up._op_context.get_data_handle()
+    want = ops.woq_linear_mul(x, hu, [ops.woq_linear_silu(x, hg)])
+    got = ops.woq_linear_silu_mul(x, hg, hu)
+    assert rel_l2(to_np_f32(got), to_np_f32(want)) < 2e-3
+    for _ in range(5):
+        assert torch.equal(ops.woq_linear_silu_mul(x, hg, hu), got)
+    odd = torch.cat([x.new_zeros(1), x.flatten()])[1:].view(1, M, K)
+    assert torch.equal(ops.woq_linear_silu_mul(odd, hg, hu), got.view(1, M, N))
