@@ -22,8 +22,9 @@
 #include <type_traits>
 
 #include "woq_common.h"
-#include "woq_internal.h"
+#include "woq_gemm_w4.h"
 #include "woq_int8_common.h"
+#include "woq_internal.h"
 
 // the three roundings of the epilogue stay separate (see woq_int8.hip)
 #pragma clang fp contract(off)
@@ -531,6 +532,50 @@ __global__ __launch_bounds__(256, (GSUB > 1 ? 2 : 3)) void woq_gemm_w4i8_kernel(
   }
 
   // ---- store: D[m][n], lane (n = r, c) holds rows m = 16 mt + 4 c + e ----
+  // Rows of whole 8-byte pieces go through the wave's stage in LDS, four columns a lane: an element at a time the 32 stores of a lane,
+  // two bytes each, and the post-op's operands, each waited for, took 7 us of any launch (M = 2048, 4096 -> 14336 217 -> 204 us in the kernel trace, M = 180, 7040 -> 5244 31 -> 25).
+  const Epilogue& ep = a.ep;
+  const bool out_f16 = ep.out_dtype == WOQ_HIP_ACT_FP16;
+  const bool vec4 = (ep.fusion == WOQ_HIP_FUSE_NONE ? out_f16 || ep.out_dtype == WOQ_HIP_ACT_BF16 : ep.out_dtype == ep.act_dtype && ep.act_dtype != WOQ_HIP_ACT_FP32) &&
+                    a.N % 4 == 0 && (((uintptr_t)ep.out | (uintptr_t)ep.other0 | (uintptr_t)ep.other1) & 7) == 0 && ((uintptr_t)ep.bias & 15) == 0;
+  if (vec4) {
+    constexpr int kStride = W8_NTW * kTileN + 4;
+    static_assert(W8_WAVES * W8_BM * kStride * 4 <= W8_NBUF * (W8_XBYTES + W8_WSTAGE), "the stage lies in the activation buffers and weight stages");
+    __syncthreads();  // (every wave has drained its requests and read its fragments)
+    float* const stage = (float*)sX + wave * (W8_BM * kStride);
+#pragma unroll
+    for (int mt = 0; mt < W8_MT; ++mt)
+#pragma unroll
+      for (int t = 0; t < W8_NTW; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) stage[(mt * 16 + 4 * c + e) * kStride + t * kTileN + r] = PER_K ? acc[mt][t][e] : acc[mt][t][e] * sa[mt][e];
+    const bool hb = ep.bias != nullptr;
+    constexpr int kPieces = W8_NTW * kTileN / 4;  // of a row
+    const int col = (lane % kPieces) * 4;
+    const int64_t n = (int64_t)nt0 * kTileN + col;
+    const f4 bias = hb && n < a.N ? *(const f4*)(ep.bias + n) : f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int it = 0; it < W8_BM * kPieces / 64; ++it) {
+      const int row = (it * 64 + lane) / kPieces, m = m0 + row;
+      if (m >= M || n >= a.N) continue;
+      const int64_t at = (int64_t)m * a.N + n;
+      u2 o0 = u2{0u, 0u}, o1 = u2{0u, 0u}, out;
+      if (ep.other0) o0 = *(const u2*)((const uint16_t*)ep.other0 + at);
+      if (ep.other1) o1 = *(const u2*)((const uint16_t*)ep.other1 + at);
+      const f4 v = *(const f4*)(stage + row * kStride + col);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float y = finalize_acc<kRegimeBF16>(v[e], hb, bias[e]);
+        if (ep.fusion != WOQ_HIP_FUSE_NONE)
+          y = post_op(round_to_act(y, ep.act_dtype), ep.fusion, ep.act_dtype, act_bits_to_f32((uint16_t)(o0[e / 2] >> (16 * (e % 2))), ep.act_dtype),
+                      act_bits_to_f32((uint16_t)(o1[e / 2] >> (16 * (e % 2))), ep.act_dtype));
+        const uint32_t bits = out_f16 ? f32_to_f16_bits(y) : f32_to_bf16_bits(y);
+        out[e / 2] = e % 2 ? out[e / 2] | (bits << 16) : bits;
+      }
+      *(u2*)((uint16_t*)ep.out + at) = out;
+    }
+    return;
+  }
 #pragma unroll
   for (int mt = 0; mt < W8_MT; ++mt)
 #pragma unroll
@@ -824,18 +869,20 @@ bool gemm_w4i8_applies(const Int8Args& a, int64_t block_k, int64_t qbk, bool per
 }
 
 // Workgroups that share the K steps of a tile: the lowest of the estimates.  A K step takes about 1.25 us whether a CU has one workgroup or
-// all that fit (three; two with 8-bit weights or K blocks inside a tile): what it waits for are its own requests and sums, so sharing K pays until
-// the chip is full, whatever K is.  The partial tiles cost 3 us and 0.4 us a megabyte.
+// all that fit (three; two with 8-bit weights or groups of 64): what it waits for are its own requests and sums, so sharing K pays until
+// the chip is full, whatever K is.  Groups of 32, four times the MFMAs and sums, fill the vector units with one workgroup a CU: 1.6 us
+// (130 tiles of 11 steps in three 34 us, in one 27).  The partial tiles cost 3 us and 0.4 us a megabyte.
 static int64_t w4i8_split_bytes(int64_t tiles, int splits) { return splits * tiles * W8_BM * W8_BN * (int64_t)sizeof(float); }
 static int w4i8_splits(int64_t tiles, int64_t ksteps, int wbits, int64_t group_size, int64_t scratch) {
-  const int64_t room = 256 * (wbits == 8 || group_size == 32 || group_size == 64 ? 2 : 3);
+  const int64_t room = 256 * (group_size == 32 ? 1 : wbits == 8 || group_size == 64 ? 2 : 3);
+  const double step = group_size == 32 ? 1.6 : 1.25;
   int best = 1;
   double us = 1e30;
   for (int s = 1; s <= 4; ++s) {
     const int64_t kts = (ksteps + s - 1) / s;
     if (s > 1 && (tiles > kSplitKCounters || kts < 4 || (s - 1) * kts >= ksteps || w4i8_split_bytes(tiles, s) > scratch)) continue;
     const double gens = tiles * s <= room ? 1.0 : (double)(tiles * s) / (double)room + 0.25;
-    const double here = (double)kts * 1.25 * gens + (s > 1 ? 3.0 + 0.4e-6 * (double)w4i8_split_bytes(tiles, s) : 0.0);
+    const double here = (double)kts * step * gens + (s > 1 ? 3.0 + 0.4e-6 * (double)w4i8_split_bytes(tiles, s) : 0.0);
     if (here < us) best = s, us = here;
   }
   return best;
