@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256) void woq_fp32_kernel(const Fp32Args f) {
 // against 2.3 us).
 // Bound: HBM and the launch up to four rows, the fp32 matrix pipes from 16 rows (16 rows, 4096 -> 11008: 9.2 us at 157 TFLOP/s).
 // Against the tiles of 32 / 128 x 128 outputs above, whose workgroups (86 at N = 11008) go through K alone with two barriers
-// every 32 values (us, INT8 per channel): 4096 -> 11008 M = 1 / 4 / 16 / 64 / 128 / 512 / 2048: 16.4 / 17.3 / 25.5 / 64 / 123 / 446 /
+// every 32 values (us, INT8 per channel): 4096 -> 11008 M = 1 / 4 / 16 / 64 / 128 / 512 / 2048: 16.4 / 17.3 (16 waves: 16.5) / 25.5 / 64 / 123 / 446 /
 // 1630 against 223 / 224 / 223 / 223 / 502 / 728 / 1868; 14336 -> 1024, M = 64 / 128 / 2048: 107 / 108 / 479 against 700 / 1761 / 1772.
 // The tiles win where K is short (fp32_few_rows).  Error against 64 bits 2e-7 .. 8e-7 in the 2-norm (one chain over all of K:
 // 1.1e-6 .. 2.2e-6).
@@ -203,7 +203,8 @@ enum { kFmtInt8, kFmtFp8, kFmtInt4, kFmtNf4 };
 template <int RT, int NTW>
 struct Fp32Decode {
   static constexpr int kRows = RT ? RT : 1;  // row tiles of a wave
-  static constexpr int kWaves = (RT <= 1 && NTW == 1) ? 16 : 8;  // narrow layers: more of K in flight per workgroup
+  // narrow layers and up to four rows: more of K in flight per workgroup (four row-blocks: the sums of 16 waves exceed 64 KiB of LDS)
+  static constexpr int kWaves = (RT <= 1 && NTW == 1) || (RT == 0 && NTW <= 3) ? 16 : 8;
   static constexpr int kMinWaves = RT <= 1 ? 4 : 2;              // per SIMD: 128 or 256 registers
 };
 
