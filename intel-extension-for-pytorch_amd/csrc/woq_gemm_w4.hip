@@ -65,7 +65,9 @@ static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t,
     const int kts = s == 1 ? ksteps : split_k_steps(ksteps, s);
     if (s > 1 && (kts < kSplitMinSteps || (s - 1) * kts >= ksteps)) break;
     const int64_t w42 = wgs(64, 128) * s, w8 = wgs(128, 256) * s;
-    auto red = [&](int shape, double a, double b) { return s == 1 ? 0.0 : a + b * (double)split_bytes(M, np, shape, s) * 1e-6; };
+    // (a short K must gain a microsecond: M = 116, 1280 -> 2973 ran 17.2 us shared by an estimate of 0.1 us less, 15.6 not)
+    const double margin = (int64_t)ksteps * kTileK4 < kSplitKPrefillMinK ? 1.0 : 0.0;
+    auto red = [&](int shape, double a, double b) { return s == 1 ? 0.0 : margin + a + b * (double)split_bytes(M, np, shape, s) * 1e-6; };
     const bool fits42 = s == 1 || split_bytes(M, np, 42, s) <= scratch, fits8 = s == 1 || split_bytes(M, np, 5, s) <= scratch;
     if (w42 <= 256 * most42 && fits42)
       offer(42, s, kts * t.t42[(w42 + 255) / 256 - 1] + red(42, 2.0 + 0.4 * s, 0.25));

@@ -1541,7 +1541,7 @@ def test_deepseek_moe_of_two_to_four_rows_an_expert_with_long_k(cuda, monkeypatc
 
 
 @pytest.mark.parametrize("M,K,N,weight_dtype,G,lowp", [
-    (128, 2048, 1024, "INT4", 128, "BF16"), (65, 1024, 512, "INT4", 32, "BF16"), (333, 3200, 1040, "INT4", 64, "BF16"), (129, 1152, 272, "INT4", 128, "FP16"),
+    (128, 2048, 1024, "INT4", 128, "BF16"), (65, 2048, 512, "INT4", 32, "BF16"), (333, 3200, 1040, "INT4", 64, "BF16"), (129, 1920, 272, "INT4", 128, "FP16"),
     (200, 3968, 528, "INT8", -1, "BF16"), (1100, 2048, 256, "INT4", 128, "BF16"), (70, 2048, 100, "NF4", 64, "BF16"),
     (128, 2048, 1024, "INT4", 128, "INT8"), (129, 1152, 272, "INT4", 32, "INT8"), (333, 3200, 1040, "INT4", 64, "INT8"), (200, 3968, 528, "INT8", -1, "INT8"),
     (500, 4096, 4096, "INT4", 128, "INT8"),
