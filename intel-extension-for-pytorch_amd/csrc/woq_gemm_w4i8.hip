@@ -532,13 +532,13 @@ __global__ __launch_bounds__(256, (GSUB > 1 ? 2 : 3)) void woq_gemm_w4i8_kernel(
   }
 
   // ---- store: D[m][n], lane (n = r, c) holds rows m = 16 mt + 4 c + e ----
-  // Rows of whole 8-byte pieces go through the wave's stage in LDS, four columns a lane: an element at a time the 32 stores of a lane,
+  // 16-bit outputs go through the wave's stage in LDS, four columns a lane (rows of whole 8-byte pieces in one access): an element at a time the 32 stores of a lane,
   // two bytes each, and the post-op's operands, each waited for, took 7 us of any launch (M = 2048, 4096 -> 14336 217 -> 204 us in the kernel trace, M = 180, 7040 -> 5244 31 -> 25).
   const Epilogue& ep = a.ep;
   const bool out_f16 = ep.out_dtype == WOQ_HIP_ACT_FP16;
-  const bool vec4 = (ep.fusion == WOQ_HIP_FUSE_NONE ? out_f16 || ep.out_dtype == WOQ_HIP_ACT_BF16 : ep.out_dtype == ep.act_dtype && ep.act_dtype != WOQ_HIP_ACT_FP32) &&
-                    a.N % 4 == 0 && (((uintptr_t)ep.out | (uintptr_t)ep.other0 | (uintptr_t)ep.other1) & 7) == 0 && ((uintptr_t)ep.bias & 15) == 0;
-  if (vec4) {
+  const bool staged = ep.fusion == WOQ_HIP_FUSE_NONE ? out_f16 || ep.out_dtype == WOQ_HIP_ACT_BF16 : ep.out_dtype == ep.act_dtype && ep.act_dtype != WOQ_HIP_ACT_FP32;
+  const bool whole = a.N % 4 == 0 && (((uintptr_t)ep.out | (uintptr_t)ep.other0 | (uintptr_t)ep.other1) & 7) == 0 && ((uintptr_t)ep.bias & 15) == 0;
+  if (staged) {
     constexpr int kStride = W8_NTW * kTileN + 4;
     static_assert(W8_WAVES * W8_BM * kStride * 4 <= W8_NBUF * (W8_XBYTES + W8_WSTAGE), "the stage lies in the activation buffers and weight stages");
     __syncthreads();  // (every wave has drained its requests and read its fragments)
@@ -553,15 +553,28 @@ __global__ __launch_bounds__(256, (GSUB > 1 ? 2 : 3)) void woq_gemm_w4i8_kernel(
     constexpr int kPieces = W8_NTW * kTileN / 4;  // of a row
     const int col = (lane % kPieces) * 4;
     const int64_t n = (int64_t)nt0 * kTileN + col;
-    const f4 bias = hb && n < a.N ? *(const f4*)(ep.bias + n) : f4{0.f, 0.f, 0.f, 0.f};
+    const int cols = n + 4 <= a.N ? 4 : (int)(a.N - n);
+    f4 bias = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (hb && e < cols) bias[e] = ep.bias[n + e];
 #pragma unroll 4
     for (int it = 0; it < W8_BM * kPieces / 64; ++it) {
       const int row = (it * 64 + lane) / kPieces, m = m0 + row;
       if (m >= M || n >= a.N) continue;
       const int64_t at = (int64_t)m * a.N + n;
       u2 o0 = u2{0u, 0u}, o1 = u2{0u, 0u}, out;
-      if (ep.other0) o0 = *(const u2*)((const uint16_t*)ep.other0 + at);
-      if (ep.other1) o1 = *(const u2*)((const uint16_t*)ep.other1 + at);
+      auto operand = [&](const void* p) {
+        const uint16_t* const v = (const uint16_t*)p + at;
+        if (whole) return *(const u2*)v;
+        u2 r = u2{v[0], 0u};
+        if (cols > 1) r[0] |= (uint32_t)v[1] << 16;
+        if (cols > 2) r[1] = v[2];
+        if (cols > 3) r[1] |= (uint32_t)v[3] << 16;
+        return r;
+      };
+      if (ep.other0) o0 = operand(ep.other0);
+      if (ep.other1) o1 = operand(ep.other1);
       const f4 v = *(const f4*)(stage + row * kStride + col);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -572,7 +585,13 @@ __global__ __launch_bounds__(256, (GSUB > 1 ? 2 : 3)) void woq_gemm_w4i8_kernel(
         const uint32_t bits = out_f16 ? f32_to_f16_bits(y) : f32_to_bf16_bits(y);
         out[e / 2] = e % 2 ? out[e / 2] | (bits << 16) : bits;
       }
-      *(u2*)((uint16_t*)ep.out + at) = out;
+      if (whole) {
+        *(u2*)((uint16_t*)ep.out + at) = out;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (e < cols) ((uint16_t*)ep.out)[at + e] = (uint16_t)(out[e / 2] >> (16 * (e % 2)));
+      }
     }
     return;
   }

@@ -1585,3 +1585,25 @@ def test_gate_and_up_of_prompts_in_one_launch(cuda, M, K, N, G):
         assert torch.equal(ops.woq_linear_silu_mul(x, hg, hu), got)
     odd = torch.cat([x.new_zeros(1), x.flatten()])[1:].view(1, M, K)
     assert torch.equal(ops.woq_linear_silu_mul(odd, hg, hu), got.view(1, M, N))
+
+
+@pytest.mark.parametrize("lowp", ["BF16", "INT8"])
+@pytest.mark.parametrize("M,K,N", [(65, 256, 31), (130, 384, 979), (64, 512, 16387), (200, 4096, 770)])
+def test_prompts_of_odd_widths_round_each_post_op_once(cuda, lowp, M, K, N):
+    """Rows that are no whole 8-byte pieces, with a bias: every post-op of the prefill kernels against the plain call and the element-wise
+    function on its output, one rounding each: sums and products bit for bit, the others to a flip of the last bf16 bit (2^-8 of
+    a value).  Operands at addresses that are no multiple of eight."""
+    ipex = _ipex()
+    mod = _woq_module(ipex, K, N, "INT4", 128, lowp, bias=True, seed=3)
+    g = torch.Generator().manual_seed(N)
+    x = torch.randn(M, K, generator=g).bfloat16().to(cuda)
+    a, b = (torch.randn(M * N + 1, generator=g).bfloat16().to(cuda)[1:].view(M, N) for _ in range(2))
+    ops, h = torch.ops.torch_ipex, mod._op_context.get_data_handle()
+    base = ops.ipex_woq_linear(x, h)
+    assert torch.equal(ops.woq_linear_add(x, h, [a]), (base.float() + a.float()).bfloat16())
+    assert torch.equal(ops.woq_linear_mul(x, h, [a]), (base.float() * a.float()).bfloat16())
+    assert torch.equal(ops.woq_linear_add_add(x, h, [a, b]), ((base.float() + a.float()).bfloat16().float() + b.float()).bfloat16())
+    assert torch.equal(ops.woq_linear_relu(x, h), torch.relu(base))
+    F = torch.nn.functional
+    for got, want in ((ops.woq_linear_gelu(x, h), F.gelu(base.float())), (ops.woq_linear_silu(x, h), F.silu(base.float()))):
+        assert torch.allclose(got.float(), want, rtol=2.0**-8, atol=1e-6)
