@@ -850,17 +850,18 @@ int launch_shape(const FpArgs& f, int g_shift, hipStream_t st, int splits = 1,
       return check_launch("woq_gemm_w4_kernel");
     }
   }
-  if constexpr (PAIR) return set_error("woq_gemm_w4_kernel: a pair needs the merged parameter tables");
-  else {
-  // more than 64 KiB of LDS per workgroup needs an opt-in (once per kernel and process)
-  static const hipError_t lds_optin =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-  if (lds_optin != hipSuccess)
-    return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin));
-  woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4><<<grid, 64 * S::WAVES, kLds, st>>>(f, g_shift, splits > 1 ? scratch->partial : nullptr,
-                                                                 splits > 1 ? scratch->counters : nullptr, kts, G4Group{});
-  return check_launch("woq_gemm_w4_kernel");
+  if constexpr (PAIR) {
+    return set_error("woq_gemm_w4_kernel: a pair needs the merged parameter tables");
+  } else {
+    // more than 64 KiB of LDS per workgroup needs an opt-in (once per kernel and process)
+    static const hipError_t lds_optin =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (lds_optin != hipSuccess)
+      return set_error("woq_gemm_w4_kernel: LDS opt-in failed: %s", hipGetErrorString(lds_optin));
+    woq_gemm_w4_kernel<REGIME, S, WBITS, FP8, false, false, NF4><<<grid, 64 * S::WAVES, kLds, st>>>(
+        f, g_shift, splits > 1 ? scratch->partial : nullptr, splits > 1 ? scratch->counters : nullptr, kts, G4Group{});
+    return check_launch("woq_gemm_w4_kernel");
   }
 }
 
