@@ -465,7 +465,7 @@ int woq_hip_moe_linear(const woq_hip_linear_params* p, const void* group, int64_
  * launch's order, so it has that launch's bits; woq_hip_moe_chained_rows: the most rows of such an expert, 0 if there is none
  * at this K and N.  Slots whose table does not say the expert's rows run K in one chain.
  * woq_hip_moe_tile_rows: the tile_rows (64, 128 or 160) with the lower estimated time for a gated layer H -> I -> H whose experts
- * have counts[e] rows (on the host).
+ * have counts[e] rows (on the host).  gate_dtype: the 8-bit one where gate and up differ (160 only if no linear is 8-bit).
  */
 int woq_hip_moe_tile_rows(const int64_t* counts, int64_t experts, int64_t H, int64_t I, int gate_dtype, int down_dtype);
 int64_t woq_hip_moe_chained_rows(int64_t K, int64_t N);

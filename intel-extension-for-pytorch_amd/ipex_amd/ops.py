@@ -944,9 +944,11 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
 
 def _moe_tile_rows(shapes, counts):
     """Rows of a slot of the prefill kernel, 64, 128 or 160, by the lower estimated time.  ``shapes``: K, N and weight dtype (wd) of the
-    three linears, ``counts``: rows of every expert."""
-    gate, down = shapes[0], shapes[2]
-    return _lib.load().woq_hip_moe_tile_rows((ctypes.c_int64 * len(counts))(*counts), len(counts), gate["K"], gate["N"], gate["wd"], down["wd"])
+    three linears, ``counts``: rows of every expert.  All three run in the same slots, and 160 rows go with 4-bit weights only: a layer
+    whose gate and up differ in type is asked for as one of 8-bit weights."""
+    gate, up, down = shapes
+    wd = _lib.DTYPE_INT8 if _lib.DTYPE_INT8 in (gate["wd"], up["wd"]) else gate["wd"]
+    return _lib.load().woq_hip_moe_tile_rows((ctypes.c_int64 * len(counts))(*counts), len(counts), gate["K"], gate["N"], wd, down["wd"])
 
 
 def _moe_expert_launches_faster(shapes, counts):

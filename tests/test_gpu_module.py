@@ -1435,6 +1435,30 @@ def test_deepseek_moe_prompt_slots_of_160_rows(cuda, monkeypatch, H, I, G, lowp)
         op(hidden, ids, [mk8(H, I, e) for e in range(E)], [mk8(H, I, e) for e in range(E)], [mk8(I, H, e) for e in range(E)], rw, False)
 
 
+def test_deepseek_moe_prompt_with_an_8_bit_up_projection(cuda, monkeypatch):
+    """Experts of 130 rows, which layers of 4-bit weights run in slots of 160: with an INT8 up projection in slots that all three linears
+    take, bit for bit the experts' own launches (no shared K at these widths)."""
+    from ipex_amd import _lib
+
+    ipex = _ipex()
+    E, H, I, rows = 32, 2048, 1024, 130
+    mk = lambda k, n, wd, G, s: _woq_module(ipex, k, n, wd, G, "BF16", seed=s)._op_context
+    gate, up, down = ([m[e % 2] for e in range(E)] for m in ([mk(H, I, "INT4", 128, s) for s in (950, 951)], [mk(H, I, "INT8", -1, s) for s in (952, 953)],
+                                                             [mk(I, H, "INT4", 128, s) for s in (954, 955)]))
+    g = torch.Generator().manual_seed(11)
+    T = E * rows
+    ids = torch.arange(E).repeat_interleave(rows)[torch.randperm(T, generator=g)].view(T, 1).to(cuda)
+    hidden = torch.randn(T, H, generator=g).bfloat16().to(cuda)
+    rw = torch.rand(T, 1, generator=g).bfloat16().to(cuda)
+    op = torch.ops.torch_ipex.deepseek_moe_woq
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "0")
+    want = op(hidden, ids, gate, up, down, rw, False)
+    monkeypatch.setenv("IPEX_AMD_MOE_GROUPED", "1")
+    got = op(hidden, ids, gate, up, down, rw, False)
+    assert _lib.last_kernel() == "moe_combine_rows"
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("T,topk,E,rows", [(65, 1, 1, 64), (512, 8, 32, 160), (1024, 8, 1024, 128), (1023, 8, 67, 160), (777, 3, 5, 160), (4097, 1, 2, 128)])
 def test_moe_route_tiles_against_sorted_lists(cuda, T, topk, E, rows):
     """Places, slots and the order of a token's contributions, at one and at 1024 experts, at remainders of the 64 entries that a wave

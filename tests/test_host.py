@@ -403,6 +403,16 @@ def test_moe_prompts_that_stay_on_the_experts_own_launches():
     assert not own(4096, 14336, i4, [4096, 4096])  # 4329 / 3105
 
 
+def test_moe_prompt_slots_of_160_rows_need_three_linears_of_4_bits():
+    from ipex_amd import _lib, ops
+
+    i4, i8 = _lib.DTYPE_INT4, _lib.DTYPE_INT8
+    pick = lambda g, u, d: ops._moe_tile_rows([dict(K=2048, N=1024, wd=g), dict(K=2048, N=1024, wd=u), dict(K=1024, N=2048, wd=d)], [130] * 32)
+    assert pick(i4, i4, i4) == 160
+    for types in ((i4, i8, i4), (i8, i4, i4), (i8, i8, i4), (i4, i4, i8), (i4, i8, i8), (i8, i8, i8)):
+        assert pick(*types) in (64, 128), types
+
+
 def test_moe_layers_on_other_devices_and_streams_do_not_wait_for_each_other():
     from ipex_amd import ops
 
