@@ -664,9 +664,16 @@ static int decode_waves(const FpArgs& f) {
   }
   return (int)w;
 }
+// Two row-blocks per workgroup from 512 row-blocks on; a single row only above 768: up to there one
+// row-block per workgroup spreads more evenly over the 256 CUs (M = 1: 8192 -> 10240 9.6 us against
+// 11.7 us, 4096 -> 8192 5.2 against 5.4 us, 4096 -> 11008 6.5 against 6.7 us; 4096 -> 14336 the other
+// way round, 7.1 against 7.8 us; M = 4, 4096 -> 11008: 7.4 us with two against 7.7 us).
+static bool two_row_blocks(const FpArgs& f) { return f.NT % 2 == 0 && (f.M == 1 ? f.NT > 768 : f.NT >= 512); }
+// Routed slots of two to four rows: eight tiles a wave only where the expert's own launch has them too (it keeps two row-blocks and
+// rounds of two tiles on wide layers), so that the fp32 sums have one order.
 bool decode_pair_applies(const FpArgs& f, bool grouped) {
   return f.x_dtype == WOQ_HIP_ACT_BF16 && f.out_dtype == WOQ_HIP_ACT_BF16 &&
-         (f.M == 1 || grouped || !eight_tiles(f, f.KT == (int64_t)decode_waves(f) * kDecodeKPW));
+         (f.M == 1 || (grouped && !two_row_blocks(f)) || !eight_tiles(f, f.KT == (int64_t)decode_waves(f) * kDecodeKPW));
 }
 
 static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t st, const MoeGroup* grp, int slots,
@@ -700,16 +707,12 @@ static int launch_decode_impl(const FpArgs& f, const uint32_t* sz, hipStream_t s
   while ((int64_t)kTileK4 << (a.tpg_shift + 1) <= f.G && a.tpg_shift < 30) ++a.tpg_shift;
   a.W = decode_waves(f);
   const bool xf16 = f.x_dtype == WOQ_HIP_ACT_FP16;
-  // Two row-blocks per workgroup from 512 row-blocks on; a single row only above 768: up to there one
-  // row-block per workgroup spreads more evenly over the 256 CUs (M = 1: 8192 -> 10240 9.6 us against
-  // 11.7 us, 4096 -> 8192 5.2 against 5.4 us, 4096 -> 11008 6.5 against 6.7 us; 4096 -> 14336 the other
-  // way round, 7.1 against 7.8 us; M = 4, 4096 -> 11008: 7.4 us with two against 7.7 us).
   // Routed slots of two to four rows fill the chip with fewer row-blocks: a workgroup of two reads the rows of activations -- as many
-  // bytes as the weights of one row-block -- half as often (17 slots, 2048 -> 7168: 27 us against 36 us; the bits are the same,
-  // so only where one round of two K tiles a wave is what the expert's own launch runs, too).
+  // bytes as the weights of one row-block -- half as often (17 slots, 2048 -> 7168: 27 us against 36 us).  Row-blocks do not
+  // change the order of the sums, tiles a wave do: not where the expert's own launch has eight.
   const bool one_round = f.KT == (int64_t)decode_waves(f) * kDecodeKPW;
   const bool many_slots = slots > 0 && f.M > 1 && !eight_tiles(f, one_round) && f.NT / 2 * slots >= 2048;
-  const bool two = f.NT % 2 == 0 && (f.M == 1 ? f.NT > 768 : f.NT >= 512 || many_slots);
+  const bool two = two_row_blocks(f) || (f.NT % 2 == 0 && many_slots);
   a.wbytes = (uint32_t)(f.NT * f.KT * kTileBytes);  // below 4 GiB (decode_kernel_applies)
   a.szbytes = (uint32_t)(f.NT * f.KG * kTileN * (int64_t)sizeof(uint32_t));
   const bool one_row = f.M == 1;

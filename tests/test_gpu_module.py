@@ -1541,16 +1541,18 @@ def test_deepseek_moe_of_few_tokens_that_name_an_expert_often(cuda, monkeypatch,
     assert sorted(row_of.cpu().tolist()) == list(range(R))
 
 
-@pytest.mark.parametrize("H,I", [(7168, 256), (4352, 512), (16384, 256), (256, 8192)])
+@pytest.mark.parametrize("H,I", [(7168, 256), (4352, 512), (16384, 256), (256, 8192), (7168, 8192), (8192, 7936)])
 def test_deepseek_moe_of_two_to_four_rows_an_expert_with_long_k(cuda, monkeypatch, H, I):
-    """Gate and up of slots of two to four rows with eight K tiles a wave in one launch, and two row-blocks a workgroup where many slots
-    share the launch: bit for bit the experts' own launches."""
+    """Gate and up of slots of two to four rows with eight K tiles a wave in one launch, two row-blocks a workgroup where many slots
+    share the launch, and wide layers, whose experts' own launches take K in rounds of two tiles a wave (from 8192 columns on; 7936 is
+    below): bit for bit the experts' own launches."""
     from ipex_amd import _lib
 
     ipex = _ipex()
     E, T, topk = 24, 24, 3
+    kinds = 3 if H * I < 2**24 else 1  # different experts
     mk = lambda k, n, s: _woq_module(ipex, k, n, "INT4", 128, "BF16", bias=True, seed=s)._op_context
-    ctxs = [[mk(H, I, 600 + e % 3) for e in range(E)], [mk(H, I, 610 + e % 3) for e in range(E)], [mk(I, H, 620 + e % 3) for e in range(E)]]
+    ctxs = [[mk(H, I, 600 + e % kinds) for e in range(E)], [mk(H, I, 610 + e % kinds) for e in range(E)], [mk(I, H, 620 + e % kinds) for e in range(E)]]
     g = torch.Generator().manual_seed(H)
     hidden = torch.randn(T, H, generator=g).bfloat16().to(cuda)
     ids = torch.stack([(t * 3 + torch.arange(3)) % (E - 4) for t in range(T)]).to(cuda)  # three or four rows each
