@@ -1014,6 +1014,11 @@ static Tensor woq_linear_silu_mul_autocast(const Tensor& input, const Tensor& W_
   return woq_linear_silu_mul(autocast_input(input), W_gate, W_up);
 }
 
+static Tensor woq_linear_expert_autocast(const Tensor& input, const Tensor& W_prepack, int64_t fusion, const std::vector<Tensor>& others) {
+  c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
+  return woq_linear_expert(autocast_input(input), W_prepack, fusion, others);
+}
+
 static Tensor woq_linear_v2_autocast(const Tensor& input, const Tensor& qweight, c10::string_view weight_dtype,
                                      std::vector<int64_t> weight_shape, std::vector<Tensor> weight_scales,
                                      optional<std::vector<Tensor>> weight_zeros, optional<std::vector<Tensor>> bias,
@@ -1088,6 +1093,7 @@ TORCH_LIBRARY_FRAGMENT(torch_ipex, m) {
   m.def("woq_linear_silu(Tensor input, Tensor W_prepack) -> Tensor");
   // silu(gate(x)) * up(x) of a gated MLP (Linear2SiluMul); no counterpart among the reference's operators, which calls the two above
   m.def("woq_linear_silu_mul(Tensor input, Tensor W_gate, Tensor W_up) -> Tensor");
+  // one linear of a routed layer's expert, for the package's own per-expert path; no counterpart in the reference
   m.def("woq_linear_expert(Tensor input, Tensor W_prepack, int fusion, Tensor[] others) -> Tensor");
   m.def("woq_linear_add(Tensor input, Tensor W_prepack, Tensor[] others) -> Tensor");
   m.def("woq_linear_add_add(Tensor input, Tensor W_prepack, Tensor[] others) -> Tensor");
@@ -1148,6 +1154,7 @@ TORCH_LIBRARY_IMPL(torch_ipex, CPU, m) {
     m.impl(name, TORCH_FN(refuse_cpu_2));
   for (const char* name : {"woq_linear_add", "woq_linear_add_add", "woq_linear_mul"}) m.impl(name, TORCH_FN(refuse_cpu_3));
   m.impl("woq_linear_silu_mul", TORCH_FN(woq_linear_silu_mul));  // raises on its CPU input
+  m.impl("woq_linear_expert", TORCH_FN(woq_linear_expert));  // raises on its CPU input
   m.impl("woq_linear", TORCH_FN(woq_linear_v2));      // raises on its CPU input
   m.impl("dequantize_nf4", TORCH_FN(dequantize_nf4));  // raises on its CPU input
 }
@@ -1162,5 +1169,6 @@ TORCH_LIBRARY_IMPL(torch_ipex, AutocastCUDA, m) {
   m.impl("woq_linear_add_add", TORCH_FN((woq_linear_binary_autocast<WOQ_HIP_FUSE_ADD_ADD, 2>)));
   m.impl("woq_linear_mul", TORCH_FN((woq_linear_binary_autocast<WOQ_HIP_FUSE_MUL, 1>)));
   m.impl("woq_linear_silu_mul", TORCH_FN(woq_linear_silu_mul_autocast));
+  m.impl("woq_linear_expert", TORCH_FN(woq_linear_expert_autocast));
   m.impl("woq_linear", TORCH_FN(woq_linear_v2_autocast));
 }

@@ -1305,6 +1305,22 @@ def test_jit_trace_save_load(cuda, tmp_path, weight_dtype, bias, M, K, N):
         assert torch.equal(loaded(x), want)
 
 
+def test_an_expert_s_linears_cast_under_autocast_as_the_other_operators(cuda):
+    from ipex_amd import _lib
+
+    ipex = _ipex()
+    mod = _woq_module(ipex, 256, 48, "INT4", 128, "BF16", seed=8)
+    h = mod._op_context.get_data_handle()
+    x = torch.randn(5, 256, generator=torch.Generator().manual_seed(8)).to(cuda)
+    ops = torch.ops.torch_ipex
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        want = ops.woq_linear_silu(x, h)
+        got = ops.woq_linear_expert(x, h, _lib.FUSE_SILU, [])
+        product = ops.woq_linear_expert(x, h, _lib.FUSE_MUL, [got])
+        assert torch.equal(product, ops.woq_linear_mul(x, h, [want]))
+    assert got.dtype == torch.bfloat16 and torch.equal(got, want)
+
+
 def test_autocast_casts_the_input_only(cuda):
     """AutocastCUDA (csrc/cpu/aten/Linear.cpp:874-883): fp32 rows under autocast(bf16) run as bf16 rows."""
     from ipex_amd.utils import synthetic

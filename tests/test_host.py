@@ -322,6 +322,17 @@ def test_ops_are_registered_with_reference_schemas():
         assert hasattr(torch.ops.ipex_prepack, name)
 
 
+@pytest.mark.parametrize("name", ["ipex_woq_linear", "woq_linear_silu", "woq_linear_mul", "woq_linear_silu_mul", "woq_linear_expert", "woq_linear"])
+def test_every_linear_op_casts_under_autocast_and_refuses_cpu_tensors(name):
+    import ipex_amd  # noqa: F401
+
+    for key in ("CPU", "CUDA", "AutocastCUDA"):
+        assert torch._C._dispatch_has_kernel_for_dispatch_key(f"torch_ipex::{name}", key), key
+    if name == "woq_linear_expert":
+        with pytest.raises(RuntimeError, match="GPU"):
+            torch.ops.torch_ipex.woq_linear_expert(torch.zeros(1, 128, dtype=torch.bfloat16), torch.tensor([1]), 0, [])
+
+
 def test_auto_split_k_predicate_is_the_library_s():
     """The problems on which woq_hip_linear shares K between workgroups by itself, asked of the library (pure host
     arithmetic): few output tiles and a long K; everything else gets no scratch."""
