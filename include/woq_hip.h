@@ -288,10 +288,13 @@ int64_t woq_hip_linear_split_k_workspace_bytes(int64_t M, int64_t N);
  * rule to keep in step.  No counterpart in the reference. */
 int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t lowp_mode);
 
-/* The scratch of one call, M of p included: woq_hip_linear_auto_split_k_workspace_bytes where that is not 0, else what the plan of a
- * prompt of more than 64 rows takes at any K -- a K below 4096 in the floating-point modes, any number of tiles under lowp_mode INT8 --, 0 where K is
- * not shared.  (A linear of a routed layer's expert asks the older function: woq_hip_linear_grouped_tiles has the bits of those
- * launches.)  woq_hip_linear_pair_scratch_bytes: of a woq_hip_linear_pair call, given in the workspace and counters of `gate`.  No counterpart in the reference. */
+/* The scratch with which woq_hip_linear (force_kernel 0) shares K between workgroups on the call p, 0 where the kernel that the call
+ * runs on does not share it.  5 to 32 rows: as the function above.  More than 64 rows: what the plan of the prefill GEMMs takes, at any K
+ * and, under lowp_mode INT8, with any number of tiles; with K of at least 4096 no more than the function above says.  The output
+ * pointers of p are not looked at; x and dense_bf16 are, for their alignment and presence.  (A linear of a routed layer's
+ * expert asks the older function: woq_hip_linear_grouped_tiles has the bits of those launches.)
+ * woq_hip_linear_pair_scratch_bytes: of a woq_hip_linear_pair call, given in the workspace and counters of `gate`.  No counterpart
+ * in the reference. */
 int64_t woq_hip_linear_scratch_bytes(const woq_hip_linear_params* p);
 int64_t woq_hip_linear_pair_scratch_bytes(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);
 

@@ -198,22 +198,102 @@ int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_
   return decode || prefill ? woq_hip_linear_split_k_workspace_bytes(M, N) : 0;
 }
 
-int64_t woq_hip_linear_scratch_bytes(const woq_hip_linear_params* p) {
-  if (!p || p->struct_size != sizeof(*p) || !valid_wdtype(p->weight_dtype) || p->M <= 0 || p->K <= 0 || p->N <= 0) return 0;
-  if (const int64_t bytes = woq_hip_linear_auto_split_k_workspace_bytes(p->M, p->K, p->N, p->lowp_mode)) return bytes;
-  if (p->M <= 64) return 0;
-  const int wbits = wdtype_is_8bit(p->weight_dtype) ? 8 : 4;
-  if (p->lowp_mode == WOQ_HIP_LOWP_INT8 && p->x_dtype != WOQ_HIP_ACT_FP32)
-    return gemm_w4i8_scratch_bytes(p->M, p->N, p->K, wbits, p->group_size);
-  if (p->K % kTileK4 != 0 || p->x_dtype == WOQ_HIP_ACT_FP32) return 0;
-  return gemm_w4_scratch_bytes(p->M, p->N, p->K / kTileK4, wbits, p->weight_dtype == WOQ_HIP_DTYPE_NF4, p->weight_dtype == WOQ_HIP_DTYPE_FP8, false);
-}
-
 // Operand i of the post-op, null where the post-op has none: a caller's parameter struct may hold another call's pointers,
 // to other shapes or freed memory, and the kernels request the operands they are given before they look at the post-op.
 static const void* post_op_operand(const woq_hip_linear_params* p, int i) {
   const bool one = p->fusion == WOQ_HIP_FUSE_ADD || p->fusion == WOQ_HIP_FUSE_MUL, two = p->fusion == WOQ_HIP_FUSE_ADD_ADD;
   return two || (one && i == 0) ? p->others[i] : nullptr;
+}
+
+// The low precision mode that a call computes in.  Shapes the blocked int8 kernels do not take run unquantized in the activation
+// dtype, which is what the reference's fallback does for lowp_mode INT8 (csrc/cpu/aten/kernels/WoqInt8GemmAPerMKrnl.cpp:143-169).
+static int effective_lowp(const woq_hip_linear_params* p) {
+  if (p->lowp_mode != WOQ_HIP_LOWP_INT8) return p->lowp_mode;
+  const int64_t bk = woq_hip_int8_block_k(p->group_size, p->K);
+  return p->x_dtype == WOQ_HIP_ACT_FP32 || (bk != 32 && bk != 64 && bk != 128) ? WOQ_HIP_LOWP_NONE : WOQ_HIP_LOWP_INT8;
+}
+
+// Sizes in tiles and groups of a call's packed weight.
+struct PackedSizes {
+  int wbits;
+  int64_t NT, KT, G, KG;
+};
+static PackedSizes packed_sizes(const woq_hip_linear_params* p) {
+  PackedSizes s;
+  s.wbits = wdtype_is_8bit(p->weight_dtype) ? 8 : 4;
+  const int tk = s.wbits == 4 ? kTileK4 : kTileK8;
+  s.NT = woq_hip_padded_n(p->N) / kTileN;
+  s.KT = woq_hip_padded_k(p->weight_dtype, p->K) / tk;
+  s.G = p->group_size > 0 ? p->group_size : s.KT * tk;
+  s.KG = p->group_size > 0 ? (p->K + s.G - 1) / s.G : 1;
+  return s;
+}
+
+static Int8Args int8_args(const woq_hip_linear_params* p, const PackedSizes& z) {
+  Int8Args a;
+  a.x = p->x; a.x_dtype = p->x_dtype; a.M = p->M; a.K = p->K; a.N = p->N; a.NT = z.NT; a.KT = z.KT;
+  a.qweight = (const uint8_t*)p->qweight; a.wbits = z.wbits; a.scales = p->scales_f32;
+  a.zeros = p->zeros_u8; a.G = z.G; a.KG = z.KG; a.bias = p->bias; a.act_quant_mode = p->act_quant_mode;
+  a.fusion = p->fusion; a.other0 = post_op_operand(p, 0); a.other1 = post_op_operand(p, 1); a.out = p->out;
+  a.out_dtype = p->out_dtype; a.workspace = p->workspace; a.workspace_bytes = p->workspace_bytes;
+  a.split_k_counters = p->split_k_counters;
+  a.debug_block_sums = p->debug_block_sums;
+  a.nf4 = p->weight_dtype == WOQ_HIP_DTYPE_NF4 ? 1 : 0;
+  a.group_size = p->group_size;
+  return a;
+}
+
+// The compute type of the floating-point kernels (csrc/cpu/aten/kernels/WoqLinearKrnl.cpp:75-112; the small-batch threshold is the
+// environment's IPEX_WOQ_SMALL_BATCH_THRESHOLD, 5 by default, csrc/cpu/aten/utils/woq.h:24); -1: none, fp32 compute or an error.
+static int fp_regime(const woq_hip_linear_params* p, int lowp) {
+  if (lowp == WOQ_HIP_LOWP_FP16 || (lowp == WOQ_HIP_LOWP_NONE && p->x_dtype == WOQ_HIP_ACT_FP16) ||
+      (lowp == WOQ_HIP_LOWP_BF16 && p->M < small_batch_threshold()))
+    return kRegimeF16;
+  if ((lowp == WOQ_HIP_LOWP_NONE && p->x_dtype == WOQ_HIP_ACT_BF16) || lowp == WOQ_HIP_LOWP_BF16) return kRegimeBF16;
+  return -1;
+}
+
+static FpArgs fp_args(const woq_hip_linear_params* p, const PackedSizes& z, int regime) {
+  FpArgs f;
+  f.x = p->x; f.x_dtype = p->x_dtype; f.M = p->M; f.K = p->K; f.N = p->N; f.NT = z.NT; f.KT = z.KT;
+  f.qweight = (const uint8_t*)p->qweight;
+  f.scales = (const uint16_t*)(regime == kRegimeF16 ? p->scales_f16 : p->scales_bf16);
+  f.zeros = p->zeros_u8; f.G = z.G; f.KG = z.KG; f.bias = p->bias; f.fusion = p->fusion;
+  f.other0 = post_op_operand(p, 0); f.other1 = post_op_operand(p, 1); f.out = p->out; f.out_dtype = p->out_dtype;
+  f.nf4 = p->weight_dtype == WOQ_HIP_DTYPE_NF4 ? 1 : 0;
+  f.fp8 = p->weight_dtype == WOQ_HIP_DTYPE_FP8 ? 1 : 0;
+  f.szb = (regime == kRegimeBF16 && !f.nf4 && !f.fp8) ? p->scale_zero_bf16 : nullptr;
+  return f;
+}
+
+// Whether a call with a dense copy (cache_weight_for_large_batch, csrc/cpu/jit/cpu/kernels/LinearWoqPacked.cpp:511-526: lowp_mode
+// BF16, at least the threshold's rows) runs on it: where it is the faster kernel, against the prefill kernel that dequantizes in
+// registers (a quarter of the bytes for the same MFMAs, and shapes of 64 rows) by the two cost models, which leave NF4 out: it and
+// weights that kernel does not take (groups that split a lane's K values) always go to the dense one.
+static bool takes_dense(const woq_hip_linear_params* p, int lowp, const FpArgs& f, int wbits, int regime) {
+  if (!p->dense_bf16 || lowp != WOQ_HIP_LOWP_BF16 || regime != kRegimeBF16 || p->M < weight_cache_batch_threshold() || p->M <= 64 ||
+      !gemm_dense_applies(f))
+    return false;
+  return f.nf4 || !gemm_w4_applies(f, wbits, regime) || gemm_dense_cost(f) < 0.97 * gemm_w4_cost(f, wbits, INT64_MAX);
+}
+
+// Follows the choice of woq_hip_linear (force_kernel 0): 0 unless the kernel that the call runs on shares K.
+int64_t woq_hip_linear_scratch_bytes(const woq_hip_linear_params* p) {
+  if (!p || p->struct_size != sizeof(*p) || !valid_wdtype(p->weight_dtype) || p->M <= 0 || p->K <= 0 || p->N <= 0) return 0;
+  if (p->group_size > 0 && p->group_size % 32 != 0) return 0;
+  const int64_t older = woq_hip_linear_auto_split_k_workspace_bytes(p->M, p->K, p->N, p->lowp_mode);
+  if (p->M <= 64 && older == 0) return 0;
+  const PackedSizes z = packed_sizes(p);
+  const int lowp = effective_lowp(p);
+  if (lowp == WOQ_HIP_LOWP_INT8)
+    return int8_linear_shares_k(int8_args(p, z)) ? gemm_w4i8_scratch_bytes(p->M, p->N, p->K, z.wbits, p->group_size) : 0;
+  const int regime = fp_regime(p, lowp);
+  if (regime < 0) return 0;
+  const FpArgs f = fp_args(p, z, regime);
+  if (p->M <= 64) return decode_dq_applies(f, z.wbits, regime) ? older : 0;
+  if (!gemm_w4_applies(f, z.wbits, regime)) return 0;
+  const int64_t bytes = gemm_w4_scratch_bytes(f.M, f.N, f.KT / (z.wbits / 4), z.wbits, f.nf4, f.fp8, false, older);
+  return bytes > 0 && !takes_dense(p, lowp, f, z.wbits, regime) ? bytes : 0;
 }
 
 int woq_hip_linear(const woq_hip_linear_params* p) {
@@ -256,13 +336,8 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
   if (p->out_dtype == WOQ_HIP_ACT_FP32 && p->x_dtype != WOQ_HIP_ACT_FP32 && p->fusion != WOQ_HIP_FUSE_NONE)
     return set_error("woq_linear: the fp32 accumulator output does not take a post-op");
 
-  const int wbits = wdtype_is_8bit(p->weight_dtype) ? 8 : 4;
-  const int tk = wbits == 4 ? kTileK4 : kTileK8;
-  const int64_t NT = woq_hip_padded_n(p->N) / kTileN;
-  const int64_t KT = woq_hip_padded_k(p->weight_dtype, p->K) / tk;
-  const int64_t Kpad = KT * tk;
-  const int64_t G = p->group_size > 0 ? p->group_size : Kpad;
-  const int64_t KG = p->group_size > 0 ? (p->K + G - 1) / G : 1;
+  const PackedSizes z = packed_sizes(p);
+  const int wbits = z.wbits;
   hipStream_t st = (hipStream_t)p->stream;
 
   const bool nf4 = p->weight_dtype == WOQ_HIP_DTYPE_NF4;
@@ -271,67 +346,31 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
   if (fp8 && p->zeros_u8) return set_error("woq_linear: FP8 weights take no zero points");
   if (fp8 && p->lowp_mode == WOQ_HIP_LOWP_INT8)
     return set_error("woq_linear: lowp_mode INT8 does not take FP8 weights");
-  int lowp = p->lowp_mode;
+  if (p->lowp_mode == WOQ_HIP_LOWP_INT8 && p->weight_dtype == WOQ_HIP_DTYPE_INT8 && p->zeros_u8)
+    return set_error("woq_linear: symmetric quantization is required for INT8 weights with lowp_mode INT8");
+  const int lowp = effective_lowp(p);
   if (lowp == WOQ_HIP_LOWP_INT8) {
-    const int64_t bk = woq_hip_int8_block_k(p->group_size, p->K);
-    const bool blocks_ok = bk == 32 || bk == 64 || bk == 128;
-    const bool mode_ok = p->act_quant_mode >= WOQ_HIP_QUANT_A_PER_TENSOR &&
-                         p->act_quant_mode <= WOQ_HIP_QUANT_A_PER_M_K_BLOCK_SYM;
-    if (p->weight_dtype == WOQ_HIP_DTYPE_INT8 && p->zeros_u8)
-      return set_error("woq_linear: symmetric quantization is required for INT8 weights with lowp_mode INT8");
-    if (p->x_dtype == WOQ_HIP_ACT_FP32 || !blocks_ok) {
-      // Shapes the blocked int8 kernel does not take run unquantized in the activation dtype,
-      // which is what the reference's fallback does for lowp_mode INT8
-      // (csrc/cpu/aten/kernels/WoqInt8GemmAPerMKrnl.cpp:143-169).
-      lowp = WOQ_HIP_LOWP_NONE;
-    } else if (!mode_ok) {
+    if (p->act_quant_mode < WOQ_HIP_QUANT_A_PER_TENSOR || p->act_quant_mode > WOQ_HIP_QUANT_A_PER_M_K_BLOCK_SYM)
       return set_error("woq_linear: lowp_mode INT8 needs an act_quant_mode in 0..7, got %d", p->act_quant_mode);
-    } else {
-      Int8Args a;
-      a.x = p->x; a.x_dtype = p->x_dtype; a.M = p->M; a.K = p->K; a.N = p->N; a.NT = NT; a.KT = KT;
-      a.qweight = (const uint8_t*)p->qweight; a.wbits = wbits; a.scales = p->scales_f32;
-      a.zeros = p->zeros_u8; a.G = G; a.KG = KG; a.bias = p->bias; a.act_quant_mode = p->act_quant_mode;
-      a.fusion = p->fusion; a.other0 = post_op_operand(p, 0); a.other1 = post_op_operand(p, 1); a.out = p->out;
-      a.out_dtype = p->out_dtype; a.workspace = p->workspace; a.workspace_bytes = p->workspace_bytes;
-      a.split_k_counters = p->split_k_counters;
-      a.debug_block_sums = p->debug_block_sums;
-      a.nf4 = nf4 ? 1 : 0;
-      a.group_size = p->group_size;
-      return launch_int8_linear(a, st);
-    }
+    return launch_int8_linear(int8_args(p, z), st);
   }
 
-  // Floating-point regimes (csrc/cpu/aten/kernels/WoqLinearKrnl.cpp:75-112; the small-batch threshold
-  // is the environment's IPEX_WOQ_SMALL_BATCH_THRESHOLD, 5 by default, csrc/cpu/aten/utils/woq.h:24).
-  int regime;
-  if (lowp == WOQ_HIP_LOWP_FP16 || (lowp == WOQ_HIP_LOWP_NONE && p->x_dtype == WOQ_HIP_ACT_FP16) ||
-      (lowp == WOQ_HIP_LOWP_BF16 && p->M < small_batch_threshold())) {
-    regime = kRegimeF16;
-  } else if ((lowp == WOQ_HIP_LOWP_NONE && p->x_dtype == WOQ_HIP_ACT_BF16) || lowp == WOQ_HIP_LOWP_BF16) {
-    regime = kRegimeBF16;
-  } else if (lowp == WOQ_HIP_LOWP_NONE && p->x_dtype == WOQ_HIP_ACT_FP32) {
+  const int regime = fp_regime(p, lowp);
+  if (regime < 0) {
+    if (lowp != WOQ_HIP_LOWP_NONE || p->x_dtype != WOQ_HIP_ACT_FP32)
+      return set_error("woq_linear: lowp_mode %d does not take x_dtype %d", lowp, p->x_dtype);
     // fp32 compute (csrc/cpu/aten/kernels/WoqLinearKrnl.cpp:142-158)
     if (p->force_kernel != 0) return set_error("woq_linear: fp32 compute has one kernel; force_kernel must be 0");
     Fp32Args a;
-    a.x = (const float*)p->x; a.M = p->M; a.K = p->K; a.N = p->N; a.NT = NT; a.KT = KT;
+    a.x = (const float*)p->x; a.M = p->M; a.K = p->K; a.N = p->N; a.NT = z.NT; a.KT = z.KT;
     a.qweight = (const uint8_t*)p->qweight; a.scales = p->scales_f32; a.zeros = p->zeros_u8;
-    a.G = G; a.KG = KG; a.bias = p->bias; a.fusion = p->fusion;
+    a.G = z.G; a.KG = z.KG; a.bias = p->bias; a.fusion = p->fusion;
     a.other0 = post_op_operand(p, 0); a.other1 = post_op_operand(p, 1); a.out = p->out; a.nf4 = nf4 ? 1 : 0;
     a.fp8 = fp8 ? 1 : 0;
     return launch_fp32(a, wbits, st);
-  } else {
-    return set_error("woq_linear: lowp_mode %d does not take x_dtype %d", lowp, p->x_dtype);
   }
 
-  FpArgs f;
-  f.x = p->x; f.x_dtype = p->x_dtype; f.M = p->M; f.K = p->K; f.N = p->N; f.NT = NT; f.KT = KT;
-  f.qweight = (const uint8_t*)p->qweight;
-  f.scales = (const uint16_t*)(regime == kRegimeF16 ? p->scales_f16 : p->scales_bf16);
-  f.zeros = p->zeros_u8; f.G = G; f.KG = KG; f.bias = p->bias; f.fusion = p->fusion;
-  f.other0 = post_op_operand(p, 0); f.other1 = post_op_operand(p, 1); f.out = p->out; f.out_dtype = p->out_dtype;
-  f.nf4 = nf4 ? 1 : 0;
-  f.fp8 = fp8 ? 1 : 0;
-  f.szb = (regime == kRegimeBF16 && !nf4 && !fp8) ? p->scale_zero_bf16 : nullptr;
+  const FpArgs f = fp_args(p, z, regime);
   SplitKScratch scratch;
   if (p->split_k_counters && p->workspace && p->workspace_bytes > 0) {
     scratch.partial = (float*)p->workspace;
@@ -340,22 +379,14 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
   }
 
   int kernel = p->force_kernel;
-  // The dense copy (cache_weight_for_large_batch, csrc/cpu/jit/cpu/kernels/LinearWoqPacked.cpp:511-526: lowp_mode
-  // BF16, at least the threshold's rows): same operands into the same MFMAs as the kernels below, so same results.
+  // The dense copy: same operands into the same MFMAs as the kernels below.
   if (kernel >= 23 && kernel <= 26) {
     if (!p->dense_bf16 || regime != kRegimeBF16 || !gemm_dense_applies(f))
       return set_error("woq_linear: the dense kernel takes dense_bf16, bf16 compute on bf16 activations and "
                        "K %% 128 == 0");
     return launch_gemm_dense(f, p->dense_bf16, wbits, st, kernel == 23 ? 0 : kernel == 24 ? 7 : kernel == 25 ? 4 : 2);
   }
-  if (kernel == 0 && p->dense_bf16 && lowp == WOQ_HIP_LOWP_BF16 && regime == kRegimeBF16 &&
-      p->M >= weight_cache_batch_threshold() && p->M > 64 && gemm_dense_applies(f)) {
-    // ... where it is the faster kernel: against the prefill kernel that dequantizes in registers (a quarter of the
-    // bytes for the same MFMAs, and shapes of 64 rows) by the two cost models, which leave NF4 out: it and weights that
-    // kernel does not take (groups that split a lane's K values) always go to the dense one
-    if (nf4 || !gemm_w4_applies(f, wbits, regime) || gemm_dense_cost(f) < 0.97 * gemm_w4_cost(f, wbits))
-      return launch_gemm_dense(f, p->dense_bf16, wbits, st, 0);
-  }
+  if (kernel == 0 && takes_dense(p, lowp, f, wbits, regime)) return launch_gemm_dense(f, p->dense_bf16, wbits, st, 0);
   if (nf4) {
     // table lookups instead of the integer decode: the dequantizing decode kernel, the prefill kernel and the two
     // general kernels carry them
@@ -466,7 +497,7 @@ int woq_hip_linear_pair_applies(const woq_hip_linear_params* gate, const woq_hip
 int64_t woq_hip_linear_pair_scratch_bytes(const woq_hip_linear_params* gate, const woq_hip_linear_params* up) {
   FpArgs f;
   int wbits, regime;
-  return pair_problem(gate, up, f, wbits, regime) && f.M > 64 ? gemm_w4_scratch_bytes(f.M, f.N, f.KT, 4, 0, 0, true) : 0;
+  return pair_problem(gate, up, f, wbits, regime) && f.M > 64 ? gemm_w4_scratch_bytes(f.M, f.N, f.KT, 4, 0, 0, true, 0) : 0;
 }
 
 int woq_hip_linear_pair(const woq_hip_linear_params* gate, const woq_hip_linear_params* up) {

@@ -154,14 +154,16 @@ int gemm_w4_split_rows(int64_t K, int64_t N) {
 // The slots of a routed layer (launch_gemm_w4_grouped) and the fp16 compute type have files of their own.
 int gemm_w4_chain_steps(const FpArgs& f, int wbits, int row_tiles) { return row_tiles <= chain_row_tiles(f.N) ? chain_steps(f.K, f.N, wbits, row_tiles) : 0; }
 
-// Estimated time of the automatic choice below, in microseconds, for the comparison with the dense kernel (gemm_dense_cost).
-double gemm_w4_cost(const FpArgs& f, int wbits) {
-  return plan_tiles(f.M, f.N, (int)(f.KT / (wbits / 4)), step_times(wbits, f.nf4, f.fp8), kSplitScratchMax).us;
+// Estimated time of the automatic choice below with that scratch, in microseconds, for the comparison with the dense kernel
+// (gemm_dense_cost).
+double gemm_w4_cost(const FpArgs& f, int wbits, int64_t scratch_bytes) {
+  return plan_tiles(f.M, f.N, (int)(f.KT / (wbits / 4)), step_times(wbits, f.nf4, f.fp8), scratch_bytes).us;
 }
 
-int64_t gemm_w4_scratch_bytes(int64_t M, int64_t N, int64_t ksteps, int wbits, int nf4, int fp8, bool pair) {
-  const TilePlan p = plan_tiles(M, pair ? 2 * N : N, (int)ksteps, step_times(wbits, nf4, fp8), kSplitScratchMax, pair);
-  return p.splits > 1 ? split_bytes(M, (pair ? 2 * N : N) + 2 * kTileN - 1, p.shape, p.splits) : 0;
+int64_t gemm_w4_scratch_bytes(int64_t M, int64_t N, int64_t ksteps, int wbits, int nf4, int fp8, bool pair, int64_t most) {
+  if (most == 0) most = kSplitScratchMax;
+  const TilePlan p = plan_tiles(M, pair ? 2 * N : N, (int)ksteps, step_times(wbits, nf4, fp8), most, pair);
+  return p.splits > 1 ? std::min(most, split_bytes(M, (pair ? 2 * N : N) + 2 * kTileN - 1, p.shape, p.splits)) : 0;
 }
 
 // Gate and up of a gated MLP as one launch, from kPairMinK input channels and kPairMinN columns of each on: it has twice the workgroups

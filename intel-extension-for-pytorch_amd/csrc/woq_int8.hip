@@ -730,6 +730,17 @@ static int dispatch_small_i8(Int8KArgs& p, hipStream_t st) {
   return launch_small_i8_cfg<WBITS, 4, 2, 1>(p, st);
 }
 
+// K values that share an activation scale in the quantization.
+static int64_t quant_block(const Int8Args& a, int64_t block_k) {
+  if (!quant_a_per_k(a.act_quant_mode)) return a.K;
+  return a.group_size <= 0 ? block_k : a.G;
+}
+
+bool int8_linear_shares_k(const Int8Args& a) {
+  const int64_t block_k = woq_hip_int8_block_k(a.group_size <= 0 ? -1 : a.G, a.K);
+  return a.M > 64 && gemm_w4i8_applies(a, block_k, quant_block(a, block_k), quant_a_per_k(a.act_quant_mode), !quant_a_is_sym(a.act_quant_mode));
+}
+
 int launch_int8_linear(const Int8Args& a, hipStream_t st) {
   const int mode = a.act_quant_mode;
   if (mode < WOQ_HIP_QUANT_A_PER_TENSOR || mode > WOQ_HIP_QUANT_A_PER_M_K_BLOCK_SYM)
@@ -769,7 +780,7 @@ int launch_int8_linear(const Int8Args& a, hipStream_t st) {
   p.xq = xq;
   p.sa = sa;
   p.za = za;
-  const int64_t qbk_quant = per_k ? (per_channel ? p.block_k : G) : a.K;
+  const int64_t qbk_quant = quant_block(a, p.block_k);
   const bool direct = gemm_w4i8_applies(a, p.block_k, qbk_quant, per_k, asym);
   if (direct && decode_i8_rows_applies(a, qbk_quant, per_m, per_k, asym)) return launch_decode_i8_rows(a, qbk_quant, per_k, st);
   if (int rc = launch_quant_impl(a.x, a.x_dtype, a.M, a.K, p.ldq, qbk_quant, mode, xq, sa, za,

@@ -195,8 +195,9 @@ bool gemm_w4s_applies(const FpArgs& f, int wbits, int regime);
 int launch_gemm_w4s(const FpArgs& f, int regime, hipStream_t st);
 int launch_gemm_w4(const FpArgs& f, int wbits, int regime, hipStream_t st, int shape = 0, int splits = 0,
                    const SplitKScratch* scratch = nullptr);
-// scratch with which the plan of a problem shares K between workgroups (pair: of gate and up together), 0 where it does not
-int64_t gemm_w4_scratch_bytes(int64_t M, int64_t N, int64_t ksteps, int wbits, int nf4, int fp8, bool pair);
+// scratch with which the plan of a problem shares K between workgroups (pair: of gate and up together), 0 where it does not;
+// most: bytes that it may take, 0: any
+int64_t gemm_w4_scratch_bytes(int64_t M, int64_t N, int64_t ksteps, int wbits, int nf4, int fp8, bool pair, int64_t most);
 // f.pair for more than 64 rows: silu(gate) * up in one launch
 bool gemm_w4_pair_applies(const FpArgs& f, int wbits, int regime);
 int launch_gemm_w4_pair(const FpArgs& f, hipStream_t st, const SplitKScratch* scratch);
@@ -212,7 +213,7 @@ int launch_gemm_w4_grouped(const FpArgs& f, int wbits, int regime, const MoeGrou
 bool gemm_dense_applies(const FpArgs& f);
 // estimated microseconds of the dense kernel / of launch_gemm_w4's automatic choice on this problem
 double gemm_dense_cost(const FpArgs& f);
-double gemm_w4_cost(const FpArgs& f, int wbits);
+double gemm_w4_cost(const FpArgs& f, int wbits, int64_t scratch_bytes);
 int launch_gemm_dense(const FpArgs& f, const void* dense, int wbits, hipStream_t st, int shape = 0);
 int launch_dense_weight(const void* qweight, int weight_dtype, int64_t N, int64_t K, const uint16_t* sb16,
                         const uint8_t* z8, int64_t G, void* out, hipStream_t st);
@@ -245,6 +246,7 @@ struct Int8Args {
 // int8 MFMA kernels that feed the stored codes to the MFMA (woq_gemm_w4i8.hip);
 // sa[m * sa_m_stride + (k / qbk) * sa_k_stride] is the activation scale of row m at k, za (asymmetric
 // modes, else nullptr) the zero point at the same index, the quantized activations then being q_a - 128.
+bool int8_linear_shares_k(const Int8Args& a);  // whether launch_int8_linear runs a prompt on its 64 x 128 tiles, which may share K
 bool gemm_w4i8_applies(const Int8Args& a, int64_t block_k, int64_t qbk, bool per_k, bool asym);
 int64_t gemm_w4i8_scratch_bytes(int64_t M, int64_t N, int64_t K, int wbits, int64_t group_size);  // beyond its workspace
 int launch_gemm_w4i8(const Int8Args& a, const uint8_t* xq, int64_t ldq, const float* sa, int64_t sa_m_stride,

@@ -434,3 +434,79 @@ def test_moe_layers_on_other_devices_and_streams_do_not_wait_for_each_other():
             assert other.acquire(blocking=False)
             other.release()
         assert not ops._moe_launch_lock(0, 1).acquire(blocking=False)
+
+
+def _linear_params(M, K, N, weight, G=128, lowp="BF16", x="BF16", aq=6, dense=False, zeros=False):
+    import ctypes
+
+    from ipex_amd import _lib
+
+    p = _lib.LinearParams()
+    p.struct_size = ctypes.sizeof(_lib.LinearParams)
+    p.M, p.K, p.N, p.weight_dtype, p.group_size = M, K, N, getattr(_lib, f"DTYPE_{weight}"), G
+    p.lowp_mode, p.x_dtype, p.out_dtype = (getattr(_lib, f"LOWP_{lowp}"), *[getattr(_lib, f"ACT_{x}")] * 2)
+    p.act_quant_mode = aq
+    p.dense_bf16 = 4096 if dense else None  # (host arithmetic: no pointer is followed)
+    p.zeros_u8 = 4096 if zeros else None
+    return p
+
+
+@pytest.mark.parametrize("kw", [
+    dict(M=1000, K=4096, N=2048, weight="INT8", G=-1, lowp="INT8"),  # more than 512 rows of 8-bit weights: the general int8 kernel
+    dict(M=600, K=2048, N=1024, weight="INT8", G=-1, lowp="INT8"),
+    dict(M=128, K=2048, N=1024, weight="INT4", G=32, lowp="INT8", aq=7),  # groups of 32 with a scale per (row, K block)
+    dict(M=128, K=2048, N=1024, weight="INT8", G=-1, lowp="INT8", aq=2),  # asymmetric rows and 8-bit weights
+    dict(M=128, K=2048, N=1024, weight="NF4", G=64, lowp="INT8"),  # NF4 in K blocks of 64
+    dict(M=128, K=2048, N=1024, weight="INT4", G=384, lowp="INT8"),  # groups of no power of two
+    dict(M=128, K=1920, N=1024, weight="INT4", G=96),  # ... under bf16 compute, short and long K
+    dict(M=128, K=4608, N=1024, weight="INT4", G=96),
+    dict(M=128, K=1920, N=1024, weight="INT4", G=96, lowp="INT8"),  # computes in bf16
+    dict(M=128, K=2048, N=1024, weight="INT8", G=64),  # 8-bit weights in groups below a K step
+    dict(M=128, K=2000, N=1024, weight="INT4", G=-1),  # K of no whole steps
+    dict(M=128, K=2048, N=1024, weight="INT4", x="FP16"),  # fp16 rows under bf16 compute, bf16 rows under fp16
+    dict(M=128, K=4096, N=1024, weight="INT4", x="FP16"),
+    dict(M=128, K=2048, N=1024, weight="INT4", lowp="FP16"),
+    dict(M=128, K=2048, N=1024, weight="INT8", G=-1, lowp="NONE", x="FP32"),  # fp32 compute
+    dict(M=128, K=4096, N=1024, weight="INT8", G=-1, lowp="NONE", x="FP32"),
+    dict(M=128, K=4096, N=1024, weight="INT4", lowp="INT8", x="FP32"),
+    dict(M=16, K=8192, N=4096, weight="INT4", G=96),  # the general kernel of few rows
+    dict(M=128, K=2048, N=2048, weight="NF4", G=64, dense=True),  # the dense copy
+    dict(M=900, K=4096, N=4096, weight="FP8", dense=True),
+    dict(M=64, K=4096, N=4096, weight="INT4"), dict(M=2048, K=4096, N=14336, weight="INT4"), dict(M=128, K=128, N=4096, weight="INT4"),
+])
+def test_calls_whose_kernel_shares_no_k_ask_for_no_scratch(kw):
+    import ctypes
+
+    from ipex_amd import _lib
+
+    assert _lib.load().woq_hip_linear_scratch_bytes(ctypes.byref(_linear_params(**kw))) == 0
+
+
+@pytest.mark.parametrize("kw", [
+    dict(M=128, K=2048, N=1024, weight="INT4"), dict(M=200, K=3968, N=528, weight="INT8", G=-1), dict(M=70, K=2048, N=100, weight="NF4", G=64),
+    dict(M=129, K=1920, N=272, weight="INT4", lowp="FP16", x="FP16"), dict(M=128, K=2048, N=2048, weight="INT4", dense=True),
+    dict(M=500, K=2048, N=1024, weight="INT8", G=-1, lowp="INT8"), dict(M=1000, K=2048, N=1024, weight="INT8", G=-1, lowp="INT8", aq=7),
+    dict(M=128, K=2048, N=1024, weight="INT4", G=64, lowp="INT8", aq=7), dict(M=128, K=2048, N=1024, weight="INT4", lowp="INT8", aq=2),
+])
+def test_scratch_of_a_call_is_its_plan_s_partial_tiles(kw):
+    """Four workgroups a tile of 64 x 128; the floating-point plan rounds its columns up by as much as two row-blocks."""
+    import ctypes
+
+    from ipex_amd import _lib
+
+    got = _lib.load().woq_hip_linear_scratch_bytes(ctypes.byref(_linear_params(**kw)))
+    columns = kw["N"] + (0 if kw.get("lowp") == "INT8" else 31)
+    assert got == 4 * -(-kw["M"] // 64) * -(-columns // 128) * 64 * 128 * 4
+
+
+def test_scratch_at_a_long_k_is_within_what_the_older_function_says():
+    import ctypes
+
+    from ipex_amd import _lib
+
+    lib = _lib.load()
+    for M, K, N in ((128, 4096, 4096), (77, 4096, 11008), (333, 11008, 4096), (1000, 7168, 4096), (2048, 4096, 512), (16, 14336, 4096)):
+        for weight, G in (("INT4", 128), ("INT8", -1), ("NF4", 64), ("FP8", 128)):
+            got = lib.woq_hip_linear_scratch_bytes(ctypes.byref(_linear_params(M, K, N, weight, G)))
+            assert 0 <= got <= lib.woq_hip_linear_auto_split_k_workspace_bytes(M, K, N, _lib.LOWP_BF16)
+            assert got > 0 or (M, K, N) != (333, 11008, 4096)
