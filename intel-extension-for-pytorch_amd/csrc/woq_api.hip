@@ -269,12 +269,13 @@ static FpArgs fp_args(const woq_hip_linear_params* p, const PackedSizes& z, int 
 // Whether a call with a dense copy (cache_weight_for_large_batch, csrc/cpu/jit/cpu/kernels/LinearWoqPacked.cpp:511-526: lowp_mode
 // BF16, at least the threshold's rows) runs on it: where it is the faster kernel, against the prefill kernel that dequantizes in
 // registers (a quarter of the bytes for the same MFMAs, and shapes of 64 rows) by the two cost models, which leave NF4 out: it and
-// weights that kernel does not take (groups that split a lane's K values) always go to the dense one.
-static bool takes_dense(const woq_hip_linear_params* p, int lowp, const FpArgs& f, int wbits, int regime) {
+// weights that kernel does not take (groups that split a lane's K values) always go to the dense one.  scratch_bytes: what the
+// packed launch could share K with.
+static bool takes_dense(const woq_hip_linear_params* p, int lowp, const FpArgs& f, int wbits, int regime, int64_t scratch_bytes) {
   if (!p->dense_bf16 || lowp != WOQ_HIP_LOWP_BF16 || regime != kRegimeBF16 || p->M < weight_cache_batch_threshold() || p->M <= 64 ||
       !gemm_dense_applies(f))
     return false;
-  return f.nf4 || !gemm_w4_applies(f, wbits, regime) || gemm_dense_cost(f) < 0.97 * gemm_w4_cost(f, wbits, INT64_MAX);
+  return f.nf4 || !gemm_w4_applies(f, wbits, regime) || gemm_dense_cost(f) < 0.97 * gemm_w4_cost(f, wbits, scratch_bytes);
 }
 
 // Follows the choice of woq_hip_linear (force_kernel 0): 0 unless the kernel that the call runs on shares K.
@@ -293,7 +294,7 @@ int64_t woq_hip_linear_scratch_bytes(const woq_hip_linear_params* p) {
   if (p->M <= 64) return decode_dq_applies(f, z.wbits, regime) ? older : 0;
   if (!gemm_w4_applies(f, z.wbits, regime)) return 0;
   const int64_t bytes = gemm_w4_scratch_bytes(f.M, f.N, f.KT / (z.wbits / 4), z.wbits, f.nf4, f.fp8, false, older);
-  return bytes > 0 && !takes_dense(p, lowp, f, z.wbits, regime) ? bytes : 0;
+  return bytes > 0 && !takes_dense(p, lowp, f, z.wbits, regime, bytes) ? bytes : 0;
 }
 
 int woq_hip_linear(const woq_hip_linear_params* p) {
@@ -386,7 +387,7 @@ int woq_hip_linear(const woq_hip_linear_params* p) {
                        "K %% 128 == 0");
     return launch_gemm_dense(f, p->dense_bf16, wbits, st, kernel == 23 ? 0 : kernel == 24 ? 7 : kernel == 25 ? 4 : 2);
   }
-  if (kernel == 0 && takes_dense(p, lowp, f, wbits, regime)) return launch_gemm_dense(f, p->dense_bf16, wbits, st, 0);
+  if (kernel == 0 && takes_dense(p, lowp, f, wbits, regime, scratch.partial ? scratch.bytes : 0)) return launch_gemm_dense(f, p->dense_bf16, wbits, st, 0);
   if (nf4) {
     // table lookups instead of the integer decode: the dequantizing decode kernel, the prefill kernel and the two
     // general kernels carry them

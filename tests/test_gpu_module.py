@@ -1649,3 +1649,21 @@ def test_prompts_of_odd_widths_round_each_post_op_once(cuda, lowp, M, K, N):
     F = torch.nn.functional
     for got, want in ((ops.woq_linear_gelu(x, h), F.gelu(base.float())), (ops.woq_linear_silu(x, h), F.silu(base.float()))):
         assert torch.allclose(got.float(), want, rtol=2.0**-8, atol=1e-6)
+
+
+@pytest.mark.parametrize("M,K,N", [(128, 2048, 2048), (512, 3968, 1024)])
+def test_the_dense_copy_is_compared_with_the_packed_launch_that_the_call_can_have(cuda, M, K, N):
+    """FP8 with a dense copy, K below 4096: the prefill kernel with K shared is the faster one, the dense kernel where a call has no
+    scratch (an expert's own launch)."""
+    from ipex_amd import _lib
+
+    g = torch.Generator().manual_seed(M)
+    w = (torch.randn(N, K, generator=g) * 20).to(torch.float8_e4m3fn).to(cuda)
+    scales = (torch.rand(N, K // 128, generator=g) * 0.01 + 0.001).to(cuda)
+    ctx = torch.ops.ipex_prepack.weight_only_qlinear_prepack(w, _lib.DTYPE_FP8, [N, K], scales, None, None, None, None, 128, _lib.LOWP_BF16, -1, True)
+    x = torch.randn(M, K, generator=g).bfloat16().to(cuda)
+    got = torch.ops.torch_ipex.ipex_woq_linear(x, ctx.get_data_handle())
+    assert _lib.last_kernel() == "woq_gemm_w4_kernel"
+    alone = torch.ops.torch_ipex.woq_linear_expert(x, ctx.get_data_handle(), 0, [])
+    assert _lib.last_kernel() == "woq_gemm_dense_kernel"
+    assert float((got.double() - alone.double()).norm() / alone.double().norm()) < 2e-3
