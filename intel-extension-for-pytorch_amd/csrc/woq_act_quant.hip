@@ -7,8 +7,8 @@
 //
 // The two-kernel form (one workgroup per quantization group for the statistics, then one thread per
 // 8 elements) reads the activations twice and, for per-(row, K block) scales, starts one workgroup
-// per 128 elements.  Here a workgroup owns a row: it loads the row once (16 bytes per lane and 512-element
-// chunk, kept as the raw 16-bit values), reduces min / max over its waves (or over the lanes of a K
+// per 128 elements.  Here a workgroup or a wave owns a row: it loads the row once (16 bytes per lane and 512-element
+// chunk, kept as the raw 16-bit values), reduces min / max over its waves or lanes (or over the lanes of a K
 // block), and quantizes from the registers.  Same arithmetic, expression by expression, as the
 // two-kernel form, so the bytes and the scales are identical.
 #include "woq_common.h"
@@ -37,17 +37,20 @@ struct AqArgs {
   int given;  // the scales (and zero points) are inputs, shared by all rows: one per tensor or per K block
 };
 
-// NCH: 512-element chunks of a (padded) row that one wave holds; the four waves of a workgroup share one row (wave w takes chunks w,
-// w + 4, ...).  A wave with a whole row is one long dependent chain -- loads, extremes, an IEEE division for every element -- that
-// few other waves of its SIMD hide at any number of rows (M = 1, K = 4096: 6.5 us; M = 180, K = 7040, a scale per K block: 17.6 us, now 6.8; M = 2048, K = 4096:
-// 14.7, now 12.6).
-template <int NCH>
+// NCH: 512-element chunks of a (padded) row that one wave holds.  SPLIT: the four waves of a workgroup share one row (wave w takes
+// chunks w, w + 4, ...); else each has a row of its own.  A wave with a whole row is one long dependent chain -- loads, extremes, an
+// IEEE division for every element, and per K block the scale's own -- that few other waves of its SIMD hide (us, a wave / four
+// waves a row: M = 180, K = 7040, a scale per K block 17.6 / 6.8; one scale a row M = 1024, K = 4096 7.7 / 6.2, M = 16384, K = 11008 258 / 155).
+// Of short rows the four waves leave lanes without data, and the exchange through LDS costs more than the chain once the rows
+// themselves fill the chip (aq_wave_a_row).
+template <int NCH, bool SPLIT>
 __global__ __launch_bounds__(256) void act_quant_rows_kernel(const AqArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int64_t m = (int64_t)blockIdx.x;
+  const int64_t m = SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
+  if (!SPLIT && m >= a.M) return;
   // chunk held in register slot c
-  auto chunk_of = [&](int c) { return wave + 4 * c; };
+  auto chunk_of = [&](int c) { return SPLIT ? wave + 4 * c : c; };
   const uint16_t* const row = a.x + m * a.K;
   const bool bf16 = a.bf16 != 0, sym = a.sym != 0, per_k = a.block_lanes_log2 >= 0;
 
@@ -88,17 +91,19 @@ __global__ __launch_bounds__(256) void act_quant_rows_kernel(const AqArgs a) {
       mn[0] = fminf(mn[0], __shfl_xor(mn[0], off));
       mx[0] = fmaxf(mx[0], __shfl_xor(mx[0], off));
     }
-    // the four waves' extremes meet in LDS (every wave of the workgroup is here: same row)
-    __shared__ float smn[4], smx[4];
-    if (lane == 0) {
-      smn[wave] = mn[0];
-      smx[wave] = mx[0];
-    }
-    __syncthreads();
+    if constexpr (SPLIT) {
+      // the four waves' extremes meet in LDS (every wave of the workgroup is here: same row)
+      __shared__ float smn[4], smx[4];
+      if (lane == 0) {
+        smn[wave] = mn[0];
+        smx[wave] = mx[0];
+      }
+      __syncthreads();
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      mn[0] = fminf(mn[0], smn[w]);
-      mx[0] = fmaxf(mx[0], smx[w]);
+      for (int w = 0; w < 4; ++w) {
+        mn[0] = fminf(mn[0], smn[w]);
+        mx[0] = fmaxf(mx[0], smx[w]);
+      }
     }
   } else {
     // the lanes of one K block are 2^block_lanes_log2 consecutive lanes, aligned
@@ -117,7 +122,7 @@ __global__ __launch_bounds__(256) void act_quant_rows_kernel(const AqArgs a) {
   } else if (!per_k) {
     int32_t z = 0;
     row_p = aq_params(mn[0], mx[0], sym, &z);
-    if (lane == 0 && wave == 0) {
+    if (lane == 0 && (!SPLIT || wave == 0)) {
       a.scales[m] = row_p.s;
       if (!sym) a.zps[m] = z;
     }
@@ -279,16 +284,29 @@ __global__ void aq_shared_finalize_kernel(int groups, int sym, float* scales, in
   if (!sym) zps[i] = z;
 }
 
+// Rows of up to 3072 values with one scale a row, from the number of rows on at which a wave a row is as fast (us, a
+// wave / four waves a row: K = 512, M = 1024 3.6 / 3.6, 1536 3.8 / 4.2, 16384 13.1 / 20.4; K = 1024 4.1 / 4.0, 4.7 / 4.9, 20.4 / 26.0; K = 1536,
+// M = 1536 5.8 / 5.2, 2048 6.1 / 6.2, 16384 26.2 / 30.0; K = 2048 .. 3072, M = 8192 19.6 / 19.3 .. 27.3 / 26.7, 16384 32.8 / 34.3 ..
+// 45.5 / 47.1; K = 4096 58.2 / 57.7).  With a scale per K block four waves are the faster ones at every size (M = 16384, K = 512
+// 22.1 / 21.3).  Given scales, nothing to exchange: from 8192 rows of a single chunk on (K = 256, a scale a tensor 17.7 / 18.5 with the
+// statistics, per K block 20.1 / 20.7, M = 16384 24.6 / 25.9; K = 1024, M = 16384, per K block 33.1 / 33.3).
+static bool aq_wave_a_row(const AqArgs& a, int64_t chunks) {
+  if (a.given) return chunks <= 1 && a.M >= 8192;
+  return a.block_lanes_log2 < 0 && chunks <= 6 && a.M >= (chunks <= 2 ? 1536 : chunks == 3 ? 2048 : 12288);
+}
+
 // the quantization pass over whole rows, for scales computed here or given
 void aq_launch_quant(const AqArgs& a, hipStream_t st) {
   const int64_t chunks = (a.ldq + 511) / 512;
   const unsigned grid = (unsigned)a.M;
-  if (chunks <= 8)
-    act_quant_rows_kernel<2><<<grid, 256, 0, st>>>(a);
+  if (aq_wave_a_row(a, chunks))
+    act_quant_rows_kernel<8, false><<<(unsigned)((a.M + 3) / 4), 256, 0, st>>>(a);
+  else if (chunks <= 8)
+    act_quant_rows_kernel<2, true><<<grid, 256, 0, st>>>(a);
   else if (chunks <= 16)
-    act_quant_rows_kernel<4><<<grid, 256, 0, st>>>(a);
+    act_quant_rows_kernel<4, true><<<grid, 256, 0, st>>>(a);
   else
-    act_quant_rows_kernel<8><<<grid, 256, 0, st>>>(a);
+    act_quant_rows_kernel<8, true><<<grid, 256, 0, st>>>(a);
 }
 
 }  // namespace

@@ -1401,6 +1401,22 @@ def test_dynamic_quant_bit_exact(cuda, mode, M, K):
         assert np.array_equal(zp.cpu().numpy().reshape(-1), zp_ref.reshape(-1))
 
 
+@pytest.mark.parametrize("mode,M,K", [
+    (6, 1535, 1024), (6, 1537, 1024), (2, 1538, 264), (2, 2047, 1536), (6, 2049, 1032), (2, 12287, 2048), (6, 12290, 3072), (6, 12289, 3080),
+    (4, 8193, 512), (0, 8191, 520), (5, 8194, 256), (7, 2049, 512),
+])
+def test_dynamic_quant_of_many_short_rows_bit_exact(cuda, mode, M, K):
+    """A wave a row or four: on both sides of the bounds in rows and in 512-element chunks, row counts that are no multiple of four."""
+    k = _kernels()
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M + K + mode)).bfloat16()
+    q, s, zp = k.dynamic_quant(x.to(cuda), 128, mode)
+    q_ref, s_ref, zp_ref = O.dynamic_quantize_per_block(to_np_f32(x), 128, mode)
+    assert np.array_equal(s.cpu().numpy().reshape(-1), s_ref.reshape(-1))
+    assert np.array_equal(q.cpu().numpy(), q_ref)
+    if mode < 4:
+        assert np.array_equal(zp.cpu().numpy().reshape(-1), zp_ref.reshape(-1))
+
+
 @pytest.mark.parametrize("mode", [2, 3, 6, 7])
 @pytest.mark.parametrize(
     "M,K,block,dtype",
