@@ -203,16 +203,16 @@ enum { kFmtInt8, kFmtFp8, kFmtInt4, kFmtNf4 };
 template <int RT, int NTW>
 struct Fp32Decode {
   static constexpr int kRows = RT ? RT : 1;  // row tiles of a wave
-  // narrow layers and up to four rows: more of K in flight per workgroup (four row-blocks: the sums of 16 waves exceed 64 KiB of LDS)
-  static constexpr int kWaves = (RT <= 1 && NTW == 1) || (RT == 0 && NTW <= 3) ? 16 : 8;
+  static constexpr int kWaves = RT <= 1 && NTW == 1 ? 16 : 8;  // narrow layers: more of K in flight per workgroup
+  // (and up to four rows of a longer K, fp32_wide_workgroup; four row-blocks: the sums of 16 waves exceed 64 KiB of LDS)
   static constexpr int kMinWaves = RT <= 1 ? 4 : 2;              // per SIMD: 128 or 256 registers
 };
 
-template <int FMT, int RT, int NTW>
-__global__ __launch_bounds__((Fp32Decode<RT, NTW>::kWaves * 64), (Fp32Decode<RT, NTW>::kMinWaves))
+template <int FMT, int RT, int NTW, int W = Fp32Decode<RT, NTW>::kWaves>
+__global__ __launch_bounds__((W * 64), (Fp32Decode<RT, NTW>::kMinWaves))
 void woq_fp32_decode_kernel(const Fp32Args f) {
   using S = Fp32Decode<RT, NTW>;
-  constexpr int W = S::kWaves, R = S::kRows;
+  constexpr int R = S::kRows;
   constexpr bool kBytes = FMT == kFmtInt8 || FMT == kFmtFp8;
   constexpr int TK = kBytes ? kTileK8 : kTileK4;
   constexpr int CH = TK / 4;        // K values of a lane in a tile, taken 16 at a time
@@ -383,10 +383,30 @@ static int fp32_decode_ntw(int64_t NT, int64_t gy) {
   return best;
 }
 
+// Up to four rows, two or three row-blocks a workgroup: sixteen waves where they have tiles.  Up to eight tiles half of sixteen waves
+// only wait at the barrier (us, 8 / 16 waves: INT8 256 -> 8192, one row 3.3 / 3.6, INT4 1024 -> 8192 4.9 / 5.1, NF4 1024 -> 11008, four rows
+// 6.6 / 6.8); one and two rows of 8-bit weights, whose tiles are half as long, gain from more on (INT8 768 -> 8192, one row 11 %
+// slower with sixteen, two rows 5 %, 1024 -> 8192 7 % and even, four rows 2 % and 7 % faster).  Longer K: INT8 8192 -> 8192, one row 22.7 / 19.8,
+// FP8 4096 -> 11008, four rows 23.0 / 20.2, INT4 1280 -> 8192 5..8 % faster (single lengths lose: INT4 2304 -> 11008, one row 10.4 / 10.8).
+template <int FMT>
+static bool fp32_wide_workgroup(const Fp32Args& f) {
+  constexpr bool kBytes = FMT == kFmtInt8 || FMT == kFmtFp8;
+  return f.KT > (kBytes && f.M <= 2 ? (f.M == 1 ? 16 : 12) : 8);
+}
+
 template <int FMT, int RT>
 static void launch_fp32_decode_rows(const Fp32Args& f, unsigned gy, hipStream_t st) {
   const int ntw = fp32_decode_ntw(f.NT, gy);
   const dim3 grid((unsigned)((f.NT + ntw - 1) / ntw), gy);
+  if constexpr (RT == 0) {
+    if ((ntw == 2 || ntw == 3) && fp32_wide_workgroup<FMT>(f)) {
+      if (ntw == 2)
+        woq_fp32_decode_kernel<FMT, RT, 2, 16><<<grid, 1024, 0, st>>>(f);
+      else
+        woq_fp32_decode_kernel<FMT, RT, 3, 16><<<grid, 1024, 0, st>>>(f);
+      return;
+    }
+  }
 #define WOQ_FP32_DECODE(N) woq_fp32_decode_kernel<FMT, RT, N><<<grid, Fp32Decode<RT, N>::kWaves * 64, 0, st>>>(f)
   switch (ntw) {
     case 1: WOQ_FP32_DECODE(1); break;

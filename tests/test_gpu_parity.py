@@ -2342,6 +2342,9 @@ def test_fp32_compute(cuda, kind, M, K, N, G, bias):
     [
         # four-row matrix instructions, one to three row-blocks per workgroup (narrow: sixteen waves), ragged widths
         ("int8", 1, 4096, 512, -1), ("int8", 2, 1000, 4100, -1), ("int8", 4, 2048, 8720, 64), ("nf4", 4, 1024, 4112, 64), ("fp8", 3, 1024, 528, 128),
+        # ... two and three of them on eight and on sixteen waves, at the last K tile of the one and the first of the other
+        ("int8", 1, 1024, 8200, -1), ("int8", 1, 1088, 8200, -1), ("int8", 2, 768, 11000, -1), ("fp8", 2, 896, 11008, 128), ("int8", 3, 512, 8200, -1),
+        ("int4", 4, 1024, 8200, 32), ("nf4", 3, 1152, 11000, 64),
         # one, two, three and four row tiles, the first and last row of each; more waves than K tiles
         ("int8", 5, 4096, 528, -1), ("int8", 16, 192, 80, -1), ("int4", 17, 1408, 96, 32), ("int8", 32, 1001, 272, -1), ("int4", 33, 512, 4112, 128),
         ("int8", 48, 640, 8224, -1), ("nf4", 49, 512, 272, 64), ("fp8", 64, 1024, 4112, 128), ("int8", 64, 512, 12304, -1),
