@@ -739,8 +739,10 @@ class _MoeGroupedPlan:
         self.x_row = torch.empty(R, dtype=torch.int64, device=device)
         # slot tables [class][expert, first row, rows][S]: experts with few / up to 16 / up to 64 rows / exactly one row
         self.S = len(gate_ctx)
-        # (and slots for the rows of experts that are cut into several)
-        self.slots = torch.empty((4, 3, self.S + R // 16), dtype=torch.int32, device=device)
+        self.slots = torch.empty((4, 3, self.S), dtype=torch.int32, device=device)
+        # ... and with slots for the rows of experts that are cut into several.  (Tables of their own: every call clears its tables, which
+        # costs a layer of few experts and one token 1.5 of 24 us with 128 unused slots in each of them.)
+        self.cut_slots = torch.empty((4, 3, self.S + R // 16), dtype=torch.int32, device=device)
         self.row_of, self.slot_of = i32(), i32()
         self.tables = []
         for rows in infos:
@@ -781,15 +783,15 @@ class _MoeGroupedPlan:
             have = _MOE_ROWS[key] = (mk(N1), mk(N1), mk(H))
         return have
 
-    def group_struct(self, linear, cls, f16_scales, gather, sz=False, tiles=False, pair=False):
+    def group_struct(self, linear, cls, f16_scales, gather, sz=False, table="slots", pair=False):
         """Device copy of the woq_hip_moe_group of one launch (built once).  ``sz``: for the integer-weight decode
-        kernels, with the (scale, zero) dword tables in place of the scales.  ``tiles``: over the slots of
-        woq_hip_moe_route_tiles.  ``pair``: with the next linear's tables as the second set."""
-        key = (linear, cls, f16_scales, gather, sz, tiles, pair)
+        kernels, with the (scale, zero) dword tables in place of the scales.  ``table``: the slot tables, ``slots``, ``cut_slots`` or
+        ``tiles`` (those of woq_hip_moe_route_tiles).  ``pair``: with the next linear's tables as the second set."""
+        key = (linear, cls, f16_scales, gather, sz, table, pair)
         st = self.structs.get(key)
         if st is None:
             ptr = lambda x: 0 if x is None else x.data_ptr()
-            slots, x_row = (self.tiles["slots"], self.tiles["x_row"]) if tiles else (self.slots, self.x_row)
+            slots, x_row = (self.tiles["slots"], self.tiles["x_row"]) if table == "tiles" else (getattr(self, table), self.x_row)
             fields = [ptr(slots[cls, i]) for i in range(3)] + [ptr(x_row) if gather else 0]
             for t in (self.tables[linear], self.tables[linear + 1] if pair else None):
                 if t is None:
@@ -802,11 +804,11 @@ class _MoeGroupedPlan:
             self.structs[key] = st
         return st
 
-    def launch(self, lib, p, linear, src, dst, cls, bound, slots, x_dtype, sz, tiles, tile_rows=0, fusion=_lib.FUSE_NONE, other=None, pair=False):
+    def launch(self, lib, p, linear, src, dst, cls, bound, slots, x_dtype, sz, table, tile_rows=0, fusion=_lib.FUSE_NONE, other=None, pair=False):
         """One linear over the slots of a size class (``pair``: gate and up as one).  ``p`` has the call's constant fields, ``sz`` per
-        linear whether it runs on the integer-weight decode kernels; ``tiles``: the slots are those of woq_hip_moe_route_tiles (all
+        linear whether it runs on the integer-weight decode kernels; ``table``: whose slots (``tiles``: all
         its classes, those with ``tile_rows`` on the prefill kernel)."""
-        key = (linear, cls, bound, x_dtype, sz[linear], tiles, tile_rows, pair)
+        key = (linear, cls, bound, x_dtype, sz[linear], table, tile_rows, pair)
         call = self.calls.get(key)
         if call is None:  # what a launch of these has in every call
             sh, t, f16 = self.shapes[linear], self.tables[linear], _f16_regime(self.shapes[linear]["lowp"], x_dtype, bound)
@@ -820,22 +822,22 @@ class _MoeGroupedPlan:
                 return False
             flags |= _lib.MOE_PAIR
         if group is None:
-            group = call[-1] = self.group_struct(linear, cls, f16, linear < 2, sz[linear], tiles, pair).data_ptr()
+            group = call[-1] = self.group_struct(linear, cls, f16, linear < 2, sz[linear], table, pair).data_ptr()
         rc = lib.woq_hip_moe_linear(p, group, slots, tile_rows, flags)
         if rc != 0:
             _lib.check(rc, "woq_linear_grouped")
         return True
 
-    def gate_up(self, lib, p, x, act, inter, cls, bound, slots, sz, tiles, tile_rows=0):
+    def gate_up(self, lib, p, x, act, inter, cls, bound, slots, sz, table, tile_rows=0):
         """silu(gate(x)) * up(x) of a size class: in one launch where there is one, else in two."""
         x_dtype = x.dtype
         key = (bound, tile_rows, x_dtype, sz[0])
         if self.pair_ok and sz[0] == sz[1] and key not in self.unpaired:
-            if self.launch(lib, p, 0, x, inter, cls, bound, slots, x_dtype, sz, tiles, tile_rows, pair=True):
+            if self.launch(lib, p, 0, x, inter, cls, bound, slots, x_dtype, sz, table, tile_rows, pair=True):
                 return
             self.unpaired.add(key)  # (asked once)
-        self.launch(lib, p, 0, x, act, cls, bound, slots, x_dtype, sz, tiles, tile_rows, _lib.FUSE_SILU)
-        self.launch(lib, p, 1, x, inter, cls, bound, slots, x_dtype, sz, tiles, tile_rows, _lib.FUSE_MUL, act)
+        self.launch(lib, p, 0, x, act, cls, bound, slots, x_dtype, sz, table, tile_rows, _lib.FUSE_SILU)
+        self.launch(lib, p, 1, x, inter, cls, bound, slots, x_dtype, sz, table, tile_rows, _lib.FUSE_MUL, act)
 
 
 def _moe_plan(gate_ctx, up_ctx, down_ctx, device, stream):
@@ -911,6 +913,8 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
     cut = T <= 16 < most and plan.S <= _lib.MOE_TILES_EXPERTS
     if cut:
         launches = [c for c in launches if c[0] != 2]
+    table = "cut_slots" if cut else "slots"
+    slots = getattr(plan, table)
     lib = _lib.load()
     ids = topk_ids.to(torch.int64).contiguous()
     rw = routing_weights.contiguous()
@@ -922,8 +926,7 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
         act, inter, y = plan.buffers(x.dtype, raw_stream)  # calls on one stream follow each other
         stream = _kernels._stream()
         _lib.check(lib.woq_hip_moe_route(ids.data_ptr(), T, topk, len(gate_ctx), split, 16, 2 if each else int(single) + (_lib.MOE_CUT if cut else 0),
-                                         plan.slots.shape[2],
-                                         plan.x_row.data_ptr(), plan.slots.data_ptr(), plan.row_of.data_ptr(),
+                                         slots.shape[2], plan.x_row.data_ptr(), slots.data_ptr(), plan.row_of.data_ptr(),
                                          plan.slot_of.data_ptr(), stream), "moe_route")
         nslots = R if each else min(R, plan.S)  # experts that can have tokens: the tables are dense
         slots_of = lambda cls: nslots + R // 16 if cut and cls == 1 else nslots
@@ -934,9 +937,9 @@ def _deepseek_moe_grouped(hidden_states, topk_ids, gate_ctx, up_ctx, down_ctx, r
         p.lowp_mode = lowp
         p.act_quant_mode = -1
         for cls, bound in launches:
-            plan.gate_up(lib, p, x, act, inter, cls, bound, slots_of(cls), [cls == 3 or (cls == 0 and single)] * 3, False)
+            plan.gate_up(lib, p, x, act, inter, cls, bound, slots_of(cls), [cls == 3 or (cls == 0 and single)] * 3, table)
         for cls, bound in launches:
-            plan.launch(lib, p, 2, inter, y, cls, bound, slots_of(cls), x.dtype, [cls == 3 or (cls == 0 and single)] * 3, False)
+            plan.launch(lib, p, 2, inter, y, cls, bound, slots_of(cls), x.dtype, [cls == 3 or (cls == 0 and single)] * 3, table)
         _lib.check(lib.woq_hip_moe_combine_rows(out.data_ptr(), code, T, H, y.data_ptr(), rw.data_ptr(), topk,
                                                 plan.row_of.data_ptr(), plan.slot_of.data_ptr(), 0, stream), "moe_combine_rows")
     return out
@@ -1022,9 +1025,9 @@ def _deepseek_moe_tiles(plan, x, topk_ids, routing_weights, host_ids, raw_stream
         p.act_quant_mode = -1
         classes = [(cls, bound, [cls == 0 and ok for ok in few], rows if cls == 3 else 0) for cls, bound in ((0, 4), (1, 16), (2, 64), (3, rows)) if used[cls]]
         for cls, bound, sz, tile in classes:
-            plan.gate_up(lib, p, x, act, inter, cls, bound, used[cls], sz, True, tile)
+            plan.gate_up(lib, p, x, act, inter, cls, bound, used[cls], sz, "tiles", tile)
         for cls, bound, sz, tile in classes:
-            plan.launch(lib, p, 2, inter, y, cls, bound, used[cls], x.dtype, sz, True, tile)
+            plan.launch(lib, p, 2, inter, y, cls, bound, used[cls], x.dtype, sz, "tiles", tile)
         _lib.check(lib.woq_hip_moe_combine_rows(out.data_ptr(), code, T, H, y.data_ptr(), rw.data_ptr(), topk,
                                                 buf["row_of"].data_ptr(), buf["slot_of"].data_ptr(), 0, stream), "moe_combine_rows")
     return out
