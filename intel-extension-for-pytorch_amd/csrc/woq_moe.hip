@@ -191,10 +191,9 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const int64_t* __restric
   for (int i = valid + threadIdx.x; i < R; i += blockDim.x) x_row[i] = 0;
 }
 
-// The same routing as a counting sort by one workgroup of W waves, W = 16 or 4: every layer of at most 1024 experts but those whose single
-// token gives every entry a slot of its own.  A wave numbers the entries of its part of the table, 64 at a time: the lanes that name
-// the same expert are found with one ballot per bit of an expert's number, and a count per (wave, expert) in LDS carries over from one
-// 64 to the next.  A scan over the experts and their waves' counts then gives every entry its place.
+// The same routing as a counting sort by one workgroup of W waves, W = 16 or 4: layers of at most 1024 experts with more than 16
+// entries.  A wave numbers the entries of its part of the table, 64 at a time: the lanes that name the same expert are found with one
+// ballot per bit of an expert's number, and a count per (wave, expert) in LDS carries over from one 64 to the next.  A scan over the experts and their waves' counts then gives every entry its place.
 // Bound: latencies -- the read of the ids, some LDS round trips, the stores.  4096 entries over 32 experts 24 -> 15 us, 128 entries
 // 9.9 -> 5.3 us (the walk of a wave over all entries for each of its experts, or every entry compared with every other).
 //   slots   [4 classes][expert, first row, rows][S].  TILES: 0: experts with fewer than split_lo rows, 1: at most split_mid, 2: at most
@@ -442,7 +441,10 @@ int launch_moe_route(const int64_t* ids, int64_t T, int64_t topk, int64_t expert
   const int64_t R = T * topk;
   if (R == 0) return 0;
   if (R > kMoeRouteMax) return set_error("moe_route: at most %d (token, slot) entries, got %lld", kMoeRouteMax, (long long)R);
-  if (use_single != 2 && (experts <= kMoeTilesExperts || (use_single & WOQ_HIP_MOE_CUT)))
+  // up to 16 entries every one compared with every other is faster than the sort with its scans over the experts (8 and 32 experts, us,
+  // compared / sorted: 2 entries 2.8 / 4.4 and 2.9 / 4.4, 8 3.2 / 4.3 and 3.3 / 4.5, 16 3.8 / 4.4 and 4.0 / 4.5, 24 4.5 / 4.5, 48 5.1 / 4.4)
+  const bool compared = (R <= 16 || experts > kMoeTilesExperts) && !(use_single & WOQ_HIP_MOE_CUT);
+  if (use_single != 2 && !compared)
     moe_route_sort_kernel<4, false><<<1, 256, 0, st>>>(ids, (int)R, (int)topk, (int)experts, (int)split_lo, (int)split_mid, 0, use_single, (int)S,
                                                        x_row, slots, row_of, slot_of);
   else

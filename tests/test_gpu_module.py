@@ -780,7 +780,7 @@ def test_moe_route_against_the_oracle_token_lists(cuda):
 
     lib = _lib.load()
     g = torch.Generator().manual_seed(5)
-    for T, topk, E, split in ((1, 8, 64, 5), (16, 8, 32, 5), (64, 6, 9, 5), (33, 4, 7, 0), (256, 8, 300, 5)):
+    for T, topk, E, split in ((1, 8, 64, 5), (2, 8, 16, 5), (4, 4, 9, 5), (6, 3, 8, 5), (16, 8, 32, 5), (64, 6, 9, 5), (33, 4, 7, 0), (256, 8, 300, 5)):
         ids = torch.stack([torch.randperm(E, generator=g)[:topk] for _ in range(T)])
         if T >= 16:
             ids[3, 1], ids[7, 0] = -1, E + 3  # not experts
