@@ -103,8 +103,11 @@ static double slot_weight(int64_t rows, int tile_rows, bool chained) {
   if (tile_rows == 128 && rows > 64) return 1.0;
   return (0.4 + 0.0047 * (double)((rows + 31) / 32 * 32)) * (chained && rows > 128 ? 1.12 : 1.0);
 }
-// Estimated microseconds of one grouped launch.  Slots of 160 are alike (an expert's rows lie evenly in them), so they run in whole
-// generations; of those of 128 the low ones fill what the tall ones leave.  From INT4 g128 / g64 / g32, us of a layer with 64, 128 and 160 rows a
+// Estimated microseconds of one grouped launch.  Slots of 160 are much alike (an expert's rows lie evenly in them), so they run in whole
+// generations of the mean slot, the last of which ends with the tallest; of those of 128 the low ones fill what the tall ones
+// leave.  (Without the tallest 160 rows were taken for experts of uneven sizes, where 128 are faster: of 159 layers of 8 to 64 experts with 60
+// to 340 rows in the mean 15 by 1..12 %, now 2; 64 / 128 / 160 rows, us: 8 x 70..147 4352 -> 2816 148 / 123 / 138, 16 x 34..513 2048 -> 7168
+// 473 / 411 / 433, 8 x 34..282 4096 -> 14336 751 / 654 / 694.)  From INT4 g128 / g64 / g32, us of a layer with 64, 128 and 160 rows a
 // slot, experts x rows: 32 x 128 7168 -> 2048 606 / 537 / 494 and 3072 -> 1024 205 / 218 / 181, 16 x 100 4096 -> 2048 190 / 164 / 161, 8 x 256
 // 7168 -> 2048 312 / 295 / 261, 16 x 250 5120 -> 1536 343 / 313 / 319, 8 x 128 4096 -> 1024 123 / 130 / 147 and 7168 -> 1024 158 / 177 / 189,
 // 8 x 75 2048 -> 512 112 / 119 / 123, 8 x 100 5120 -> 2048 144 / 149 / 149, 8 x 450 1024 -> 2048 151 / 152 / 157.
@@ -112,16 +115,18 @@ static double grouped_us(const int64_t* counts, int64_t experts, int64_t K, int6
   const StepTimes& t = step_times(wbits, 0, 0);
   const double steps = (double)((K + kTileK4 - 1) / kTileK4);
   int64_t slots = 0;
-  double weight = 0;
+  double weight = 0, tallest = 0;
   for (int64_t e = 0; e < experts; ++e) {
     const int64_t n = counts[e];
     if (n <= 64) continue;
     const bool chained = tile_rows == 160 && (n + 63) / 64 <= chain_row_tiles(N_own) && chain_steps(K, N_own, wbits, (int)((n + 63) / 64));
     const int64_t own = (n + tile_rows - 1) / tile_rows;
     slots += own;
-    if (tile_rows == 160)
-      weight += (double)own * slot_weight((n + own - 1) / own, 160, chained);
-    else
+    if (tile_rows == 160) {
+      const double each = slot_weight((n + own - 1) / own, 160, chained);
+      weight += (double)own * each;
+      tallest = std::max(tallest, each);
+    } else
       weight += (double)(n / tile_rows) + (n % tile_rows ? slot_weight(n % tile_rows, 128, false) : 0.0);
   }
   if (tile_rows == 64) {
@@ -131,8 +136,9 @@ static double grouped_us(const int64_t* counts, int64_t experts, int64_t K, int6
     return (steps * t.t42[most - 1] + kSlotUs42) * ((double)w / (256 * most) + 0.25);
   }
   const double cols = (double)((N + 255) / 256);
-  const double each = tile_rows == 160 ? weight / (double)slots : 1.0, w = cols * (tile_rows == 160 ? (double)slots : weight);
-  return (steps * (w <= 192 ? t.t8 : t.t8f) * 1.05 * each + kSlotUs8) * std::ceil(w / 256);
+  const double mean = weight / (double)slots, w = cols * (tile_rows == 160 ? (double)slots : weight), gens = std::ceil(w / 256);
+  const double us = steps * (w <= 192 ? t.t8 : t.t8f) * 1.05;
+  return tile_rows == 160 ? us * (mean * gens + tallest - mean) + kSlotUs8 * gens : (us + kSlotUs8) * gens;
 }
 int gemm_w4_tile_rows(const int64_t* counts, int64_t experts, const int64_t* K, const int64_t* N, const int* wbits) {
   int best = 64;

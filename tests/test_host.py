@@ -424,6 +424,21 @@ def test_moe_prompt_slots_of_160_rows_need_three_linears_of_4_bits():
         assert pick(*types) in (64, 128), types
 
 
+def test_moe_prompt_slots_at_measured_points():
+    """Rows of a slot, INT4 (64 / 128 / 160 rows, us): experts of uneven sizes keep 128 rows, even ones take 160."""
+    from ipex_amd import _lib, ops
+
+    def pick(H, I, counts):
+        return ops._moe_tile_rows([dict(K=H, N=I, wd=_lib.DTYPE_INT4)] * 2 + [dict(K=I, N=H, wd=_lib.DTYPE_INT4)], counts)
+
+    assert pick(4352, 2816, [90, 147, 109, 117, 121, 70, 72, 138]) == 128  # 148 / 123 / 138
+    assert pick(2048, 7168, [440, 287, 130, 56, 167, 350, 86, 106, 114, 513, 128, 134, 215, 212, 104, 34]) == 128  # 473 / 411 / 433
+    assert pick(4096, 14336, [200, 282, 156, 119, 251, 273, 49, 34]) == 128  # 751 / 654 / 694
+    assert pick(3072, 1024, [141, 57, 273, 217, 308, 121, 54, 331, 80, 12, 176, 184, 97, 477, 138, 178]) == 128  # 152 / 141 / 150
+    assert pick(7168, 2048, [128] * 16 + [153, 110] * 8) == 160  # 598 / 540 / 497
+    assert pick(4352, 2816, [66, 75, 84, 84, 78, 68, 83, 60]) == 160  # 13 % below 128
+
+
 def test_moe_layers_on_other_devices_and_streams_do_not_wait_for_each_other():
     from ipex_amd import ops
 
