@@ -313,10 +313,11 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
   // silu(gate(x)) * up(x), in one launch where the library has one (woq_hip_linear_pair), else in the two that the ops
   // woq_linear_silu and woq_linear_mul make
   static Tensor run_pair(WoqLinearOpContext& gate, WoqLinearOpContext& up, const Tensor& x_in) {
+    Tensor x2 = x_in;
     const int64_t M = x_in.numel() > 0 && x_in.size(-1) == gate.K_ ? x_in.numel() / gate.K_ : 0;
     if (M >= 1 && gate.K_ == up.K_ && gate.N_ == up.N_ && !gate.g_src_.defined() && !up.g_src_.defined() &&
         gate.packed_.device() == x_in.device() && up.packed_.device() == x_in.device() && x_in.scalar_type() == at::kBFloat16) {
-      Tensor x2 = x_in.is_contiguous() ? x_in : x_in.contiguous();
+      if (!x2.is_contiguous()) x2 = x2.contiguous();
       if ((uintptr_t)x2.data_ptr() % 16) x2 = x2.clone();  // the kernels read activation rows with 16-byte loads
       std::vector<int64_t> out_sizes = x_in.sizes().vec();
       out_sizes.back() = gate.N_;
@@ -348,7 +349,7 @@ class WoqLinearOpContext : public torch::CustomClassHolder {
         return out;
       }
     }
-    return up.run(x_in, WOQ_HIP_FUSE_MUL, {gate.run(x_in, WOQ_HIP_FUSE_SILU, {})});
+    return up.run(x2, WOQ_HIP_FUSE_MUL, {gate.run(x2, WOQ_HIP_FUSE_SILU, {})});  // (x2: copied once where rows had to be)
   }
 
   int64_t handle() const { return handle_; }

@@ -1629,6 +1629,23 @@ def test_gate_and_up_of_prompts_in_one_launch(cuda, M, K, N, G):
     assert torch.equal(ops.woq_linear_silu_mul(odd, hg, hu), got.view(1, M, N))
 
 
+@pytest.mark.parametrize("odd", ["strided", "misaligned"])
+def test_gate_and_up_in_two_launches_copy_their_rows_once(cuda, odd):
+    """A prompt that keeps two launches (K of two steps, not shared): one copy of rows that are not contiguous or not aligned, and two outputs."""
+    ipex = _ipex()
+    M, K, N = 70, 256, 48
+    gate, up = (_woq_module(ipex, K, N, seed=s) for s in (46, 47))
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).bfloat16().to(cuda)
+    view = x.t().contiguous().t() if odd == "strided" else torch.cat([x.new_zeros(1), x.flatten()])[1:].view(M, K)
+    ops = torch.ops.torch_ipex
+    hg, hu = gate._op_context.get_data_handle(), up._op_context.get_data_handle()
+    want = ops.woq_linear_mul(x, hu, [ops.woq_linear_silu(x, hg)])
+    first = torch.cuda.memory_stats()["allocation.all.allocated"]
+    got = ops.woq_linear_silu_mul(view, hg, hu)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - first == 3
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("lowp", ["BF16", "INT8"])
 @pytest.mark.parametrize("M,K,N", [(65, 256, 31), (130, 384, 979), (64, 512, 16387), (200, 4096, 770)])
 def test_prompts_of_odd_widths_round_each_post_op_once(cuda, lowp, M, K, N):
