@@ -1608,20 +1608,63 @@ def test_prompts_share_k_whatever_its_length(cuda, M, K, N, weight_dtype, G, low
         assert torch.equal(torch.ops.torch_ipex.ipex_woq_linear(x, handle), got)
 
 
-@pytest.mark.parametrize("M,K,N,G", [(65, 1024, 512, 128), (128, 1152, 528, 32), (129, 4096, 1040, 64), (200, 2048, 3000, 128), (64 * 5, 1024, 8208, -1),
-                                     (512, 4096, 11008, 128)])
-def test_gate_and_up_of_prompts_in_one_launch(cuda, M, K, N, G):
+def _pair_scratch(M, K, N, G):
+    """What the library says of gate and up of a gated MLP (host arithmetic: no pointer is followed): None for two launches, else the bytes
+    with which the one launch shares K."""
+    import ctypes
+
+    from ipex_amd import _lib
+
+    p = [_lib.LinearParams(), _lib.LinearParams()]
+    for q in p:
+        q.struct_size = ctypes.sizeof(_lib.LinearParams)
+        q.M, q.K, q.N, q.weight_dtype, q.group_size, q.lowp_mode = M, K, N, _lib.DTYPE_INT4, G, _lib.LOWP_BF16
+        q.x_dtype = q.out_dtype = _lib.ACT_BF16
+        q.x = q.out = q.qweight = q.scale_zero_bf16 = 4096
+    lib, refs = _lib.load(), [ctypes.byref(q) for q in p]
+    return lib.woq_hip_linear_pair_scratch_bytes(*refs) if lib.woq_hip_linear_pair_applies(*refs) else None
+
+
+@pytest.mark.parametrize("sym", [False, True])
+@pytest.mark.parametrize("M,K,N,G,kind", [
+    (65, 1024, 512, 128, "one"), (128, 1152, 528, 32, "one"), (200, 2048, 3000, 128, "one"), (64 * 5, 1024, 8208, -1, "one"), (2048, 1024, 528, 128, "one"),
+    (129, 4096, 1040, 64, "shared"), (200, 7168, 2064, 32, "shared"), (512, 7168, 2048, 128, "shared"),  # 64 x 128 tiles in four, three and two
+    (1000, 7168, 2048, 128, "shared"),  # 128 x 256 in two
+    (65, 896, 512, 128, "two"), (65, 1024, 496, 128, "two"), (512, 4096, 11008, 128, "two"),
+])
+def test_gate_and_up_of_prompts_in_one_launch(cuda, M, K, N, G, kind, sym):
     """Beyond 64 rows: one launch over both weights, with or without shared K, against two launches (fp32 sums in another order at most:
-    flips of a last bf16 bit, 2e-3 in the 2-norm); every call has the same bits."""
+    flips of a last bf16 bit, 2e-3 in the 2-norm); every call has the same bits.  One launch makes the output and, where it shares K,
+    its scratch; two make an intermediate tensor besides."""
     from helpers import rel_l2, to_np_f32
 
     ipex = _ipex()
-    gate, up = (_woq_module(ipex, K, N, "INT4", G, "BF16", bias=True, seed=s) for s in (44, 45))
+    if sym:
+        from ipex_amd import _lib
+
+        g = torch.Generator().manual_seed(K + N)
+        groups = K // G if G > 0 else 1
+        mk = lambda: torch.ops.ipex_prepack.weight_only_qlinear_prepack(
+            torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8).to(cuda), _lib.DTYPE_INT4, [N, K],
+            (torch.rand(N, groups, generator=g) * 0.002 + 0.001).to(cuda), None, torch.randn(N, generator=g).to(cuda), None, None, G, _lib.LOWP_BF16, -1, False)
+        contexts = mk(), mk()
+    else:
+        mods = [_woq_module(ipex, K, N, "INT4", G, "BF16", bias=True, seed=s) for s in (44, 45)]
+        contexts = [m._op_context for m in mods]
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(cuda)
     ops = torch.ops.torch_ipex
-    hg, hu = gate._op_context.get_data_handle(), up._op_context.get_data_handle()
+    hg, hu = (c.get_data_handle() for c in contexts)
     want = ops.woq_linear_mul(x, hu, [ops.woq_linear_silu(x, hg)])
+    scratch = _pair_scratch(M, K, N, G)
+    assert kind == ("two" if scratch is None else "shared" if scratch else "one")
+    count = lambda: [torch.cuda.memory_stats()[k] for k in ("allocation.all.allocated", "requested_bytes.all.allocated")]
+    before = count()
     got = ops.woq_linear_silu_mul(x, hg, hu)
+    made, size = (b - a for a, b in zip(before, count()))
+    if scratch is not None:
+        assert (made, size) == (1 + (scratch > 0), 2 * M * N + scratch)
+    else:
+        assert made >= 2 and size >= 4 * M * N
     assert rel_l2(to_np_f32(got), to_np_f32(want)) < 2e-3
     for _ in range(5):
         assert torch.equal(ops.woq_linear_silu_mul(x, hg, hu), got)
