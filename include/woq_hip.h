@@ -283,9 +283,9 @@ int64_t woq_hip_linear_split_k_workspace_bytes(int64_t M, int64_t N);
 
 /* The same size for the problems on which woq_hip_linear shares K between workgroups BY ITSELF (force_kernel 0):
  * few output tiles and a long K -- 5..32 rows with K >= 8192 and N <= 4096 in the floating-point modes, more than
- * 64 rows with K >= 4096, either at most 1024 rows or at most 128 tiles of 64 rows x 128 columns (lowp_mode INT8: the latter) -- and 0 for every other problem, where scratch and
- * counters would go unused.  A caller that allocates per call asks this function; there is no second copy of the
- * rule to keep in step.  No counterpart in the reference. */
+ * 64 rows with K >= 4096, either at most 1024 rows or at most 128 tiles of 64 rows x 128 columns (lowp_mode INT8: the latter) -- and 0
+ * for every other size.  By the sizes alone: woq_hip_linear_scratch_bytes below, which a caller that allocates per call asks, leaves
+ * out what runs on other kernels and knows shorter K.  No counterpart in the reference. */
 int64_t woq_hip_linear_auto_split_k_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t lowp_mode);
 
 /* The scratch with which woq_hip_linear (force_kernel 0) shares K between workgroups on the call p, 0 where the kernel that the call
@@ -307,9 +307,11 @@ int woq_hip_linear(const woq_hip_linear_params* p);
 /* The front half of a gated MLP in one launch: out = silu(x Wg^T + bg) * (x Wu^T + bu), rounded as woq_hip_linear on `gate` with the
  * silu and then on `up` with the mul round it (Linear2SiluMul).  The K sums may be added in another order with 17 to 32 rows, with 5
  * to 16 rows where woq_hip_linear shares K (woq_hip_linear_auto_split_k_workspace_bytes), and with 33 to 64 rows and more than
- * 16384 columns, where it takes the prefill kernel.  Both parameter sets name the same x, out, sizes, modes and stream, no post-op.  For the problems of woq_hip_linear_pair_applies: INT4 and INT8 weights with their scale_zero_bf16
- * tables (and scale_zero_f16x2 for rows that compute in fp16), bf16 rows, lowp_mode BF16 or NONE; beyond 64 rows INT4 weights without a dense copy, K of at least
- * 1024 and a multiple of 128, at least 512 columns, where the estimated time is the lower one (K may be shared otherwise than in two launches). */
+ * 16384 columns, where it takes the prefill kernel.  Both parameter sets name the same x, out, sizes, modes and stream, no post-op.
+ * For the problems of woq_hip_linear_pair_applies: INT4 and INT8 weights with their scale_zero_bf16 tables (and scale_zero_f16x2 for
+ * rows that compute in fp16), bf16 rows, lowp_mode BF16 or NONE; beyond 64 rows INT4 weights without a dense copy, K of at least 1024
+ * and a multiple of 128, at least 512 columns, where the estimated time is the lower one (K may be shared otherwise than in two
+ * launches). */
 int woq_hip_linear_pair_applies(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);
 int woq_hip_linear_pair(const woq_hip_linear_params* gate, const woq_hip_linear_params* up);
 
@@ -408,8 +410,8 @@ int woq_hip_moe_scale_add_rows(void* out, int dtype, int64_t T, int64_t H, const
  *   larger M on the others; M <= 16 and M > 16 also select a kernel with one or four row tiles, hence the size classes); p's weight, scale, zero
  *   point and bias pointers are ignored -- except that a non-NULL scale_zero_f16x2 says that the group's scales table
  *   holds the experts' (fp16 scale, fp16 128 + zero) dword tables: the call then runs the single-row decode kernel
- *   (M must be at most 4: the classes of experts with exactly one row and with fewer than five; 4-bit weights in groups of 32, 64 or 128 * 2^k, K a multiple of 256,
- *   fp16 compute).  x: the rows the slots read, out / others[0]: [routed rows, N].  group: DEVICE
+ *   (M must be at most 4: the classes of experts with exactly one row and with fewer than five; 4-bit weights in groups of 32, 64 or
+ *   128 * 2^k, K a multiple of 256, fp16 compute).  x: the rows the slots read, out / others[0]: [routed rows, N].  group: DEVICE
  *   pointer to a woq_hip_moe_group.  Rows of a slot are row0 .. row0 + rows - 1 of out; they read row x_row[row] of x,
  *   or the same row when x_row is NULL.  Needs what the dequantizing decode kernel needs: K a multiple of the weight tile,
  *   a power-of-two or per-channel group size, an even number of 16-column blocks, rows in the compute type (bf16 rows

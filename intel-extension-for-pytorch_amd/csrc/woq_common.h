@@ -56,6 +56,9 @@ __device__ __forceinline__ uint16_t f32_to_f16_bits(float f) {
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t b) {
   return (float)bitcast<_Float16>(b);
 }
+__device__ __forceinline__ float act_bits_to_f32(uint16_t bits, int dtype) {
+  return dtype == WOQ_HIP_ACT_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
+}
 
 // Nibble position of K-element e (0..7) inside one dword of the packed INT4 layout.
 __host__ __device__ __forceinline__ constexpr int nibble_pos(int e) {
@@ -254,6 +257,20 @@ __device__ __forceinline__ void store_act(void* p, int dtype, int64_t i, float v
     ((uint16_t*)p)[i] = f32_to_f16_bits(v);
   else
     ((float*)p)[i] = v;
+}
+
+// Post-op of epilogue_store on a value of the activation dtype; the result is rounded by the store.
+__device__ __forceinline__ float post_op(float y, int fusion, int act_dtype, float other0, float other1) {
+  switch (fusion) {
+    case WOQ_HIP_FUSE_GELU_ERF: return gelu_erf(y);
+    case WOQ_HIP_FUSE_GELU_TANH: return gelu_tanh(y);
+    case WOQ_HIP_FUSE_RELU: return y > 0.0f ? y : 0.0f;
+    case WOQ_HIP_FUSE_SILU: return silu(y);
+    case WOQ_HIP_FUSE_ADD: return y + other0;
+    case WOQ_HIP_FUSE_ADD_ADD: return round_to_act(y + other0, act_dtype) + other1;
+    case WOQ_HIP_FUSE_MUL: return y * other0;
+    default: return y;
+  }
 }
 
 // Epilogue shared by every kernel: bias + regime rounding, optional post-op, store.

@@ -184,8 +184,8 @@ __global__ __launch_bounds__(256) void woq_fp32_kernel(const Fp32Args f) {
     }
 }
 
-// Few rows (decode), and prompts of any length where K is long (64 rows a workgroup): a workgroup owns NTW row-blocks of 16 output columns for all K, its W waves split
-// K, and every operand goes from memory straight into the registers that feed the MFMA.  A packed weight tile already
+// Few rows (decode), and prompts of any length where K is long (64 rows a workgroup): a workgroup owns NTW row-blocks of 16 output
+// columns for all K, its W waves split K, and every operand goes from memory straight into the registers that feed the MFMA.  A packed weight tile already
 // has the B layout of v_mfma_f32_16x16x4_f32: lane r + 16 c holds consecutive K values of row r, so MFMA number e of a
 // tile takes each lane's value e, and the A operand of lane m + 16 c is x[m] at the same K, read as 16-byte pieces.
 // Up to four rows (RT 0) the MFMA is v_mfma_f32_4x4x1_16b: its block l / 4 has the columns 4 (l / 4 % 4) .. + 3 and

@@ -125,24 +125,6 @@ __device__ __forceinline__ u4 g4_dequant_m(uint32_t d, const G4Masks& k, uint32_
   return r;
 }
 
-__device__ __forceinline__ float act_bits_to_f32(uint16_t bits, int dtype) {
-  return dtype == WOQ_HIP_ACT_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
-}
-
-// Post-op of epilogue_store on a value of the activation dtype; the result is rounded by the store.
-__device__ __forceinline__ float post_op(float y, int fusion, int act_dtype, float other0, float other1) {
-  switch (fusion) {
-    case WOQ_HIP_FUSE_GELU_ERF: return gelu_erf(y);
-    case WOQ_HIP_FUSE_GELU_TANH: return gelu_tanh(y);
-    case WOQ_HIP_FUSE_RELU: return y > 0.0f ? y : 0.0f;
-    case WOQ_HIP_FUSE_SILU: return silu(y);
-    case WOQ_HIP_FUSE_ADD: return y + other0;
-    case WOQ_HIP_FUSE_ADD_ADD: return round_to_act(y + other0, act_dtype) + other1;
-    case WOQ_HIP_FUSE_MUL: return y * other0;
-    default: return y;
-  }
-}
-
 // GROUPED (mixture of experts): the row tile of a workgroup is a slot of the routing tables -- at most G4_BM routed rows of
 // one expert, whose tensors come from the group's pointer tables; a slot without an expert ends at once.
 // 32 experts 7168 -> 2048 -> 7168, top-8, 512 tokens: 3738 us with three launches per expert (each on 32 to 192 workgroups),

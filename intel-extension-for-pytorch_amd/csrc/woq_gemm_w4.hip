@@ -86,8 +86,8 @@ static TilePlan plan_tiles(int64_t M, int64_t N, int ksteps, const StepTimes& t,
 }
 static const StepTimes& step_times(int wbits, int nf4, int fp8) { return wbits == 8 ? (fp8 ? kStepsFp8 : kSteps8) : nf4 ? kStepsNf4 : kSteps4; }
 
-// K steps of a chain for an expert (whose own launch has scratch from kSplitKPrefillMinK on) of 64 (i - 1) < rows <= 64 i rows, i = 2 ..: as its own launch shares them with the scratch
-// that woq_hip_linear_auto_split_k_workspace_bytes asks for (0: one chain).
+// K steps of a chain for an expert (whose own launch has scratch from kSplitKPrefillMinK on) of 64 (i - 1) < rows <= 64 i rows,
+// i = 2 ..: as its own launch shares them with the scratch that woq_hip_linear_auto_split_k_workspace_bytes asks for (0: one chain).
 static int chain_steps(int64_t K, int64_t N, int wbits, int row_tiles) {
   const int ksteps = (int)(K / kTileK4);
   const TilePlan p = plan_tiles(64 * row_tiles, N, ksteps, step_times(wbits, 0, 0), K >= kSplitKPrefillMinK ? kSplitScratchMax : 0);
@@ -172,11 +172,13 @@ int64_t gemm_w4_scratch_bytes(int64_t M, int64_t N, int64_t ksteps, int wbits, i
   return p.splits > 1 ? std::min(most, split_bytes(M, (pair ? 2 * N : N) + 2 * kTileN - 1, p.shape, p.splits)) : 0;
 }
 
-// Gate and up of a gated MLP as one launch, from kPairMinK input channels and kPairMinN columns of each on: it has twice the workgroups
-// where one of them leaves the chip idle, and the gate's rows stay in registers.  MLP of three linears, us, before / now (with K shared
-// below 4096 as well): M = 196, 3072 -> 3200 82.9 / 45.5, M = 363, 1536 -> 3456 68.4 / 39.7, M = 121, 1408 -> 5504 59.3 / 36.6, M = 180,
-// 2304 -> 12928 103.7 / 68.3; blocks M = 396, 3840 -> 6528 210 / 172, M = 101, 7168 -> 13056 200 / 164.  (Smaller layers keep two
-// launches, whose bits they have.)
+// Gate and up of a gated MLP as one launch: it has twice the workgroups where one of them leaves the chip idle, and the gate's rows stay
+// in registers, where two launches store them, read them and pass the post-op's epilogue twice (which costs a launch of its own 6 us,
+// M = 1024, 4096 -> 14336: 105 us without, 166 with the silu, 221 with the product).  Two launches / the pair, us, g128: 1024 -> 512, M = 65
+// 29.8 / 10.1, 4096 31.8 / 16.1; 2048 -> 5504, M = 128 37.5 / 15.6, 512 68 / 32, 4096 265 / 205; 4096 -> 14336, M = 128 69 / 45, 512 138 / 114,
+// 2048 774 / 450, 4096 1000 / 854; 8192 -> 28672, M = 128 167 / 113, 4096 3370 / 3109.  Nowhere slower by more than 3 % up to 4096 rows
+// (where the estimate keeps two launches the two are the same).  The lower bounds are not of speed -- 256 -> 512, M = 256 would be
+// 22.6 / 6.8 --: smaller layers have the bits of the two launches.
 constexpr int64_t kPairMinK = 1024, kPairMinN = 512;
 bool gemm_w4_pair_applies(const FpArgs& f, int wbits, int regime) {
   if (wbits != 4 || regime != kRegimeBF16 || f.nf4 || !f.szb || !f.szb_b || f.M <= 64 || f.K < kPairMinK || f.N < kPairMinN) return false;

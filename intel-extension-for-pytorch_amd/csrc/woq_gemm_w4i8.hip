@@ -22,7 +22,6 @@
 #include <type_traits>
 
 #include "woq_common.h"
-#include "woq_gemm_w4.h"
 #include "woq_int8_common.h"
 #include "woq_internal.h"
 
@@ -532,11 +531,13 @@ __global__ __launch_bounds__(256, (GSUB > 1 ? 2 : 3)) void woq_gemm_w4i8_kernel(
   }
 
   // ---- store: D[m][n], lane (n = r, c) holds rows m = 16 mt + 4 c + e ----
-  // 16-bit outputs go through the wave's stage in LDS, four columns a lane (rows of whole 8-byte pieces in one access): an element at a time the 32 stores of a lane,
-  // two bytes each, and the post-op's operands, each waited for, took 7 us of any launch (M = 2048, 4096 -> 14336 217 -> 204 us in the kernel trace, M = 180, 7040 -> 5244 31 -> 25).
+  // 16-bit outputs go through the wave's stage in LDS, four columns a lane (rows of whole 8-byte pieces in one access): an element at
+  // a time the 32 stores of a lane, two bytes each, and the post-op's operands, each waited for, took 7 us of any launch (M = 2048,
+  // 4096 -> 14336 217 -> 204 us in the kernel trace, M = 180, 7040 -> 5244 31 -> 25).
   const Epilogue& ep = a.ep;
   const bool out_f16 = ep.out_dtype == WOQ_HIP_ACT_FP16;
-  const bool staged = ep.fusion == WOQ_HIP_FUSE_NONE ? out_f16 || ep.out_dtype == WOQ_HIP_ACT_BF16 : ep.out_dtype == ep.act_dtype && ep.act_dtype != WOQ_HIP_ACT_FP32;
+  const bool staged = ep.fusion == WOQ_HIP_FUSE_NONE ? out_f16 || ep.out_dtype == WOQ_HIP_ACT_BF16
+                                                     : ep.out_dtype == ep.act_dtype && ep.act_dtype != WOQ_HIP_ACT_FP32;
   const bool whole = a.N % 4 == 0 && (((uintptr_t)ep.out | (uintptr_t)ep.other0 | (uintptr_t)ep.other1) & 7) == 0 && ((uintptr_t)ep.bias & 15) == 0;
   if (staged) {
     constexpr int kStride = W8_NTW * kTileN + 4;

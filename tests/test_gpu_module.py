@@ -497,6 +497,19 @@ def _woq_module(ipex, K, N, weight_dtype="INT4", group_size=128, lowp="BF16", bi
     return q.convert(q.prepare(model, qmap, inplace=True), inplace=True)[0]
 
 
+def _int4_context(K, N, G, seed, sym=False, device="cuda"):
+    """A context of random INT4 codes, scales around 0.002 and a bias (no float weight to quantize: wide layers are made at once)."""
+    from ipex_amd import _lib
+
+    g = torch.Generator(device=device).manual_seed(seed)
+    groups = K // G if G > 0 else 1
+    codes = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8, device=device)
+    scales = torch.rand(N, groups, generator=g, device=device) * 0.002 + 0.001
+    zeros = None if sym else torch.randint(4, 12, (N, groups), generator=g, device=device).float()
+    bias = torch.randn(N, generator=g, device=device)
+    return torch.ops.ipex_prepack.weight_only_qlinear_prepack(codes, _lib.DTYPE_INT4, [N, K], scales, zeros, bias, None, None, G, _lib.LOWP_BF16, -1, False)
+
+
 @pytest.mark.parametrize("M", [3, 40, 150])
 def test_llm_linear_fusion_modules_match_unfused_composition(cuda, M):
     """Each fusion module against the same WOQ linear followed by the torch elementwise op
@@ -1564,11 +1577,10 @@ def test_deepseek_moe_of_two_to_four_rows_an_expert_with_long_k(cuda, monkeypatc
     below): bit for bit the experts' own launches."""
     from ipex_amd import _lib
 
-    ipex = _ipex()
+    _ipex()
     E, T, topk = 24, 24, 3
-    kinds = 3 if H * I < 2**24 else 1  # different experts
-    mk = lambda k, n, s: _woq_module(ipex, k, n, "INT4", 128, "BF16", bias=True, seed=s)._op_context
-    ctxs = [[mk(H, I, 600 + e % kinds) for e in range(E)], [mk(H, I, 610 + e % kinds) for e in range(E)], [mk(I, H, 620 + e % kinds) for e in range(E)]]
+    mk = lambda k, n, s: [_int4_context(k, n, 128, s + e) for e in range(3)]
+    ctxs = [[kinds[e % 3] for e in range(E)] for kinds in (mk(H, I, 600), mk(H, I, 610), mk(I, H, 620))]
     g = torch.Generator().manual_seed(H)
     hidden = torch.randn(T, H, generator=g).bfloat16().to(cuda)
     ids = torch.stack([(t * 3 + torch.arange(3)) % (E - 4) for t in range(T)]).to(cuda)  # three or four rows each
@@ -1640,14 +1652,7 @@ def test_gate_and_up_of_prompts_in_one_launch(cuda, M, K, N, G, kind, sym):
 
     ipex = _ipex()
     if sym:
-        from ipex_amd import _lib
-
-        g = torch.Generator().manual_seed(K + N)
-        groups = K // G if G > 0 else 1
-        mk = lambda: torch.ops.ipex_prepack.weight_only_qlinear_prepack(
-            torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8).to(cuda), _lib.DTYPE_INT4, [N, K],
-            (torch.rand(N, groups, generator=g) * 0.002 + 0.001).to(cuda), None, torch.randn(N, generator=g).to(cuda), None, None, G, _lib.LOWP_BF16, -1, False)
-        contexts = mk(), mk()
+        contexts = [_int4_context(K, N, G, seed, sym=True) for seed in (44, 45)]
     else:
         mods = [_woq_module(ipex, K, N, "INT4", G, "BF16", bias=True, seed=s) for s in (44, 45)]
         contexts = [m._op_context for m in mods]
