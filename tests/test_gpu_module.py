@@ -1642,6 +1642,7 @@ def _pair_scratch(M, K, N, G):
     (65, 1024, 512, 128, "one"), (128, 1152, 528, 32, "one"), (200, 2048, 3000, 128, "one"), (64 * 5, 1024, 8208, -1, "one"), (2048, 1024, 528, 128, "one"),
     (129, 4096, 1040, 64, "shared"), (200, 7168, 2064, 32, "shared"), (512, 7168, 2048, 128, "shared"),  # 64 x 128 tiles in four, three and two
     (1000, 7168, 2048, 128, "shared"),  # 128 x 256 in two
+    (65, 1024, 1001, -1, "one"), (129, 4096, 1037, 64, "shared"), (333, 2048, 5503, 128, "one"),  # rows of no whole 8-byte pieces
     (65, 896, 512, 128, "two"), (65, 1024, 496, 128, "two"), (512, 4096, 11008, 128, "two"),
 ])
 def test_gate_and_up_of_prompts_in_one_launch(cuda, M, K, N, G, kind, sym):
